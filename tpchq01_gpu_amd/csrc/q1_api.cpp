@@ -186,17 +186,15 @@ static const void*& col(q1_columns& c, int i) {
 }
 static const void* colc(const q1_columns& c, int i) { return col(const_cast<q1_columns&>(c), i); }
 
+// Sets t->fast: whether the table's values lie inside the TPC-H domain.  The columns of a
+// pushdown table are those of a compressed one.
 static q1_status measure_domain(q1_ctx* ctx, q1_table* t) {
-  const int64_t init[8] = {INT64_MAX, INT64_MIN, INT64_MAX, INT64_MIN,
-                           INT64_MAX, INT64_MIN, INT64_MAX, INT64_MIN};
-  int64_t out[8];
-  Q1_HIP(ctx, hipMemcpyAsync(ctx->d_stats, init, sizeof(init), hipMemcpyHostToDevice, ctx->stream));
-  q1_status s = launch_domain(t->layout, t->dev, t->rows, ctx->d_stats, ctx->stream);
-  if (s != Q1_OK) return fail(ctx, s, "domain statistics kernel launch failed");
-  Q1_HIP(ctx, hipMemcpyAsync(out, ctx->d_stats, sizeof(out), hipMemcpyDeviceToHost, ctx->stream));
+  const q1_layout l = t->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? Q1_LAYOUT_COMPRESSED : t->layout;
+  *ctx->h_outside = 0;
+  q1_status s = launch_domain_check(l, t->dev, t->rows, ctx->d_outside, ctx->stream);
+  if (s != Q1_OK) return fail(ctx, s, "domain check kernel launch failed");
   Q1_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  t->domain = Domain{out[0], out[1], out[2], out[3], out[4], out[5], out[6], out[7]};
-  t->fast = t->rows == 0 || domain_is_tpch(t->layout, t->domain);
+  t->fast = *ctx->h_outside == 0;
   return Q1_OK;
 }
 
@@ -335,7 +333,8 @@ q1_status q1_init(int device, q1_ctx** out) {
   ok = ok && hipEventCreate(&ctx->ev_h2d_begin) == hipSuccess && hipEventCreate(&ctx->ev_h2d_end) == hipSuccess;
   ok = ok && hipMalloc(&ctx->d_aggr, sizeof(q1_device_aggregates)) == hipSuccess;
   ok = ok && hipHostMalloc(&ctx->h_aggr, sizeof(q1_device_aggregates), hipHostMallocDefault) == hipSuccess;
-  ok = ok && hipMalloc(&ctx->d_stats, 8 * sizeof(int64_t)) == hipSuccess;
+  ok = ok && hipHostMalloc(&ctx->h_outside, sizeof(uint32_t), hipHostMallocMapped) == hipSuccess &&
+       hipHostGetDevicePointer((void**)&ctx->d_outside, ctx->h_outside, 0) == hipSuccess;
   ok = ok && hipMalloc(&ctx->spread.tables, kSpreadTables * sizeof(q1_device_aggregates)) == hipSuccess;
   ok = ok && hipMemset(ctx->spread.tables, 0, kSpreadTables * sizeof(q1_device_aggregates)) == hipSuccess;
   // the scratch of q1_enqueue_noalloc on this device (once per device and process)
@@ -369,7 +368,6 @@ void q1_shutdown(q1_ctx* ctx) {
   if (ctx->batch) batch_destroy(ctx->batch);
   stream_state_release(ctx);
   if (ctx->workspace) (void)hipFree(ctx->workspace);
-  if (ctx->d_stats) (void)hipFree(ctx->d_stats);
   if (ctx->spread.tables) (void)hipFree(ctx->spread.tables);
   for (auto& kv : ctx->stream_spreads) {
     // the caller's stream may still run the last launch that used them
@@ -379,6 +377,7 @@ void q1_shutdown(q1_ctx* ctx) {
   }
   ctx->stream_spreads.clear();
   if (ctx->h_aggr) (void)hipHostFree(ctx->h_aggr);
+  if (ctx->h_outside) (void)hipHostFree(ctx->h_outside);
   if (ctx->d_aggr) (void)hipFree(ctx->d_aggr);
   for (hipEvent_t e : {ctx->ev_begin, ctx->ev_end, ctx->ev_h2d_begin, ctx->ev_h2d_end})
     if (e) (void)hipEventDestroy(e);
@@ -477,16 +476,7 @@ q1_status q1_table_upload(q1_ctx* ctx, q1_layout layout, const q1_columns* host,
   ctx->last.h2d_ms = ms;
   ctx->last.wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
   ctx->last.bytes_read = t->device_bytes;
-  if (layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN) {
-    // The domain of a pushdown table is that of its compressed columns.
-    q1_table tmp = *t;
-    tmp.layout = Q1_LAYOUT_COMPRESSED;
-    s = measure_domain(ctx, &tmp);
-    t->domain = tmp.domain;
-    t->fast = tmp.fast;
-  } else {
-    s = measure_domain(ctx, t);
-  }
+  s = measure_domain(ctx, t);
   if (s != Q1_OK) {
     release_table(t);
     return s;
@@ -517,15 +507,11 @@ q1_status q1_table_wrap(q1_ctx* ctx, q1_layout layout, const q1_columns* device,
   t->dev = *device;
   for (int i = 0; i < 8; i++)
     if (!b[i]) col(t->dev, i) = nullptr;
-  q1_table tmp = *t;
-  if (layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN) tmp.layout = Q1_LAYOUT_COMPRESSED;
-  const q1_status s = measure_domain(ctx, &tmp);
+  const q1_status s = measure_domain(ctx, t);
   if (s != Q1_OK) {
     delete t;
     return s;
   }
-  t->domain = tmp.domain;
-  t->fast = tmp.fast;
   ctx->tables.insert(t);
   *out = t;
   return Q1_OK;
@@ -536,13 +522,7 @@ q1_status q1_table_refresh_domain(q1_ctx* ctx, q1_table* t) {
   if (!ctx || !t || t->ctx != ctx) return fail(ctx, Q1_EINVAL, "bad argument");
   GUARD_BEGIN
   std::lock_guard<std::mutex> g(ctx->lock);
-  q1_table tmp = *t;
-  if (t->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN) tmp.layout = Q1_LAYOUT_COMPRESSED;
-  const q1_status s = measure_domain(ctx, &tmp);
-  if (s != Q1_OK) return s;
-  t->domain = tmp.domain;
-  t->fast = tmp.fast;
-  return Q1_OK;
+  return measure_domain(ctx, t);
   GUARD_END(ctx)
 }
 
@@ -616,7 +596,6 @@ q1_status q1_build_filter(q1_ctx* ctx, const q1_table* compressed, int32_t cutof
   t->rows = compressed->rows;
   t->dev = compressed->dev;
   t->dev.ship_date = nullptr;
-  t->domain = compressed->domain;
   t->fast = compressed->fast;
   t->filter_cutoff = cutoff_day;
   ctx->tables.insert(t);

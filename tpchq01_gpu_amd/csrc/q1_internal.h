@@ -18,7 +18,6 @@ struct q1_table {
   uint64_t rows = 0;
   q1_columns dev{};
   void* owned[8] = {};           // allocations this table frees
-  q1::Domain domain{};
   bool fast = false;             // inside the TPC-H value domain
   uint64_t device_bytes = 0;
   int32_t filter_cutoff = 0;     // pushdown tables: the cutoff their bitmap encodes
@@ -57,7 +56,8 @@ struct q1_ctx {
   hipEvent_t ev_begin = nullptr, ev_end = nullptr, ev_h2d_begin = nullptr, ev_h2d_end = nullptr;
   q1_device_aggregates* d_aggr = nullptr;  // one table for q1_run
   q1_device_aggregates* h_aggr = nullptr;  // pinned host copy
-  int64_t* d_stats = nullptr;              // 8 words for domain statistics
+  uint32_t* h_outside = nullptr;           // pinned word the domain check writes
+  uint32_t* d_outside = nullptr;           // ... as the device addresses it
   void* workspace = nullptr;
   uint64_t workspace_bytes = 0;
   q1_timing last{};

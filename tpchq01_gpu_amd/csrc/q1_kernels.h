@@ -8,8 +8,8 @@
 
 namespace q1 {
 
-// Value domain of a table, measured on the device when the table is created.  Inside the
-// TPC-H domain the narrow 32-bit kernels are exact; outside it the 64-bit kernels run.
+// Value ranges of host columns.  Inside the TPC-H domain the narrow 32-bit kernels are exact;
+// outside it the 64-bit kernels run.  Device tables are checked by launch_domain_check.
 struct Domain {
   int64_t min_disc, max_disc, min_tax, max_tax, min_qty, max_qty, min_price, max_price;
 };
@@ -76,9 +76,10 @@ q1_status launch_zero(q1_device_aggregates* table, uint32_t count, void* stream)
 q1_status launch_generate(q1_layout layout, uint64_t seed, uint64_t rows, const q1_columns& cols,
                           void* stream);
 
-// Device-side domain statistics of a table into `out_dev` (8 int64 slots: min/max pairs).
-q1_status launch_domain(q1_layout layout, const q1_columns& cols, uint64_t rows, int64_t* out_dev,
-                        void* stream);
+// Device-side domain check of a table's columns: *outside (device-visible) is set to 1 if any
+// value lies outside the TPC-H domain, and not written otherwise.
+q1_status launch_domain_check(q1_layout layout, const q1_columns& cols, uint64_t rows, uint32_t* outside,
+                              void* stream);
 
 // Device-side pushdown producer: filter bitmap of a compressed ship_date column.
 q1_status launch_build_filter(const uint16_t* ship, uint64_t rows, int32_t cutoff_day,

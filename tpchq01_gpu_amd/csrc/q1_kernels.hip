@@ -130,48 +130,105 @@ __global__ void generate_rows(uint64_t seed, uint64_t rows, q1_columns c) {
   }
 }
 
-// min/max of discount, tax, quantity, price: out[0..7] = {min,max} x {disc,tax,qty,price}.
+// The value-domain check: *outside becomes 1 if any discount, tax, quantity or price lies
+// outside the TPC-H domain (domain_is_tpch's limits), and is left alone otherwise.
+// HBM bounds it: 7 (compressed), 14 or 32 bytes per row are read once and nothing is written
+// for a table inside the domain.  Each column is read as 16-byte vectors with no regard to
+// rows: a limit of the form 2^k - 1 is a test of bits, so a lane ORs what it reads of such a
+// column and tests the OR; quantities in hundredths (at most 6300) keep a maximum.  A block
+// takes kDomainRows rows: its 14 to 16 non-temporal loads per lane, each a contiguous
+// stretch of the block's share of a column, are all issued before any is used.
+// Measured with its launch and wait: 60M compressed rows 72 us, 600M 610 us (6.9 TB/s), 600M
+// uncompressed 1.19 ms (7.0), 600M reference 2.66 ms (7.2).  Grid-strided columns one after
+// another, four vectors in flight per lane, took 83 us, 709 us, 1.37 ms and 3.04 ms; the
+// per-row minimum and maximum of every column, merged with eight 64-bit atomics per
+// wavefront into one line, took 1.55 ms at 60M compressed rows.
 template <int L>
-__global__ void domain_stats(q1_columns c, uint64_t rows, int64_t* out) {
-  int64_t mn[4] = {INT64_MAX, INT64_MAX, INT64_MAX, INT64_MAX};
-  int64_t mx[4] = {INT64_MIN, INT64_MIN, INT64_MIN, INT64_MIN};
-  for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < rows;
-       r += (uint64_t)gridDim.x * blockDim.x) {
-    int64_t v[4];
-    if (L == Q1_LAYOUT_REFERENCE) {
-      v[0] = ((const int64_t*)c.discount)[r];
-      v[1] = ((const int64_t*)c.tax)[r];
-      v[2] = ((const int64_t*)c.quantity)[r];
-      v[3] = ((const int64_t*)c.extended_price)[r];
-    } else if (L == Q1_LAYOUT_UNCOMPRESSED) {
-      v[0] = ((const int8_t*)c.discount)[r];
-      v[1] = ((const int8_t*)c.tax)[r];
-      v[2] = ((const int32_t*)c.quantity)[r];
-      v[3] = ((const int64_t*)c.extended_price)[r];
+constexpr int kDomainRows = L == Q1_LAYOUT_REFERENCE ? 2048 : L == Q1_LAYOUT_UNCOMPRESSED ? 4096 : 8192;
+
+// A lane's vectors of one block's share of a column of T values, at most LIMIT each.
+template <typename T, uint32_t LIMIT, int ROWS>
+struct DomainColumn {
+  static constexpr bool kBits = (LIMIT & (LIMIT + 1)) == 0;
+  static constexpr int kPer = 16 / sizeof(T);              // values per vector
+  static constexpr int kVectors = ROWS / kPer / 256;       // vectors per lane
+  static_assert(kVectors >= 1 && (kBits || sizeof(T) >= 4), "whole vectors; byte columns have limits 2^k - 1");
+  uint4 v[kVectors];
+
+  // WHOLE: the block's rows all lie in the column; otherwise vectors past its last whole
+  // one are taken as zero.
+  template <bool WHOLE>
+  __device__ __forceinline__ void load(const void* col, uint64_t block, uint64_t rows) {
+    const uint64_t first = block * (ROWS / kPer) + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kVectors; k++) {
+      const uint64_t i = first + k * 256;
+      v[k] = WHOLE || i < rows / kPer ? nt_load(reinterpret_cast<const uint4*>(col) + i) : make_uint4(0, 0, 0, 0);
+    }
+  }
+  __device__ __forceinline__ bool outside() const {
+    uint4 a = v[0];
+#pragma unroll
+    for (int k = 1; k < kVectors; k++) {
+      if (kBits) {
+        a.x |= v[k].x; a.y |= v[k].y; a.z |= v[k].z; a.w |= v[k].w;
+      } else {
+        a.x = max(a.x, v[k].x); a.y = max(a.y, v[k].y); a.z = max(a.z, v[k].z); a.w = max(a.w, v[k].w);
+      }
+    }
+    if constexpr (kBits) {
+      constexpr uint32_t low = sizeof(T) == 1 ? (~LIMIT & 0xFFu) * 0x01010101u : ~LIMIT;
+      constexpr uint32_t high = sizeof(T) == 8 ? 0xFFFFFFFFu : low;
+      return ((a.x | a.z) & low) != 0 || ((a.y | a.w) & high) != 0;
     } else {
-      v[0] = ((const uint8_t*)c.discount)[r];
-      v[1] = ((const uint8_t*)c.tax)[r];
-      v[2] = ((const uint8_t*)c.quantity)[r];
-      v[3] = ((const uint32_t*)c.extended_price)[r];
-    }
-    for (int i = 0; i < 4; i++) {
-      mn[i] = v[i] < mn[i] ? v[i] : mn[i];
-      mx[i] = v[i] > mx[i] ? v[i] : mx[i];
+      return max(a.x, a.z) > LIMIT || max(a.y, a.w) > (sizeof(T) == 8 ? 0u : LIMIT);
     }
   }
-  for (int i = 0; i < 4; i++) {
-    for (int m = 32; m >= 1; m >>= 1) {
-      const int64_t omn = __shfl_xor(mn[i], m, 64), omx = __shfl_xor(mx[i], m, 64);
-      mn[i] = omn < mn[i] ? omn : mn[i];
-      mx[i] = omx > mx[i] ? omx : mx[i];
-    }
+  // One of the up to 15 values behind the column's last whole vector.
+  __device__ __forceinline__ static bool tail_outside(const void* col, uint64_t rows) {
+    const uint64_t r = rows / kPer * kPer + threadIdx.x;
+    if (r >= rows) return false;
+    const int64_t x = (int64_t)reinterpret_cast<const T*>(col)[r];
+    return x < 0 || x > (int64_t)LIMIT;
   }
-  if ((threadIdx.x & 63) == 0) {
-    for (int i = 0; i < 4; i++) {
-      atomicMin((long long*)&out[2 * i], (long long)mn[i]);
-      atomicMax((long long*)&out[2 * i + 1], (long long)mx[i]);
-    }
+};
+
+template <typename Narrow, typename Qty, uint32_t QTY_LIMIT, typename Price, int ROWS>
+__device__ __forceinline__ bool block_outside(const q1_columns& c, uint64_t rows) {
+  DomainColumn<Narrow, 15, ROWS> d, x;
+  DomainColumn<Qty, QTY_LIMIT, ROWS> q;
+  DomainColumn<Price, (1u << 24) - 1, ROWS> p;
+  const uint64_t b = blockIdx.x;
+  bool tail = false;
+  if ((b + 1) * ROWS <= rows) {
+    d.template load<true>(c.discount, b, rows);
+    x.template load<true>(c.tax, b, rows);
+    q.template load<true>(c.quantity, b, rows);
+    p.template load<true>(c.extended_price, b, rows);
+  } else {
+    d.template load<false>(c.discount, b, rows);
+    x.template load<false>(c.tax, b, rows);
+    q.template load<false>(c.quantity, b, rows);
+    p.template load<false>(c.extended_price, b, rows);
+    tail = d.tail_outside(c.discount, rows) | x.tail_outside(c.tax, rows) | q.tail_outside(c.quantity, rows) |
+           p.tail_outside(c.extended_price, rows);
   }
+  return tail | d.outside() | x.outside() | q.outside() | p.outside();
+}
+
+template <int L>
+__global__ void __launch_bounds__(256) domain_check(q1_columns c, uint64_t rows, uint32_t* outside) {
+  bool bad;
+  if constexpr (L == Q1_LAYOUT_REFERENCE)
+    bad = block_outside<int64_t, int64_t, 6300, int64_t, kDomainRows<L>>(c, rows);
+  else if constexpr (L == Q1_LAYOUT_UNCOMPRESSED)
+    bad = block_outside<int8_t, int32_t, 6300, int64_t, kDomainRows<L>>(c, rows);
+  else
+    bad = block_outside<uint8_t, uint8_t, 63, uint32_t, kDomainRows<L>>(c, rows);
+  // The word is in host memory: a wavefront writes it once, and only if nobody has yet.
+  if (ballot(bad) && (threadIdx.x & 63) == 0 &&
+      __hip_atomic_load(outside, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0)
+    __hip_atomic_store(outside, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The pushdown producer (src/main.cu:362-389 semantics, runtime cutoff).  A lane turns the
@@ -362,17 +419,20 @@ q1_status launch_generate(q1_layout layout, uint64_t seed, uint64_t rows, const 
   return hip_status(hipGetLastError());
 }
 
-q1_status launch_domain(q1_layout layout, const q1_columns& cols, uint64_t rows, int64_t* out_dev,
-                        void* stream) {
+q1_status launch_domain_check(q1_layout layout, const q1_columns& cols, uint64_t rows, uint32_t* outside,
+                              void* stream) {
   if (rows == 0) return Q1_OK;
-  uint64_t blocks = (rows + 255) / 256;
-  if (blocks > 4096) blocks = 4096;
+  const uint64_t per = layout == Q1_LAYOUT_REFERENCE      ? kDomainRows<Q1_LAYOUT_REFERENCE>
+                       : layout == Q1_LAYOUT_UNCOMPRESSED ? kDomainRows<Q1_LAYOUT_UNCOMPRESSED>
+                                                          : kDomainRows<Q1_LAYOUT_COMPRESSED>;
+  const uint64_t blocks = (rows + per - 1) / per;
+  if (blocks * 256 > 0xFFFFFFFFull) return Q1_EINVAL;  // HIP counts work-items in 32 bits
   const dim3 grid((uint32_t)blocks), block(256);
   const hipStream_t s = (hipStream_t)stream;
   switch (layout) {
-    case Q1_LAYOUT_REFERENCE: hipLaunchKernelGGL(domain_stats<Q1_LAYOUT_REFERENCE>, grid, block, 0, s, cols, rows, out_dev); break;
-    case Q1_LAYOUT_UNCOMPRESSED: hipLaunchKernelGGL(domain_stats<Q1_LAYOUT_UNCOMPRESSED>, grid, block, 0, s, cols, rows, out_dev); break;
-    default: hipLaunchKernelGGL(domain_stats<Q1_LAYOUT_COMPRESSED>, grid, block, 0, s, cols, rows, out_dev); break;
+    case Q1_LAYOUT_REFERENCE: hipLaunchKernelGGL(domain_check<Q1_LAYOUT_REFERENCE>, grid, block, 0, s, cols, rows, outside); break;
+    case Q1_LAYOUT_UNCOMPRESSED: hipLaunchKernelGGL(domain_check<Q1_LAYOUT_UNCOMPRESSED>, grid, block, 0, s, cols, rows, outside); break;
+    default: hipLaunchKernelGGL(domain_check<Q1_LAYOUT_COMPRESSED>, grid, block, 0, s, cols, rows, outside); break;
   }
   return hip_status(hipGetLastError());
 }
