@@ -132,7 +132,9 @@ typedef struct {
 #define Q1_LAUNCH_ASSUME_TPCH_DOMAIN 1u
 
 typedef struct {
-  double kernel_ms;      /* device time of the last run (HIP events around the kernels) */
+  double kernel_ms;      /* device time of the last run: q1_run and q1_run_split by the device's
+                            clock, from the first block's start to the folded result; the
+                            others by HIP events around the kernels */
   double h2d_ms;         /* device time of host-to-device copies of the last call */
   double wall_ms;        /* host wall-clock of the last call */
   uint64_t bytes_read;   /* algorithmic column bytes the last run read */
@@ -212,7 +214,7 @@ q1_status q1_last_timing(q1_ctx* ctx, q1_timing* out);
 /* The drop-in kernel launch: accumulate rows [row_begin, row_begin+num_tuples) of the
  * device columns into the caller-zeroed device table `aggregates` on `hip_stream`
  * (NULL = the context stream).  Launches on disjoint ranges compose by addition.
- * Large grids merge through spread tables: the context's on the context stream, a set
+ * Large grids merge through partial tables: the context's on the context stream, a set
  * made on a caller stream's first large launch (kept until q1_shutdown, at most 16
  * streams; a stream under graph capture or beyond those merges directly). */
 q1_status q1_enqueue(q1_ctx* ctx, q1_placement placement, q1_layout layout,
@@ -222,8 +224,8 @@ q1_status q1_enqueue(q1_ctx* ctx, q1_placement placement, q1_layout layout,
 /* No counterpart in the reference: q1_enqueue that allocates nothing (no hipMalloc, hipFree
  * or allocating library call), for callers that cannot allocate device memory -- code
  * under HIP graph capture, serving loops that forbid allocation.  Same arguments, results
- * and errors as q1_enqueue.  Its scratch (the spread-merge tables of grids of 176 blocks or
- * more, and the global placement's per-block tables) is a static array of 8 MiB + 24 KiB
+ * and errors as q1_enqueue.  Its scratch (the partial tables of grids of 144 blocks or
+ * more, and the global placement's per-block tables) is a static array of 8 MiB + 33 KiB
  * per GPU, set up by q1_init and held until the process ends; a launch needing more (the
  * global placement with more than 34952 blocks) gets Q1_EINVAL.  Every call on one GPU
  * shares that array: calls that overlap on one GPU (other streams or threads) race, so the

@@ -101,11 +101,11 @@ q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
   return Q1_OK;
 }
 
-// The spread tables of a caller's stream for a large fast launch, made on the stream's
-// first such launch; nullptr (merge directly) while the stream is being captured into a
+// The merge set of a caller's stream for a large launch, made on the stream's first such
+// launch; nullptr (merge directly) while the stream is being captured into a
 // graph, where nothing may be allocated or waited for outside the capture, once
-// kMaxStreamSpreads streams have tables, or if making them fails.  A stream that has
-// tables first waits for the event of their last use.
+// kMaxStreamSpreads streams have one, or if making it fails.  A stream that has
+// one first waits for the event of its last use.
 static StreamSpread* stream_spread(q1_ctx* ctx, void* stream) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
@@ -121,9 +121,9 @@ static StreamSpread* stream_spread(q1_ctx* ctx, void* stream) {
   }
   if (ctx->stream_spreads.size() >= kMaxStreamSpreads) return nullptr;
   StreamSpread ss;
-  if (hipMalloc(&ss.spread.tables, kSpreadTables * sizeof(q1_device_aggregates)) != hipSuccess) return nullptr;
+  if (hipMalloc(&ss.set, sizeof(MergeSet)) != hipSuccess) return nullptr;
   if (hipEventCreateWithFlags(&ss.done, hipEventDisableTiming) != hipSuccess) {
-    (void)hipFree(ss.spread.tables);
+    (void)hipFree(ss.set);
     return nullptr;
   }
   return &ctx->stream_spreads.emplace(stream, ss).first->second;
@@ -131,32 +131,57 @@ static StreamSpread* stream_spread(q1_ctx* ctx, void* stream) {
 
 q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
                   const LaunchShape& shape, void* stream, bool table_outside) {
-  // Launches on one stream run one after another, so they can share one set of spread
-  // tables: the context's for the context stream, a set of the stream's own for a
-  // caller's stream (large fast launches only; the others merge directly).
-  Spread* sp = nullptr;
-  bool* dirty = nullptr;
+  // Launches on one stream run one after another, so they can share one merge set: the
+  // context's for the context stream, a set of the stream's own for a caller's stream
+  // (large launches only; the others merge directly).
+  MergeSet* set = nullptr;
   StreamSpread* other = nullptr;
   if (stream == (void*)ctx->stream) {
-    if (ctx->spread.tables) {
-      sp = &ctx->spread;
-      dirty = &ctx->spread_dirty;
-    }
-  } else if (fast && shape.blocks >= kSpreadMinBlocks) {
-    if ((other = stream_spread(ctx, stream))) {
-      sp = &other->spread;
-      dirty = &other->dirty;
+    set = ctx->set;
+  } else if (shape.blocks >= kSpreadMinBlocks && (other = stream_spread(ctx, stream))) {
+    set = other->set;
+    if (!other->zeroed) {
+      const q1_status z = launch_zero(set, stream);
+      if (z != Q1_OK) return z;
+      other->zeroed = true;
     }
   }
-  if (sp && *dirty) {
-    const q1_status z = launch_zero(sp->tables, kSpreadTables, stream);
-    if (z != Q1_OK) return z;
-    *dirty = false;
-  }
-  const q1_status s = launch_scan(placement, layout, fast, a, shape, ctx->workspace, stream, sp, table_outside);
-  if (s != Q1_OK && sp) *dirty = true;
+  const q1_status s = launch_scan(placement, layout, fast, a, shape, ctx->workspace, stream, set, table_outside);
   if (other && hipEventRecord(other->done, (hipStream_t)stream) != hipSuccess) other->usable = false;
   return s;
+}
+
+q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, ScanArgs a,
+                       const LaunchShape& shape, bool table_outside) {
+  a.host = ctx->d_result;
+  a.sequence = ++ctx->sequence;
+  if (shape.blocks == 0) {
+    std::memset(ctx->h_result, 0, sizeof(HostResult));
+    ctx->h_result->sequence = a.sequence;
+    return Q1_OK;
+  }
+  const q1_status s = scan_on(ctx, placement, layout, fast, a, shape, (void*)ctx->stream, table_outside);
+  return s == Q1_OK ? Q1_OK : fail(ctx, s, "scan kernel launch failed");
+}
+
+// The kernel's last store is the launch's number in pinned host memory: a short launch is
+// awaited by watching for it (an empty kernel launched and awaited so takes 6.2 us, 10.9
+// with the stream's wait), a longer one, after kWatchMicroseconds, by the stream's own wait,
+// which lets the processor go and then costs at most 5 % of the call.
+constexpr int kWatchMicroseconds = 100;
+q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms) {
+  const HostResult* r = ctx->h_result;
+  auto arrived = [&] { return __atomic_load_n(&r->sequence, __ATOMIC_ACQUIRE) == ctx->sequence; };
+  const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(kWatchMicroseconds);
+  while (!arrived() && std::chrono::steady_clock::now() < until)
+    for (int i = 0; i < 16 && !arrived(); i++) __builtin_ia32_pause();
+  if (!arrived()) {
+    Q1_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (!arrived()) return fail(ctx, Q1_EDEVICE, "the scan kernel ended without a result");
+  }
+  q1_aggregates_to_result(&r->sums, out);
+  *kernel_ms = ctx->clock_khz > 0 ? (double)(r->clock_end - r->clock_begin) / ctx->clock_khz : 0.0;
+  return Q1_OK;
 }
 
 // Column sizes in bytes, in q1_columns order.
@@ -335,8 +360,12 @@ q1_status q1_init(int device, q1_ctx** out) {
   ok = ok && hipHostMalloc(&ctx->h_aggr, sizeof(q1_device_aggregates), hipHostMallocDefault) == hipSuccess;
   ok = ok && hipHostMalloc(&ctx->h_outside, sizeof(uint32_t), hipHostMallocMapped) == hipSuccess &&
        hipHostGetDevicePointer((void**)&ctx->d_outside, ctx->h_outside, 0) == hipSuccess;
-  ok = ok && hipMalloc(&ctx->spread.tables, kSpreadTables * sizeof(q1_device_aggregates)) == hipSuccess;
-  ok = ok && hipMemset(ctx->spread.tables, 0, kSpreadTables * sizeof(q1_device_aggregates)) == hipSuccess;
+  ok = ok && hipHostMalloc(&ctx->h_result, sizeof(HostResult), hipHostMallocMapped) == hipSuccess &&
+       hipHostGetDevicePointer((void**)&ctx->d_result, ctx->h_result, 0) == hipSuccess;
+  if (ok) std::memset(ctx->h_result, 0, sizeof(HostResult));
+  ok = ok && hipDeviceGetAttribute(&ctx->clock_khz, hipDeviceAttributeWallClockRate, device) == hipSuccess;
+  ok = ok && hipMalloc(&ctx->set, sizeof(MergeSet)) == hipSuccess;
+  ok = ok && hipMemset(ctx->set, 0, sizeof(MergeSet)) == hipSuccess;
   // the scratch of q1_enqueue_noalloc on this device (once per device and process)
   ok = ok && noalloc_setup(device, ctx->stream) == Q1_OK;
   ok = ok && hipDeviceSynchronize() == hipSuccess;
@@ -368,16 +397,17 @@ void q1_shutdown(q1_ctx* ctx) {
   if (ctx->batch) batch_destroy(ctx->batch);
   stream_state_release(ctx);
   if (ctx->workspace) (void)hipFree(ctx->workspace);
-  if (ctx->spread.tables) (void)hipFree(ctx->spread.tables);
+  if (ctx->set) (void)hipFree(ctx->set);
   for (auto& kv : ctx->stream_spreads) {
     // the caller's stream may still run the last launch that used them
     (void)hipEventSynchronize(kv.second.done);
-    (void)hipFree(kv.second.spread.tables);
+    (void)hipFree(kv.second.set);
     (void)hipEventDestroy(kv.second.done);
   }
   ctx->stream_spreads.clear();
   if (ctx->h_aggr) (void)hipHostFree(ctx->h_aggr);
   if (ctx->h_outside) (void)hipHostFree(ctx->h_outside);
+  if (ctx->h_result) (void)hipHostFree(ctx->h_result);
   if (ctx->d_aggr) (void)hipFree(ctx->d_aggr);
   for (hipEvent_t e : {ctx->ev_begin, ctx->ev_end, ctx->ev_h2d_begin, ctx->ev_h2d_end})
     if (e) (void)hipEventDestroy(e);
@@ -687,25 +717,16 @@ static q1_status run_locked(q1_ctx* ctx, const q1_table* t, uint64_t row_begin, 
   if (s != Q1_OK) return fail(ctx, s, why);
   s = ensure_workspace(ctx, scan_workspace_bytes(p, shape));
   if (s != Q1_OK) return s;
-  ScanArgs a;
+  ScanArgs a{};
   a.cols = t->dev;
   a.row_begin = row_begin;
   a.row_end = row_begin + row_count;
   a.cutoff_day = t->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t->filter_cutoff : cutoff_day;
-  a.out = ctx->d_aggr;
   const auto w0 = std::chrono::steady_clock::now();
-  s = launch_zero(ctx->d_aggr, 1, ctx->stream);
-  if (s != Q1_OK) return fail(ctx, s, "zero kernel launch failed");
-  Q1_HIP(ctx, hipEventRecord(ctx->ev_begin, ctx->stream));
-  s = scan_on(ctx, p, t->layout, t->fast, a, shape, ctx->stream, !t->fast);
-  if (s != Q1_OK) return fail(ctx, s, "scan kernel launch failed");
-  Q1_HIP(ctx, hipEventRecord(ctx->ev_end, ctx->stream));
-  Q1_HIP(ctx, hipMemcpyAsync(ctx->h_aggr, ctx->d_aggr, sizeof(q1_device_aggregates), hipMemcpyDeviceToHost,
-                             ctx->stream));
-  Q1_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  float ms = 0;
-  (void)hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end);
-  q1_aggregates_to_result(ctx->h_aggr, out);
+  double ms = 0;
+  s = scan_to_host(ctx, p, t->layout, t->fast, a, shape, !t->fast);
+  if (s == Q1_OK) s = wait_result(ctx, out, &ms);
+  if (s != Q1_OK) return s;
   ctx->last = q1_timing{};
   ctx->last.kernel_ms = ms;
   ctx->last.wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
@@ -755,13 +776,13 @@ q1_status q1_enqueue_noalloc(q1_ctx* ctx, q1_placement placement, q1_layout layo
   const char* why = "";
   q1_status s = make_shape(p, layout, &l, row_begin, row_begin + num_tuples, &shape, &why);
   if (s != Q1_OK) return fail(ctx, s, why);
-  ScanArgs a;
+  ScanArgs a{};
   a.cols = *device;
   a.row_begin = row_begin;
   a.row_end = row_begin + num_tuples;
   a.cutoff_day = cutoff_day;
   a.out = aggregates;
-  // the device's static scratch array instead of the context's spread tables and workspace
+  // the device's static scratch array instead of the context's merge set and workspace
   s = noalloc_launch_scan(ctx->device, p, layout, (l.flags & Q1_LAUNCH_ASSUME_TPCH_DOMAIN) != 0, a, shape,
                           hip_stream ? hip_stream : (void*)ctx->stream, &why);
   return s == Q1_OK ? Q1_OK : fail(ctx, s, why);
@@ -797,7 +818,7 @@ q1_status q1_enqueue(q1_ctx* ctx, q1_placement placement, q1_layout layout, cons
     return fail(ctx, Q1_EINVAL, "the global placement enqueues on the context stream only");
   s = ensure_workspace(ctx, scan_workspace_bytes(p, shape));
   if (s != Q1_OK) return s;
-  ScanArgs a;
+  ScanArgs a{};
   a.cols = *device;
   a.row_begin = row_begin;
   a.row_end = row_begin + num_tuples;

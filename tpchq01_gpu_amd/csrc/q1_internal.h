@@ -31,17 +31,17 @@ constexpr int kStreamCount = 4;
 struct q1_batch_state;  // q1_batch.cpp
 namespace q1 {
 struct StreamState;     // q1_stream.cpp: the host-resident streaming pipeline
-// Spread tables of one caller stream (q1_enqueue on a stream other than the context's).
-// `done` is recorded after every launch that uses them and the next launch waits for it,
+// The merge set of one caller stream (q1_enqueue on a stream other than the context's).
+// `done` is recorded after every launch that uses it and the next launch waits for it,
 // so a stream created at the address of a destroyed one never overlaps the old stream's
 // last use; `usable` is cleared if that bookkeeping ever fails.
 struct StreamSpread {
-  Spread spread{};
+  MergeSet* set = nullptr;
   hipEvent_t done = nullptr;
-  bool dirty = true;   // zeroed by the first launch that uses them
+  bool zeroed = false;   // the first launch that uses it clears it
   bool usable = true;
 };
-// Caller streams that get spread tables; launches on further streams merge directly.
+// Caller streams that get a merge set; launches on further streams merge directly.
 constexpr size_t kMaxStreamSpreads = 16;
 // A launch shape tuned on ranges of `rows` rows ("launch_at" lines of the tuning file).
 struct SizedLaunch {
@@ -54,7 +54,11 @@ struct q1_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev_begin = nullptr, ev_end = nullptr, ev_h2d_begin = nullptr, ev_h2d_end = nullptr;
-  q1_device_aggregates* d_aggr = nullptr;  // one table for q1_run
+  q1::HostResult* h_result = nullptr;      // pinned: what q1_run's kernel leaves for the host
+  q1::HostResult* d_result = nullptr;      // ... as the device addresses it
+  uint64_t sequence = 0;                   // number of the last launch that wrote h_result
+  int32_t clock_khz = 0;                   // rate of the device clock in h_result
+  q1_device_aggregates* d_aggr = nullptr;  // the table q1_run_streaming's chunks add into
   q1_device_aggregates* h_aggr = nullptr;  // pinned host copy
   uint32_t* h_outside = nullptr;           // pinned word the domain check writes
   uint32_t* d_outside = nullptr;           // ... as the device addresses it
@@ -78,9 +82,8 @@ struct q1_ctx {
                           Q1_PLACE_IN_REGISTERS};
   q1_batch_state* batch = nullptr;
   q1::StreamState* streaming = nullptr;    // cached staging buffers and streams of q1_run_streaming
-  q1::Spread spread{};                     // spread-merge tables of the context stream
-  bool spread_dirty = false;               // a failed launch may have left partials in them
-  std::unordered_map<void*, q1::StreamSpread> stream_spreads;  // caller streams' spread tables
+  q1::MergeSet* set = nullptr;             // merge set of the context stream
+  std::unordered_map<void*, q1::StreamSpread> stream_spreads;  // caller streams' merge sets
   std::unordered_set<q1_table*> tables;    // live tables (released device memory at shutdown)
   std::mutex lock;                         // serialises calls that share the context stream
 };
@@ -97,10 +100,16 @@ void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, uint64_t rows
                     q1_launch* out, bool any_value_kernel = false);
 uint64_t algorithmic_bytes(q1_layout layout, uint64_t rows);
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes);
-// launch_scan with the context's spread tables when `stream` is the context stream.
+// launch_scan with the merge set of `stream` (the context's or a caller's).
 // table_outside: the rows come from a table known to hold values outside the domain.
 q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
                   const LaunchShape& shape, void* stream, bool table_outside = false);
+// The same on the context stream with the sums going to ctx->h_result, and the wait for
+// them: fills *out and returns the kernel's device time in *kernel_ms.  A launch with no
+// blocks leaves zeros.
+q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, ScanArgs a,
+                       const LaunchShape& shape, bool table_outside);
+q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms);
 void batch_destroy(q1_batch_state* b);
 // The batched kernel's plan, shared by q1_run_batch and the server: rows per lane (the
 // tuned value of the layout and placement, at most batch_max_lane_rows), the default

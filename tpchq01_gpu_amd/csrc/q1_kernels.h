@@ -29,48 +29,72 @@ struct LaunchShape {
   uint32_t blocks, threads, tiles_per_thread;
 };
 
+// Spread merge.  Thousands of blocks adding into one 48-word table serialise on those
+// words' atomics at the end of the grid; instead block b of a launch merges into
+// tables[b % kSpreadTables] of a merge set, and the last block to finish folds the tables
+// into the destination.  A set is all zero before a launch and after it (the fold clears
+// what it read), and must not be shared by launches that can overlap.
+constexpr uint32_t kSpreadTables = 64;      // power of two
+struct MergeSet {
+  q1_device_aggregates tables[kSpreadTables];
+  // Blocks that have merged: those of one table (the blocks b with the same b mod 64) count
+  // in finished[b % 64], each on a cache line of its own, and the last of them in
+  // tables_finished, so that no counter sees more than a 64th of a large grid.
+  struct alignas(128) Count {
+    uint32_t n;
+  } finished[kSpreadTables];
+  Count tables_finished;
+  uint64_t clock_begin;       // device clock at the start of block 0
+};
+
+// What a launch leaves in pinned host memory for a caller that waits for it.
+struct HostResult {
+  q1_device_aggregates sums;
+  uint64_t clock_begin, clock_end;  // device clock at the start of block 0 and at the fold
+  uint64_t sequence;                // the launch's number, written after everything else
+};
+
 // Kernel-level request: accumulate rows [row_begin, row_end) of `cols` into `out`.
 struct ScanArgs {
   q1_columns cols;          // device pointers
   uint64_t row_begin, row_end;
   int32_t cutoff_day;       // MonetDB day number (ignored for pushdown)
   q1_device_aggregates* out;
-  uint32_t out_mask;        // set by launch_scan: block b merges into out[b & out_mask]
-};
-
-// Spread merge.  Thousands of blocks adding into one 48-word table serialise on those
-// words' atomics at the end of the grid; instead block b of a large launch merges into
-// tables[b % kSpreadTables] and a one-block fold kernel adds the tables into the
-// destination and clears them.  The tables must be zero before the launch (the fold
-// leaves them zero) and must not be shared by launches that can overlap: one set per
-// stream that serialises its launches.
-constexpr uint32_t kSpreadTables = 64;      // power of two
-// Smaller grids merge directly.  Device-scope atomics on one address from all compute
-// units serialise: a grid's direct merge costs about 0.03 us per block against the fold's
-// fixed 4.5 us, so direct merging wins below about 165-190 blocks (measured on 5K-6M-row
-// launches: 49 blocks 11 us direct / 15 us spread, 489 blocks 28 / 15 us, 977 blocks 49 /
-// 16 us).
-constexpr uint32_t kSpreadMinBlocks = 176;
-struct Spread {
-  q1_device_aggregates* tables;  // kSpreadTables zeroed tables
+  // Set by launch_scan: block b merges into out[b & out_mask]; with a merge set, `out` are
+  // the set's tables and the last block folds them into *dest (added), or, when dest is
+  // null, into *host (stored, with the clocks and `sequence`; host memory as the device
+  // addresses it).
+  uint32_t out_mask;
+  MergeSet* set;
+  q1_device_aggregates* dest;
+  HostResult* host;
+  uint64_t sequence;
 };
 
 // Validate and complete a launch shape for `rows` rows (0 fields filled from defaults).
 q1_status make_shape(q1_placement placement, q1_layout layout, const q1_launch* launch,
                      uint64_t row_begin, uint64_t row_end, LaunchShape* shape, const char** why);
 
-// Enqueue the scan kernel.  `fast` selects the narrow (TPC-H domain) kernels.  With a
-// `spread` (may be null) a fast launch of at least kSpreadMinBlocks blocks merges through
-// the spread tables and is followed by the fold kernel on the same stream.
+// Smaller grids add straight into a device destination.  Device-scope atomics on one address
+// from all compute units serialise, about 0.03 us per block; counting the blocks and the
+// fold add a fixed 3 us.  Back-to-back q1_enqueue of 64 lanes x 64 rows blocks, direct /
+// through a set: 64 blocks 12.2 / 14.8 us, 128 blocks 14.5 / 15.1, 176 blocks 16.1 / 15.1,
+// 512 blocks 30.8 / 16.5, 4096 blocks 167 / 35.5.
+constexpr uint32_t kSpreadMinBlocks = 144;
+
+// Where a scan's sums go.  host: stored into a.host (needs `set`; every grid merges through
+// it).  Otherwise added into *a.out, through `set` when there is one and the grid has at
+// least kSpreadMinBlocks blocks.
 // fast: the rows lie inside the TPC-H domain.  Otherwise an any-value kernel runs;
 // table_outside picks the one for tables known to hold values outside the domain.
 q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
-                      const LaunchShape& shape, void* workspace, void* stream, const Spread* spread = nullptr,
+                      const LaunchShape& shape, void* workspace, void* stream, MergeSet* set = nullptr,
                       bool table_outside = false);
 uint64_t scan_workspace_bytes(q1_placement placement, const LaunchShape& shape);
 
-// Zero a device aggregate table (a fill kernel, safe inside graph capture).
+// Zero device aggregate tables or a merge set (a fill kernel, safe inside graph capture).
 q1_status launch_zero(q1_device_aggregates* table, uint32_t count, void* stream);
+q1_status launch_zero(MergeSet* set, void* stream);
 
 // Device-side generator: rows [0, rows) of `layout` into the device columns.
 q1_status launch_generate(q1_layout layout, uint64_t seed, uint64_t rows, const q1_columns& cols,

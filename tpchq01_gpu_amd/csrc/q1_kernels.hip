@@ -358,19 +358,22 @@ uint64_t scan_workspace_bytes(q1_placement placement, const LaunchShape& shape) 
 }
 
 q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const ScanArgs& args,
-                      const LaunchShape& shape, void* workspace, void* stream, const Spread* spread,
-                      bool table_outside) {
+                      const LaunchShape& shape, void* workspace, void* stream, MergeSet* set, bool table_outside) {
+  if (args.host && !set) return Q1_EINVAL;
   if (shape.blocks == 0) return Q1_OK;
   const hipStream_t s = (hipStream_t)stream;
   const uint32_t nwaves = shape.threads / 64;
   ScanArgs a = args;
   a.out_mask = 0;
+  a.set = nullptr;
+  a.dest = nullptr;
+  if (set && (a.host || shape.blocks >= kSpreadMinBlocks)) {
+    a.set = set;
+    a.dest = a.host ? nullptr : args.out;
+    a.out = set->tables;
+    a.out_mask = kSpreadTables - 1;
+  }
   if (fast) {
-    const bool spread_merge = spread && spread->tables && shape.blocks >= kSpreadMinBlocks;
-    if (spread_merge) {
-      a.out = spread->tables;
-      a.out_mask = kSpreadTables - 1;
-    }
     const uint64_t lane_rows = (uint64_t)shape.tiles_per_thread * tile_rows(layout);
     const bool shared = placement == Q1_PLACE_PER_THREAD_SHARED_MEM;
     // The packed slot holds quantities in whole units: the compressed layouts only.
@@ -384,11 +387,6 @@ q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const
     lds += nwaves * kNumGroups * NF * 8;
     hipLaunchKernelGGL(fast_kernel(layout, variant, shape.threads), dim3(shape.blocks), dim3(shape.threads), lds,
                        s, a, shape.tiles_per_thread, (uint64_t*)workspace);
-    if (spread_merge) {
-      const q1_status st = hip_status(hipGetLastError());
-      if (st != Q1_OK) return st;
-      hipLaunchKernelGGL(fold_spread, dim3(1), dim3(256), 0, s, spread->tables, args.out);
-    }
   } else {
     const uint32_t lds = shared_table_bytes(shape.threads) + nwaves * kNumGroups * 8 * 8;
     hipLaunchKernelGGL(general_kernel(layout, shape.threads, table_outside), dim3(shape.blocks), dim3(shape.threads),
@@ -397,13 +395,19 @@ q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const
   return hip_status(hipGetLastError());
 }
 
-q1_status launch_zero(q1_device_aggregates* table, uint32_t count, void* stream) {
-  const uint64_t n = (uint64_t)count * (sizeof(q1_device_aggregates) / 8);
+static q1_status zero(void* p, uint64_t bytes, void* stream) {
+  const uint64_t n = bytes / 8;
   if (n == 0) return Q1_OK;
   hipLaunchKernelGGL(zero_words, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                     (uint64_t*)table, n);
+                     (uint64_t*)p, n);
   return hip_status(hipGetLastError());
 }
+
+q1_status launch_zero(q1_device_aggregates* table, uint32_t count, void* stream) {
+  return zero(table, (uint64_t)count * sizeof(q1_device_aggregates), stream);
+}
+
+q1_status launch_zero(MergeSet* set, void* stream) { return zero(set, sizeof(MergeSet), stream); }
 
 q1_status launch_generate(q1_layout layout, uint64_t seed, uint64_t rows, const q1_columns& cols,
                           void* stream) {

@@ -12,7 +12,7 @@
 //     with its latency; a client waiting for a request of a launched batch waits for the
 //     device itself and publishes the batch first if it gets there first.
 // Large requests (at least exclusive_bytes of columns to scan) run alone, through q1_run's
-// scan kernel with its tuned launch and the slot's own spread tables, and one at a time in
+// scan kernel with its tuned launch and the slot's own merge set, and one at a time in
 // arrival order: two large scans sharing the device would both finish late, which is what
 // sets the latency tail.  Smaller requests batch beside them on the other slots, so a short
 // request that arrives while a large one runs starts at once instead of queueing behind it.
@@ -82,8 +82,10 @@ struct Slot {
   hipGraphNode_t kernel_node = nullptr;  // the batched kernel's node (its grid is set per batch)
   hipKernelNodeParams kernel_params{};
   uint32_t grid = 0;             // the batched kernel's tuned (persistent) grid
-  q1::Spread spread{};           // the slot's own spread-merge tables (lone requests)
-  bool spread_dirty = false;     // a failed launch may have left partial sums in them
+  q1::MergeSet* set = nullptr;   // the slot's own merge set (lone requests)
+  q1::HostResult* h_result = nullptr;  // pinned: what a lone request's kernel leaves
+  q1::HostResult* h_result_dev = nullptr;  // ... as the device addresses it
+  bool lone = false;             // the batch's result is in h_result
   std::vector<Pending> batch;
   Clock::time_point started;
   uint32_t batch_id = 0;
@@ -207,74 +209,43 @@ q1_status prepare_slot(q1_server* sv, Slot& s, uint32_t cap, q1_layout layout) {
 q1_status launch_slot(q1_server* sv, Slot& s) {
   const uint32_t n = (uint32_t)s.batch.size();
   const q1_table* t0 = s.batch[0].req.table;
-  if (s.single) {
-    // One request on a table outside the TPC-H domain: the 64-bit scan kernel.
-    q1_status st = prepare_slot(sv, s, 16, t0->layout);
-    if (st != Q1_OK) return st;
+  s.lone = false;
+  if (n == 1) {
+    // A lone request runs the scan kernel of q1_run with its tuned launch (the batched
+    // kernel's list of entries buys nothing for one request), or the 64-bit scan kernel on a
+    // table outside the TPC-H domain, merging through the slot's own set.
     const q1_request& r = s.batch[0].req;
+    q1_placement p = Q1_PLACE_IN_REGISTERS;
+    q1_launch l{256, 1024, 0, 0};
+    if (!s.single) {
+      p = q1::resolve_placement(sv->ctx, t0->layout, Q1_PLACE_AUTO);
+      q1::resolve_launch(sv->ctx, t0->layout, p, r.row_count, nullptr, &l);
+    }
     q1::LaunchShape shape;
     const char* why = "";
-    q1_launch l{256, 1024, 0, 0};
-    st = q1::make_shape(Q1_PLACE_IN_REGISTERS, t0->layout, &l, r.row_begin, r.row_begin + r.row_count, &shape, &why);
-    if (st != Q1_OK) return st;
-    q1::ScanArgs a;
-    a.cols = t0->dev;
-    a.row_begin = r.row_begin;
-    a.row_end = r.row_begin + r.row_count;
-    a.cutoff_day = t0->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t0->filter_cutoff : r.cutoff_day;
-    a.out = s.d_out;
-    st = q1::launch_zero(s.d_out, 1, s.stream);
-    if (st == Q1_OK)
-      st = q1::launch_scan(Q1_PLACE_IN_REGISTERS, t0->layout, false, a, shape, nullptr, s.stream, nullptr, true);
-    if (st == Q1_OK && hipMemcpyAsync(s.h_out, s.d_out, sizeof(q1_device_aggregates), hipMemcpyDeviceToHost,
-                                      s.stream) != hipSuccess)
-      st = Q1_EDEVICE;
-    if (st == Q1_OK && hipEventRecord(s.done, s.stream) != hipSuccess) {
-      (void)hipStreamSynchronize(s.stream);
-      st = Q1_EDEVICE;
+    q1_status st = q1::make_shape(p, t0->layout, &l, r.row_begin, r.row_begin + r.row_count, &shape, &why);
+    if (s.single && st != Q1_OK) return st;
+    if (st == Q1_OK && q1::scan_workspace_bytes(p, shape) == 0) {
+      q1::ScanArgs a{};
+      a.cols = t0->dev;
+      a.row_begin = r.row_begin;
+      a.row_end = r.row_begin + r.row_count;
+      a.cutoff_day = t0->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t0->filter_cutoff : r.cutoff_day;
+      a.host = s.h_result_dev;
+      std::memset(s.h_result, 0, sizeof(*s.h_result));  // stays so when there are no rows
+      st = q1::launch_scan(p, t0->layout, !s.single, a, shape, nullptr, s.stream, s.set, s.single);
+      if (st == Q1_OK && hipEventRecord(s.done, s.stream) != hipSuccess) {
+        (void)hipStreamSynchronize(s.stream);
+        st = Q1_EDEVICE;
+      }
+      s.lone = st == Q1_OK;
+      return st;
     }
-    return st;
   }
   uint32_t cap = 16;
   while (cap < n) cap <<= 1;
   q1_status st = prepare_slot(sv, s, cap, t0->layout);
   if (st != Q1_OK) return st;
-  if (n == 1 && s.spread.tables) {
-    // A lone request runs the scan kernel of q1_run with its tuned launch (the batched
-    // kernel's list of entries buys nothing for one request), merging large grids through
-    // the slot's own spread tables.
-    const q1_request& r = s.batch[0].req;
-    q1_placement p = q1::resolve_placement(sv->ctx, t0->layout, Q1_PLACE_AUTO);
-    q1_launch l;
-    q1::resolve_launch(sv->ctx, t0->layout, p, r.row_count, nullptr, &l);
-    q1::LaunchShape shape;
-    const char* why = "";
-    st = q1::make_shape(p, t0->layout, &l, r.row_begin, r.row_begin + r.row_count, &shape, &why);
-    if (st == Q1_OK && q1::scan_workspace_bytes(p, shape) == 0) {
-      q1::ScanArgs a;
-      a.cols = t0->dev;
-      a.row_begin = r.row_begin;
-      a.row_end = r.row_begin + r.row_count;
-      a.cutoff_day = t0->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t0->filter_cutoff : r.cutoff_day;
-      a.out = s.d_out;
-      if (s.spread_dirty) {
-        st = q1::launch_zero(s.spread.tables, q1::kSpreadTables, s.stream);
-        if (st != Q1_OK) return st;
-        s.spread_dirty = false;
-      }
-      st = q1::launch_zero(s.d_out, 1, s.stream);
-      if (st == Q1_OK) st = q1::launch_scan(p, t0->layout, true, a, shape, nullptr, s.stream, &s.spread);
-      if (st != Q1_OK) s.spread_dirty = true;
-      if (st == Q1_OK && hipMemcpyAsync(s.h_out, s.d_out, sizeof(q1_device_aggregates), hipMemcpyDeviceToHost,
-                                        s.stream) != hipSuccess)
-        st = Q1_EDEVICE;
-      if (st == Q1_OK && hipEventRecord(s.done, s.stream) != hipSuccess) {
-        (void)hipStreamSynchronize(s.stream);
-        st = Q1_EDEVICE;
-      }
-      return st;
-    }
-  }
   const uint32_t lane_rows = q1::batch_lane_rows(sv->ctx, t0->layout, sv->placement);
   q1::BatchDesc* d = reinterpret_cast<q1::BatchDesc*>(s.h_buf + 1);
   uint64_t entries = 0;
@@ -339,7 +310,7 @@ void publish(q1_server* sv, Slot& s, q1_status st, uint32_t id) {
   for (size_t i = 0; i < s.batch.size(); i++) {
     Finished f;
     f.status = st;
-    if (st == Q1_OK) q1_aggregates_to_result(&s.h_out[i], &f.result);
+    if (st == Q1_OK) q1_aggregates_to_result(s.lone ? &s.h_result->sums : &s.h_out[i], &f.result);
     f.stats.submit_to_start_us =
         std::chrono::duration<double, std::micro>(s.started - s.batch[i].submitted).count();
     f.stats.latency_us = std::chrono::duration<double, std::micro>(now - s.batch[i].submitted).count();
@@ -509,14 +480,15 @@ q1_status q1_server_create(q1_ctx* ctx, const q1_server_config* cfg, q1_server**
     const q1_placement best = ctx->best[Q1_LAYOUT_COMPRESSED];
     sv->placement = best == Q1_PLACE_PER_THREAD_SHARED_MEM ? best : Q1_PLACE_IN_REGISTERS;
     sv->slots.resize(c.max_inflight);
-    const size_t spread_bytes = q1::kSpreadTables * sizeof(q1_device_aggregates);
     for (auto& s : sv->slots) {
       if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess ||
           hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess ||
-          hipMalloc(&s.spread.tables, spread_bytes) != hipSuccess ||
-          hipMemset(s.spread.tables, 0, spread_bytes) != hipSuccess) {
+          hipHostMalloc(&s.h_result, sizeof(q1::HostResult), hipHostMallocMapped) != hipSuccess ||
+          hipHostGetDevicePointer((void**)&s.h_result_dev, s.h_result, 0) != hipSuccess ||
+          hipMalloc(&s.set, sizeof(q1::MergeSet)) != hipSuccess ||
+          hipMemset(s.set, 0, sizeof(q1::MergeSet)) != hipSuccess) {
         q1_server_destroy(sv);
-        return q1::fail(ctx, Q1_EDEVICE, "stream or spread-table creation failed");
+        return q1::fail(ctx, Q1_EDEVICE, "stream or merge-set creation failed");
       }
     }
     if (hipDeviceSynchronize() != hipSuccess) {
@@ -663,7 +635,8 @@ void q1_server_destroy(q1_server* sv) {
   for (auto& s : sv->slots) {
     if (s.stream) (void)hipStreamSynchronize(s.stream);
     free_slot_buffers(s);
-    if (s.spread.tables) (void)hipFree(s.spread.tables);
+    if (s.set) (void)hipFree(s.set);
+    if (s.h_result) (void)hipHostFree(s.h_result);
     if (s.done) (void)hipEventDestroy(s.done);
     if (s.stream) (void)hipStreamDestroy(s.stream);
   }

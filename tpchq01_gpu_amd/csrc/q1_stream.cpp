@@ -175,7 +175,7 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
       LaunchShape shape;
       s = make_shape(p, layout, &l, 0, n, &shape, &why);
       if (s != Q1_OK) return drain_fail(s, why);
-      ScanArgs a;
+      ScanArgs a{};
       a.cols = dst;
       a.row_begin = 0;
       a.row_end = n;
@@ -235,34 +235,25 @@ q1_status q1_run_split(q1_ctx* ctx, const q1_table* t, const q1_columns* host, u
     if (s != Q1_OK) return fail(ctx, s, why);
     s = ensure_workspace(ctx, scan_workspace_bytes(p, shape));
     if (s != Q1_OK) return s;
-    ScanArgs a;
+    ScanArgs a{};
     a.cols = t->dev;
     a.row_begin = 0;
     a.row_end = split;
     a.cutoff_day = t->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t->filter_cutoff : cutoff_day;
-    a.out = ctx->d_aggr;
     const auto w0 = std::chrono::steady_clock::now();
-    s = launch_zero(ctx->d_aggr, 1, ctx->stream);
-    if (s == Q1_OK && hipEventRecord(ctx->ev_begin, ctx->stream) != hipSuccess) s = Q1_EDEVICE;
-    if (s == Q1_OK) s = scan_on(ctx, p, t->layout, t->fast, a, shape, ctx->stream, !t->fast);
-    if (s == Q1_OK && hipEventRecord(ctx->ev_end, ctx->stream) != hipSuccess) s = Q1_EDEVICE;
-    if (s == Q1_OK &&
-        hipMemcpyAsync(ctx->h_aggr, ctx->d_aggr, sizeof(q1_device_aggregates), hipMemcpyDeviceToHost, ctx->stream) !=
-            hipSuccess)
-      s = Q1_EDEVICE;
-    if (s != Q1_OK) return fail(ctx, s, "device part of the split failed to launch");
+    s = scan_to_host(ctx, p, t->layout, t->fast, a, shape, !t->fast);
+    if (s != Q1_OK) return s;
     // The host share runs while the device works.
     q1_result cpu{};
     const auto c0 = std::chrono::steady_clock::now();
     s = q1_cpu_run(t->layout, host, split, rows - split, a.cutoff_day, cpu_threads, &cpu);
     const double cms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - c0).count();
-    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return fail(ctx, Q1_EDEVICE, "device part of the split failed");
-    if (s != Q1_OK) return fail(ctx, s, "host part of the split failed");
     q1_result gpu;
-    q1_aggregates_to_result(ctx->h_aggr, &gpu);
+    double ms = 0;
+    const q1_status device = wait_result(ctx, &gpu, &ms);
+    if (device != Q1_OK) return device;
+    if (s != Q1_OK) return fail(ctx, s, "host part of the split failed");
     q1_result_merge(&gpu, &cpu, out);
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end);
     ctx->last = q1_timing{};
     ctx->last.kernel_ms = ms;
     ctx->last.wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
