@@ -880,7 +880,6 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
 // 2^28 over a tile; the product in the high half, below 16 * 15 * 2^24 < 2^32), so a row
 // costs three adds per group: that word, the packed count|discount|quantity and the charge.
 struct AccRegisters {
-  static constexpr bool kPackedSmall = false;
   uint32_t ns[kNumGroups];
   uint64_t npd[kNumGroups];
   uint64_t ch[kNumGroups], pr[kNumGroups], dp[kNumGroups];
@@ -969,7 +968,6 @@ __device__ __forceinline__ uint64_t small_to_small64(uint32_t s) {
 // of it (real data fills four of the six groups), and its four 64-bit adds run under the
 // lanes' mask: count, discount and quantity share one word (pack_small64).
 struct AccPerThread {
-  static constexpr bool kPackedSmall = false;
   uint64_t sm[kNumGroups], pr[kNumGroups], dp[kNumGroups], ch[kNumGroups];
   __device__ __forceinline__ void init(char*) {
 #pragma unroll
@@ -1020,7 +1018,6 @@ struct AccPerThread {
 // 64 rows 1.46 ms, 256 rows 1.35 ms, 1024 rows 1.19 ms.
 constexpr uint32_t kLocalFlushRows = 1024;
 struct AccLocal {
-  static constexpr bool kPackedSmall = false;
   // Per group: narrow sums of at most 16 rows as in AccRegisters (pack_small word; price
   // and discount product in one 64-bit word), folded every 16 rows into 64-bit
   // register sums of at most kLocalFlushRows rows (count, discount and quantity in the
@@ -1124,6 +1121,58 @@ struct AccLocal {
   static constexpr uint32_t lds_bytes(uint32_t) { return 0; }
 };
 
+// The LDS tables of the shared placement: [group][word][thread] words of 64 bits, W words per
+// group.  A wavefront clears, updates and sums only its own 64 threads' words of every row,
+// and LDS operations of a wavefront take effect in order, so none of it needs a barrier.
+// Clearing: one 16-byte store covers a wavefront's words of two rows.
+template <int B, int W>
+__device__ __forceinline__ void clear_wave_table(uint64_t* tab) {
+  const uint32_t wave = thread_index() >> 6, lane = thread_index() & 63;
+  uint64_t* p = tab + (lane >> 5) * B + wave * 64 + (lane & 31) * 2;
+#pragma unroll
+  for (int row = 0; row < W * kNumGroups; row += 2) *reinterpret_cast<uint4*>(p + row * B) = make_uint4(0, 0, 0, 0);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Sums a wavefront's part of the table over its threads into red[wave][group][NF].  Lane 8g + k
+// takes group g and threads k, k + 8, ... (rotated by g, so that the groups' reads fall on
+// different banks), then the eight lanes of a group are added with DPP.  All groups go at
+// once: about 200 vector instructions per wavefront, where a butterfly over all lanes for
+// each word of each group took 1,560 -- half the vector work of a block of 128 rows per
+// lane, and 2 us of every short launch.  Kernel time of 5,003 compressed rows 10.5 -> 8.5 us,
+// of 1M rows 12.3 -> 10.4, of 6M rows 20.9 -> 18.6; the 256-request batch 1,019 -> 977 us
+// per call; 600M rows 847 -> 843 us.
+__device__ __forceinline__ void add_eight(uint32_t& v) {
+  v += (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
+  v += (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
+  v += (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, false);  // row_half_mirror
+}
+__device__ __forceinline__ void add_eight(uint64_t& v) {
+  v += dpp_u64<0xB1>(v);
+  v += dpp_u64<0x4E>(v);
+  v += dpp_u64<0x141>(v);
+}
+template <int B, int W, class GroupSums>
+__device__ __forceinline__ void sum_wave_table(const uint64_t* tab, uint64_t* red) {
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const uint32_t wave = thread_index() >> 6, lane = thread_index() & 63, g = lane >> 3, k = lane & 7;
+  GroupSums sums;
+  if (g < kNumGroups) {
+    const uint64_t* p = tab + g * (W * B) + wave * 64 + k;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; i++) {
+      uint64_t w[W];
+#pragma unroll
+      for (int j = 0; j < W; j++) w[j] = p[j * B + 8 * ((i + g) & 7)];
+      sums.add(w);
+    }
+  }
+  sums.reduce([](auto& v) { add_eight(v); });
+  if (g < kNumGroups && k == 0) sums.store(red + (wave * kNumGroups + g) * NF);
+}
+
 // Q1_PLACE_PER_THREAD_SHARED_MEM: each lane owns a table in LDS laid out
 // [group][field][thread] (consecutive lanes -> consecutive 8-byte words, so a wavefront's
 // update of any mix of groups is bank-conflict free); rows are added with return-less
@@ -1139,8 +1188,7 @@ struct AccShared {
   uint64_t* tab;  // dynamic LDS: 6 * 4 * B words
   __device__ __forceinline__ void init(char* lds) {
     tab = reinterpret_cast<uint64_t*>(lds);
-#pragma unroll
-    for (int i = 0; i < 4 * kNumGroups; i++) tab[i * B + thread_index()] = 0;
+    clear_wave_table<B, 4>(tab);
   }
   __device__ __forceinline__ void add(const FastRow& r) {
     // Nearly every row passes: lay the atomics out inline, with no branch around them.
@@ -1157,20 +1205,58 @@ struct AccShared {
     }
   }
   __device__ __forceinline__ void flush(bool = false) {}
-  // NARROW tables hand over the packed (count | discount | quantity) word in F_CNT: at
-  // most 256 rows per lane, a wavefront's sum of it still fits every field (count
-  // < 2^17, discount < 2^20, quantity < 2^27), so the block merge sums one word for three.
-  static constexpr bool kPackedSmall = NARROW;
+  // The wavefront's sums of one group's words (sum_wave_table).  A wavefront's sum of the
+  // packed word fits its fields for NARROW tables (count <= 64 * 256, discount < 2^18,
+  // quantity <= 64 * 256 * 6300 < 2^27); the others take the fields apart first.
+  struct GroupSums {
+    uint64_t small = 0, price = 0, dprod = 0, charge = 0;
+    uint32_t cnt = 0, disc = 0;
+    uint64_t qty = 0;
+    __device__ __forceinline__ void add(const uint64_t (&w)[4]) {
+      if (NARROW) {
+        small += w[0];
+      } else {
+        cnt += (uint32_t)w[0] & ((1u << 17) - 1);
+        disc += (uint32_t)(w[0] >> 17) & ((1u << 20) - 1);
+        qty += w[0] >> 37;
+      }
+      price += w[1];
+      dprod += w[2];
+      charge += w[3];
+    }
+    template <class F>
+    __device__ __forceinline__ void reduce(F f) {
+      if (NARROW) {
+        f(small);
+      } else {
+        f(cnt);
+        f(disc);
+        f(qty);
+      }
+      f(price);
+      f(dprod);
+      f(charge);
+    }
+    __device__ __forceinline__ void store(uint64_t* r) const {
+      if (NARROW) {
+        unpack_small64(small, r);
+      } else {
+        r[F_CNT] = cnt;
+        r[F_DISC] = disc;
+        r[F_QTY] = qty;
+      }
+      r[F_PRICE] = price;
+      r[F_DPROD] = dprod;
+      r[F_CHARGE] = charge;
+    }
+  };
+  __device__ __forceinline__ void wave_totals(uint64_t* red) const { sum_wave_table<B, 4, GroupSums>(tab, red); }
+  // The lane's own sums (scan_any and scan_wide add their wide ones to them).
   __device__ __forceinline__ void totals(LaneTotals& o, char*) const {
 #pragma unroll
     for (int g = 0; g < kNumGroups; g++) {
       const uint64_t* base = tab + g * (4 * B) + thread_index();
-      if (NARROW) {
-        o.v[g][F_CNT] = base[0];
-        o.v[g][F_QTY] = o.v[g][F_DISC] = 0;
-      } else {
-        unpack_small64(base[0], o.v[g]);
-      }
+      unpack_small64(base[0], o.v[g]);
       o.v[g][F_PRICE] = base[B];
       o.v[g][F_DPROD] = base[2 * B];
       o.v[g][F_CHARGE] = base[3 * B];
@@ -1195,8 +1281,7 @@ struct AccSharedPacked {
   uint64_t* tab;  // dynamic LDS: 6 * 3 * B words
   __device__ __forceinline__ void init(char* lds) {
     tab = reinterpret_cast<uint64_t*>(lds);
-#pragma unroll
-    for (int i = 0; i < 3 * kNumGroups; i++) tab[i * B + thread_index()] = 0;
+    clear_wave_table<B, 3>(tab);
   }
   __device__ __forceinline__ void add(const FastRow& r) {
     // Nearly every row passes: lay the atomics out inline, with no branch around them.
@@ -1210,22 +1295,36 @@ struct AccSharedPacked {
     }
   }
   __device__ __forceinline__ void flush(bool = false) {}
-  // The block merge gets count, discount and quantity re-packed in the pack_small64 layout
-  // (a wavefront's sums of them fit it: count <= 64 * 256, discount <= 64 * 3840,
-  // quantity <= 64 * 16128), so it sums one word for the three.
-  static constexpr bool kPackedSmall = true;
-  __device__ __forceinline__ void totals(LaneTotals& o, char*) const {
-#pragma unroll
-    for (int g = 0; g < kNumGroups; g++) {
-      const uint64_t* base = tab + g * (3 * B) + thread_index();
-      const uint64_t w0 = base[0], w1 = base[B];
-      o.v[g][F_PRICE] = w0 & 0xFFFFFFFFull;
-      o.v[g][F_CNT] = (w1 >> 48) | ((w0 >> 32) & 0xFFFull) << 17 | (w0 >> 44) << 37;
-      o.v[g][F_QTY] = o.v[g][F_DISC] = 0;
-      o.v[g][F_DPROD] = w1 & ((1ull << 48) - 1);
-      o.v[g][F_CHARGE] = base[2 * B];
+  // The wavefront's sums of one group's words (sum_wave_table): slot 0 is taken apart, slot
+  // 1's fields hold a wavefront's sums (product < 2^42, count <= 64 * 256).
+  struct GroupSums {
+    uint64_t price = 0, dprod_cnt = 0, charge = 0;
+    uint32_t disc = 0, qty = 0;
+    __device__ __forceinline__ void add(const uint64_t (&w)[3]) {
+      price += (uint32_t)w[0];
+      disc += (uint32_t)(w[0] >> 32) & 0xFFFu;
+      qty += (uint32_t)(w[0] >> 44);
+      dprod_cnt += w[1];
+      charge += w[2];
     }
-  }
+    template <class F>
+    __device__ __forceinline__ void reduce(F f) {
+      f(price);
+      f(disc);
+      f(qty);
+      f(dprod_cnt);
+      f(charge);
+    }
+    __device__ __forceinline__ void store(uint64_t* r) const {
+      r[F_PRICE] = price;
+      r[F_DISC] = disc;
+      r[F_QTY] = qty;
+      r[F_DPROD] = dprod_cnt & ((1ull << 48) - 1);
+      r[F_CNT] = dprod_cnt >> 48;
+      r[F_CHARGE] = charge;
+    }
+  };
+  __device__ __forceinline__ void wave_totals(uint64_t* red) const { sum_wave_table<B, 3, GroupSums>(tab, red); }
   static constexpr uint32_t lds_bytes(uint32_t) { return packed_table_bytes(B); }
 };
 
@@ -1241,7 +1340,6 @@ struct AccSharedPacked {
 // fits 64 bits (price < 2^46, discount product < 2^50, charge < 2^60).
 __device__ __forceinline__ void atomic_add128(uint64_t* lo_p, uint64_t* hi_p, uint64_t lo, uint64_t hi);
 struct AccGlobal {
-  static constexpr bool kPackedSmall = false;
   static constexpr int W = 5;  // words per group: count|disc, qty, price, dprod, charge
   AccRegisters regs;
   uint64_t* tab;               // [W][6] words of this block
@@ -1340,36 +1438,25 @@ __device__ __forceinline__ void atomic_add128(uint64_t* lo_p, uint64_t* hi_p, ui
   if (hi + carry) atomicAdd((unsigned long long*)hi_p, (unsigned long long)(hi + carry));
 }
 
-// Block-wide reduction of LaneTotals (exact: lane sums fit uint64, block sums are taken
-// in 128 bits) and the merge into `out`.  `red` is LDS scratch of
-// (blockDim/64) * 6 * NF uint64 words.  qty_scale turns layout units into x100.
-// PACKED: t.v[g][F_CNT] holds the packed (count | discount | quantity) word of the
-// lane (pack_small64 layout) and F_QTY / F_DISC are unused.
-template <bool PACKED = false>
-__device__ void block_merge(const LaneTotals& t, uint64_t* red, q1_device_aggregates* out,
-                            uint64_t qty_scale) {
-  const uint32_t wave = thread_index() >> 6, lane = thread_index() & 63, nwaves = blockDim.x >> 6;
+// A wavefront's sums of LaneTotals (exact: they fit uint64) into red[wave][group][NF].
+__device__ void sum_lane_totals(const LaneTotals& t, uint64_t* red) {
+  const uint32_t wave = thread_index() >> 6, lane = thread_index() & 63;
 #pragma unroll
   for (int g = 0; g < kNumGroups; g++) {
     const bool any = ballot(t.v[g][F_CNT] != 0) != 0;
     uint64_t* r = red + (wave * kNumGroups + g) * NF;
 #pragma unroll
     for (int f = 0; f < NF; f++) {
-      if (PACKED && (f == F_QTY || f == F_DISC)) continue;
-      const uint64_t s = any ? wave_sum_u64(t.v[g][f]) : 0;
-      if (lane == 0) {
-        if (PACKED && f == F_CNT) {
-          uint64_t u[NF];
-          unpack_small64(s, u);
-          r[F_CNT] = u[F_CNT];
-          r[F_DISC] = u[F_DISC];
-          r[F_QTY] = u[F_QTY];
-        } else {
-          r[f] = s;
-        }
-      }
+      const uint64_t sum = any ? wave_sum_u64(t.v[g][f]) : 0;
+      if (lane == 0) r[f] = sum;
     }
   }
+}
+
+// The block's merge into `out`: the wavefronts' sums red[wave][group][NF] are added in 128
+// bits.  qty_scale turns layout units into x100.
+__device__ __forceinline__ void block_merge(const uint64_t* red, q1_device_aggregates* out, uint64_t qty_scale) {
+  const uint32_t nwaves = blockDim.x >> 6;
   __syncthreads();
   // Thread g*NF + f sums field f of group g over the waves (128-bit) and issues that
   // field's atomics, so a block's destination atomics go out together.
@@ -1650,12 +1737,16 @@ __device__ __forceinline__ void scan_block(const ScanArgs& a, uint64_t block, ui
     // through the block's table in global memory
     acc.merge(out, qty_scale);
   } else {
-    LaneTotals tot;
-    acc.totals(tot, reinterpret_cast<char*>(lds));
     // The reduction scratch follows the placement's own LDS table.
     uint64_t* red = lds + Acc::lds_bytes(B) / 8;
-    __syncthreads();
-    block_merge<Acc::kPackedSmall>(tot, red, out, qty_scale);
+    if constexpr (kSplit) {
+      acc.wave_totals(red);
+    } else {
+      LaneTotals tot;
+      acc.totals(tot, reinterpret_cast<char*>(lds));
+      sum_lane_totals(tot, red);
+    }
+    block_merge(red, out, qty_scale);
   }
 }
 
