@@ -116,8 +116,10 @@ typedef struct {
 
 /* Launch shape (the reference's --threads-per-block / --tuples-per-thread,
  * src/main.cu:255-360, 627-650).  Zero fields mean "from the autotuning table"; launches
- * of q1_enqueue and q1_run_streaming without Q1_LAUNCH_ASSUME_TPCH_DOMAIN run the
- * any-value kernel, whose zero fields mean 256 threads and 1024 tuples per thread. */
+ * of q1_enqueue and q1_run_streaming without Q1_LAUNCH_ASSUME_TPCH_DOMAIN, and queries on
+ * tables outside the TPC-H domain, run the any-value kernel, whose zero fields mean a shape
+ * of its own for the number of rows.  That kernel takes at most 128 (compressed) or 256 rows
+ * per lane: a larger tuples_per_thread becomes more blocks. */
 typedef struct {
   uint32_t threads_per_block; /* 64, 128 or 256 (the batched kernel: 256) */
   uint32_t tuples_per_thread; /* multiple of 16 */
@@ -127,7 +129,7 @@ typedef struct {
 
 /* q1_enqueue only: the caller asserts the columns lie in the TPC-H value domain
  * (discount <= 15, tax <= 15, quantity <= 63 units, extended_price < 2^24) so the narrow
- * 32-bit kernels may run; without it the 64-bit kernels run.  Tables created through
+ * 32-bit kernels may run; without it the any-value kernel runs.  Tables created through
  * this library measure their own domain. */
 #define Q1_LAUNCH_ASSUME_TPCH_DOMAIN 1u
 

@@ -47,6 +47,17 @@ q1_placement resolve_placement(q1_ctx* ctx, q1_layout layout, q1_placement p) {
   return p == Q1_PLACE_AUTO ? ctx->best[layout] : p;
 }
 
+// The any-value kernel's shape: 128 lanes x 128 rows, or 64 rows where 128 would give fewer
+// than 16 blocks per compute unit (the last of few rounds of large blocks leaves compute
+// units idle), and less only to have 4 blocks per compute unit (a block's fixed cost shows).
+// Compressed / uncompressed / reference at 60M rows: 128 x 64 93 / 190 / 341 us, 128 x 128
+// 98 / 200 / 354, 256 x 128 97 / 199 / 371; 6M rows: 128 x 32 20 / 33 / 46, 128 x 64 20 / 30 /
+// 45, 128 x 128 27 / 44 / 48; 1M rows: 128 x 16 12 / 14 / 15, 128 x 64 15 / 21 / 21.  256 lanes
+// are 1 % faster on 600M compressed rows and 12 % slower on 60M reference rows, whose
+// tables then leave a compute unit one block.
+constexpr uint32_t kAnyThreads = 128, kAnyTuples = 128;
+constexpr uint64_t kAnyBlocksPerCu = 16;
+
 // The tuned shape for a range of `rows` rows: of the shapes tuned at several row counts,
 // the one whose row count is nearest by ratio (the larger on a tie); the single tuned
 // shape when the table has none.
@@ -67,25 +78,31 @@ static q1_launch tuned_for_rows(const q1_ctx* ctx, q1_layout layout, q1_placemen
   return t;
 }
 
-void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, uint64_t rows, const q1_launch* in,
-                    q1_launch* out, bool any_value_kernel) {
-  const q1_launch t = tuned_for_rows(ctx, layout, p, rows);
-  const bool any_value = any_value_kernel && !(in && (in->flags & Q1_LAUNCH_ASSUME_TPCH_DOMAIN));
-  const uint32_t tuned_threads = any_value ? 256 : t.threads_per_block;
-  const uint32_t tuned_tuples = any_value ? 1024 : t.tuples_per_thread;
-  out->threads_per_block = in && in->threads_per_block ? in->threads_per_block : tuned_threads;
-  out->tuples_per_thread = in && in->tuples_per_thread ? in->tuples_per_thread : tuned_tuples;
+void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, uint64_t rows, const q1_launch* in,
+                    q1_launch* out, bool table) {
+  q1_launch t{kAnyThreads, kAnyTuples, 0, 0};
+  if (fast)
+    t = tuned_for_rows(ctx, layout, p, rows);
+  else if (in && in->num_blocks)
+    // a caller's grid is held against the tuned shape for a table, 256 x 1024 for raw pointers
+    t = table ? tuned_for_rows(ctx, layout, p, rows) : q1_launch{256, 1024, 0, 0};
+  out->threads_per_block = in && in->threads_per_block ? in->threads_per_block : t.threads_per_block;
+  out->tuples_per_thread = in && in->tuples_per_thread ? in->tuples_per_thread : t.tuples_per_thread;
   out->num_blocks = in ? in->num_blocks : 0;
   out->flags = in ? in->flags : 0;
+  // A caller-chosen value is kept as given.
+  if ((in && in->tuples_per_thread) || out->num_blocks) return;
   // A range smaller than the row counts the shape was tuned at halves its tuples_per_thread
-  // until the grid has at least 4 blocks per compute unit, so small requests still spread
-  // over the whole chip.  A caller-chosen value is kept as given.
-  if (!(in && in->tuples_per_thread) && !out->num_blocks) {
-    const uint64_t want = 4ull * (uint64_t)(ctx->compute_units > 0 ? ctx->compute_units : 256);
-    const uint64_t tpb = out->threads_per_block ? out->threads_per_block : 256;
-    while (out->tuples_per_thread > 16 && rows < want * tpb * out->tuples_per_thread)
+  // until the grid has at least `per_cu` blocks per compute unit, so small requests still
+  // spread over the whole chip.
+  const uint64_t tpb = out->threads_per_block ? out->threads_per_block : 256;
+  auto halve = [&](uint64_t per_cu, uint32_t least) {
+    const uint64_t want = per_cu * (uint64_t)(ctx->compute_units > 0 ? ctx->compute_units : 256);
+    while (out->tuples_per_thread > least && rows < want * tpb * out->tuples_per_thread)
       out->tuples_per_thread = std::max<uint32_t>(16, (out->tuples_per_thread / 2) & ~15u);
-  }
+  };
+  if (!fast) halve(kAnyBlocksPerCu, kAnyTuples / 2);
+  halve(4, 16);
 }
 
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
@@ -130,7 +147,7 @@ static StreamSpread* stream_spread(q1_ctx* ctx, void* stream) {
 }
 
 q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
-                  const LaunchShape& shape, void* stream, bool table_outside) {
+                  const LaunchShape& shape, void* stream) {
   // Launches on one stream run one after another, so they can share one merge set: the
   // context's for the context stream, a set of the stream's own for a caller's stream
   // (large launches only; the others merge directly).
@@ -146,13 +163,13 @@ q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fa
       other->zeroed = true;
     }
   }
-  const q1_status s = launch_scan(placement, layout, fast, a, shape, ctx->workspace, stream, set, table_outside);
+  const q1_status s = launch_scan(placement, layout, fast, a, shape, ctx->workspace, stream, set);
   if (other && hipEventRecord(other->done, (hipStream_t)stream) != hipSuccess) other->usable = false;
   return s;
 }
 
 q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, ScanArgs a,
-                       const LaunchShape& shape, bool table_outside) {
+                       const LaunchShape& shape) {
   a.host = ctx->d_result;
   a.sequence = ++ctx->sequence;
   if (shape.blocks == 0) {
@@ -160,7 +177,7 @@ q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bo
     ctx->h_result->sequence = a.sequence;
     return Q1_OK;
   }
-  const q1_status s = scan_on(ctx, placement, layout, fast, a, shape, (void*)ctx->stream, table_outside);
+  const q1_status s = scan_on(ctx, placement, layout, fast, a, shape, (void*)ctx->stream);
   return s == Q1_OK ? Q1_OK : fail(ctx, s, "scan kernel launch failed");
 }
 
@@ -710,10 +727,10 @@ static q1_status run_locked(q1_ctx* ctx, const q1_table* t, uint64_t row_begin, 
     return fail(ctx, Q1_EINVAL, "row range outside the table");
   const q1_placement p = resolve_placement(ctx, t->layout, placement);
   q1_launch l;
-  resolve_launch(ctx, t->layout, p, row_count, launch, &l);
+  resolve_launch(ctx, t->layout, p, t->fast, row_count, launch, &l);
   LaunchShape shape;
   const char* why = "";
-  q1_status s = make_shape(p, t->layout, &l, row_begin, row_begin + row_count, &shape, &why);
+  q1_status s = make_shape(p, t->layout, t->fast, &l, row_begin, row_begin + row_count, &shape, &why);
   if (s != Q1_OK) return fail(ctx, s, why);
   s = ensure_workspace(ctx, scan_workspace_bytes(p, shape));
   if (s != Q1_OK) return s;
@@ -724,7 +741,7 @@ static q1_status run_locked(q1_ctx* ctx, const q1_table* t, uint64_t row_begin, 
   a.cutoff_day = t->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t->filter_cutoff : cutoff_day;
   const auto w0 = std::chrono::steady_clock::now();
   double ms = 0;
-  s = scan_to_host(ctx, p, t->layout, t->fast, a, shape, !t->fast);
+  s = scan_to_host(ctx, p, t->layout, t->fast, a, shape);
   if (s == Q1_OK) s = wait_result(ctx, out, &ms);
   if (s != Q1_OK) return s;
   ctx->last = q1_timing{};
@@ -734,7 +751,7 @@ static q1_status run_locked(q1_ctx* ctx, const q1_table* t, uint64_t row_begin, 
   ctx->last.bytes_read = algorithmic_bytes(t->layout, row_count);
   ctx->last.num_blocks = shape.blocks;
   ctx->last.threads_per_block = shape.threads;
-  ctx->last.tuples_per_thread = l.tuples_per_thread;
+  ctx->last.tuples_per_thread = shape.tiles_per_thread * layout_tile_rows(t->layout);
   ctx->last.placement = t->fast ? (uint32_t)p : (uint32_t)Q1_PLACE_IN_REGISTERS_PER_THREAD;
   return Q1_OK;
 }
@@ -771,10 +788,11 @@ q1_status q1_enqueue_noalloc(q1_ctx* ctx, q1_placement placement, q1_layout layo
   }
   const q1_placement p = resolve_placement(ctx, layout, placement);
   q1_launch l;
-  resolve_launch(ctx, layout, p, num_tuples, launch, &l, true);
+  const bool fast = in_domain_flag(launch);
+  resolve_launch(ctx, layout, p, fast, num_tuples, launch, &l, false);
   LaunchShape shape;
   const char* why = "";
-  q1_status s = make_shape(p, layout, &l, row_begin, row_begin + num_tuples, &shape, &why);
+  q1_status s = make_shape(p, layout, fast, &l, row_begin, row_begin + num_tuples, &shape, &why);
   if (s != Q1_OK) return fail(ctx, s, why);
   ScanArgs a{};
   a.cols = *device;
@@ -783,7 +801,7 @@ q1_status q1_enqueue_noalloc(q1_ctx* ctx, q1_placement placement, q1_layout layo
   a.cutoff_day = cutoff_day;
   a.out = aggregates;
   // the device's static scratch array instead of the context's merge set and workspace
-  s = noalloc_launch_scan(ctx->device, p, layout, (l.flags & Q1_LAUNCH_ASSUME_TPCH_DOMAIN) != 0, a, shape,
+  s = noalloc_launch_scan(ctx->device, p, layout, fast, a, shape,
                           hip_stream ? hip_stream : (void*)ctx->stream, &why);
   return s == Q1_OK ? Q1_OK : fail(ctx, s, why);
   GUARD_END(ctx)
@@ -806,10 +824,11 @@ q1_status q1_enqueue(q1_ctx* ctx, q1_placement placement, q1_layout layout, cons
   }
   const q1_placement p = resolve_placement(ctx, layout, placement);
   q1_launch l;
-  resolve_launch(ctx, layout, p, num_tuples, launch, &l, true);
+  const bool fast = in_domain_flag(launch);
+  resolve_launch(ctx, layout, p, fast, num_tuples, launch, &l, false);
   LaunchShape shape;
   const char* why = "";
-  q1_status s = make_shape(p, layout, &l, row_begin, row_begin + num_tuples, &shape, &why);
+  q1_status s = make_shape(p, layout, fast, &l, row_begin, row_begin + num_tuples, &shape, &why);
   if (s != Q1_OK) return fail(ctx, s, why);
   void* stream = hip_stream ? hip_stream : (void*)ctx->stream;
   // The global placement's workspace is per launch: size it and keep launches that
@@ -824,7 +843,6 @@ q1_status q1_enqueue(q1_ctx* ctx, q1_placement placement, q1_layout layout, cons
   a.row_end = row_begin + num_tuples;
   a.cutoff_day = cutoff_day;
   a.out = aggregates;
-  const bool fast = (l.flags & Q1_LAUNCH_ASSUME_TPCH_DOMAIN) != 0;
   s = scan_on(ctx, p, layout, fast, a, shape, stream);
   return s == Q1_OK ? Q1_OK : fail(ctx, s, "scan kernel launch failed");
   GUARD_END(ctx)
@@ -851,7 +869,7 @@ q1_status q1_tuning_set(q1_ctx* ctx, q1_layout layout, q1_placement placement, c
     return fail(ctx, Q1_EINVAL, "bad argument");
   LaunchShape shape;
   const char* why = "";
-  const q1_status s = make_shape(placement, layout, best, 0, 1, &shape, &why);
+  const q1_status s = make_shape(placement, layout, true, best, 0, 1, &shape, &why);
   if (s != Q1_OK) return fail(ctx, s, why);
   ctx->tuning[layout][placement] = *best;
   ctx->tuning[layout][placement].num_blocks = 0;
@@ -868,7 +886,7 @@ q1_status q1_tuning_get(q1_ctx* ctx, q1_layout layout, q1_placement placement, q
 q1_status q1_tuning_resolve(q1_ctx* ctx, q1_layout layout, q1_placement placement, uint64_t rows,
                             q1_launch* out) {
   if (!ctx || !out || !valid_layout(layout) || !valid_placement(placement)) return Q1_EINVAL;
-  resolve_launch(ctx, layout, resolve_placement(ctx, layout, placement), rows, nullptr, out);
+  resolve_launch(ctx, layout, resolve_placement(ctx, layout, placement), true, rows, nullptr, out);
   return Q1_OK;
 }
 

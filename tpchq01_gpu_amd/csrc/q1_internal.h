@@ -92,23 +92,22 @@ namespace q1 {
 q1_status fail(q1_ctx* ctx, q1_status s, const std::string& why);
 q1_status hip_fail(q1_ctx* ctx, hipError_t e, const char* what);
 q1_placement resolve_placement(q1_ctx* ctx, q1_layout layout, q1_placement p);
-// Fills a launch from the caller's, with the tuned values where it leaves them 0.  Launches
-// without Q1_LAUNCH_ASSUME_TPCH_DOMAIN that run the any-value kernel (q1_enqueue,
-// q1_run_streaming) take that kernel's own defaults instead: it runs every placement
-// alike, and is fastest with 256 threads and 1024 rows per lane.
-void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, uint64_t rows, const q1_launch* in,
-                    q1_launch* out, bool any_value_kernel = false);
+// Fills a launch from the caller's, with the tuned values where it leaves them 0.  fast: for
+// the narrow kernels; launches that run the any-value kernel take that kernel's own shape
+// instead, since it runs every placement alike.  table: the columns are a table's.
+void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, uint64_t rows, const q1_launch* in,
+                    q1_launch* out, bool table = true);
+inline bool in_domain_flag(const q1_launch* l) { return l && (l->flags & Q1_LAUNCH_ASSUME_TPCH_DOMAIN); }
 uint64_t algorithmic_bytes(q1_layout layout, uint64_t rows);
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes);
 // launch_scan with the merge set of `stream` (the context's or a caller's).
-// table_outside: the rows come from a table known to hold values outside the domain.
 q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
-                  const LaunchShape& shape, void* stream, bool table_outside = false);
+                  const LaunchShape& shape, void* stream);
 // The same on the context stream with the sums going to ctx->h_result, and the wait for
 // them: fills *out and returns the kernel's device time in *kernel_ms.  A launch with no
 // blocks leaves zeros.
 q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, ScanArgs a,
-                       const LaunchShape& shape, bool table_outside);
+                       const LaunchShape& shape);
 q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms);
 void batch_destroy(q1_batch_state* b);
 // The batched kernel's plan, shared by q1_run_batch and the server: rows per lane (the

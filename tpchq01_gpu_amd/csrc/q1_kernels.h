@@ -71,8 +71,15 @@ struct ScanArgs {
   uint64_t sequence;
 };
 
+// Rows per lane for which the any-value kernel's LDS words are exact.
+constexpr uint32_t any_value_lane_rows(q1_layout l) {
+  return l == Q1_LAYOUT_COMPRESSED || l == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? 128 : 256;
+}
+
 // Validate and complete a launch shape for `rows` rows (0 fields filled from defaults).
-q1_status make_shape(q1_placement placement, q1_layout layout, const q1_launch* launch,
+// fast: for the narrow kernels.  The any-value kernel takes no more than
+// any_value_lane_rows rows per lane: a larger tuples_per_thread becomes more blocks.
+q1_status make_shape(q1_placement placement, q1_layout layout, bool fast, const q1_launch* launch,
                      uint64_t row_begin, uint64_t row_end, LaunchShape* shape, const char** why);
 
 // Smaller grids add straight into a device destination.  Device-scope atomics on one address
@@ -85,11 +92,9 @@ constexpr uint32_t kSpreadMinBlocks = 144;
 // Where a scan's sums go.  host: stored into a.host (needs `set`; every grid merges through
 // it).  Otherwise added into *a.out, through `set` when there is one and the grid has at
 // least kSpreadMinBlocks blocks.
-// fast: the rows lie inside the TPC-H domain.  Otherwise an any-value kernel runs;
-// table_outside picks the one for tables known to hold values outside the domain.
+// fast: the rows lie inside the TPC-H domain.  Otherwise the any-value kernel runs.
 q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
-                      const LaunchShape& shape, void* workspace, void* stream, MergeSet* set = nullptr,
-                      bool table_outside = false);
+                      const LaunchShape& shape, void* workspace, void* stream, MergeSet* set = nullptr);
 uint64_t scan_workspace_bytes(q1_placement placement, const LaunchShape& shape);
 
 // Zero device aggregate tables or a merge set (a fill kernel, safe inside graph capture).

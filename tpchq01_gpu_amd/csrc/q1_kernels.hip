@@ -284,13 +284,21 @@ FastFn fast_kernel(q1_layout l, int p, uint32_t threads) {
   }
 }
 
-// outside: the table is known to hold values outside the domain.
-GenFn general_kernel(q1_layout l, uint32_t threads, bool outside) {
+GenFn any_kernel(q1_layout l, uint32_t threads) {
   switch (l) {
-    case Q1_LAYOUT_REFERENCE: return outside ? wide_kernel_reference(threads) : any_kernel_reference(threads);
-    case Q1_LAYOUT_UNCOMPRESSED: return outside ? wide_kernel_uncompressed(threads) : any_kernel_uncompressed(threads);
-    case Q1_LAYOUT_COMPRESSED: return outside ? wide_kernel_compressed(threads) : any_kernel_compressed(threads);
-    default: return outside ? wide_kernel_pushdown(threads) : any_kernel_pushdown(threads);
+    case Q1_LAYOUT_REFERENCE: return any_kernel_reference(threads);
+    case Q1_LAYOUT_UNCOMPRESSED: return any_kernel_uncompressed(threads);
+    case Q1_LAYOUT_COMPRESSED: return any_kernel_compressed(threads);
+    default: return any_kernel_pushdown(threads);
+  }
+}
+
+uint32_t any_kernel_lds(q1_layout l, uint32_t threads) {
+  switch (l) {
+    case Q1_LAYOUT_REFERENCE: return any_kernel_lds_reference(threads);
+    case Q1_LAYOUT_UNCOMPRESSED: return any_kernel_lds_uncompressed(threads);
+    case Q1_LAYOUT_COMPRESSED: return any_kernel_lds_compressed(threads);
+    default: return any_kernel_lds_pushdown(threads);
   }
 }
 
@@ -312,7 +320,7 @@ bool domain_is_tpch(q1_layout layout, const Domain& d) {
          d.max_qty <= max_qty && d.min_price >= 0 && d.max_price < (1ll << 24);
 }
 
-q1_status make_shape(q1_placement placement, q1_layout layout, const q1_launch* launch,
+q1_status make_shape(q1_placement placement, q1_layout layout, bool fast, const q1_launch* launch,
                      uint64_t row_begin, uint64_t row_end, LaunchShape* shape, const char** why) {
   const uint32_t trows = tile_rows(layout);
   uint32_t threads = launch && launch->threads_per_block ? launch->threads_per_block : 256;
@@ -329,10 +337,10 @@ q1_status make_shape(q1_placement placement, q1_layout layout, const q1_launch* 
     *why = "unknown placement";
     return Q1_EINVAL;
   }
-  const uint32_t tiles_per_thread = tpt / trows;
+  uint32_t tiles_per_thread = tpt / trows;
   const uint64_t first = align_rows_down(row_begin) / trows, end = (row_end + trows - 1) / trows;
   const uint64_t tiles = end > first ? end - first : 0;
-  const uint64_t per_block = (uint64_t)threads * tiles_per_thread;
+  uint64_t per_block = (uint64_t)threads * tiles_per_thread;
   uint64_t blocks = (tiles + per_block - 1) / per_block;
   if (launch && launch->num_blocks) {
     // A caller-chosen grid must still cover the range with the chosen tuples per thread.
@@ -341,6 +349,12 @@ q1_status make_shape(q1_placement placement, q1_layout layout, const q1_launch* 
       return Q1_EINVAL;
     }
     blocks = launch->num_blocks;
+  }
+  if (!fast && tpt > any_value_lane_rows(layout)) {
+    tiles_per_thread = any_value_lane_rows(layout) / trows;
+    per_block = (uint64_t)threads * tiles_per_thread;
+    const uint64_t needed = (tiles + per_block - 1) / per_block;
+    blocks = needed > blocks ? needed : blocks;
   }
   // HIP's grid size counts work-items in 32 bits.
   if (blocks * threads > 0xFFFFFFFFull) {
@@ -358,7 +372,7 @@ uint64_t scan_workspace_bytes(q1_placement placement, const LaunchShape& shape) 
 }
 
 q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const ScanArgs& args,
-                      const LaunchShape& shape, void* workspace, void* stream, MergeSet* set, bool table_outside) {
+                      const LaunchShape& shape, void* workspace, void* stream, MergeSet* set) {
   if (args.host && !set) return Q1_EINVAL;
   if (shape.blocks == 0) return Q1_OK;
   const hipStream_t s = (hipStream_t)stream;
@@ -388,9 +402,8 @@ q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const
     hipLaunchKernelGGL(fast_kernel(layout, variant, shape.threads), dim3(shape.blocks), dim3(shape.threads), lds,
                        s, a, shape.tiles_per_thread, (uint64_t*)workspace);
   } else {
-    const uint32_t lds = shared_table_bytes(shape.threads) + nwaves * kNumGroups * 8 * 8;
-    hipLaunchKernelGGL(general_kernel(layout, shape.threads, table_outside), dim3(shape.blocks), dim3(shape.threads),
-                       lds, s, a, shape.tiles_per_thread);
+    hipLaunchKernelGGL(any_kernel(layout, shape.threads), dim3(shape.blocks), dim3(shape.threads),
+                       any_kernel_lds(layout, shape.threads), s, a, shape.tiles_per_thread);
   }
   return hip_status(hipGetLastError());
 }

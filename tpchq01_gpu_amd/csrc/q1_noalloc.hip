@@ -66,7 +66,7 @@ q1_status noalloc_launch_scan(int device, q1_placement placement, q1_layout layo
   }
   void* workspace = static_cast<char*>(base) + sizeof(MergeSet);
   const q1_status s =
-      launch_scan(placement, layout, fast, a, shape, workspace, stream, static_cast<MergeSet*>(base), false);
+      launch_scan(placement, layout, fast, a, shape, workspace, stream, static_cast<MergeSet*>(base));
   if (s != Q1_OK) *why = "scan kernel launch failed";
   return s;
 }

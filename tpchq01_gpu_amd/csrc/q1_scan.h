@@ -27,7 +27,7 @@
 //   small    = 1 | disc << 5 | qty << 13       (count, discount, quantity in one dword)
 //   dprod    = disc * price                     (then sum_disc_price = 100*sum_price - sum_dprod)
 //   charge   = (100-disc)*(100+tax) * price     (v_mul_u32_u24 + v_mul_hi_u32_u24)
-// Outside the domain the "general" kernel computes in wrapping int64 with 128-bit
+// Outside the domain the any-value kernel computes in wrapping int64 with 128-bit
 // signed sums, which is the reference CPU kernels' arithmetic for any input.
 #pragma once
 
@@ -44,7 +44,6 @@ namespace {
 
 constexpr int kMaxBlock = 256;
 constexpr int kBatchBlock = (int)kBatchThreads;  // the batched kernel's block size
-constexpr uint32_t kNoGroup = 7;
 
 // ------------------------------------------------------------------------------------
 // Small helpers
@@ -97,10 +96,12 @@ struct FastRow {
   __device__ __forceinline__ bool counts() const { return pass && gid < kNumGroups; }
 };
 
-// One row of the general path.
+// One row of the any-value path, for layouts whose values are wider than 32 bits.
 struct WideRow {
+  bool pass;
   uint32_t gid;
   int64_t qty, price, disc, tax;
+  __device__ __forceinline__ bool counts() const { return pass && gid < kNumGroups; }
 };
 
 // ------------------------------------------------------------------------------------
@@ -180,15 +181,6 @@ struct CompressedTile {
       }
     }
   }
-  // Every row of the tile inside the TPC-H value domain (discount, tax <= 15, quantity
-  // <= 63 units, price < 2^24); rows zeroed by load_edge pass.
-  __device__ __forceinline__ bool in_domain() const {
-    const uint32_t dd = d.x | d.y | d.z | d.w, xx = x.x | x.y | x.z | x.w, qq = q.x | q.y | q.z | q.w;
-    uint32_t pp = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) pp |= p[k].x | p[k].y | p[k].z | p[k].w;
-    return ((dd | xx) & 0xF0F0F0F0u) == 0 && (qq & 0xC0C0C0C0u) == 0 && (pp & 0xFF000000u) == 0;
-  }
   // `cut` is the cutoff relative to the frame of reference (may be < 0 or > 65535).
   __device__ __forceinline__ bool pass(int j, int32_t cut) const {
     if (PUSHDOWN) return (flt >> j) & 1;
@@ -230,16 +222,6 @@ struct CompressedTile {
     FastRow r;
     r.pass = EDGE ? ((valid >> j & 1) && pass(j, cut)) : pass(j, cut);
     r.gid = gid(j);
-    r.qty = byte(q, j);
-    r.disc = byte(d, j);
-    r.tax = byte(x, j);
-    r.price = comp(p[j >> 2], j & 3);
-    return r;
-  }
-  __device__ __forceinline__ WideRow wide(int j, int32_t cut, uint32_t valid) const {
-    WideRow r;
-    const bool ok = (valid >> j & 1) && pass(j, cut);
-    r.gid = ok ? gid(j) : kNoGroup;
     r.qty = byte(q, j);
     r.disc = byte(d, j);
     r.tax = byte(x, j);
@@ -307,12 +289,6 @@ struct CompressedStreamTile {
       }
     }
   }
-  // Every row of the tile inside the TPC-H value domain (discount, tax <= 15, quantity
-  // <= 63 units, price < 2^24); rows zeroed by load_edge pass.
-  __device__ __forceinline__ bool in_domain() const {
-    return ((d | x) & 0xF0F0F0F0u) == 0 && (q & 0xC0C0C0C0u) == 0 &&
-           ((p.x | p.y | p.z | p.w) & 0xFF000000u) == 0;
-  }
   // `cut` is the cutoff relative to the frame of reference (may be < 0 or > 65535).
   __device__ __forceinline__ bool pass(int j, int32_t cut) const {
     if (PUSHDOWN) return (flt >> j) & 1;
@@ -365,16 +341,6 @@ struct CompressedStreamTile {
     FastRow r;
     r.pass = EDGE ? ((valid >> j & 1) && pass(j, cut)) : pass(j, cut);
     r.gid = gid(j);
-    r.qty = byte(q, j);
-    r.disc = byte(d, j);
-    r.tax = byte(x, j);
-    r.price = comp(p, j);
-    return r;
-  }
-  __device__ __forceinline__ WideRow wide(int j, int32_t cut, uint32_t valid) const {
-    WideRow r;
-    const bool ok = (valid >> j & 1) && pass(j, cut);
-    r.gid = ok ? gid(j) : kNoGroup;
     r.qty = byte(q, j);
     r.disc = byte(d, j);
     r.tax = byte(x, j);
@@ -436,19 +402,6 @@ struct UncompressedTile {
   __device__ __forceinline__ bool pass(int j, int32_t cut) const {
     return (int32_t)comp(s[j >> 2], j & 3) <= cut;
   }
-  // Every row inside the TPC-H value domain (discount, tax in [0, 15], quantity in
-  // [0, 6300] hundredths, price in [0, 2^24)); rows zeroed by load_edge pass.
-  __device__ __forceinline__ bool in_domain() const {
-    uint32_t qmax = 0, phi = 0, plo = 0;
-#pragma unroll
-    for (int k = 0; k < 2; k++) qmax = max(qmax, max(max(q[k].x, q[k].y), max(q[k].z, q[k].w)));
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      plo |= p[k].x | p[k].z;
-      phi |= p[k].y | p[k].w;
-    }
-    return qmax <= 6300u && phi == 0 && (plo & 0xFF000000u) == 0 && ((d.x | d.y | x.x | x.y) & 0xF0F0F0F0u) == 0;
-  }
   // Character flags encode to slots 0..5 only.
   __device__ __forceinline__ static constexpr uint32_t bad_codes() { return 0; }
   __device__ __forceinline__ void drop_bad_codes() {}
@@ -467,16 +420,6 @@ struct UncompressedTile {
     r.disc = byte8(d, j);
     r.tax = byte8(x, j);
     r.price = comp(p[j >> 1], 2 * (j & 1));
-    return r;
-  }
-  __device__ __forceinline__ WideRow wide(int j, int32_t cut, uint32_t valid) const {
-    WideRow r;
-    const bool ok = (valid >> j & 1) && pass(j, cut);
-    r.gid = ok ? gid(j) : kNoGroup;
-    r.qty = (int32_t)comp(q[j >> 2], j & 3);
-    r.disc = (int8_t)byte8(d, j);
-    r.tax = (int8_t)byte8(x, j);
-    r.price = (int64_t)((uint64_t)comp(p[j >> 1], 2 * (j & 1) + 1) << 32 | comp(p[j >> 1], 2 * (j & 1)));
     return r;
   }
 };
@@ -529,12 +472,6 @@ struct UncompressedStreamTile {
     return encode_return_flag(byte(rf, j)) << 1 | encode_line_status(byte(ls, j));
   }
   __device__ __forceinline__ bool pass(int j, int32_t cut) const { return (int32_t)comp(s, j) <= cut; }
-  // Every row inside the TPC-H value domain (discount, tax in [0, 15], quantity in
-  // [0, 6300] hundredths, price in [0, 2^24)); rows zeroed by load_edge pass.
-  __device__ __forceinline__ bool in_domain() const {
-    return max(q.x, q.y) <= 6300u && (p.y | p.w) == 0 && ((p.x | p.z) & 0xFF000000u) == 0 &&
-           ((d | x) & 0xF0F0u) == 0;
-  }
   // Character flags encode to slots 0..5 only.
   __device__ __forceinline__ static constexpr uint32_t bad_codes() { return 0; }
   __device__ __forceinline__ void drop_bad_codes() {}
@@ -555,10 +492,11 @@ struct UncompressedStreamTile {
     r.price = comp(p, 2 * j);
     return r;
   }
+  template <bool EDGE>
   __device__ __forceinline__ WideRow wide(int j, int32_t cut, uint32_t valid) const {
     WideRow r;
-    const bool ok = (valid >> j & 1) && pass(j, cut);
-    r.gid = ok ? gid(j) : kNoGroup;
+    r.pass = EDGE ? ((valid >> j & 1) && pass(j, cut)) : pass(j, cut);
+    r.gid = gid(j);
     r.qty = (int32_t)comp(q, j);
     r.disc = (int8_t)byte(d, j);
     r.tax = (int8_t)byte(x, j);
@@ -621,19 +559,6 @@ struct ReferenceTile {
     return encode_return_flag((rf >> (8 * j)) & 0xFFu) << 1 | encode_line_status((ls >> (8 * j)) & 0xFFu);
   }
   __device__ __forceinline__ bool pass(int j, int32_t cut) const { return (int32_t)comp(s, j) <= cut; }
-  // Every row inside the TPC-H value domain (int64 discount, tax in [0, 15], quantity in
-  // [0, 6300], price in [0, 2^24)); rows zeroed by load_edge pass.
-  __device__ __forceinline__ bool in_domain() const {
-    uint32_t hi = 0, qmax = 0, plo = 0, dx = 0;
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-      hi |= q[k].y | q[k].w | p[k].y | p[k].w | d[k].y | d[k].w | x[k].y | x[k].w;
-      qmax = max(qmax, max(q[k].x, q[k].z));
-      plo |= p[k].x | p[k].z;
-      dx |= d[k].x | d[k].z | x[k].x | x[k].z;
-    }
-    return hi == 0 && qmax <= 6300u && (plo & 0xFF000000u) == 0 && (dx & ~15u) == 0;
-  }
   // Character flags encode to slots 0..5 only.
   __device__ __forceinline__ static constexpr uint32_t bad_codes() { return 0; }
   __device__ __forceinline__ void drop_bad_codes() {}
@@ -652,16 +577,6 @@ struct ReferenceTile {
     r.disc = lo32(d, j);
     r.tax = lo32(x, j);
     r.price = lo32(p, j);
-    return r;
-  }
-  __device__ __forceinline__ WideRow wide(int j, int32_t cut, uint32_t valid) const {
-    WideRow r;
-    const bool ok = (valid >> j & 1) && pass(j, cut);
-    r.gid = ok ? gid(j) : kNoGroup;
-    r.qty = get64(q, j);
-    r.disc = get64(d, j);
-    r.tax = get64(x, j);
-    r.price = get64(p, j);
     return r;
   }
 };
@@ -716,13 +631,6 @@ struct ReferenceStreamTile {
     return encode_return_flag((rf >> (8 * j)) & 0xFFu) << 1 | encode_line_status((ls >> (8 * j)) & 0xFFu);
   }
   __device__ __forceinline__ bool pass(int j, int32_t cut) const { return (int32_t)comp(s, j) <= cut; }
-  // Every row inside the TPC-H value domain (int64 discount, tax in [0, 15], quantity in
-  // [0, 6300], price in [0, 2^24)); rows zeroed by load_edge pass.
-  __device__ __forceinline__ bool in_domain() const {
-    const uint32_t hi = q.y | q.w | p.y | p.w | d.y | d.w | x.y | x.w;
-    return hi == 0 && max(q.x, q.z) <= 6300u && ((p.x | p.z) & 0xFF000000u) == 0 &&
-           ((d.x | d.z | x.x | x.z) & ~15u) == 0;
-  }
   // Character flags encode to slots 0..5 only.
   __device__ __forceinline__ static constexpr uint32_t bad_codes() { return 0; }
   __device__ __forceinline__ void drop_bad_codes() {}
@@ -743,10 +651,11 @@ struct ReferenceStreamTile {
     r.price = lo32(p, j);
     return r;
   }
+  template <bool EDGE>
   __device__ __forceinline__ WideRow wide(int j, int32_t cut, uint32_t valid) const {
     WideRow r;
-    const bool ok = (valid >> j & 1) && pass(j, cut);
-    r.gid = ok ? gid(j) : kNoGroup;
+    r.pass = EDGE ? ((valid >> j & 1) && pass(j, cut)) : pass(j, cut);
+    r.gid = gid(j);
     r.qty = get64(q, j);
     r.disc = get64(d, j);
     r.tax = get64(x, j);
@@ -880,6 +789,7 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
 // 2^28 over a tile; the product in the high half, below 16 * 15 * 2^24 < 2^32), so a row
 // costs three adds per group: that word, the packed count|discount|quantity and the charge.
 struct AccRegisters {
+  static constexpr bool kWideRows = false;
   uint32_t ns[kNumGroups];
   uint64_t npd[kNumGroups];
   uint64_t ch[kNumGroups], pr[kNumGroups], dp[kNumGroups];
@@ -968,6 +878,7 @@ __device__ __forceinline__ uint64_t small_to_small64(uint32_t s) {
 // of it (real data fills four of the six groups), and its four 64-bit adds run under the
 // lanes' mask: count, discount and quantity share one word (pack_small64).
 struct AccPerThread {
+  static constexpr bool kWideRows = false;
   uint64_t sm[kNumGroups], pr[kNumGroups], dp[kNumGroups], ch[kNumGroups];
   __device__ __forceinline__ void init(char*) {
 #pragma unroll
@@ -1018,6 +929,7 @@ struct AccPerThread {
 // 64 rows 1.46 ms, 256 rows 1.35 ms, 1024 rows 1.19 ms.
 constexpr uint32_t kLocalFlushRows = 1024;
 struct AccLocal {
+  static constexpr bool kWideRows = false;
   // Per group: narrow sums of at most 16 rows as in AccRegisters (pack_small word; price
   // and discount product in one 64-bit word), folded every 16 rows into 64-bit
   // register sums of at most kLocalFlushRows rows (count, discount and quantity in the
@@ -1135,7 +1047,7 @@ __device__ __forceinline__ void clear_wave_table(uint64_t* tab) {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Sums a wavefront's part of the table over its threads into red[wave][group][NF].  Lane 8g + k
+// Sums a wavefront's part of the table over its threads into red[wave][group][words].  Lane 8g + k
 // takes group g and threads k, k + 8, ... (rotated by g, so that the groups' reads fall on
 // different banks), then the eight lanes of a group are added with DPP.  All groups go at
 // once: about 200 vector instructions per wavefront, where a butterfly over all lanes for
@@ -1170,7 +1082,7 @@ __device__ __forceinline__ void sum_wave_table(const uint64_t* tab, uint64_t* re
     }
   }
   sums.reduce([](auto& v) { add_eight(v); });
-  if (g < kNumGroups && k == 0) sums.store(red + (wave * kNumGroups + g) * NF);
+  if (g < kNumGroups && k == 0) sums.store(red + (wave * kNumGroups + g) * GroupSums::kWords);
 }
 
 // Q1_PLACE_PER_THREAD_SHARED_MEM: each lane owns a table in LDS laid out
@@ -1185,6 +1097,7 @@ constexpr uint32_t shared_table_bytes(uint32_t threads) { return 4u * kNumGroups
 // register pair to build per row); the slot's high word stays zero.
 template <int B, bool NARROW = false>
 struct AccShared {
+  static constexpr bool kWideRows = false;
   uint64_t* tab;  // dynamic LDS: 6 * 4 * B words
   __device__ __forceinline__ void init(char* lds) {
     tab = reinterpret_cast<uint64_t*>(lds);
@@ -1209,6 +1122,7 @@ struct AccShared {
   // packed word fits its fields for NARROW tables (count <= 64 * 256, discount < 2^18,
   // quantity <= 64 * 256 * 6300 < 2^27); the others take the fields apart first.
   struct GroupSums {
+    static constexpr int kWords = NF;
     uint64_t small = 0, price = 0, dprod = 0, charge = 0;
     uint32_t cnt = 0, disc = 0;
     uint64_t qty = 0;
@@ -1251,17 +1165,6 @@ struct AccShared {
     }
   };
   __device__ __forceinline__ void wave_totals(uint64_t* red) const { sum_wave_table<B, 4, GroupSums>(tab, red); }
-  // The lane's own sums (scan_any and scan_wide add their wide ones to them).
-  __device__ __forceinline__ void totals(LaneTotals& o, char*) const {
-#pragma unroll
-    for (int g = 0; g < kNumGroups; g++) {
-      const uint64_t* base = tab + g * (4 * B) + thread_index();
-      unpack_small64(base[0], o.v[g]);
-      o.v[g][F_PRICE] = base[B];
-      o.v[g][F_DPROD] = base[2 * B];
-      o.v[g][F_CHARGE] = base[3 * B];
-    }
-  }
   static constexpr uint32_t lds_bytes(uint32_t) { return shared_table_bytes(B); }
 };
 
@@ -1278,6 +1181,7 @@ constexpr uint32_t packed_table_bytes(uint32_t threads) { return 3u * kNumGroups
 
 template <int B>
 struct AccSharedPacked {
+  static constexpr bool kWideRows = false;
   uint64_t* tab;  // dynamic LDS: 6 * 3 * B words
   __device__ __forceinline__ void init(char* lds) {
     tab = reinterpret_cast<uint64_t*>(lds);
@@ -1298,6 +1202,7 @@ struct AccSharedPacked {
   // The wavefront's sums of one group's words (sum_wave_table): slot 0 is taken apart, slot
   // 1's fields hold a wavefront's sums (product < 2^42, count <= 64 * 256).
   struct GroupSums {
+    static constexpr int kWords = NF;
     uint64_t price = 0, dprod_cnt = 0, charge = 0;
     uint32_t disc = 0, qty = 0;
     __device__ __forceinline__ void add(const uint64_t (&w)[3]) {
@@ -1340,6 +1245,7 @@ struct AccSharedPacked {
 // fits 64 bits (price < 2^46, discount product < 2^50, charge < 2^60).
 __device__ __forceinline__ void atomic_add128(uint64_t* lo_p, uint64_t* hi_p, uint64_t lo, uint64_t hi);
 struct AccGlobal {
+  static constexpr bool kWideRows = false;
   static constexpr int W = 5;  // words per group: count|disc, qty, price, dprod, charge
   AccRegisters regs;
   uint64_t* tab;               // [W][6] words of this block
@@ -1577,6 +1483,21 @@ __device__ __forceinline__ void finish_scan(const ScanArgs& a) {
 // ------------------------------------------------------------------------------------
 // Row bodies of one tile group.
 // ------------------------------------------------------------------------------------
+// Row j of a tile into an accumulator, in the row form the accumulator takes.  SLOT: the
+// caller knows that the row's slot is below 6.
+template <bool EDGE, bool SLOT, class Tile, class Acc>
+__device__ __forceinline__ void add_row(const Tile& tile, int j, Acc& acc, int32_t cut, uint32_t valid) {
+  if constexpr (Acc::kWideRows) {
+    const WideRow r = tile.template wide<EDGE>(j, cut, valid);
+    if (SLOT) __builtin_assume(r.gid < kNumGroups);
+    acc.add(r);
+  } else {
+    const FastRow r = tile.template fast<EDGE>(j, cut, valid);
+    if (SLOT) __builtin_assume(r.gid < kNumGroups);
+    acc.add(r);
+  }
+}
+
 // A whole group inside the range.  Rows with the unused return-flag code are first made
 // to fail the filter (a wavefront-uniform branch that real data never takes), so every
 // row's slot is below 6 and the slot test drops out of the row body.
@@ -1593,11 +1514,7 @@ __device__ __forceinline__ void add_whole_group(TileGroup<Tile, U>& grp, Acc& ac
 #pragma unroll
   for (int m = 0; m < U; m++)
 #pragma unroll
-    for (int j = 0; j < TILE; j++) {
-      const FastRow r = grp.tile[m].template fast<false>(j, cut, 0);
-      __builtin_assume(r.gid < kNumGroups);
-      acc.add(r);
-    }
+    for (int j = 0; j < TILE; j++) add_row<false, true>(grp.tile[m], j, acc, cut, 0);
 }
 
 // Any group: tiles may be unused, or partial at the range's ends.
@@ -1608,19 +1525,64 @@ __device__ __forceinline__ void add_any_group(const TileGroup<Tile, U>& grp, Acc
 #pragma unroll
     for (int m = 0; m < U; m++)
 #pragma unroll
-      for (int j = 0; j < TILE; j++) acc.add(grp.tile[m].template fast<false>(j, cut, 0));
+      for (int j = 0; j < TILE; j++) add_row<false, false>(grp.tile[m], j, acc, cut, 0);
   } else {
 #pragma unroll
     for (int m = 0; m < U; m++) {
       if (!grp.use[m]) continue;
       if (!grp.edge[m]) {
 #pragma unroll
-        for (int j = 0; j < TILE; j++) acc.add(grp.tile[m].template fast<false>(j, cut, 0));
+        for (int j = 0; j < TILE; j++) add_row<false, false>(grp.tile[m], j, acc, cut, 0);
       } else {
 #pragma unroll
-        for (int j = 0; j < TILE; j++) acc.add(grp.tile[m].template fast<true>(j, cut, grp.valid[m]));
+        for (int j = 0; j < TILE; j++) add_row<true, false>(grp.tile[m], j, acc, cut, grp.valid[m]);
       }
     }
+  }
+}
+
+// The tiles base + k * B + lane (k < tiles_per_thread) of a block's lanes into an LDS table.
+// Groups k in [k_lo, k_end) are whole and inside the range for every lane of the
+// block: the tiles of group k are base + (k + m) * B + lane, and they all lie in
+// [whole_begin, whole_end), the tiles with no row outside [row_begin, row_end).  They
+// run a branch-free body; the few others (the range's first and last groups) a
+// guarded one.  A dropped row's ship date 0xFFFF must fail the filter: compressed
+// cutoffs of 65535 and above (beyond the year 2170) take the guarded body throughout.
+template <int L, class Tile, int B, class Acc>
+__device__ __forceinline__ void add_tiles(const ScanArgs& a, uint64_t base, uint32_t tiles_per_thread, Acc& acc,
+                                          int32_t cut) {
+  constexpr int TILE = Tile::TILE;
+  constexpr int U = Tile::GROUP;
+  const uint64_t end_tile = (a.row_end + TILE - 1) / TILE;
+  const uint64_t whole_begin = (a.row_begin + TILE - 1) / TILE, whole_end = a.row_end / TILE;
+  uint32_t k_lo = 0, k_end = 0;
+  if ((L != Q1_LAYOUT_COMPRESSED || cut < 65535) && whole_end > base) {
+    const uint64_t lo = base >= whole_begin ? 0 : (whole_begin - base + B - 1) / B;
+    const uint64_t klo = (lo + U - 1) / U * U;
+    uint64_t kmax = (whole_end - base) / B;  // groups with k + U <= kmax are inside
+    if (kmax > tiles_per_thread) kmax = tiles_per_thread;
+    if (kmax >= klo + U) {
+      k_lo = (uint32_t)klo;
+      k_end = (uint32_t)(klo + (kmax - klo) / U * U);
+    }
+  }
+  uint32_t k = 0;
+  for (; k < k_lo; k += U) {
+    TileGroup<Tile, U> grp;
+    grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
+             a.row_end);
+    add_any_group(grp, acc, cut);
+  }
+  for (; k < k_end; k += U) {
+    TileGroup<Tile, U> grp;
+    grp.load_plain(a.cols, base + (uint64_t)k * B + thread_index(), B);
+    add_whole_group(grp, acc, cut);
+  }
+  for (; k < tiles_per_thread; k += U) {
+    TileGroup<Tile, U> grp;
+    grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
+             a.row_end);
+    add_any_group(grp, acc, cut);
   }
 }
 
@@ -1661,45 +1623,7 @@ __device__ __forceinline__ void scan_block(const ScanArgs& a, uint64_t block, ui
 
   constexpr bool kSplit = P == Q1_PLACE_PER_THREAD_SHARED_MEM || P == kPlaceSharedNarrow || P == kPlaceSharedPacked;
   if constexpr (kSplit) {
-    // Groups k in [k_lo, k_end) are whole and inside the range for every lane of the
-    // block: the tiles of group k are base + (k + m) * B + lane, and they all lie in
-    // [whole_begin, whole_end), the tiles with no row outside [row_begin, row_end).  They
-    // run a branch-free body; the few others (the range's first and last groups) a
-    // guarded one.  A dropped row's ship date 0xFFFF must fail the filter: compressed
-    // cutoffs of 65535 and above (beyond the year 2170) take the guarded body throughout.
-    const uint64_t whole_begin = (a.row_begin + TILE - 1) / TILE, whole_end = a.row_end / TILE;
-    uint32_t k_lo = 0, k_end = 0;
-    if ((L != Q1_LAYOUT_COMPRESSED || cut < 65535) && whole_end > base) {
-      const uint64_t lo = base >= whole_begin ? 0 : (whole_begin - base + B - 1) / B;
-      const uint64_t klo = (lo + U - 1) / U * U;
-      uint64_t kmax = (whole_end - base) / B;  // groups with k + U <= kmax are inside
-      if (kmax > tiles_per_thread) kmax = tiles_per_thread;
-      if (kmax >= klo + U) {
-        k_lo = (uint32_t)klo;
-        k_end = (uint32_t)(klo + (kmax - klo) / U * U);
-      }
-    }
-    uint32_t k = 0, n = 0;
-    for (; k < k_lo; k += U, n++) {
-      TileGroup<Tile, U> grp;
-      grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
-               a.row_end);
-      add_any_group(grp, acc, cut);
-      if ((n + 1) % FLUSH == 0) acc.flush();  // at most 16 rows per lane between flushes
-    }
-    for (; k < k_end; k += U, n++) {
-      TileGroup<Tile, U> grp;
-      grp.load_plain(a.cols, base + (uint64_t)k * B + thread_index(), B);
-      add_whole_group(grp, acc, cut);
-      if ((n + 1) % FLUSH == 0) acc.flush();
-    }
-    for (; k < tiles_per_thread; k += U, n++) {
-      TileGroup<Tile, U> grp;
-      grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
-               a.row_end);
-      add_any_group(grp, acc, cut);
-      if ((n + 1) % FLUSH == 0) acc.flush();
-    }
+    add_tiles<L, Tile, B>(a, base, tiles_per_thread, acc, cut);
   } else {
     // The register-table placements keep one guarded loop: a second copy of the row body
     // costs them registers (spills, lower occupancy) that the saved instructions do not
@@ -1760,382 +1684,284 @@ scan_fast(ScanArgs a, uint32_t host_tiles_per_thread, uint64_t* ws) {
 }
 
 // ------------------------------------------------------------------------------------
-// The any-value scan kernel (tables outside the TPC-H domain, and q1_enqueue without
+// The any-value scan kernel (tables outside the TPC-H domain, and launches without
 // Q1_LAUNCH_ASSUME_TPCH_DOMAIN): exact for every input with the reference's arithmetic,
-// wrapping int64 per-row products and 128-bit signed sums.  Each lane tests its tile:
-// a tile whose rows all lie inside the TPC-H value domain goes through the narrow
-// per-lane LDS table of the shared placement (exact there: no product can wrap); any
-// other tile goes through a per-lane 64-bit register table.  At the end the narrow table
-// is folded into the wide one (disc_price = 100 * price - disc * price, all
-// non-negative), and the block merges in 128 bits.  In-domain data runs at the speed of
-// the narrow kernel; a wavefront pays for the wide path only on tiles that need it.
+// wrapping int64 per-row products and 128-bit signed sums, whatever the values.  It is the
+// shared placement's kernel with LDS tables whose words hold any value of the layout's
+// types, so a row takes the same branch-free path inside and outside the domain: streaming
+// tiles, 3 (compressed), 5 (uncompressed) or 7 (reference) return-less 64-bit LDS atomics.
+// The fields of a word are exact for any_value_lane_rows rows per lane, which make_shape
+// keeps to.
+// Bound by HBM, as the narrow kernel: 600M compressed rows 0.82-0.84 ms (narrow 0.83), 60M
+// uncompressed 190 us, 60M reference 341 us (6.7 TB/s).  Testing each tile for the domain and
+// sending the others to 128-bit sums in registers or private memory took 281 us for 60M
+// compressed rows with two thirds of them outside (now 93), and 27 us for a 1M-row launch,
+// whose blocks each reduced both kinds of sums (now 12).
 // ------------------------------------------------------------------------------------
-struct Wide128 {
-  uint64_t lo;
-  uint64_t hi;
-  __device__ __forceinline__ void add64s(int64_t v) {
-    const uint64_t nlo = lo + (uint64_t)v;
-    hi += (uint64_t)(v >> 63) + (nlo < lo);
-    lo = nlo;
+// A wavefront's sums of one group in red[wave][group][NA]: 64-bit (wrapping, as the
+// reference's int64 sums), the products as 128-bit word pairs.
+enum { A_QTY, A_PRICE, A_DISC, A_CNT, A_DP_LO, A_DP_HI, A_CH_LO, A_CH_HI, NA };
+
+__device__ __forceinline__ void store_i128(uint64_t* lo_hi, __int128 v) {
+  lo_hi[0] = (uint64_t)v;
+  lo_hi[1] = (uint64_t)((unsigned __int128)v >> 64);
+}
+// The two halves of the sum of up to 2^23 int64 values, split into unsigned low and signed
+// high 32-bit words.
+__device__ __forceinline__ __int128 join_i128(uint64_t lo_sum, int64_t hi_sum) {
+  return (__int128)hi_sum * ((__int128)1 << 32) + (__int128)lo_sum;
+}
+// a word's signed sum in bits [0,40) and the rest of it, sum >> 40 (below 2^24)
+__device__ __forceinline__ int64_t low40(uint64_t w) { return (int64_t)(w << 24) >> 24; }
+__device__ __forceinline__ uint32_t high24(uint64_t w) { return (uint32_t)((w - (uint64_t)low40(w)) >> 40); }
+
+// Compressed layouts: quantity, discount and tax are bytes and the price has 32 bits, so every
+// product fits 64 bits and a lane's sums over 128 rows fit three words:
+//   word 0: price (< 2^39) in bits [0,39), discount (< 2^15) in [39,54), count in [54,62)
+//   word 1: discount x price (< 2^47) in [0,47), quantity (< 2^15) in [47,62)
+//   word 2: (f + 55025) x price, f = (100 - discount)(100 + tax) in [-55025, 35500] (< 2^56)
+// Two multiplications a row beyond the narrow table's, both with a 64-bit result.
+template <int B>
+struct AnyCompressed {
+  static constexpr bool kWideRows = false;
+  static constexpr int W = 3;
+  static_assert(any_value_lane_rows(Q1_LAYOUT_COMPRESSED) <= 128, "the fields' widths");
+  static constexpr uint32_t kFactorBias = 55025;
+  uint64_t* tab;
+  __device__ __forceinline__ void init(uint64_t* lds) {
+    tab = lds;
+    clear_wave_table<B, W>(tab);
   }
-};
-
-// The sums of one slot for rows outside the TPC-H domain: 64-bit (wrapping, as the
-// reference's int64 sums) and 128-bit products.
-struct WideSums {
-  uint64_t qty, price, disc, cnt;
-  Wide128 dp, ch;
-};
-
-template <class Tile>
-__device__ __forceinline__ void add_wide_rows(const Tile& tile, WideSums* wide, int32_t cut, uint32_t valid) {
-#pragma unroll
-  for (int j = 0; j < Tile::TILE; j++) {
-    const WideRow r = tile.wide(j, cut, valid);
-    if (r.gid < kNumGroups) {
-      const int64_t disc_1 = (int64_t)(100ull - (uint64_t)r.disc);
-      const int64_t disc_price = (int64_t)((uint64_t)disc_1 * (uint64_t)r.price);
-      const int64_t charge = (int64_t)((uint64_t)disc_price * (uint64_t)(r.tax + 100));
-      WideSums& t = wide[r.gid];
-      t.qty += (uint64_t)r.qty;
-      t.price += (uint64_t)r.price;
-      t.disc += (uint64_t)r.disc;
-      t.cnt += 1;
-      t.dp.add64s(disc_price);
-      t.ch.add64s(charge);
+  __device__ __forceinline__ void add(const FastRow& r) {
+    if (__builtin_expect(r.counts(), 1)) {
+      uint64_t* base = tab + r.gid * (W * B) + thread_index();
+      const uint32_t f = (uint32_t)(__mul24(100 - (int)r.disc, 100 + (int)r.tax) + (int)kFactorBias);
+      const uint64_t w0 = (uint64_t)r.price | (uint64_t)(r.disc << 7 | 1u << 22) << 32;
+      const uint64_t w1 = (uint64_t)r.disc * r.price + ((uint64_t)(r.qty << 15) << 32);
+      __hip_atomic_fetch_add(base, w0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_fetch_add(base + B, w1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_fetch_add(base + 2 * B, (uint64_t)f * r.price, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
   }
+  struct GroupSums {
+    static constexpr int kWords = NA;
+    uint64_t price = 0, dprod = 0, charge = 0;
+    uint32_t disc = 0, cnt = 0, qty = 0;
+    __device__ __forceinline__ void add(const uint64_t (&w)[W]) {
+      price += w[0] & ((1ull << 39) - 1);
+      disc += (uint32_t)(w[0] >> 39) & 0x7FFFu;
+      cnt += (uint32_t)(w[0] >> 54);
+      dprod += w[1] & ((1ull << 47) - 1);
+      qty += (uint32_t)(w[1] >> 47);
+      charge += w[2];
+    }
+    template <class F>
+    __device__ __forceinline__ void reduce(F f) {
+      f(price);
+      f(disc);
+      f(cnt);
+      f(dprod);
+      f(qty);
+      f(charge);
+    }
+    // over a wavefront: price < 2^45, discount x price < 2^53, word 2 < 2^62
+    __device__ __forceinline__ void store(uint64_t* r) const {
+      r[A_QTY] = qty;
+      r[A_PRICE] = price;
+      r[A_DISC] = disc;
+      r[A_CNT] = cnt;
+      store_i128(r + A_DP_LO, (__int128)((int64_t)(100 * price) - (int64_t)dprod));
+      store_i128(r + A_CH_LO, (__int128)((int64_t)charge - (int64_t)(kFactorBias * price)));
+    }
+  };
+  __device__ __forceinline__ void wave_totals(uint64_t* red) const { sum_wave_table<B, W, GroupSums>(tab, red); }
+  static constexpr uint32_t lds_bytes(uint32_t threads) { return W * kNumGroups * 8u * threads; }
+};
+
+// A wrapping 64-bit product whose second factor is a signed 32-bit value.
+__device__ __forceinline__ uint64_t mul_64_s32(uint64_t a, int32_t f) {
+  const uint32_t lo = (uint32_t)a, hi = (uint32_t)(a >> 32);
+  const uint64_t p = (uint64_t)lo * (uint32_t)f;
+  const uint32_t top = (uint32_t)(p >> 32) + hi * (uint32_t)f - (f < 0 ? lo : 0u);
+  return (uint64_t)top << 32 | (uint32_t)p;
 }
 
-// A group of tiles some of whose rows may lie outside the domain: each lane sends each of
-// its tiles to the narrow LDS table or to its wide table.
-template <class Tile, int U, class Acc>
-__device__ __forceinline__ void add_group_any_value(const TileGroup<Tile, U>& grp, Acc& narrow, WideSums* wide,
-                                                    bool& wide_used, int32_t cut, bool whole) {
-  constexpr int TILE = Tile::TILE;
+// Uncompressed layout: int64 price, int32 quantity, int8 discount and tax; the products are
+// split into unsigned low and signed high halves.  A lane's sums over 256 rows fit five words:
+//   word 0: low halves of disc_price (< 2^40) in bits [0,48), count in [48,57)
+//   word 1: high halves of disc_price (signed) in [0,40), discount + 128 in [40,56)
+//   word 2: low halves of charge in [0,40), low half-word of quantity in [40,64)
+//   word 3: high halves of charge (signed) in [0,40), high half-word of quantity + 2^15 in [40,64)
+//   word 4: price (wrapping)
+template <int B>
+struct AnyUncompressed {
+  static constexpr bool kWideRows = true;
+  static constexpr int W = 5;
+  static_assert(any_value_lane_rows(Q1_LAYOUT_UNCOMPRESSED) <= 256, "the fields' widths");
+  uint64_t* tab;
+  __device__ __forceinline__ void init(uint64_t* lds) {
+    tab = lds;
+    clear_wave_table<B, W>(tab);
+  }
+  __device__ __forceinline__ void add(const WideRow& r) {
+    if (__builtin_expect(r.counts(), 1)) {
+      uint64_t* base = tab + r.gid * (W * B) + thread_index();
+      const int32_t disc = (int32_t)r.disc, qty = (int32_t)r.qty, d1 = 100 - disc;
+      const uint64_t dp = mul_64_s32((uint64_t)r.price, d1);
+      const uint64_t ch = mul_64_s32((uint64_t)r.price, __mul24(d1, 100 + (int32_t)r.tax));
+      const uint64_t w[W] = {(uint64_t)(uint32_t)dp | 1ull << 48,
+                             (uint64_t)((int64_t)dp >> 32) + ((uint64_t)(uint32_t)(disc + 128) << 40),
+                             (uint64_t)(uint32_t)ch | (uint64_t)((uint32_t)qty & 0xFFFFu) << 40,
+                             (uint64_t)((int64_t)ch >> 32) + ((uint64_t)(uint32_t)((qty >> 16) + 32768) << 40),
+                             (uint64_t)r.price};
 #pragma unroll
-  for (int m = 0; m < U; m++) {
-    if (!whole && !grp.use[m]) continue;
-    const Tile& tile = grp.tile[m];
-    const bool edge = !whole && grp.edge[m];
-    const uint32_t valid = whole ? (1u << TILE) - 1 : grp.valid[m];
-    if (tile.in_domain()) {
-      if (!edge) {
-#pragma unroll
-        for (int j = 0; j < TILE; j++) narrow.add(tile.template fast<false>(j, cut, 0));
-      } else {
-#pragma unroll
-        for (int j = 0; j < TILE; j++) narrow.add(tile.template fast<true>(j, cut, valid));
-      }
-    } else {
-      if (!wide_used) {  // the lane's first row outside the domain
-#pragma unroll
-        for (int g = 0; g < kNumGroups; g++) wide[g] = WideSums{0, 0, 0, 0, {0, 0}, {0, 0}};
-        wide_used = true;
-      }
-      add_wide_rows(tile, wide, cut, valid);
+      for (int i = 0; i < W; i++)
+        __hip_atomic_fetch_add(base + i * B, w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
+  }
+  struct GroupSums {
+    static constexpr int kWords = NA;
+    uint64_t dp_lo_cnt = 0, dp_hi = 0, ch_lo = 0, ch_hi = 0, price = 0;
+    uint32_t disc = 0, qty_lo = 0, qty_hi = 0;
+    __device__ __forceinline__ void add(const uint64_t (&w)[W]) {
+      dp_lo_cnt += w[0];  // a wavefront's sums fit the fields
+      dp_hi += (uint64_t)low40(w[1]);
+      disc += high24(w[1]);
+      ch_lo += w[2] & ((1ull << 40) - 1);
+      qty_lo += (uint32_t)(w[2] >> 40);
+      ch_hi += (uint64_t)low40(w[3]);
+      qty_hi += high24(w[3]);
+      price += w[4];
+    }
+    template <class F>
+    __device__ __forceinline__ void reduce(F f) {
+      f(dp_lo_cnt);
+      f(dp_hi);
+      f(disc);
+      f(ch_lo);
+      f(qty_lo);
+      f(ch_hi);
+      f(qty_hi);
+      f(price);
+    }
+    __device__ __forceinline__ void store(uint64_t* r) const {
+      const int64_t cnt = (int64_t)(dp_lo_cnt >> 48);
+      r[A_QTY] = (uint64_t)((int64_t)qty_lo + ((int64_t)qty_hi - 32768 * cnt) * 65536);
+      r[A_PRICE] = price;
+      r[A_DISC] = (uint64_t)((int64_t)disc - 128 * cnt);
+      r[A_CNT] = (uint64_t)cnt;
+      store_i128(r + A_DP_LO, join_i128(dp_lo_cnt & ((1ull << 48) - 1), (int64_t)dp_hi));
+      store_i128(r + A_CH_LO, join_i128(ch_lo, (int64_t)ch_hi));
+    }
+  };
+  __device__ __forceinline__ void wave_totals(uint64_t* red) const { sum_wave_table<B, W, GroupSums>(tab, red); }
+  static constexpr uint32_t lds_bytes(uint32_t threads) { return W * kNumGroups * 8u * threads; }
+};
+
+// Reference layout: every value int64.  Seven words: low halves of disc_price with the count
+// in bits [48,57), its high halves, low and high halves of charge, and the wrapping sums of
+// price, quantity and discount.
+template <int B>
+struct AnyReference {
+  static constexpr bool kWideRows = true;
+  static constexpr int W = 7;
+  static_assert(any_value_lane_rows(Q1_LAYOUT_REFERENCE) <= 256, "the fields' widths");
+  uint64_t* tab;
+  __device__ __forceinline__ void init(uint64_t* lds) {
+    tab = lds;
+    clear_wave_table<B, W>(tab);
+  }
+  __device__ __forceinline__ void add(const WideRow& r) {
+    if (__builtin_expect(r.counts(), 1)) {
+      uint64_t* base = tab + r.gid * (W * B) + thread_index();
+      const uint64_t dp = (100ull - (uint64_t)r.disc) * (uint64_t)r.price;
+      const uint64_t ch = dp * (100ull + (uint64_t)r.tax);
+      const uint64_t w[W] = {(uint64_t)(uint32_t)dp | 1ull << 48, (uint64_t)((int64_t)dp >> 32),
+                             (uint64_t)(uint32_t)ch,              (uint64_t)((int64_t)ch >> 32),
+                             (uint64_t)r.price,                   (uint64_t)r.qty,
+                             (uint64_t)r.disc};
+#pragma unroll
+      for (int i = 0; i < W; i++)
+        __hip_atomic_fetch_add(base + i * B, w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  }
+  struct GroupSums {
+    static constexpr int kWords = NA;
+    uint64_t w[W] = {};
+    __device__ __forceinline__ void add(const uint64_t (&v)[W]) {
+#pragma unroll
+      for (int i = 0; i < W; i++) w[i] += v[i];
+    }
+    template <class F>
+    __device__ __forceinline__ void reduce(F f) {
+#pragma unroll
+      for (int i = 0; i < W; i++) f(w[i]);
+    }
+    __device__ __forceinline__ void store(uint64_t* r) const {
+      r[A_QTY] = w[5];
+      r[A_PRICE] = w[4];
+      r[A_DISC] = w[6];
+      r[A_CNT] = w[0] >> 48;
+      store_i128(r + A_DP_LO, join_i128(w[0] & ((1ull << 48) - 1), (int64_t)w[1]));
+      store_i128(r + A_CH_LO, join_i128(w[2], (int64_t)w[3]));
+    }
+  };
+  __device__ __forceinline__ void wave_totals(uint64_t* red) const { sum_wave_table<B, W, GroupSums>(tab, red); }
+  static constexpr uint32_t lds_bytes(uint32_t threads) { return W * kNumGroups * 8u * threads; }
+};
+
+template <int L, int B> struct AnyOf { using A = AnyCompressed<B>; };
+template <int B> struct AnyOf<Q1_LAYOUT_UNCOMPRESSED, B> { using A = AnyUncompressed<B>; };
+template <int B> struct AnyOf<Q1_LAYOUT_REFERENCE, B> { using A = AnyReference<B>; };
+
+// The block's merge: thread 8g + i of wavefront 0 adds word (or word pair) i of group g over
+// the wavefronts and issues its atomics.
+template <int B>
+__device__ __forceinline__ void any_merge(const uint64_t* red, q1_device_aggregates* out, uint64_t qty_scale) {
+  __syncthreads();
+  const uint32_t g = thread_index() >> 3, f = thread_index() & 7;
+  if (g >= kNumGroups || f == A_DP_HI || f == A_CH_HI) return;
+  const bool pair = f == A_DP_LO || f == A_CH_LO;
+  uint64_t lo = 0, hi = 0;
+#pragma unroll
+  for (int w = 0; w < B / 64; w++) {
+    const uint64_t* r = red + (w * kNumGroups + g) * NA + f;
+    lo += r[0];
+    if (pair) hi += r[1] + (lo < r[0]);
+  }
+  if (f == A_QTY) lo *= qty_scale;
+  if (pair) {
+    atomic_add128(f == A_DP_LO ? &out->sum_disc_price_lo[g] : &out->sum_charge_lo[g],
+                  f == A_DP_LO ? &out->sum_disc_price_hi[g] : &out->sum_charge_hi[g], lo, hi);
+  } else if (lo) {
+    uint64_t* d = f == A_QTY     ? out->sum_qty
+                  : f == A_PRICE ? out->sum_base_price
+                  : f == A_DISC  ? out->sum_disc
+                                 : out->count;
+    atomicAdd((unsigned long long*)(d + g), (unsigned long long)lo);
   }
 }
 
 template <int L, int B>
 __global__ void __launch_bounds__(B)
 scan_any(ScanArgs a, uint32_t host_tiles_per_thread) {
-  begin_scan(a);
-  // The LDS placement's streaming tiles; the host counts tiles of TileOf<L>.
   using Tile = typename ScanTileOf<L, kPlaceSharedNarrow>::T;
+  using Acc = typename AnyOf<L, B>::A;
   constexpr int TILE = Tile::TILE;
-  constexpr int U = Tile::GROUP;
-  constexpr int SUB = TileOf<L>::T::TILE / TILE;
+  constexpr int SUB = TileOf<L>::T::TILE / TILE;  // the host counts tiles of TileOf<L>
+  constexpr uint64_t kQtyScale =
+      (L == Q1_LAYOUT_COMPRESSED || L == Q1_LAYOUT_COMPRESSED_PUSHDOWN) ? kQuantityScaleCompressed : 1;
   extern __shared__ uint64_t lds[];
-
-  const uint32_t tiles_per_thread = host_tiles_per_thread * SUB;
-  const int32_t cut = column_cutoff<L>(a.cutoff_day);
-  const uint64_t first_tile = a.row_begin / kRowAlign * kRowAlign / TILE;  // as the host counts them
-  const uint64_t end_tile = (a.row_end + TILE - 1) / TILE;
-  const uint64_t base = first_tile + (uint64_t)blockIdx.x * B * tiles_per_thread;
-
-  AccShared<B> narrow;
-  narrow.init(reinterpret_cast<char*>(lds));
-  // Indexed by slot at run time, so it lives in the lane's private memory and costs no
-  // registers; only lanes with rows outside the domain clear, update and read it.
-  WideSums wide[kNumGroups];
-  bool wide_used = false;
-
-  // Whole groups as in scan_fast: when every row of a wavefront's group lies in the domain
-  // it takes the branch-free body; otherwise its lanes sort their tiles.
-  const uint64_t whole_begin = (a.row_begin + TILE - 1) / TILE, whole_end = a.row_end / TILE;
-  uint32_t k_lo = 0, k_end = 0;
-  if ((L != Q1_LAYOUT_COMPRESSED || cut < 65535) && whole_end > base) {
-    const uint64_t lo = base >= whole_begin ? 0 : (whole_begin - base + B - 1) / B;
-    const uint64_t klo = (lo + U - 1) / U * U;
-    uint64_t kmax = (whole_end - base) / B;
-    if (kmax > tiles_per_thread) kmax = tiles_per_thread;
-    if (kmax >= klo + U) {
-      k_lo = (uint32_t)klo;
-      k_end = (uint32_t)(klo + (kmax - klo) / U * U);
-    }
-  }
-  uint32_t k = 0;
-  for (; k < k_lo; k += U) {
-    TileGroup<Tile, U> grp;
-    grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
-             a.row_end);
-    add_group_any_value(grp, narrow, wide, wide_used, cut, false);
-  }
-  for (; k < k_end; k += U) {
-    TileGroup<Tile, U> grp;
-    grp.load_plain(a.cols, base + (uint64_t)k * B + thread_index(), B);
-    bool in = true;
-#pragma unroll
-    for (int m = 0; m < U; m++) in = in & grp.tile[m].in_domain();
-    if (ballot(!in) == 0)
-      add_whole_group(grp, narrow, cut);
-    else
-      add_group_any_value(grp, narrow, wide, wide_used, cut, true);
-  }
-  for (; k < tiles_per_thread; k += U) {
-    TileGroup<Tile, U> grp;
-    grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
-             a.row_end);
-    add_group_any_value(grp, narrow, wide, wide_used, cut, false);
-  }
-
-  uint64_t qty[kNumGroups], price[kNumGroups], disc[kNumGroups], cnt[kNumGroups];
-  Wide128 dp[kNumGroups], ch[kNumGroups];
-#pragma unroll
-  for (int g = 0; g < kNumGroups; g++) {
-    qty[g] = price[g] = disc[g] = cnt[g] = 0;
-    dp[g].lo = dp[g].hi = ch[g].lo = ch[g].hi = 0;
-  }
-  if (wide_used) {
-#pragma unroll
-    for (int g = 0; g < kNumGroups; g++) {
-      qty[g] = wide[g].qty;
-      price[g] = wide[g].price;
-      disc[g] = wide[g].disc;
-      cnt[g] = wide[g].cnt;
-      dp[g] = wide[g].dp;
-      ch[g] = wide[g].ch;
-    }
-  }
-
-  // Fold the lane's narrow table into its wide one.  Lane sums of the narrow table are
-  // exact and far below 2^63 (at most 16384 rows per lane).
-  {
-    LaneTotals nt;
-    narrow.totals(nt, reinterpret_cast<char*>(lds));
-#pragma unroll
-    for (int g = 0; g < kNumGroups; g++) {
-      qty[g] += nt.v[g][F_QTY];
-      price[g] += nt.v[g][F_PRICE];
-      disc[g] += nt.v[g][F_DISC];
-      cnt[g] += nt.v[g][F_CNT];
-      dp[g].add64s((int64_t)(100u * nt.v[g][F_PRICE] - nt.v[g][F_DPROD]));
-      ch[g].add64s((int64_t)nt.v[g][F_CHARGE]);
-    }
-  }
-
-  // Block merge in 128 bits for every field; the scratch follows the narrow table.
-  const uint32_t wave = thread_index() >> 6, lane = thread_index() & 63, nwaves = B >> 6;
-  constexpr int NW = 8;  // qty, price, disc, cnt, dp.lo, dp.hi, ch.lo, ch.hi
-  uint64_t* red = lds + shared_table_bytes(B) / 8;  // nwaves * 6 * NW words
-#pragma unroll
-  for (int g = 0; g < kNumGroups; g++) {
-    uint64_t s64[4] = {qty[g], price[g], disc[g], cnt[g]};
-    Wide128 w[2] = {dp[g], ch[g]};
-    if (ballot(cnt[g] != 0)) {
-#pragma unroll
-      for (int f = 0; f < 4; f++) s64[f] = wave_sum_u64(s64[f]);
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) {
-#pragma unroll
-        for (int f = 0; f < 2; f++) {
-          const uint64_t olo = __shfl_xor(w[f].lo, m, 64), ohi = __shfl_xor(w[f].hi, m, 64);
-          const uint64_t nlo = w[f].lo + olo;
-          w[f].hi += ohi + (nlo < olo);
-          w[f].lo = nlo;
-        }
-      }
-    } else {
-      s64[0] = s64[1] = s64[2] = s64[3] = 0;
-      w[0].lo = w[0].hi = w[1].lo = w[1].hi = 0;
-    }
-    if (lane == 0) {
-      uint64_t* r = red + (wave * kNumGroups + g) * NW;
-      r[0] = s64[0]; r[1] = s64[1]; r[2] = s64[2]; r[3] = s64[3];
-      r[4] = w[0].lo; r[5] = w[0].hi; r[6] = w[1].lo; r[7] = w[1].hi;
-    }
-  }
-  __syncthreads();
-  if (thread_index() < kNumGroups) {
-    const int g = thread_index();
-    uint64_t s[4] = {0, 0, 0, 0};
-    Wide128 w[2] = {{0, 0}, {0, 0}};
-    for (uint32_t v = 0; v < nwaves; v++) {
-      const uint64_t* r = red + (v * kNumGroups + g) * NW;
-      for (int f = 0; f < 4; f++) s[f] += r[f];
-      for (int f = 0; f < 2; f++) {
-        const uint64_t nlo = w[f].lo + r[4 + 2 * f];
-        w[f].hi += r[5 + 2 * f] + (nlo < w[f].lo);
-        w[f].lo = nlo;
-      }
-    }
-    if (s[3]) {
-      const uint64_t qs =
-          (L == Q1_LAYOUT_COMPRESSED || L == Q1_LAYOUT_COMPRESSED_PUSHDOWN) ? kQuantityScaleCompressed : 1;
-      q1_device_aggregates* out = a.out + (blockIdx.x & a.out_mask);
-      atomicAdd((unsigned long long*)&out->sum_qty[g], (unsigned long long)(s[0] * qs));
-      atomicAdd((unsigned long long*)&out->sum_base_price[g], (unsigned long long)s[1]);
-      atomicAdd((unsigned long long*)&out->sum_disc[g], (unsigned long long)s[2]);
-      atomicAdd((unsigned long long*)&out->count[g], (unsigned long long)s[3]);
-      atomic_add128(&out->sum_disc_price_lo[g], &out->sum_disc_price_hi[g], w[0].lo, w[0].hi);
-      atomic_add128(&out->sum_charge_lo[g], &out->sum_charge_hi[g], w[1].lo, w[1].hi);
-    }
-  }
-  finish_scan(a);
-}
-
-// The any-value kernel for tables known to hold values outside the domain (q1_run and the
-// server on such tables): 16-row tiles, each lane's tile tested as above, and the wide
-// sums in registers, so a table with every row outside the domain still runs at a few
-// times the fast kernel's time instead of the private-memory table's.
-template <int L, int B>
-__global__ void __launch_bounds__(B)
-scan_wide(ScanArgs a, uint32_t tiles_per_thread) {
   begin_scan(a);
-  using Tile = typename TileOf<L>::T;
-  constexpr int TILE = Tile::TILE;
-  extern __shared__ uint64_t lds[];
-
-  const int32_t cut = column_cutoff<L>(a.cutoff_day);
+  const uint32_t tiles_per_thread = host_tiles_per_thread * SUB;
   const uint64_t first_tile = a.row_begin / kRowAlign * kRowAlign / TILE;  // as the host counts them
-  const uint64_t end_tile = (a.row_end + TILE - 1) / TILE;
-  const uint64_t base = first_tile + (uint64_t)blockIdx.x * B * tiles_per_thread;
-
-  AccShared<B> narrow;
-  narrow.init(reinterpret_cast<char*>(lds));
-  uint64_t qty[kNumGroups], price[kNumGroups], disc[kNumGroups], cnt[kNumGroups];
-  Wide128 dp[kNumGroups], ch[kNumGroups];
-#pragma unroll
-  for (int g = 0; g < kNumGroups; g++) {
-    qty[g] = price[g] = disc[g] = cnt[g] = 0;
-    dp[g].lo = dp[g].hi = ch[g].lo = ch[g].hi = 0;
-  }
-
-  constexpr int U = Tile::GROUP;
-  for (uint32_t k = 0; k < tiles_per_thread; k += U) {
-    TileGroup<Tile, U> grp;
-    grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
-             a.row_end);
-#pragma unroll
-    for (int m = 0; m < U; m++) {
-      if (!grp.use[m]) continue;
-      const Tile& tile = grp.tile[m];
-      if (tile.in_domain()) {
-        if (!grp.edge[m]) {
-#pragma unroll
-          for (int j = 0; j < TILE; j++) narrow.add(tile.template fast<false>(j, cut, 0));
-        } else {
-#pragma unroll
-          for (int j = 0; j < TILE; j++) narrow.add(tile.template fast<true>(j, cut, grp.valid[m]));
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < TILE; j++) {
-          const WideRow r = tile.wide(j, cut, grp.valid[m]);
-          const int64_t disc_1 = (int64_t)(100ull - (uint64_t)r.disc);
-          const int64_t disc_price = (int64_t)((uint64_t)disc_1 * (uint64_t)r.price);
-          const int64_t charge = (int64_t)((uint64_t)disc_price * (uint64_t)(r.tax + 100));
-#pragma unroll
-          for (int g = 0; g < kNumGroups; g++) {
-            if (r.gid == (uint32_t)g) {
-              qty[g] += (uint64_t)r.qty;
-              price[g] += (uint64_t)r.price;
-              disc[g] += (uint64_t)r.disc;
-              cnt[g] += 1;
-              dp[g].add64s(disc_price);
-              ch[g].add64s(charge);
-            }
-          }
-        }
-      }
-    }
-  }
-
-  // Fold the lane's narrow table into its wide one.  Lane sums of the narrow table are
-  // exact and far below 2^63 (at most 16384 rows per lane).
-  {
-    LaneTotals nt;
-    narrow.totals(nt, reinterpret_cast<char*>(lds));
-#pragma unroll
-    for (int g = 0; g < kNumGroups; g++) {
-      qty[g] += nt.v[g][F_QTY];
-      price[g] += nt.v[g][F_PRICE];
-      disc[g] += nt.v[g][F_DISC];
-      cnt[g] += nt.v[g][F_CNT];
-      dp[g].add64s((int64_t)(100u * nt.v[g][F_PRICE] - nt.v[g][F_DPROD]));
-      ch[g].add64s((int64_t)nt.v[g][F_CHARGE]);
-    }
-  }
-
-  // Block merge in 128 bits for every field; the scratch follows the narrow table.
-  const uint32_t wave = thread_index() >> 6, lane = thread_index() & 63, nwaves = B >> 6;
-  constexpr int NW = 8;  // qty, price, disc, cnt, dp.lo, dp.hi, ch.lo, ch.hi
-  uint64_t* red = lds + shared_table_bytes(B) / 8;  // nwaves * 6 * NW words
-#pragma unroll
-  for (int g = 0; g < kNumGroups; g++) {
-    uint64_t s64[4] = {qty[g], price[g], disc[g], cnt[g]};
-    Wide128 w[2] = {dp[g], ch[g]};
-    if (ballot(cnt[g] != 0)) {
-#pragma unroll
-      for (int f = 0; f < 4; f++) s64[f] = wave_sum_u64(s64[f]);
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) {
-#pragma unroll
-        for (int f = 0; f < 2; f++) {
-          const uint64_t olo = __shfl_xor(w[f].lo, m, 64), ohi = __shfl_xor(w[f].hi, m, 64);
-          const uint64_t nlo = w[f].lo + olo;
-          w[f].hi += ohi + (nlo < olo);
-          w[f].lo = nlo;
-        }
-      }
-    } else {
-      s64[0] = s64[1] = s64[2] = s64[3] = 0;
-      w[0].lo = w[0].hi = w[1].lo = w[1].hi = 0;
-    }
-    if (lane == 0) {
-      uint64_t* r = red + (wave * kNumGroups + g) * NW;
-      r[0] = s64[0]; r[1] = s64[1]; r[2] = s64[2]; r[3] = s64[3];
-      r[4] = w[0].lo; r[5] = w[0].hi; r[6] = w[1].lo; r[7] = w[1].hi;
-    }
-  }
-  __syncthreads();
-  if (thread_index() < kNumGroups) {
-    const int g = thread_index();
-    uint64_t s[4] = {0, 0, 0, 0};
-    Wide128 w[2] = {{0, 0}, {0, 0}};
-    for (uint32_t v = 0; v < nwaves; v++) {
-      const uint64_t* r = red + (v * kNumGroups + g) * NW;
-      for (int f = 0; f < 4; f++) s[f] += r[f];
-      for (int f = 0; f < 2; f++) {
-        const uint64_t nlo = w[f].lo + r[4 + 2 * f];
-        w[f].hi += r[5 + 2 * f] + (nlo < w[f].lo);
-        w[f].lo = nlo;
-      }
-    }
-    if (s[3]) {
-      const uint64_t qs =
-          (L == Q1_LAYOUT_COMPRESSED || L == Q1_LAYOUT_COMPRESSED_PUSHDOWN) ? kQuantityScaleCompressed : 1;
-      q1_device_aggregates* out = a.out + (blockIdx.x & a.out_mask);
-      atomicAdd((unsigned long long*)&out->sum_qty[g], (unsigned long long)(s[0] * qs));
-      atomicAdd((unsigned long long*)&out->sum_base_price[g], (unsigned long long)s[1]);
-      atomicAdd((unsigned long long*)&out->sum_disc[g], (unsigned long long)s[2]);
-      atomicAdd((unsigned long long*)&out->count[g], (unsigned long long)s[3]);
-      atomic_add128(&out->sum_disc_price_lo[g], &out->sum_disc_price_hi[g], w[0].lo, w[0].hi);
-      atomic_add128(&out->sum_charge_lo[g], &out->sum_charge_hi[g], w[1].lo, w[1].hi);
-    }
-  }
+  Acc acc;
+  acc.init(lds);
+  add_tiles<L, Tile, B>(a, first_tile + (uint64_t)blockIdx.x * B * tiles_per_thread, tiles_per_thread, acc,
+                        column_cutoff<L>(a.cutoff_day));
+  uint64_t* red = lds + Acc::lds_bytes(B) / 8;
+  acc.wave_totals(red);
+  any_merge<B>(red, a.out + (blockIdx.x & a.out_mask), kQtyScale);
   finish_scan(a);
 }
 
@@ -2250,10 +2076,9 @@ template <int L>
 GenFn any_fn(uint32_t threads) {
   return threads == 64 ? scan_any<L, 64> : threads == 128 ? scan_any<L, 128> : scan_any<L, 256>;
 }
-
 template <int L>
-GenFn wide_fn(uint32_t threads) {
-  return threads == 64 ? scan_wide<L, 64> : threads == 128 ? scan_wide<L, 128> : scan_wide<L, 256>;
+uint32_t any_lds(uint32_t threads) {
+  return AnyOf<L, 64>::A::lds_bytes(threads) + threads / 64 * kNumGroups * NA * 8;
 }
 
 // The batched kernel's variants: the shared placement runs the narrow per-lane table (the
@@ -2271,7 +2096,7 @@ void* batch_fn(q1_placement p) {
 #define Q1_DECLARE_LAYOUT_KERNELS(NAME)                  \
   FastFn fast_kernel_##NAME(int placement, uint32_t threads); \
   GenFn any_kernel_##NAME(uint32_t threads);             \
-  GenFn wide_kernel_##NAME(uint32_t threads);            \
+  uint32_t any_kernel_lds_##NAME(uint32_t threads);      \
   void* batch_kernel_##NAME(q1_placement placement);
 Q1_DECLARE_LAYOUT_KERNELS(reference)
 Q1_DECLARE_LAYOUT_KERNELS(uncompressed)
@@ -2281,7 +2106,7 @@ Q1_DECLARE_LAYOUT_KERNELS(pushdown)
 #define Q1_DEFINE_LAYOUT_KERNELS(L, NAME)                                                          \
   FastFn fast_kernel_##NAME(int placement, uint32_t threads) { return fast_fn<L>(placement, threads); } \
   GenFn any_kernel_##NAME(uint32_t threads) { return any_fn<L>(threads); }                         \
-  GenFn wide_kernel_##NAME(uint32_t threads) { return wide_fn<L>(threads); }                       \
+  uint32_t any_kernel_lds_##NAME(uint32_t threads) { return any_lds<L>(threads); }                 \
   void* batch_kernel_##NAME(q1_placement placement) { return batch_fn<L>(placement); }
 
 }  // namespace q1

@@ -215,15 +215,13 @@ q1_status launch_slot(q1_server* sv, Slot& s) {
     // kernel's list of entries buys nothing for one request), or the 64-bit scan kernel on a
     // table outside the TPC-H domain, merging through the slot's own set.
     const q1_request& r = s.batch[0].req;
-    q1_placement p = Q1_PLACE_IN_REGISTERS;
-    q1_launch l{256, 1024, 0, 0};
-    if (!s.single) {
-      p = q1::resolve_placement(sv->ctx, t0->layout, Q1_PLACE_AUTO);
-      q1::resolve_launch(sv->ctx, t0->layout, p, r.row_count, nullptr, &l);
-    }
+    const q1_placement p =
+        s.single ? Q1_PLACE_IN_REGISTERS : q1::resolve_placement(sv->ctx, t0->layout, Q1_PLACE_AUTO);
+    q1_launch l;
+    q1::resolve_launch(sv->ctx, t0->layout, p, !s.single, r.row_count, nullptr, &l);
     q1::LaunchShape shape;
     const char* why = "";
-    q1_status st = q1::make_shape(p, t0->layout, &l, r.row_begin, r.row_begin + r.row_count, &shape, &why);
+    q1_status st = q1::make_shape(p, t0->layout, !s.single, &l, r.row_begin, r.row_begin + r.row_count, &shape, &why);
     if (s.single && st != Q1_OK) return st;
     if (st == Q1_OK && q1::scan_workspace_bytes(p, shape) == 0) {
       q1::ScanArgs a{};
@@ -233,7 +231,7 @@ q1_status launch_slot(q1_server* sv, Slot& s) {
       a.cutoff_day = t0->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t0->filter_cutoff : r.cutoff_day;
       a.host = s.h_result_dev;
       std::memset(s.h_result, 0, sizeof(*s.h_result));  // stays so when there are no rows
-      st = q1::launch_scan(p, t0->layout, !s.single, a, shape, nullptr, s.stream, s.set, s.single);
+      st = q1::launch_scan(p, t0->layout, !s.single, a, shape, nullptr, s.stream, s.set);
       if (st == Q1_OK && hipEventRecord(s.done, s.stream) != hipSuccess) {
         (void)hipStreamSynchronize(s.stream);
         st = Q1_EDEVICE;

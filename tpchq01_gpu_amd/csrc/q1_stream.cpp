@@ -21,6 +21,7 @@ struct StreamState {
   std::vector<q1_columns> staging;
   std::vector<void*> allocs;
   std::vector<void*> workspace;
+  std::vector<MergeSet*> set;   // each stream's launches merge through its own
   uint64_t workspace_bytes = 0;
 };
 
@@ -30,6 +31,7 @@ static void stream_state_free(StreamState* st) {
   for (void* p : st->allocs) (void)hipFree(p);
   for (void* p : st->workspace)
     if (p) (void)hipFree(p);
+  for (MergeSet* p : st->set) (void)hipFree(p);
   for (hipEvent_t e : st->done) (void)hipEventDestroy(e);
   for (hipStream_t s : st->s) (void)hipStreamDestroy(s);
   delete st;
@@ -69,6 +71,10 @@ static q1_status prepare(q1_ctx* ctx, q1_layout layout, uint64_t chunk_rows, int
     st->s.push_back(s);
     if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return give_up(Q1_EDEVICE, "event creation failed");
     st->done.push_back(e);
+    MergeSet* set = nullptr;
+    if (hipMalloc(&set, sizeof(MergeSet)) != hipSuccess) return give_up(Q1_ENOMEM, "staging allocation failed");
+    st->set.push_back(set);
+    if (launch_zero(set, s) != Q1_OK) return give_up(Q1_EDEVICE, "zero kernel failed");
     q1_columns c{};
     const void** slots[8] = {&c.ship_date, &c.quantity, &c.extended_price, &c.discount,
                              &c.tax, &c.return_flag, &c.line_status, &c.filter};
@@ -110,13 +116,14 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
     std::lock_guard<std::mutex> g(ctx->lock);
     const q1_placement p = resolve_placement(ctx, layout, placement);
     q1_launch l;
-    resolve_launch(ctx, layout, p, chunk_rows, launch, &l, true);
+    const bool fast = in_domain_flag(launch);
+    resolve_launch(ctx, layout, p, fast, chunk_rows, launch, &l, false);
     StreamState* st = nullptr;
     q1_status s = prepare(ctx, layout, chunk_rows, num_streams, &st);
     if (s != Q1_OK) return s;
     LaunchShape full_shape;
     const char* why = "";
-    s = make_shape(p, layout, &l, 0, chunk_rows, &full_shape, &why);
+    s = make_shape(p, layout, fast, &l, 0, chunk_rows, &full_shape, &why);
     if (s != Q1_OK) return fail(ctx, s, why);
     const uint64_t ws_bytes = scan_workspace_bytes(p, full_shape);
     if (ws_bytes > st->workspace_bytes) {
@@ -127,7 +134,6 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
       }
       st->workspace_bytes = ws_bytes;
     }
-    const bool fast = (l.flags & Q1_LAUNCH_ASSUME_TPCH_DOMAIN) != 0;
     uint64_t elem[8];
     column_bytes_local(layout, 1, elem);  // per-row bytes of the unpacked columns
     const bool packed = layout == Q1_LAYOUT_COMPRESSED || layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN;
@@ -173,7 +179,7 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
         bytes += len;
       }
       LaunchShape shape;
-      s = make_shape(p, layout, &l, 0, n, &shape, &why);
+      s = make_shape(p, layout, fast, &l, 0, n, &shape, &why);
       if (s != Q1_OK) return drain_fail(s, why);
       ScanArgs a{};
       a.cols = dst;
@@ -181,7 +187,7 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
       a.row_end = n;
       a.cutoff_day = cutoff_day;
       a.out = ctx->d_aggr;
-      s = launch_scan(p, layout, fast, a, shape, st->workspace[(size_t)idx], ss);
+      s = launch_scan(p, layout, fast, a, shape, st->workspace[(size_t)idx], ss, st->set[(size_t)idx]);
       if (s != Q1_OK) return drain_fail(s, "scan kernel launch failed");
     }
     for (int i = 0; i < num_streams; i++) {
@@ -228,10 +234,10 @@ q1_status q1_run_split(q1_ctx* ctx, const q1_table* t, const q1_columns* host, u
     std::lock_guard<std::mutex> g(ctx->lock);
     const q1_placement p = resolve_placement(ctx, t->layout, placement);
     q1_launch l;
-    resolve_launch(ctx, t->layout, p, split, launch, &l);
+    resolve_launch(ctx, t->layout, p, t->fast, split, launch, &l);
     LaunchShape shape;
     const char* why = "";
-    q1_status s = make_shape(p, t->layout, &l, 0, split, &shape, &why);
+    q1_status s = make_shape(p, t->layout, t->fast, &l, 0, split, &shape, &why);
     if (s != Q1_OK) return fail(ctx, s, why);
     s = ensure_workspace(ctx, scan_workspace_bytes(p, shape));
     if (s != Q1_OK) return s;
@@ -241,7 +247,7 @@ q1_status q1_run_split(q1_ctx* ctx, const q1_table* t, const q1_columns* host, u
     a.row_end = split;
     a.cutoff_day = t->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t->filter_cutoff : cutoff_day;
     const auto w0 = std::chrono::steady_clock::now();
-    s = scan_to_host(ctx, p, t->layout, t->fast, a, shape, !t->fast);
+    s = scan_to_host(ctx, p, t->layout, t->fast, a, shape);
     if (s != Q1_OK) return s;
     // The host share runs while the device works.
     q1_result cpu{};
