@@ -136,13 +136,14 @@ __global__ void generate_rows(uint64_t seed, uint64_t rows, q1_columns c) {
 // for a table inside the domain.  Each column is read as 16-byte vectors with no regard to
 // rows: a limit of the form 2^k - 1 is a test of bits, so a lane ORs what it reads of such a
 // column and tests the OR; quantities in hundredths (at most 6300) keep a maximum.  A block
-// takes kDomainRows rows: its 14 to 16 non-temporal loads per lane, each a contiguous
-// stretch of the block's share of a column, are all issued before any is used.
-// Measured with its launch and wait: 60M compressed rows 72 us, 600M 610 us (6.9 TB/s), 600M
-// uncompressed 1.19 ms (7.0), 600M reference 2.66 ms (7.2).  Grid-strided columns one after
-// another, four vectors in flight per lane, took 83 us, 709 us, 1.37 ms and 3.04 ms; the
-// per-row minimum and maximum of every column, merged with eight 64-bit atomics per
-// wavefront into one line, took 1.55 ms at 60M compressed rows.
+// takes kDomainRows rows: its 14 to 16 loads per lane, each a contiguous stretch of the
+// block's share of a column, are all issued before any is used.  The loads are ordinary ones,
+// which pass through the memory-side cache and so write back what the columns' producer
+// left there: after them the first query of 600M freshly written rows takes 880 us, after
+// non-temporal ones 990 (checks 0.67 and 0.61 ms).
+// With its launch and wait, 60M compressed rows take 72 us.  Grid-strided columns one after
+// another, four vectors in flight per lane, took 83 us; the per-row minimum and maximum of
+// every column, merged with eight 64-bit atomics per wavefront into one line, 1.55 ms.
 template <int L>
 constexpr int kDomainRows = L == Q1_LAYOUT_REFERENCE ? 2048 : L == Q1_LAYOUT_UNCOMPRESSED ? 4096 : 8192;
 
@@ -163,7 +164,7 @@ struct DomainColumn {
 #pragma unroll
     for (int k = 0; k < kVectors; k++) {
       const uint64_t i = first + k * 256;
-      v[k] = WHOLE || i < rows / kPer ? nt_load(reinterpret_cast<const uint4*>(col) + i) : make_uint4(0, 0, 0, 0);
+      v[k] = WHOLE || i < rows / kPer ? reinterpret_cast<const uint4*>(col)[i] : make_uint4(0, 0, 0, 0);
     }
   }
   __device__ __forceinline__ bool outside() const {
