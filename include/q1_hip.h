@@ -134,14 +134,15 @@ typedef struct {
 #define Q1_LAUNCH_ASSUME_TPCH_DOMAIN 1u
 
 typedef struct {
-  double kernel_ms;      /* device time of the last run: q1_run and q1_run_split by the device's
-                            clock, from the first block's start to the folded result; the
-                            others by HIP events around the kernels */
+  double kernel_ms;      /* device time of the last run: q1_run, q1_run_split and q1_run_batch
+                            by the device's clock, from the first block's start to the folded
+                            result; the others by HIP events around the kernels */
   double h2d_ms;         /* device time of host-to-device copies of the last call */
   double wall_ms;        /* host wall-clock of the last call */
   uint64_t bytes_read;   /* algorithmic column bytes the last run read */
   uint64_t rows;         /* rows scanned */
-  uint32_t num_blocks;   /* grid of the last kernel */
+  uint32_t num_blocks;   /* grid of the last kernel; q1_run_batch: this and the next two are the
+                            shape the batch was planned with, of which a small batch runs less */
   uint32_t threads_per_block;
   uint32_t tuples_per_thread;
   uint32_t placement;
@@ -241,7 +242,7 @@ void q1_aggregates_to_result(const q1_device_aggregates* host_copy, q1_result* o
 /* Exact 128-bit merge of two results (out = a + b). */
 void q1_result_merge(const q1_result* a, const q1_result* b, q1_result* out);
 
-/* --- batched (new): many requests in one persistent, hipGraph-replayed launch ------ */
+/* --- batched (new): many requests in one launch ----------------------------------- */
 typedef struct {
   const q1_table* table;
   uint64_t row_begin;
@@ -254,11 +255,12 @@ typedef struct {
  * q1_run of that request alone.  Requests of one layout on tables inside the TPC-H domain
  * share one launch; any other mix runs request by request.  `launch` may be NULL; its
  * threads_per_block must be 0 or 256; tuples_per_thread (rows per lane of each block of a
- * request; 0 = the tuned value) a multiple of 16, at most 256 for the shared placement and
- * 16384 for the register one; num_blocks (the resident grid, below 2^24) 0 = the tuned
- * blocks per compute unit x compute units.  The context keeps the batch's buffers between
- * calls of one capacity (the next power of two >= n, at least 16): the descriptors, the
- * results and 24 KiB of partial tables per request for the first 1024 requests. */
+ * request; 0 = the tuned value, less for a batch too small to fill the device) a multiple of
+ * 16, at most 256 for the shared placement and 16384 for the register one; num_blocks (the
+ * grid, below 2^24, whose blocks stride through the batch's) 0 = one per block of the batch,
+ * up to the tuned blocks per compute unit x compute units.  The context keeps the batch's
+ * buffers between calls, grown to the largest batch so far: the descriptors, the results and
+ * up to 65536 partial tables of 512 B. */
 q1_status q1_run_batch(q1_ctx* ctx, const q1_request* reqs, uint32_t n, const q1_launch* launch,
                        q1_result* outs);
 

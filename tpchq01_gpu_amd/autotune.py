@@ -51,7 +51,7 @@ from . import PACKAGE_DIR, q1
 THREADS = [64, 128, 256]
 TUPLES = [16, 32, 64, 128, 256, 512, 1024, 2048, 4096, 8192, 16384]
 ROWS = [600_000_000, 60_000_000, 6_000_000]
-BATCH_BLOCKS_PER_CU = [1, 2, 3, 4, 6, 8]
+BATCH_BLOCKS_PER_CU = [4, 8, 16, 32, 64]
 STREAM_CHUNKS = [1 << 20, 1 << 21, 1 << 22, 1 << 23, 1 << 24, 1 << 25, 1 << 26]
 STREAM_COUNTS = [1, 2, 3, 4, 6, 8]
 BATCH_LANE_ROWS = {q1.IN_REGISTERS: [256, 512, 1024, 2048], q1.PER_THREAD_SHARED_MEM: [64, 128, 192, 256]}
@@ -116,7 +116,7 @@ def sweep_batch(ctx: q1.Context, layout: int, spec, placements, reps: int, log=p
                 for lr in lane_rows[p]:
                     launch = q1.make_launch(0, lr, per_cu * cus)
                     best = float("inf")
-                    for r in range(reps + 1):    # the first call captures the graph
+                    for r in range(reps + 1):    # the first call makes the buffers
                         ctx.check(q1.lib.q1_run_batch(ctx.handle, reqs, n, C.byref(launch), outs), "q1_run_batch")
                         if r:
                             best = min(best, ctx.last_timing().kernel_ms)
@@ -201,9 +201,9 @@ BATCH_TIE = 0.01
 def best_batch_table(batch_results, tie=BATCH_TIE):
     """The batched kernel's shape per (layout, placement): of the shapes within `tie` of the
     fastest, the one with the most blocks per compute unit (then the fastest of those).
-    Grids that leave wave slots empty measured within 1 % of full ones on the batch alone,
-    but 5 % slower with other tables resident too (1.18 against 1.125 ms for 3 against 8
-    blocks per CU), so among shapes the sweep cannot tell apart the full grid is kept."""
+    The more blocks, the more of the list's balance is left to the hardware's dispatch (one
+    block per entry measures 4 % faster than 8 blocks per compute unit that stride through
+    the list), so among shapes the sweep cannot tell apart the largest grid is kept."""
     fastest = {}
     for r in batch_results:
         k = (r["layout"], r["placement"])

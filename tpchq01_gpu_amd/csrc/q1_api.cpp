@@ -158,7 +158,7 @@ q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fa
   } else if (shape.blocks >= kSpreadMinBlocks && (other = stream_spread(ctx, stream))) {
     set = other->set;
     if (!other->zeroed) {
-      const q1_status z = launch_zero(set, stream);
+      const q1_status z = launch_zero(set, sizeof(MergeSet), stream);
       if (z != Q1_OK) return z;
       other->zeroed = true;
     }
@@ -186,9 +186,8 @@ q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bo
 // with the stream's wait), a longer one, after kWatchMicroseconds, by the stream's own wait,
 // which lets the processor go and then costs at most 5 % of the call.
 constexpr int kWatchMicroseconds = 100;
-q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms) {
-  const HostResult* r = ctx->h_result;
-  auto arrived = [&] { return __atomic_load_n(&r->sequence, __ATOMIC_ACQUIRE) == ctx->sequence; };
+q1_status wait_sequence(q1_ctx* ctx, const uint64_t* word, uint64_t sequence) {
+  auto arrived = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) == sequence; };
   const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(kWatchMicroseconds);
   while (!arrived() && std::chrono::steady_clock::now() < until)
     for (int i = 0; i < 16 && !arrived(); i++) __builtin_ia32_pause();
@@ -196,8 +195,19 @@ q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms) {
     Q1_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (!arrived()) return fail(ctx, Q1_EDEVICE, "the scan kernel ended without a result");
   }
+  return Q1_OK;
+}
+
+double clock_ms(const q1_ctx* ctx, uint64_t begin, uint64_t end) {
+  return ctx->clock_khz > 0 ? (double)(end - begin) / ctx->clock_khz : 0.0;
+}
+
+q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms) {
+  const HostResult* r = ctx->h_result;
+  const q1_status s = wait_sequence(ctx, &r->sequence, ctx->sequence);
+  if (s != Q1_OK) return s;
   q1_aggregates_to_result(&r->sums, out);
-  *kernel_ms = ctx->clock_khz > 0 ? (double)(r->clock_end - r->clock_begin) / ctx->clock_khz : 0.0;
+  *kernel_ms = clock_ms(ctx, r->clock_begin, r->clock_end);
   return Q1_OK;
 }
 
@@ -411,7 +421,10 @@ void q1_shutdown(q1_ctx* ctx) {
     t->rows = 0;
   }
   ctx->tables.clear();
-  if (ctx->batch) batch_destroy(ctx->batch);
+  if (ctx->batch) {
+    batch_free(ctx->batch);
+    delete ctx->batch;
+  }
   stream_state_release(ctx);
   if (ctx->workspace) (void)hipFree(ctx->workspace);
   if (ctx->set) (void)hipFree(ctx->set);

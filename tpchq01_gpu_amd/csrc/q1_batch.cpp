@@ -1,15 +1,9 @@
 // q1_run_batch: many filter-aggregate requests (uneven row counts, their own cutoffs) in
-// one persistent launch, captured once into a hipGraph and replayed:
-//   H2D copy of the request descriptors (pinned staging) -> the batched kernel -> the fold
-//   of each request's spread tables, which stores the results straight into the pinned
-//   host results (over PCIe).
-// A batch of more than kBatchSpreadRequests requests gives spread tables to the first
-// kBatchSpreadRequests only, so its graph is: H2D copy -> zero the device results (a fill
-// kernel, never a memset node) -> the batched kernel -> the fold, adding into the device
-// results -> D2H copy of the results.
-// The spread tables are zeroed once when allocated; every fold clears the tables it read.
-// The graph is rebuilt only when the capacity bucket, layout, placement or grid changes;
-// each call only rewrites the pinned descriptor buffer before the replay.
+// one launch of the batched kernel: the descriptors are copied to the device, the kernel runs
+// every request's blocks, and the last block of each request stores its result straight into
+// the pinned host results, with a done record after all of them that the caller waits for.
+// Two commands on the stream and no per-batch set-up: a batch of any size runs at once in
+// the same buffers.
 #include <algorithm>
 #include <chrono>
 #include <cstring>
@@ -17,41 +11,23 @@
 
 #include "q1_internal.h"
 
-struct q1_batch_state {
-  q1_layout layout = Q1_LAYOUT_COMPRESSED;
-  q1_placement placement = Q1_PLACE_IN_REGISTERS;
-  uint32_t capacity = 0, blocks = 0, threads = 0;
-  q1::BatchHeader* h_buf = nullptr;  // pinned: header + capacity descriptors
-  q1::BatchHeader* d_buf = nullptr;
-  q1_device_aggregates* h_out = nullptr;  // pinned
-  q1_device_aggregates* d_out = nullptr;
-  q1_device_aggregates* d_spread = nullptr;  // spread_requests x kSpreadTables tables
-  uint32_t spread_requests = 0;
-  q1_device_aggregates* h_out_dev = nullptr;  // h_out as the device addresses it (folds store there)
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-};
-
 namespace q1 {
 
-void batch_destroy(q1_batch_state* b) {
-  if (!b) return;
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
+void batch_free(BatchBuffers* b) {
   if (b->h_buf) (void)hipHostFree(b->h_buf);
   if (b->h_out) (void)hipHostFree(b->h_out);
   if (b->d_buf) (void)hipFree(b->d_buf);
-  if (b->d_out) (void)hipFree(b->d_out);
-  if (b->d_spread) (void)hipFree(b->d_spread);
-  delete b;
+  if (b->control) (void)hipFree(b->control);
+  *b = BatchBuffers{};
 }
 
-static uint64_t buf_bytes(uint32_t cap) { return sizeof(BatchHeader) + (uint64_t)cap * sizeof(BatchDesc); }
+static uint64_t buf_bytes(uint32_t n) {
+  return sizeof(BatchHeader) + (uint64_t)n * (sizeof(BatchDesc) + sizeof(uint32_t));
+}
 
 // Rows per lane: the autotuner's batch value for the layout and placement, else the
 // scan's tuned value, within the batched kernel's limit.
-uint32_t batch_lane_rows(q1_ctx* ctx, q1_layout layout, q1_placement p) {
-  p = batch_placement(p);
+static uint32_t batch_lane_rows(q1_ctx* ctx, q1_layout layout, q1_placement p) {
   const uint32_t most = batch_max_lane_rows(p);
   const uint32_t batch_tuned = ctx->batch_tuning[layout][p].tuples_per_thread;
   if (batch_tuned >= 16 && batch_tuned <= most) return batch_tuned / 16 * 16;
@@ -59,87 +35,148 @@ uint32_t batch_lane_rows(q1_ctx* ctx, q1_layout layout, q1_placement p) {
   return tuned >= 16 && tuned <= most ? tuned / 16 * 16 : std::min<uint32_t>(256, most);
 }
 
+static uint32_t compute_units(const q1_ctx* ctx) { return (uint32_t)(ctx->compute_units > 0 ? ctx->compute_units : 256); }
+
 // Grid: the autotuner's blocks per compute unit for the layout and placement, else as many
 // blocks as are resident at once.
-uint32_t batch_default_blocks(q1_ctx* ctx, q1_layout layout, q1_placement p) {
-  p = batch_placement(p);
-  const uint32_t cus = (uint32_t)(ctx->compute_units > 0 ? ctx->compute_units : 256);
+static uint32_t batch_default_blocks(q1_ctx* ctx, q1_layout layout, q1_placement p) {
   const uint32_t per_cu = ctx->batch_tuning[layout][p].num_blocks;
-  return cus * (per_cu ? per_cu : batch_blocks_per_cu(layout, p));
+  return compute_units(ctx) * (per_cu ? per_cu : batch_blocks_per_cu(layout, p));
 }
 
-uint64_t batch_describe(BatchDesc* d, const q1_request& r, uint64_t first, uint32_t lane_rows) {
-  const q1_table* t = r.table;
-  d->cols = t->dev;
-  d->row_begin = r.row_begin;
-  d->row_end = r.row_begin + r.row_count;
-  d->block_begin = first;
-  d->cutoff_day = t->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t->filter_cutoff : r.cutoff_day;
-  d->pad = 0;
+static uint64_t request_blocks(const q1_request& r, uint32_t lane_rows) {
   if (r.row_count == 0) return 0;
-  const uint64_t trows = layout_tile_rows(t->layout);
-  const uint64_t tiles = (d->row_end + trows - 1) / trows - align_rows_down(d->row_begin) / trows;
+  const uint64_t trows = layout_tile_rows(r.table->layout);
+  const uint64_t tiles = (r.row_begin + r.row_count + trows - 1) / trows - align_rows_down(r.row_begin) / trows;
   const uint64_t per_block = (uint64_t)kBatchThreads * (lane_rows / trows);
   return (tiles + per_block - 1) / per_block;
 }
 
-static q1_status build_state(q1_ctx* ctx, q1_layout layout, q1_placement placement, uint32_t cap,
-                             uint32_t threads, uint32_t blocks) {
-  q1_batch_state* b = ctx->batch;
-  if (b && b->layout == layout && b->placement == placement && b->capacity == cap && b->threads == threads &&
-      b->blocks == blocks)
+// Makes room for n requests and `tables` merge tables.  The stream's earlier launches with
+// the buffers have finished.
+static q1_status reserve(BatchBuffers* b, uint32_t n, uint32_t tables, hipStream_t stream, const char** why) {
+  auto give_up = [&](q1_status s, const char* text) {
+    *why = text;
+    return s;
+  };
+  if (b->capacity < n) {
+    uint32_t cap = 16;
+    while (cap < n) cap <<= 1;
+    if (b->h_buf) (void)hipHostFree(b->h_buf);
+    if (b->h_out) (void)hipHostFree(b->h_out);
+    if (b->d_buf) (void)hipFree(b->d_buf);
+    b->h_buf = b->d_buf = nullptr;
+    b->h_out = b->h_out_dev = nullptr;
+    b->capacity = 0;
+    const uint64_t out_bytes = (uint64_t)cap * sizeof(q1_device_aggregates) + sizeof(BatchDone);
+    if (hipHostMalloc(&b->h_buf, buf_bytes(cap), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&b->h_out, out_bytes, hipHostMallocMapped) != hipSuccess ||
+        hipHostGetDevicePointer((void**)&b->h_out_dev, b->h_out, 0) != hipSuccess ||
+        hipMalloc(&b->d_buf, buf_bytes(cap)) != hipSuccess)
+      return give_up(Q1_ENOMEM, "batch buffers could not be allocated");
+    std::memset((void*)b->h_out, 0, out_bytes);
+    b->capacity = cap;
+  }
+  if (!b->control || b->tables < tables) {
+    uint32_t t = 64;
+    while (t < tables) t <<= 1;
+    if (b->control) (void)hipFree(b->control);
+    b->control = nullptr;
+    b->tables = 0;
+    const uint64_t bytes = sizeof(BatchControl) + (uint64_t)t * sizeof(MergeTable);
+    if (hipMalloc(&b->control, bytes) != hipSuccess)
+      return give_up(Q1_ENOMEM, "batch tables could not be allocated");
+    if (launch_zero(b->control, bytes, stream) != Q1_OK) {
+      (void)hipFree(b->control);
+      b->control = nullptr;
+      return give_up(Q1_EDEVICE, "clearing the batch tables failed");
+    }
+    b->tables = t;
+  }
+  return Q1_OK;
+}
+
+q1_status batch_launch(q1_ctx* ctx, BatchBuffers* b, const q1_request* reqs, uint32_t n, q1_placement placement,
+                       uint32_t lane_rows, uint32_t grid, hipStream_t stream, uint32_t* lane_rows_planned,
+                       uint32_t* grid_planned, const char** why) {
+  auto give_up = [&](q1_status s, const char* text) {
+    *why = text;
+    return s;
+  };
+  const q1_layout layout = reqs[0].table->layout;
+  placement = batch_placement(placement);
+  *lane_rows_planned = lane_rows ? lane_rows : batch_lane_rows(ctx, layout, placement);
+  *grid_planned = grid ? grid : batch_default_blocks(ctx, layout, placement);
+  if (!lane_rows) {
+    // The tuned rows per lane, halved while the batch has fewer than 4 blocks per compute
+    // unit, so that a small batch spreads over the chip too.
+    lane_rows = *lane_rows_planned;
+    uint64_t rows = 0;
+    for (uint32_t i = 0; i < n; i++) rows += reqs[i].row_count;
+    while (lane_rows > 16 && rows < 4ull * compute_units(ctx) * kBatchThreads * lane_rows)
+      lane_rows = std::max<uint32_t>(16, (lane_rows / 2) & ~15u);
+  }
+  // A request's tables: as a scan of its blocks would have, fewer for all while the batch
+  // would need more than kBatchMaxTables.
+  uint64_t entries = 0, tables = 0;
+  uint32_t most = kSpreadTables;
+  for (;; most >>= 1) {
+    entries = tables = 0;
+    for (uint32_t i = 0; i < n; i++) {
+      const uint64_t blocks = request_blocks(reqs[i], lane_rows);
+      entries += blocks;
+      tables += std::min(merge_tables(blocks), most);
+    }
+    if (tables <= kBatchMaxTables || most == 1) break;
+  }
+  if (entries >= (1ull << 31)) return give_up(Q1_EINVAL, "batch too large (2^31 blocks of rows)");
+  const q1_status s = reserve(b, n, (uint32_t)tables, stream, why);
+  if (s != Q1_OK) return s;
+  BatchDesc* d = reinterpret_cast<BatchDesc*>(b->h_buf + 1);
+  uint32_t* first = reinterpret_cast<uint32_t*>(d + n);
+  MergeTable* next = reinterpret_cast<MergeTable*>(b->control + 1);
+  uint32_t block = 0, with_rows = 0;
+  for (uint32_t i = 0; i < n; i++) {
+    const q1_request& r = reqs[i];
+    const q1_table* t = r.table;
+    const uint32_t blocks = (uint32_t)request_blocks(r, lane_rows);
+    const uint32_t own = std::min(merge_tables(blocks), most);
+    d[i].cols = t->dev;
+    d[i].row_begin = r.row_begin;
+    d[i].row_end = r.row_begin + r.row_count;
+    d[i].tables = next;
+    d[i].table_mask = own - 1;
+    d[i].first_block = first[i] = block;
+    d[i].blocks = blocks;
+    d[i].cutoff_day = t->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? t->filter_cutoff : r.cutoff_day;
+    next += own;
+    block += blocks;
+    if (blocks)
+      with_rows++;
+    else
+      std::memset((void*)&b->h_out[i], 0, sizeof(q1_device_aggregates));
+  }
+  b->sequence++;
+  BatchHeader* h = b->h_buf;
+  *h = BatchHeader{};
+  h->n = n;
+  h->with_rows = with_rows;
+  h->total_blocks = block;
+  h->tiles_per_thread = lane_rows / layout_tile_rows(layout);
+  h->sequence = b->sequence;
+  if (!with_rows) {
+    BatchDone* done = const_cast<BatchDone*>(b->done());
+    *done = BatchDone{0, 0, b->sequence};
     return Q1_OK;
-  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return fail(ctx, Q1_EDEVICE, "stream sync failed");
-  batch_destroy(b);
-  ctx->batch = nullptr;
-  b = new q1_batch_state();
-  b->layout = layout;
-  b->placement = placement;
-  b->capacity = cap;
-  b->threads = threads;
-  b->blocks = blocks;
-  b->spread_requests = std::min(cap, kBatchSpreadRequests);
-  const uint64_t spread_bytes = (uint64_t)b->spread_requests * kSpreadTables * sizeof(q1_device_aggregates);
-  bool ok = hipHostMalloc(&b->h_buf, buf_bytes(cap), hipHostMallocDefault) == hipSuccess &&
-            hipHostMalloc(&b->h_out, cap * sizeof(q1_device_aggregates), hipHostMallocMapped) == hipSuccess &&
-            hipHostGetDevicePointer((void**)&b->h_out_dev, b->h_out, 0) == hipSuccess &&
-            hipMalloc(&b->d_buf, buf_bytes(cap)) == hipSuccess &&
-            hipMalloc(&b->d_out, cap * sizeof(q1_device_aggregates)) == hipSuccess &&
-            hipMalloc(&b->d_spread, spread_bytes) == hipSuccess &&
-            hipMemsetAsync(b->d_spread, 0, spread_bytes, ctx->stream) == hipSuccess &&
-            hipStreamSynchronize(ctx->stream) == hipSuccess;  // before the capture, not inside it
-  if (!ok) {
-    batch_destroy(b);
-    return fail(ctx, Q1_ENOMEM, "batch buffers could not be allocated");
   }
-  std::memset(b->h_buf, 0, buf_bytes(cap));
-  // Capture the whole step once.
-  hipStream_t s = ctx->stream;
-  q1_status st = Q1_OK;
-  if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) st = Q1_EDEVICE;
-  if (st == Q1_OK && hipMemcpyAsync(b->d_buf, b->h_buf, buf_bytes(cap), hipMemcpyHostToDevice, s) != hipSuccess)
-    st = Q1_EDEVICE;
-  const bool store = b->spread_requests == cap;  // every request has spread tables
-  if (st == Q1_OK && !store) st = launch_zero(b->d_out, cap, s);
-  if (st == Q1_OK)
-    st = launch_batch(layout, placement, b->d_buf, b->d_out, b->d_spread, b->spread_requests,
-                      store ? b->h_out_dev : nullptr, blocks, threads, s);
-  if (st == Q1_OK && !store &&
-      hipMemcpyAsync(b->h_out, b->d_out, cap * sizeof(q1_device_aggregates), hipMemcpyDeviceToHost, s) != hipSuccess)
-    st = Q1_EDEVICE;
-  hipGraph_t g = nullptr;
-  const hipError_t ec = hipStreamEndCapture(s, &g);
-  if (st != Q1_OK || ec != hipSuccess || !g) {
-    if (g) (void)hipGraphDestroy(g);
-    batch_destroy(b);
-    return fail(ctx, Q1_EDEVICE, "capturing the batch graph failed");
+  if (!grid) grid = std::min(block, *grid_planned);
+  if (hipMemcpyAsync(b->d_buf, b->h_buf, buf_bytes(n), hipMemcpyHostToDevice, stream) != hipSuccess)
+    return give_up(Q1_EDEVICE, "copying the batch descriptors failed");
+  BatchDone* done = reinterpret_cast<BatchDone*>(b->h_out_dev + b->capacity);
+  if (launch_batch(layout, placement, b->d_buf, n, b->control, b->h_out_dev, done, grid, stream) != Q1_OK) {
+    (void)hipStreamSynchronize(stream);  // the copy still reads the pinned descriptors
+    return give_up(Q1_EDEVICE, "batch kernel launch failed");
   }
-  b->graph = g;
-  if (hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0) != hipSuccess) {
-    batch_destroy(b);
-    return fail(ctx, Q1_EDEVICE, "instantiating the batch graph failed");
-  }
-  ctx->batch = b;
   return Q1_OK;
 }
 
@@ -159,7 +196,7 @@ extern "C" q1_status q1_run_batch(q1_ctx* ctx, const q1_request* reqs, uint32_t 
       return fail(ctx, Q1_EINVAL, "request row range outside its table");
   }
   try {
-    // One persistent launch needs one layout and the TPC-H domain; any other mix runs
+    // One launch needs one layout and the TPC-H domain; any other mix runs
     // request by request (same results, no batching).
     const q1_layout layout = reqs[0].table->layout;
     bool batchable = true;
@@ -176,57 +213,40 @@ extern "C" q1_status q1_run_batch(q1_ctx* ctx, const q1_request* reqs, uint32_t 
     std::lock_guard<std::mutex> g(ctx->lock);
     const q1_placement p = batch_placement(ctx->best[layout]);
     // The batched kernel runs 256-thread blocks; the grid and rows per lane are tunable.
-    const uint32_t threads = kBatchThreads;
-    if (launch && launch->threads_per_block && launch->threads_per_block != threads)
+    if (launch && launch->threads_per_block && launch->threads_per_block != kBatchThreads)
       return fail(ctx, Q1_EINVAL, "the batched kernel runs 256 threads per block");
-    uint32_t lane_rows = batch_lane_rows(ctx, layout, p);
-    if (launch && launch->tuples_per_thread) {
-      lane_rows = launch->tuples_per_thread;
-      if (lane_rows % 16 != 0 || lane_rows > batch_max_lane_rows(p))
-        return fail(ctx, Q1_EINVAL,
-                    "batched tuples_per_thread must be a multiple of 16, at most 256 (shared placement) or 16384");
-    }
-    const uint32_t blocks =
-        launch && launch->num_blocks ? launch->num_blocks : batch_default_blocks(ctx, layout, p);
+    const uint32_t lane_rows = launch ? launch->tuples_per_thread : 0, grid = launch ? launch->num_blocks : 0;
+    if (lane_rows % 16 != 0 || lane_rows > batch_max_lane_rows(p))
+      return fail(ctx, Q1_EINVAL,
+                  "batched tuples_per_thread must be a multiple of 16, at most 256 (shared placement) or 16384");
     // The grid's work-items (blocks x 256) must stay below 2^32.
-    if (blocks >= (1u << 24)) return fail(ctx, Q1_EINVAL, "batched num_blocks must be below 2^24");
-    uint32_t cap = 16;
-    while (cap < n) cap <<= 1;
-    q1_status s = build_state(ctx, layout, p, cap, threads, blocks);
-    if (s != Q1_OK) return s;
-    q1_batch_state* b = ctx->batch;
-    BatchDesc* d = reinterpret_cast<BatchDesc*>(b->h_buf + 1);
-    uint64_t entries = 0, rows = 0;
+    if (grid >= (1u << 24)) return fail(ctx, Q1_EINVAL, "batched num_blocks must be below 2^24");
+    if (!ctx->batch) ctx->batch = new BatchBuffers();
+    BatchBuffers* b = ctx->batch;
+    const auto w0 = std::chrono::steady_clock::now();
+    uint32_t plan_rows = 0, plan_grid = 0;
+    const char* why = "";
+    q1_status s = batch_launch(ctx, b, reqs, n, p, lane_rows, grid, ctx->stream, &plan_rows, &plan_grid, &why);
+    if (s != Q1_OK) return fail(ctx, s, why);
+    s = wait_sequence(ctx, &b->done()->sequence, b->sequence);
+    if (s != Q1_OK) {
+      // The tables may hold partial sums: the next call makes new ones.
+      batch_free(b);
+      return s;
+    }
+    uint64_t rows = 0;
     for (uint32_t i = 0; i < n; i++) {
-      entries += batch_describe(&d[i], reqs[i], entries, lane_rows);
+      q1_aggregates_to_result(&b->h_out[i], &outs[i]);
       rows += reqs[i].row_count;
     }
-    if (entries >= (1ull << 31)) return fail(ctx, Q1_EINVAL, "batch too large (2^31 blocks of rows)");
-    b->h_buf->n = n;
-    b->h_buf->total_blocks = entries;
-    b->h_buf->tiles_per_thread = lane_rows / layout_tile_rows(layout);
-    b->h_buf->spread_requests = b->spread_requests;
-    const auto w0 = std::chrono::steady_clock::now();
-    if (hipEventRecord(ctx->ev_begin, ctx->stream) != hipSuccess ||
-        hipGraphLaunch(b->exec, ctx->stream) != hipSuccess || hipEventRecord(ctx->ev_end, ctx->stream) != hipSuccess ||
-        hipStreamSynchronize(ctx->stream) != hipSuccess) {
-      // The spread tables may hold partial sums: the next call rebuilds the state.
-      (void)hipStreamSynchronize(ctx->stream);
-      batch_destroy(ctx->batch);
-      ctx->batch = nullptr;
-      return fail(ctx, Q1_EDEVICE, "batch graph launch failed");
-    }
-    for (uint32_t i = 0; i < n; i++) q1_aggregates_to_result(&b->h_out[i], &outs[i]);
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end);
     ctx->last = q1_timing{};
-    ctx->last.kernel_ms = ms;
+    ctx->last.kernel_ms = clock_ms(ctx, b->done()->clock_begin, b->done()->clock_end);
     ctx->last.wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
     ctx->last.rows = rows;
     ctx->last.bytes_read = algorithmic_bytes(layout, rows);
-    ctx->last.num_blocks = blocks;
-    ctx->last.threads_per_block = threads;
-    ctx->last.tuples_per_thread = lane_rows;
+    ctx->last.num_blocks = plan_grid;
+    ctx->last.threads_per_block = kBatchThreads;
+    ctx->last.tuples_per_thread = plan_rows;
     ctx->last.placement = (uint32_t)p;
     return Q1_OK;
   } catch (const std::exception& e) {

@@ -28,8 +28,8 @@ struct q1_table {
 constexpr uint64_t kStreamChunkRows = 1ull << 24;
 constexpr int kStreamCount = 4;
 
-struct q1_batch_state;  // q1_batch.cpp
 namespace q1 {
+struct BatchBuffers;
 struct StreamState;     // q1_stream.cpp: the host-resident streaming pipeline
 // The merge set of one caller stream (q1_enqueue on a stream other than the context's).
 // `done` is recorded after every launch that uses it and the next launch waits for it,
@@ -80,7 +80,7 @@ struct q1_ctx {
   int stream_count[4] = {};
   q1_placement best[4] = {Q1_PLACE_IN_REGISTERS, Q1_PLACE_IN_REGISTERS, Q1_PLACE_IN_REGISTERS,
                           Q1_PLACE_IN_REGISTERS};
-  q1_batch_state* batch = nullptr;
+  q1::BatchBuffers* batch = nullptr;       // q1_run_batch's buffers
   q1::StreamState* streaming = nullptr;    // cached staging buffers and streams of q1_run_streaming
   q1::MergeSet* set = nullptr;             // merge set of the context stream
   std::unordered_map<void*, q1::StreamSpread> stream_spreads;  // caller streams' merge sets
@@ -109,13 +109,33 @@ q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fa
 q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, ScanArgs a,
                        const LaunchShape& shape);
 q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms);
-void batch_destroy(q1_batch_state* b);
-// The batched kernel's plan, shared by q1_run_batch and the server: rows per lane (the
-// tuned value of the layout and placement, at most batch_max_lane_rows), the default
-// grid (every block resident at once), and descriptor r of a batch, whose blocks start at
-// list entry `first`; batch_describe returns the request's number of blocks.
-uint32_t batch_lane_rows(q1_ctx* ctx, q1_layout layout, q1_placement p);
-uint32_t batch_default_blocks(q1_ctx* ctx, q1_layout layout, q1_placement p);
-uint64_t batch_describe(BatchDesc* d, const q1_request& r, uint64_t first, uint32_t lane_rows);
+// Waits until a launch on the context stream has written `sequence` to *word (pinned).
+q1_status wait_sequence(q1_ctx* ctx, const uint64_t* word, uint64_t sequence);
+double clock_ms(const q1_ctx* ctx, uint64_t begin, uint64_t end);
+
+// The buffers of batched launches on one stream, kept between launches and grown when a
+// larger batch comes: the descriptors (pinned and on the device), the results (pinned,
+// written by the kernel) and the requests' merge tables.
+struct BatchBuffers {
+  uint32_t capacity = 0;                    // requests
+  uint32_t tables = 0;
+  BatchHeader* h_buf = nullptr;             // header, descriptors, first blocks
+  BatchHeader* d_buf = nullptr;
+  q1_device_aggregates* h_out = nullptr;    // results, then a BatchDone
+  q1_device_aggregates* h_out_dev = nullptr;  // ... as the device addresses them
+  BatchControl* control = nullptr;          // on the device, the tables behind it
+  uint64_t sequence = 0;                    // of the last launch
+  const BatchDone* done() const { return reinterpret_cast<const BatchDone*>(h_out + capacity); }
+};
+void batch_free(BatchBuffers* b);
+// Launches n requests of one layout inside the domain on `stream` (whose earlier launches with
+// these buffers have finished): results in b->h_out[0 .. n-1] once b->done() holds
+// b->sequence, or the stream has got there.  lane_rows and grid of 0 take the tuned rows per
+// lane, less for a batch too small to fill the chip, and a block per entry up to the tuned
+// grid.  *lane_rows_planned, *grid_planned: the tuned shape or the caller's.  *why: what
+// failed (ctx is only read: the server's threads launch without its lock).
+q1_status batch_launch(q1_ctx* ctx, BatchBuffers* b, const q1_request* reqs, uint32_t n, q1_placement placement,
+                       uint32_t lane_rows, uint32_t grid, hipStream_t stream, uint32_t* lane_rows_planned,
+                       uint32_t* grid_planned, const char** why);
 void stream_state_release(q1_ctx* ctx);
 }  // namespace q1

@@ -30,20 +30,34 @@ struct LaunchShape {
 };
 
 // Spread merge.  Thousands of blocks adding into one 48-word table serialise on those
-// words' atomics at the end of the grid; instead block b of a launch merges into
-// tables[b % kSpreadTables] of a merge set, and the last block to finish folds the tables
-// into the destination.  A set is all zero before a launch and after it (the fold clears
-// what it read), and must not be shared by launches that can overlap.
-constexpr uint32_t kSpreadTables = 64;      // power of two
+// words' atomics at the end of the grid; instead the blocks of a range merge into several
+// tables, block b into table b mod their number, and the last block to finish folds the
+// tables into the destination.  Tables are all zero before a launch and after it (the fold
+// clears what it read), and must not be shared by launches that can overlap.
+// A table takes up to 16 blocks while there are fewer than 64: the fold reads fewer tables,
+// and 16 blocks' atomics on one table still pass within 0.5 us.  Kernel time with 64 / 32-4
+// tables: 64 blocks 8.3 / 6.5 us, 128 blocks 8.7 / 6.7, 293 blocks 8.8 / 7.4; a table per 2,
+// 4, 8 or 16 blocks: a 256-request batch 911, 908, 899, 896 us.
+constexpr uint32_t kBlocksPerTable = 16;
+constexpr uint32_t kSpreadTables = 64;      // the most tables a range merges into; a power of two
+struct alignas(128) MergeTable {
+  q1_device_aggregates sums;
+  // Blocks that have merged here count in `merged`, the last of them in the range's first
+  // table's tables_merged, so that no counter sees more than its share of a large grid.
+  alignas(128) uint32_t merged;
+  uint32_t tables_merged;
+};
+static_assert(sizeof(MergeTable) == 512, "sums and counters on cache lines of their own");
+// How many tables the blocks of a range merge into (a power of two, at most the blocks).
+inline uint32_t merge_tables(uint64_t blocks) {
+  uint32_t t = 1;
+  while (t < kSpreadTables && (uint64_t)t * kBlocksPerTable < blocks) t <<= 1;
+  return t;
+}
+
+// The tables of a stream's scan launches.
 struct MergeSet {
-  q1_device_aggregates tables[kSpreadTables];
-  // Blocks that have merged: those of one table (the blocks b with the same b mod 64) count
-  // in finished[b % 64], each on a cache line of its own, and the last of them in
-  // tables_finished, so that no counter sees more than a 64th of a large grid.
-  struct alignas(128) Count {
-    uint32_t n;
-  } finished[kSpreadTables];
-  Count tables_finished;
+  MergeTable table[kSpreadTables];
   uint64_t clock_begin;       // device clock at the start of block 0
 };
 
@@ -60,13 +74,12 @@ struct ScanArgs {
   uint64_t row_begin, row_end;
   int32_t cutoff_day;       // MonetDB day number (ignored for pushdown)
   q1_device_aggregates* out;
-  // Set by launch_scan: block b merges into out[b & out_mask]; with a merge set, `out` are
-  // the set's tables and the last block folds them into *dest (added), or, when dest is
-  // null, into *host (stored, with the clocks and `sequence`; host memory as the device
-  // addresses it).
-  uint32_t out_mask;
+  // Set by launch_scan: without a merge set the blocks add into *out.  With one, block b
+  // merges into the set's table b & table_mask, and the last block folds the tables into
+  // *host (stored, with the clocks and `sequence`; host memory as the device addresses it),
+  // or, when host is null, into *out (added).
+  uint32_t table_mask;
   MergeSet* set;
-  q1_device_aggregates* dest;
   HostResult* host;
   uint64_t sequence;
 };
@@ -97,9 +110,8 @@ q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const
                       const LaunchShape& shape, void* workspace, void* stream, MergeSet* set = nullptr);
 uint64_t scan_workspace_bytes(q1_placement placement, const LaunchShape& shape);
 
-// Zero device aggregate tables or a merge set (a fill kernel, safe inside graph capture).
-q1_status launch_zero(q1_device_aggregates* table, uint32_t count, void* stream);
-q1_status launch_zero(MergeSet* set, void* stream);
+// Zero device memory (whole 64-bit words; a fill kernel, safe inside graph capture).
+q1_status launch_zero(void* p, uint64_t bytes, void* stream);
 
 // Device-side generator: rows [0, rows) of `layout` into the device columns.
 q1_status launch_generate(q1_layout layout, uint64_t seed, uint64_t rows, const q1_columns& cols,
@@ -115,47 +127,54 @@ q1_status launch_build_filter(const uint16_t* ship, uint64_t rows, int32_t cutof
                               uint32_t* filter, void* stream);
 
 // Batched scan: one launch over many requests of one layout, TPC-H domain.  The device
-// buffer starts with a BatchHeader followed by `n` BatchDesc records.  Request r is cut
-// into the blocks launch_scan would run over its rows alone (256 lanes x
+// buffer starts with a BatchHeader followed by `n` BatchDesc records and the n first blocks.
+// Request r is cut into the blocks launch_scan would run over its rows alone (256 lanes x
 // tiles_per_thread tiles each); the blocks of all requests, in request order, form one
-// list of total_blocks entries.  A resident grid of G blocks works through the list with a
-// fixed stride (block b runs entries b, b + G, b + 2G, ...).  Entry v of request r merges
-// into spread table v mod 64 of the request (spread + 64 r) when r < spread_requests, and
-// into outs[r] otherwise; after the kernel, fold_spread (one block per request with spread
-// tables) adds each request's 64 tables into outs[r] and clears them.
+// list of total_blocks entries.  A grid of G blocks works through the list with a
+// fixed stride (block b runs entries b, b + G, b + 2G, ...).  The entries of a request merge
+// through tables of its own as a scan's blocks do, and the last of them stores the sums into
+// results[r], in pinned host memory.
 struct BatchDesc {
   q1_columns cols;
   uint64_t row_begin, row_end;
-  uint64_t block_begin;       // request's first entry in the block list
+  MergeTable* tables;         // table_mask + 1 of them, all zero
+  uint32_t table_mask;
+  uint32_t first_block;       // request's first entry in the block list
+  uint32_t blocks;            // its entries
   int32_t cutoff_day;
-  uint32_t pad;
 };
 struct BatchHeader {
-  uint64_t n;                 // requests
-  uint64_t total_blocks;      // entries of the block list (below 2^31)
+  uint32_t n;                 // requests
+  uint32_t with_rows;         // requests with entries
+  uint32_t total_blocks;      // entries of the block list (below 2^31)
   uint32_t tiles_per_thread;  // tiles of layout_tile_rows rows per lane and entry
-  uint32_t spread_requests;   // requests 0 .. spread_requests-1 merge through spread tables
+  uint64_t sequence;          // written to the done record at the end
   uint64_t pad[5];
 };
+// All zero before a batch and after it.
+struct alignas(128) BatchControl {
+  uint64_t clock_begin;       // device clock at the start of block 0
+  uint32_t requests_done;
+};
+// What a batch leaves in pinned host memory after its results.
+struct BatchDone {
+  uint64_t clock_begin, clock_end;
+  uint64_t sequence;          // written after everything else
+};
 constexpr uint32_t kBatchThreads = 256;
-// Requests of a batch that get spread tables: 64 x 384 B each, at most 24 MiB.
-constexpr uint32_t kBatchSpreadRequests = 1024;
+// The tables of a batch: a request with many blocks gets up to kSpreadTables of them while
+// all fit (32 MiB).
+constexpr uint32_t kBatchMaxTables = 65536;
 uint32_t layout_tile_rows(q1_layout layout);
 // The placement the batched kernel runs for a requested one (shared or in registers),
 // the largest rows per lane it accepts for it, and how many of its blocks fit on a CU.
 q1_placement batch_placement(q1_placement p);
 uint32_t batch_max_lane_rows(q1_placement p);
 uint32_t batch_blocks_per_cu(q1_layout layout, q1_placement p);
-// The batched kernel over the list in dev_buffer, then, with `spread` (spread_requests x
-// kSpreadTables tables, all zero), the fold of the first spread_requests requests' tables:
-// added into outs, or, with store_results (a device-visible pointer to the results in
-// pinned host memory, when every request has spread tables), stored there directly.
-q1_status launch_batch(q1_layout layout, q1_placement placement, BatchHeader* dev_buffer,
-                       q1_device_aggregates* outs, q1_device_aggregates* spread, uint32_t spread_requests,
-                       q1_device_aggregates* store_results, uint32_t blocks, uint32_t threads, void* stream);
-// The host function launch_batch launches for (layout, placement), e.g. to find its node in
-// a captured graph.
-const void* batch_kernel_function(q1_layout layout, q1_placement placement);
+// The batched kernel over the list in dev_buffer (of n requests).
+q1_status launch_batch(q1_layout layout, q1_placement placement, const BatchHeader* dev_buffer, uint32_t n,
+                       BatchControl* control, q1_device_aggregates* results, BatchDone* done, uint32_t blocks,
+                       void* stream);
 
 // The scratch of q1_enqueue_noalloc (q1_noalloc.hip): a static per-device array holding the
 // spread tables and kNoallocWorkspaceBytes of per-block tables for the global placement.

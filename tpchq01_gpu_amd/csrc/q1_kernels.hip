@@ -1,5 +1,4 @@
-// gfx950 utility kernels (zero fill, spread-table fold, generator, domain statistics,
-// pushdown producer), kernel dispatch and the host-side launch helpers of the TPC-H Q1
+// gfx950 utility kernels (zero fill, generator, domain check, pushdown producer), kernel dispatch and the host-side launch helpers of the TPC-H Q1
 // path.  The scan kernels themselves are in q1_scan.h, instantiated per layout.
 #include "q1_scan.h"
 
@@ -7,82 +6,11 @@ namespace q1 {
 namespace {
 
 // ------------------------------------------------------------------------------------
-// Utility kernels: zero fill, generator, domain statistics, pushdown producer.
+// Utility kernels: zero fill, generator, domain check, pushdown producer.
 // ------------------------------------------------------------------------------------
 __global__ void zero_words(uint64_t* p, uint64_t n) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
-}
-
-// Adds the kSpreadTables spread tables into `out` and clears them.  One block of four
-// wavefronts; lane k reads table k, so every load of the block is issued at once and the
-// sums are wavefront butterflies.  The 48 words of a table split over the waves:
-//   wave 0: sum_qty, sum_base_price       (words  0..11, 64-bit)
-//   wave 1: sum_disc_price lo/hi pairs    (words 12..23, 128-bit)
-//   wave 2: sum_charge lo/hi pairs        (words 24..35, 128-bit)
-//   wave 3: sum_disc, count               (words 36..47, 64-bit)
-// Each wave clears only the words it read, after its sums consumed them.
-static_assert(kSpreadTables == 64, "the fold gives each table one lane of a wavefront");
-static_assert(sizeof(q1_device_aggregates) == 48 * 8, "8 fields x 6 groups");
-// Block b folds tables[64 b .. 64 b + 63] into out[b] (one block for a scan's tables, one
-// per request for a batch's).  STORE: out[b] receives the sums with plain stores (every
-// word, zeros included) instead of atomic adds, for a destination that holds nothing yet:
-// a batch's results in pinned host memory, which the stores reach over PCIe.
-template <bool STORE>
-__device__ __forceinline__ void fold_tables(q1_device_aggregates* tables, q1_device_aggregates* out) {
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  uint64_t* mine = reinterpret_cast<uint64_t*>(tables + (uint64_t)blockIdx.x * kSpreadTables + lane) + wave * 12;
-  uint64_t* dst = reinterpret_cast<uint64_t*>(out + blockIdx.x) + wave * 12;
-  uint64_t v[12];
-#pragma unroll
-  for (int i = 0; i < 12; i++) v[i] = mine[i];
-  // After the butterflies every lane holds every sum; lane i then adds word (or pair) i,
-  // so the wave's destination atomics are issued together rather than one after another.
-  if (wave == 0 || wave == 3) {
-    uint64_t my = 0;
-#pragma unroll
-    for (int i = 0; i < 12; i++) {
-      const uint64_t sum = wave_sum_u64(v[i]);
-      my = lane == (uint32_t)i ? sum : my;
-    }
-    if (STORE) {
-      if (lane < 12) dst[lane] = my;
-    } else if (lane < 12 && my) {
-      atomicAdd((unsigned long long*)&dst[lane], (unsigned long long)my);
-    }
-  } else {
-    uint64_t my_lo = 0, my_hi = 0;
-#pragma unroll
-    for (int g = 0; g < kNumGroups; g++) {
-      uint64_t lo = v[g], hi = v[6 + g];
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) {
-        const uint64_t olo = __shfl_xor(lo, m, 64), ohi = __shfl_xor(hi, m, 64);
-        const uint64_t nlo = lo + olo;
-        hi += ohi + (nlo < lo);
-        lo = nlo;
-      }
-      my_lo = lane == (uint32_t)g ? lo : my_lo;
-      my_hi = lane == (uint32_t)g ? hi : my_hi;
-    }
-    if (lane < (uint32_t)kNumGroups) {
-      if (STORE) {
-        dst[lane] = my_lo;
-        dst[6 + lane] = my_hi;
-      } else {
-        atomic_add128(&dst[lane], &dst[6 + lane], my_lo, my_hi);
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 12; i++) mine[i] = 0;
-}
-
-__global__ void __launch_bounds__(256) fold_spread(q1_device_aggregates* tables, q1_device_aggregates* out) {
-  fold_tables<false>(tables, out);
-}
-__global__ void __launch_bounds__(256) fold_spread_store(q1_device_aggregates* tables, q1_device_aggregates* out) {
-  fold_tables<true>(tables, out);
 }
 
 // One thread per 32-row group writes the rows' values and the packed words of the group.
@@ -379,15 +307,8 @@ q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const
   const hipStream_t s = (hipStream_t)stream;
   const uint32_t nwaves = shape.threads / 64;
   ScanArgs a = args;
-  a.out_mask = 0;
-  a.set = nullptr;
-  a.dest = nullptr;
-  if (set && (a.host || shape.blocks >= kSpreadMinBlocks)) {
-    a.set = set;
-    a.dest = a.host ? nullptr : args.out;
-    a.out = set->tables;
-    a.out_mask = kSpreadTables - 1;
-  }
+  a.set = set && (a.host || shape.blocks >= kSpreadMinBlocks) ? set : nullptr;
+  a.table_mask = merge_tables(shape.blocks) - 1;
   if (fast) {
     const uint64_t lane_rows = (uint64_t)shape.tiles_per_thread * tile_rows(layout);
     const bool shared = placement == Q1_PLACE_PER_THREAD_SHARED_MEM;
@@ -409,19 +330,13 @@ q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const
   return hip_status(hipGetLastError());
 }
 
-static q1_status zero(void* p, uint64_t bytes, void* stream) {
+q1_status launch_zero(void* p, uint64_t bytes, void* stream) {
   const uint64_t n = bytes / 8;
   if (n == 0) return Q1_OK;
   hipLaunchKernelGGL(zero_words, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                      (uint64_t*)p, n);
   return hip_status(hipGetLastError());
 }
-
-q1_status launch_zero(q1_device_aggregates* table, uint32_t count, void* stream) {
-  return zero(table, (uint64_t)count * sizeof(q1_device_aggregates), stream);
-}
-
-q1_status launch_zero(MergeSet* set, void* stream) { return zero(set, sizeof(MergeSet), stream); }
 
 q1_status launch_generate(q1_layout layout, uint64_t seed, uint64_t rows, const q1_columns& cols,
                           void* stream) {
@@ -503,30 +418,16 @@ uint32_t batch_blocks_per_cu(q1_layout layout, q1_placement p) {
   return (uint32_t)per_cu;
 }
 
-q1_status launch_batch(q1_layout layout, q1_placement placement, BatchHeader* buf, q1_device_aggregates* outs,
-                       q1_device_aggregates* spread, uint32_t spread_requests, q1_device_aggregates* store_results,
-                       uint32_t blocks, uint32_t threads, void* stream) {
+q1_status launch_batch(q1_layout layout, q1_placement placement, const BatchHeader* buf, uint32_t n,
+                       BatchControl* control, q1_device_aggregates* results, BatchDone* done, uint32_t blocks,
+                       void* stream) {
   placement = batch_placement(placement);
-  if (threads != (uint32_t)kBatchBlock || blocks == 0 || (spread_requests && !spread) ||
-      (store_results && !spread_requests))
-    return Q1_EINVAL;
+  if (blocks == 0) return Q1_EINVAL;
   const BatchDesc* descs = reinterpret_cast<const BatchDesc*>(buf + 1);
-  void* args[] = {(void*)&buf, (void*)&descs, (void*)&outs, (void*)&spread};
-  const hipStream_t s = (hipStream_t)stream;
-  q1_status st = hip_status(
-      hipLaunchKernel(batch_kernel(layout, placement), dim3(blocks), dim3(threads), args, batch_lds(layout, placement), s));
-  if (st == Q1_OK && spread_requests) {
-    if (store_results)
-      hipLaunchKernelGGL(fold_spread_store, dim3(spread_requests), dim3(256), 0, s, spread, store_results);
-    else
-      hipLaunchKernelGGL(fold_spread, dim3(spread_requests), dim3(256), 0, s, spread, outs);
-    st = hip_status(hipGetLastError());
-  }
-  return st;
-}
-
-const void* batch_kernel_function(q1_layout layout, q1_placement placement) {
-  return batch_kernel(layout, batch_placement(placement));
+  const uint32_t* first = reinterpret_cast<const uint32_t*>(descs + n);
+  void* args[] = {(void*)&buf, (void*)&descs, (void*)&first, (void*)&control, (void*)&results, (void*)&done};
+  return hip_status(hipLaunchKernel(batch_kernel(layout, placement), dim3(blocks), dim3(kBatchBlock), args,
+                                    batch_lds(layout, placement), (hipStream_t)stream));
 }
 
 }  // namespace q1

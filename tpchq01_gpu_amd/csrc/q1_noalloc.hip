@@ -37,7 +37,7 @@ q1_status noalloc_setup(int device, void* stream) {
   void* p = nullptr;
   if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) return Q1_EDEVICE;
   // the merge set starts at zero (a fill kernel, no memset node)
-  q1_status s = launch_zero(static_cast<MergeSet*>(p), stream);
+  q1_status s = launch_zero(p, sizeof(MergeSet), stream);
   if (s == Q1_OK && hipStreamSynchronize((hipStream_t)stream) != hipSuccess) s = Q1_EDEVICE;
   if (s != Q1_OK) return s;
   g_scratch[device] = p;

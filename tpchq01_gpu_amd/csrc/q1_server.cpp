@@ -5,9 +5,9 @@
 //     joins the pending queue (bounded: Q1_EBUSY when full).
 //   scheduler thread: whenever an in-flight slot is free, admits pending requests in
 //     arrival order (optionally holding them back batch_window_us for more while other
-//     batches are still running) and launches them as one batch on the slot's stream (a
-//     hipGraph per slot: descriptor copy, batched kernel, and the fold of the requests'
-//     spread tables, which stores the results into the slot's pinned host buffer).
+//     batches are still running) and launches them as one batch on the slot's stream (the
+//     descriptor copy and the batched kernel, which stores the results into the slot's pinned
+//     host buffer).
 //   completion: a thread per slot waits for the slot's batch and publishes every result
 //     with its latency; a client waiting for a request of a launched batch waits for the
 //     device itself and publishes the batch first if it gets there first.
@@ -16,11 +16,10 @@
 // arrival order: two large scans sharing the device would both finish late, which is what
 // sets the latency tail.  Smaller requests batch beside them on the other slots, so a short
 // request that arrives while a large one runs starts at once instead of queueing behind it.
-// A batch runs the persistent batched kernel with its tuned grid, or one block per entry
-// when the batch has fewer entries than that grid.
+// A batch runs the batched kernel as q1_run_batch does.
 // Admission by device memory: a request pins its table's columns (counted once per table
 // while any of its requests is in flight) and its descriptor and result table.
-// Requests on tables outside the TPC-H value domain run alone through the 64-bit kernel.
+// Requests on tables outside the TPC-H value domain run alone through the any-value kernel.
 #include <algorithm>
 #include <chrono>
 #include <condition_variable>
@@ -53,7 +52,8 @@ struct Where {
   uint32_t batch_id;
 };
 
-uint64_t request_state_bytes() { return sizeof(q1::BatchDesc) + sizeof(q1_device_aggregates); }
+// A request's share of the memory budget beside its table (stated in q1_hip.h).
+uint64_t request_state_bytes() { return 480; }
 
 // Device bytes of a table's columns (what a request on it keeps resident).
 uint64_t table_bytes(const q1_table* t) {
@@ -67,21 +67,9 @@ uint64_t table_bytes(const q1_table* t) {
 struct Slot {
   hipStream_t stream = nullptr;
   hipEvent_t done = nullptr;
-  uint32_t capacity = 0;
-  q1_layout layout = Q1_LAYOUT_COMPRESSED;
-  bool single = false;           // a lone request through the 64-bit scan kernel
-  q1::BatchHeader* h_buf = nullptr;
-  q1::BatchHeader* d_buf = nullptr;
-  q1_device_aggregates* h_out = nullptr;
-  q1_device_aggregates* d_out = nullptr;
-  q1_device_aggregates* d_spread = nullptr;  // the batch's per-request spread tables
-  uint32_t spread_requests = 0;
-  q1_device_aggregates* h_out_dev = nullptr;  // h_out as the device addresses it
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  hipGraphNode_t kernel_node = nullptr;  // the batched kernel's node (its grid is set per batch)
-  hipKernelNodeParams kernel_params{};
-  uint32_t grid = 0;             // the batched kernel's tuned (persistent) grid
+  bool single = false;           // a lone request on a table outside the TPC-H domain
+  q1::BatchBuffers batched;      // the slot's batches
+  std::vector<q1_request> requests;  // of the batch being launched
   q1::MergeSet* set = nullptr;   // the slot's own merge set (lone requests)
   q1::HostResult* h_result = nullptr;  // pinned: what a lone request's kernel leaves
   q1::HostResult* h_result_dev = nullptr;  // ... as the device addresses it
@@ -117,94 +105,6 @@ struct q1_server {
 
 namespace {
 
-void free_slot_buffers(Slot& s) {
-  if (s.exec) (void)hipGraphExecDestroy(s.exec);
-  if (s.graph) (void)hipGraphDestroy(s.graph);
-  if (s.h_buf) (void)hipHostFree(s.h_buf);
-  if (s.h_out) (void)hipHostFree(s.h_out);
-  if (s.d_buf) (void)hipFree(s.d_buf);
-  if (s.d_out) (void)hipFree(s.d_out);
-  if (s.d_spread) (void)hipFree(s.d_spread);
-  s.d_spread = nullptr;
-  s.spread_requests = 0;
-  s.h_out_dev = nullptr;
-  s.exec = nullptr;
-  s.graph = nullptr;
-  s.kernel_node = nullptr;
-  s.h_buf = s.d_buf = nullptr;
-  s.h_out = s.d_out = nullptr;
-  s.capacity = 0;
-}
-
-// (Re)builds a slot's buffers and graph for `cap` requests of `layout`.
-q1_status prepare_slot(q1_server* sv, Slot& s, uint32_t cap, q1_layout layout) {
-  if (s.capacity == cap && s.layout == layout && s.exec) return Q1_OK;
-  free_slot_buffers(s);
-  const uint64_t bb = sizeof(q1::BatchHeader) + (uint64_t)cap * sizeof(q1::BatchDesc);
-  const uint64_t ob = (uint64_t)cap * sizeof(q1_device_aggregates);
-  s.spread_requests = std::min(cap, q1::kBatchSpreadRequests);
-  const uint64_t sb = (uint64_t)s.spread_requests * q1::kSpreadTables * sizeof(q1_device_aggregates);
-  if (hipHostMalloc(&s.h_buf, bb, hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc(&s.h_out, ob, hipHostMallocMapped) != hipSuccess ||
-      hipHostGetDevicePointer((void**)&s.h_out_dev, s.h_out, 0) != hipSuccess || hipMalloc(&s.d_buf, bb) != hipSuccess ||
-      hipMalloc(&s.d_out, ob) != hipSuccess || hipMalloc(&s.d_spread, sb) != hipSuccess) {
-    free_slot_buffers(s);
-    return Q1_ENOMEM;
-  }
-  // zeroed once, before the capture (every fold clears the tables it read)
-  if (hipMemsetAsync(s.d_spread, 0, sb, s.stream) != hipSuccess || hipStreamSynchronize(s.stream) != hipSuccess) {
-    free_slot_buffers(s);
-    return Q1_EDEVICE;
-  }
-  std::memset(s.h_buf, 0, bb);
-  const uint32_t blocks = q1::batch_default_blocks(sv->ctx, layout, sv->placement);
-  q1_status st = Q1_OK;
-  if (hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal) != hipSuccess) st = Q1_EDEVICE;
-  if (st == Q1_OK && hipMemcpyAsync(s.d_buf, s.h_buf, bb, hipMemcpyHostToDevice, s.stream) != hipSuccess) st = Q1_EDEVICE;
-  // With spread tables for every request the fold stores the results into h_out itself.
-  const bool store = s.spread_requests == cap;
-  if (st == Q1_OK && !store) st = q1::launch_zero(s.d_out, cap, s.stream);
-  if (st == Q1_OK)
-    st = q1::launch_batch(layout, sv->placement, s.d_buf, s.d_out, s.d_spread, s.spread_requests,
-                          store ? s.h_out_dev : nullptr, blocks, q1::kBatchThreads, s.stream);
-  if (st == Q1_OK && !store && hipMemcpyAsync(s.h_out, s.d_out, ob, hipMemcpyDeviceToHost, s.stream) != hipSuccess)
-    st = Q1_EDEVICE;
-  hipGraph_t g = nullptr;
-  const hipError_t ec = hipStreamEndCapture(s.stream, &g);
-  if (st != Q1_OK || ec != hipSuccess || !g) {
-    if (g) (void)hipGraphDestroy(g);
-    free_slot_buffers(s);
-    return Q1_EDEVICE;
-  }
-  s.graph = g;
-  if (hipGraphInstantiate(&s.exec, g, nullptr, nullptr, 0) != hipSuccess) {
-    free_slot_buffers(s);
-    return Q1_EDEVICE;
-  }
-  // The batched kernel's node, whose grid each launch sets to the batch's entries.  If it
-  // cannot be found the captured (resident) grid stays.
-  size_t count = 0;
-  if (hipGraphGetNodes(g, nullptr, &count) == hipSuccess && count) {
-    std::vector<hipGraphNode_t> nodes(count);
-    if (hipGraphGetNodes(g, nodes.data(), &count) == hipSuccess) {
-      const void* fn = q1::batch_kernel_function(layout, sv->placement);
-      for (hipGraphNode_t node : nodes) {
-        hipGraphNodeType type;
-        hipKernelNodeParams kp{};
-        if (hipGraphNodeGetType(node, &type) == hipSuccess && type == hipGraphNodeTypeKernel &&
-            hipGraphKernelNodeGetParams(node, &kp) == hipSuccess && kp.func == fn) {
-          s.kernel_node = node;
-          s.kernel_params = kp;
-        }
-      }
-    }
-  }
-  s.grid = blocks;
-  s.capacity = cap;
-  s.layout = layout;
-  return Q1_OK;
-}
-
 // Launches the slot's batch; called with the server lock released, on the server's device.
 q1_status launch_slot(q1_server* sv, Slot& s) {
   const uint32_t n = (uint32_t)s.batch.size();
@@ -212,7 +112,7 @@ q1_status launch_slot(q1_server* sv, Slot& s) {
   s.lone = false;
   if (n == 1) {
     // A lone request runs the scan kernel of q1_run with its tuned launch (the batched
-    // kernel's list of entries buys nothing for one request), or the 64-bit scan kernel on a
+    // kernel's list of entries buys nothing for one request), or the any-value kernel on a
     // table outside the TPC-H domain, merging through the slot's own set.
     const q1_request& r = s.batch[0].req;
     const q1_placement p =
@@ -240,35 +140,19 @@ q1_status launch_slot(q1_server* sv, Slot& s) {
       return st;
     }
   }
-  uint32_t cap = 16;
-  while (cap < n) cap <<= 1;
-  q1_status st = prepare_slot(sv, s, cap, t0->layout);
-  if (st != Q1_OK) return st;
-  const uint32_t lane_rows = q1::batch_lane_rows(sv->ctx, t0->layout, sv->placement);
-  q1::BatchDesc* d = reinterpret_cast<q1::BatchDesc*>(s.h_buf + 1);
-  uint64_t entries = 0;
-  for (uint32_t i = 0; i < n; i++) entries += q1::batch_describe(&d[i], s.batch[i].req, entries, lane_rows);
-  if (entries >= (1ull << 31)) return Q1_EINVAL;
-  s.h_buf->n = n;
-  s.h_buf->total_blocks = entries;
-  s.h_buf->tiles_per_thread = lane_rows / q1::layout_tile_rows(t0->layout);
-  s.h_buf->spread_requests = s.spread_requests;
-  if (s.kernel_node) {
-    // The tuned persistent grid, or one block per entry for a batch with fewer entries
-    // (block b then runs entry b only).
-    hipKernelNodeParams kp = s.kernel_params;
-    kp.gridDim = dim3((uint32_t)std::min<uint64_t>(std::max<uint64_t>(entries, 1), s.grid));
-    if (hipGraphExecKernelNodeSetParams(s.exec, s.kernel_node, &kp) != hipSuccess) s.kernel_node = nullptr;
-  }
-  if (hipGraphLaunch(s.exec, s.stream) != hipSuccess || hipEventRecord(s.done, s.stream) != hipSuccess) {
-    // The graph may still be reading the slot's pinned buffers: let it finish before the
-    // caller frees the slot for the next batch, and rebuild the slot (its spread tables
-    // may hold partial sums).
+  s.requests.clear();
+  for (const Pending& p : s.batch) s.requests.push_back(p.req);
+  uint32_t lane_rows = 0, grid = 0;
+  const char* why = "";
+  q1_status st = q1::batch_launch(sv->ctx, &s.batched, s.requests.data(), n, sv->placement, 0, 0, s.stream, &lane_rows,
+                                  &grid, &why);
+  if (st == Q1_OK && hipEventRecord(s.done, s.stream) != hipSuccess) {
+    // The kernel may still be writing the slot's pinned results: let it finish before the
+    // caller frees the slot for the next batch.
     (void)hipStreamSynchronize(s.stream);
-    free_slot_buffers(s);
-    return Q1_EDEVICE;
+    st = Q1_EDEVICE;
   }
-  return Q1_OK;
+  return st;
 }
 
 // Device bytes admitting `r` would add to what the in-flight work pins.
@@ -308,7 +192,7 @@ void publish(q1_server* sv, Slot& s, q1_status st, uint32_t id) {
   for (size_t i = 0; i < s.batch.size(); i++) {
     Finished f;
     f.status = st;
-    if (st == Q1_OK) q1_aggregates_to_result(s.lone ? &s.h_result->sums : &s.h_out[i], &f.result);
+    if (st == Q1_OK) q1_aggregates_to_result(s.lone ? &s.h_result->sums : &s.batched.h_out[i], &f.result);
     f.stats.submit_to_start_us =
         std::chrono::duration<double, std::micro>(s.started - s.batch[i].submitted).count();
     f.stats.latency_us = std::chrono::duration<double, std::micro>(now - s.batch[i].submitted).count();
@@ -632,7 +516,7 @@ void q1_server_destroy(q1_server* sv) {
     if (s.waiter.joinable()) s.waiter.join();
   for (auto& s : sv->slots) {
     if (s.stream) (void)hipStreamSynchronize(s.stream);
-    free_slot_buffers(s);
+    q1::batch_free(&s.batched);
     if (s.set) (void)hipFree(s.set);
     if (s.h_result) (void)hipHostFree(s.h_result);
     if (s.done) (void)hipEventDestroy(s.done);

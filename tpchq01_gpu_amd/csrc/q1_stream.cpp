@@ -74,7 +74,7 @@ static q1_status prepare(q1_ctx* ctx, q1_layout layout, uint64_t chunk_rows, int
     MergeSet* set = nullptr;
     if (hipMalloc(&set, sizeof(MergeSet)) != hipSuccess) return give_up(Q1_ENOMEM, "staging allocation failed");
     st->set.push_back(set);
-    if (launch_zero(set, s) != Q1_OK) return give_up(Q1_EDEVICE, "zero kernel failed");
+    if (launch_zero(set, sizeof(MergeSet), s) != Q1_OK) return give_up(Q1_EDEVICE, "zero kernel failed");
     q1_columns c{};
     const void** slots[8] = {&c.ship_date, &c.quantity, &c.extended_price, &c.discount,
                              &c.tax, &c.return_flag, &c.line_status, &c.filter};
@@ -145,7 +145,7 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
       (void)hipStreamSynchronize(ctx->stream);
       return fail(ctx, code, why);
     };
-    s = launch_zero(ctx->d_aggr, 1, ctx->stream);
+    s = launch_zero(ctx->d_aggr, sizeof(q1_device_aggregates), ctx->stream);
     if (s != Q1_OK) return fail(ctx, s, "zero kernel failed");
     if (hipEventRecord(ctx->ev_begin, ctx->stream) != hipSuccess) return fail(ctx, Q1_EDEVICE, "event record failed");
     for (hipStream_t ss : st->s)
