@@ -63,3 +63,36 @@ def test_grids_of_every_merge(ctx, oracle, layout, wide):
                 q1.lib.q1_aggregates_to_result(C.byref(got), C.byref(r))
                 assert _as_dicts(q1.result_to_list(r)) == [{k: 3 * v for k, v in g.items()} for g in want]
     t.free()
+
+
+def test_more_launches_in_flight_than_merge_sets(ctx, oracle):
+    """1,200 launches enqueued at once on four streams, more than the 256 merge sets: the ones
+    without a set merge directly, and the next ones find their sets zero."""
+    import torch
+    rows, chunk = 400_000, 200_000
+    ref, cols = _columns(q1.COMPRESSED, rows, False)
+    want, _ = oracle.naive(ref, 0, rows, 729999)
+    t = ctx.upload(q1.COMPRESSED, cols, rows)
+    dev = t.device_columns()
+    launch = q1.make_launch(LANES, LANE_ROWS, 0, q1.LAUNCH_ASSUME_TPCH_DOMAIN)   # 196 blocks each
+    streams = [torch.cuda.Stream() for _ in range(4)]
+    for turn in range(2):
+        sums = [torch.zeros(48, dtype=torch.int64, device="cuda") for _ in streams]
+        busy = torch.zeros(1 << 28, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        for s in streams:       # the launches queue up behind these
+            with torch.cuda.stream(s):
+                for _ in range(20):
+                    busy.add_(1)
+        for i in range(300):
+            for s, out in zip(streams, sums):
+                ctx.check(q1.lib.q1_enqueue(ctx.handle, q1.PER_THREAD_SHARED_MEM, q1.COMPRESSED, C.byref(launch),
+                                            out.data_ptr(), C.byref(dev), chunk * (i % 2), chunk, 729999,
+                                            s.cuda_stream), "q1_enqueue")
+        torch.cuda.synchronize()
+        for out in sums:
+            got = q1.DeviceAggregates.from_buffer_copy(np.ascontiguousarray(out.cpu().numpy()).tobytes())
+            r = q1.Result()
+            q1.lib.q1_aggregates_to_result(C.byref(got), C.byref(r))
+            assert _as_dicts(q1.result_to_list(r)) == [{k: 150 * v for k, v in g.items()} for g in want]
+    t.free()

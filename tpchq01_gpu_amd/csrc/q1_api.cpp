@@ -47,16 +47,24 @@ q1_placement resolve_placement(q1_ctx* ctx, q1_layout layout, q1_placement p) {
   return p == Q1_PLACE_AUTO ? ctx->best[layout] : p;
 }
 
-// The any-value kernel's shape: 128 lanes x 128 rows, or 64 rows where 128 would give fewer
-// than 16 blocks per compute unit (the last of few rounds of large blocks leaves compute
-// units idle), and less only to have 4 blocks per compute unit (a block's fixed cost shows).
-// Compressed / uncompressed / reference at 60M rows: 128 x 64 93 / 190 / 341 us, 128 x 128
-// 98 / 200 / 354, 256 x 128 97 / 199 / 371; 6M rows: 128 x 32 20 / 33 / 46, 128 x 64 20 / 30 /
-// 45, 128 x 128 27 / 44 / 48; 1M rows: 128 x 16 12 / 14 / 15, 128 x 64 15 / 21 / 21.  256 lanes
-// are 1 % faster on 600M compressed rows and 12 % slower on 60M reference rows, whose
-// tables then leave a compute unit one block.
-constexpr uint32_t kAnyThreads = 128, kAnyTuples = 128;
-constexpr uint64_t kAnyBlocksPerCu = 16;
+// The any-value kernel's shape.  Lanes per block: 256 for the compressed layouts, 128 for the
+// others, whose LDS tables of 61 and 86 KB per 256 lanes leave a compute unit two blocks or
+// one (60M reference rows 371 us with 256 lanes, 354 with 128; 2M compressed rows 10.0 and
+// 11.2 us, 600M 0.82 and 0.83 ms).  Rows per lane: 128, or 64 where 128 would give fewer than
+// 2048 lanes per compute unit (the last of few rounds of large blocks leaves compute units
+// idle), and less only to have half the lanes whose tables fit a compute unit's LDS (a
+// block's fixed cost shows; 2M reference rows 18.9 us with 32 rows per lane, 23.3 with 16,
+// whose 1,024 blocks are a third more than fit).
+// Compressed / uncompressed / reference: 60M rows with 64 rows per lane 94 / 190 / 341 us,
+// with 128 98 / 200 / 354; 6M rows with 32 18 / 33 / 46, with 64 21 / 30 / 45, with 128 29 /
+// 44 / 48; 1M rows with 16 12 / 14 / 15, with 64 15 / 21 / 21.
+constexpr uint32_t kAnyTuples = 128, kAnyManyLanes = 2048;
+static uint32_t any_value_lanes(q1_layout l) {
+  return l == Q1_LAYOUT_REFERENCE ? 192 : l == Q1_LAYOUT_UNCOMPRESSED ? 320 : 512;
+}
+static uint32_t any_value_threads(q1_layout l) {
+  return l == Q1_LAYOUT_COMPRESSED || l == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? 256 : 128;
+}
 
 // The tuned shape for a range of `rows` rows: of the shapes tuned at several row counts,
 // the one whose row count is nearest by ratio (the larger on a tie); the single tuned
@@ -80,7 +88,7 @@ static q1_launch tuned_for_rows(const q1_ctx* ctx, q1_layout layout, q1_placemen
 
 void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, uint64_t rows, const q1_launch* in,
                     q1_launch* out, bool table) {
-  q1_launch t{kAnyThreads, kAnyTuples, 0, 0};
+  q1_launch t{any_value_threads(layout), kAnyTuples, 0, 0};
   if (fast)
     t = tuned_for_rows(ctx, layout, p, rows);
   else if (in && in->num_blocks)
@@ -93,16 +101,20 @@ void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, ui
   // A caller-chosen value is kept as given.
   if ((in && in->tuples_per_thread) || out->num_blocks) return;
   // A range smaller than the row counts the shape was tuned at halves its tuples_per_thread
-  // until the grid has at least `per_cu` blocks per compute unit, so small requests still
-  // spread over the whole chip.
+  // until the grid has at least `lanes` lanes (for the tuned shapes 4 blocks) per compute unit,
+  // so small requests still spread over the whole chip.
   const uint64_t tpb = out->threads_per_block ? out->threads_per_block : 256;
-  auto halve = [&](uint64_t per_cu, uint32_t least) {
-    const uint64_t want = per_cu * (uint64_t)(ctx->compute_units > 0 ? ctx->compute_units : 256);
-    while (out->tuples_per_thread > least && rows < want * tpb * out->tuples_per_thread)
+  auto halve = [&](uint64_t lanes, uint32_t least) {
+    const uint64_t want = lanes * (uint64_t)(ctx->compute_units > 0 ? ctx->compute_units : 256);
+    while (out->tuples_per_thread > least && rows < want * out->tuples_per_thread)
       out->tuples_per_thread = std::max<uint32_t>(16, (out->tuples_per_thread / 2) & ~15u);
   };
-  if (!fast) halve(kAnyBlocksPerCu, kAnyTuples / 2);
-  halve(4, 16);
+  if (fast) {
+    halve(4 * tpb, 16);
+  } else {
+    halve(kAnyManyLanes, kAnyTuples / 2);
+    halve(any_value_lanes(layout), 16);
+  }
 }
 
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
@@ -118,53 +130,53 @@ q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
   return Q1_OK;
 }
 
-// The merge set of a caller's stream for a large launch, made on the stream's first such
-// launch; nullptr (merge directly) while the stream is being captured into a
-// graph, where nothing may be allocated or waited for outside the capture, once
-// kMaxStreamSpreads streams have one, or if making it fails.  A stream that has
-// one first waits for the event of its last use.
-static StreamSpread* stream_spread(q1_ctx* ctx, void* stream) {
+constexpr int kPoolWaitMs = 2;  // longer than any scan of 1.5G compressed rows
+
+// A free set of the pool for a large launch on a caller's stream, its index in *index; nullptr
+// (merge directly) while the stream is being captured into a graph, whose replays would use
+// the set again, or when the sets stay in flight.
+static MergeSet* pool_set(q1_ctx* ctx, void* stream, size_t* index) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
-  auto it = ctx->stream_spreads.find(stream);
-  if (it != ctx->stream_spreads.end()) {
-    StreamSpread& ss = it->second;
-    if (!ss.usable) return nullptr;
-    if (hipStreamWaitEvent((hipStream_t)stream, ss.done, 0) != hipSuccess) {
-      ss.usable = false;
-      return nullptr;
-    }
-    return &ss;
+  SetPool& pool = ctx->pool;
+  // Launches on one stream end in order, so the set after the last one given is the first to
+  // come free unless streams of very different pace share the pool.
+  auto free_set = [&](size_t i) { return __atomic_load_n(&pool.done[i], __ATOMIC_ACQUIRE) == pool.last[i]; };
+  auto take = [&](size_t i) {
+    pool.cursor = (i + 1) % kPoolSets;
+    pool.stalled = false;
+    *index = i;
+    return pool.sets + i;
+  };
+  for (size_t looked = 0; looked < 8; looked++)
+    if (free_set((pool.cursor + looked) % kPoolSets)) return take((pool.cursor + looked) % kPoolSets);
+  // All in flight: the caller is 256 launches ahead of the device.  Waiting for the oldest
+  // keeps it there; a direct merge would cost this launch up to 0.03 us per block.  A stream
+  // that does not move (it may be waiting for the caller) is waited for once only.
+  if (!pool.stalled) {
+    const size_t i = pool.cursor;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(kPoolWaitMs);
+    while (!free_set(i) && std::chrono::steady_clock::now() < until) __builtin_ia32_pause();
+    if (free_set(i)) return take(i);
+    pool.stalled = true;
   }
-  if (ctx->stream_spreads.size() >= kMaxStreamSpreads) return nullptr;
-  StreamSpread ss;
-  if (hipMalloc(&ss.set, sizeof(MergeSet)) != hipSuccess) return nullptr;
-  if (hipEventCreateWithFlags(&ss.done, hipEventDisableTiming) != hipSuccess) {
-    (void)hipFree(ss.set);
-    return nullptr;
-  }
-  return &ctx->stream_spreads.emplace(stream, ss).first->second;
+  pool.cursor = (pool.cursor + 8) % kPoolSets;
+  return nullptr;
 }
 
-q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
+q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& args,
                   const LaunchShape& shape, void* stream) {
-  // Launches on one stream run one after another, so they can share one merge set: the
-  // context's for the context stream, a set of the stream's own for a caller's stream
-  // (large launches only; the others merge directly).
-  MergeSet* set = nullptr;
-  StreamSpread* other = nullptr;
-  if (stream == (void*)ctx->stream) {
-    set = ctx->set;
-  } else if (shape.blocks >= kSpreadMinBlocks && (other = stream_spread(ctx, stream))) {
-    set = other->set;
-    if (!other->zeroed) {
-      const q1_status z = launch_zero(set, sizeof(MergeSet), stream);
-      if (z != Q1_OK) return z;
-      other->zeroed = true;
-    }
+  if (stream == (void*)ctx->stream)  // its launches run one after another
+    return launch_scan(placement, layout, fast, args, shape, ctx->workspace, stream, ctx->set);
+  ScanArgs a = args;
+  size_t i = 0;
+  MergeSet* set = shape.blocks >= kSpreadMinBlocks ? pool_set(ctx, stream, &i) : nullptr;
+  if (set) {
+    a.done = ctx->pool.done_dev + i;
+    a.sequence = ++ctx->pool.sequence;
   }
   const q1_status s = launch_scan(placement, layout, fast, a, shape, ctx->workspace, stream, set);
-  if (other && hipEventRecord(other->done, (hipStream_t)stream) != hipSuccess) other->usable = false;
+  if (s == Q1_OK && set) ctx->pool.last[i] = a.sequence;
   return s;
 }
 
@@ -393,6 +405,12 @@ q1_status q1_init(int device, q1_ctx** out) {
   ok = ok && hipDeviceGetAttribute(&ctx->clock_khz, hipDeviceAttributeWallClockRate, device) == hipSuccess;
   ok = ok && hipMalloc(&ctx->set, sizeof(MergeSet)) == hipSuccess;
   ok = ok && hipMemset(ctx->set, 0, sizeof(MergeSet)) == hipSuccess;
+  SetPool& pool = ctx->pool;
+  ok = ok && hipMalloc(&pool.sets, kPoolSets * sizeof(MergeSet)) == hipSuccess &&
+       hipMemset(pool.sets, 0, kPoolSets * sizeof(MergeSet)) == hipSuccess &&
+       hipHostMalloc(&pool.done, kPoolSets * sizeof(uint64_t), hipHostMallocMapped) == hipSuccess &&
+       hipHostGetDevicePointer((void**)&pool.done_dev, pool.done, 0) == hipSuccess;
+  if (ok) std::memset(pool.done, 0, kPoolSets * sizeof(uint64_t));
   // the scratch of q1_enqueue_noalloc on this device (once per device and process)
   ok = ok && noalloc_setup(device, ctx->stream) == Q1_OK;
   ok = ok && hipDeviceSynchronize() == hipSuccess;
@@ -428,13 +446,9 @@ void q1_shutdown(q1_ctx* ctx) {
   stream_state_release(ctx);
   if (ctx->workspace) (void)hipFree(ctx->workspace);
   if (ctx->set) (void)hipFree(ctx->set);
-  for (auto& kv : ctx->stream_spreads) {
-    // the caller's stream may still run the last launch that used them
-    (void)hipEventSynchronize(kv.second.done);
-    (void)hipFree(kv.second.set);
-    (void)hipEventDestroy(kv.second.done);
-  }
-  ctx->stream_spreads.clear();
+  if (ctx->pool.sets) (void)hipDeviceSynchronize();  // callers' streams may still use the pool
+  if (ctx->pool.sets) (void)hipFree(ctx->pool.sets);
+  if (ctx->pool.done) (void)hipHostFree(ctx->pool.done);
   if (ctx->h_aggr) (void)hipHostFree(ctx->h_aggr);
   if (ctx->h_outside) (void)hipHostFree(ctx->h_outside);
   if (ctx->h_result) (void)hipHostFree(ctx->h_result);

@@ -5,7 +5,6 @@
 
 #include <mutex>
 #include <string>
-#include <unordered_map>
 #include <unordered_set>
 #include <vector>
 
@@ -31,18 +30,20 @@ constexpr int kStreamCount = 4;
 namespace q1 {
 struct BatchBuffers;
 struct StreamState;     // q1_stream.cpp: the host-resident streaming pipeline
-// The merge set of one caller stream (q1_enqueue on a stream other than the context's).
-// `done` is recorded after every launch that uses it and the next launch waits for it,
-// so a stream created at the address of a destroyed one never overlaps the old stream's
-// last use; `usable` is cleared if that bookkeeping ever fails.
-struct StreamSpread {
-  MergeSet* set = nullptr;
-  hipEvent_t done = nullptr;
-  bool zeroed = false;   // the first launch that uses it clears it
-  bool usable = true;
+// Merge sets for launches on callers' streams: each launch in flight has one of its own, so
+// nothing orders the streams (or a destroyed stream and one made at its address).  A launch's
+// last block writes the launch's number to its set's word in `done`, and a set is free again
+// once the number is there.
+constexpr size_t kPoolSets = 256;  
+struct SetPool {
+  MergeSet* sets = nullptr;       // kPoolSets
+  uint64_t* done = nullptr;       // pinned words
+  uint64_t* done_dev = nullptr;   // ... as the device addresses them
+  uint64_t last[kPoolSets] = {};  // number of the last launch given the set
+  uint64_t sequence = 0;
+  size_t cursor = 0;
+  bool stalled = false;           // the last wait for a set was in vain
 };
-// Caller streams that get a merge set; launches on further streams merge directly.
-constexpr size_t kMaxStreamSpreads = 16;
 // A launch shape tuned on ranges of `rows` rows ("launch_at" lines of the tuning file).
 struct SizedLaunch {
   uint64_t rows;
@@ -83,7 +84,7 @@ struct q1_ctx {
   q1::BatchBuffers* batch = nullptr;       // q1_run_batch's buffers
   q1::StreamState* streaming = nullptr;    // cached staging buffers and streams of q1_run_streaming
   q1::MergeSet* set = nullptr;             // merge set of the context stream
-  std::unordered_map<void*, q1::StreamSpread> stream_spreads;  // caller streams' merge sets
+  q1::SetPool pool;                        // merge sets of launches on callers' streams
   std::unordered_set<q1_table*> tables;    // live tables (released device memory at shutdown)
   std::mutex lock;                         // serialises calls that share the context stream
 };
@@ -100,7 +101,8 @@ void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, ui
 inline bool in_domain_flag(const q1_launch* l) { return l && (l->flags & Q1_LAUNCH_ASSUME_TPCH_DOMAIN); }
 uint64_t algorithmic_bytes(q1_layout layout, uint64_t rows);
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes);
-// launch_scan with the merge set of `stream` (the context's or a caller's).
+// launch_scan with the context's merge set on the context stream, one of the pool's on a
+// caller's.
 q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
                   const LaunchShape& shape, void* stream);
 // The same on the context stream with the sums going to ctx->h_result, and the wait for

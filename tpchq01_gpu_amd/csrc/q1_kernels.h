@@ -77,10 +77,12 @@ struct ScanArgs {
   // Set by launch_scan: without a merge set the blocks add into *out.  With one, block b
   // merges into the set's table b & table_mask, and the last block folds the tables into
   // *host (stored, with the clocks and `sequence`; host memory as the device addresses it),
-  // or, when host is null, into *out (added).
+  // or, when host is null, into *out (added; `sequence` then goes to *done if not null, once
+  // the set is zero again).
   uint32_t table_mask;
   MergeSet* set;
   HostResult* host;
+  uint64_t* done;
   uint64_t sequence;
 };
 

@@ -321,13 +321,15 @@ q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const
                    : shared                     ? shared_table_bytes(shape.threads)
                                                 : 0;
     lds += nwaves * kNumGroups * NF * 8;
-    hipLaunchKernelGGL(fast_kernel(layout, variant, shape.threads), dim3(shape.blocks), dim3(shape.threads), lds,
-                       s, a, shape.tiles_per_thread, (uint64_t*)workspace);
-  } else {
-    hipLaunchKernelGGL(any_kernel(layout, shape.threads), dim3(shape.blocks), dim3(shape.threads),
-                       any_kernel_lds(layout, shape.threads), s, a, shape.tiles_per_thread);
+    uint32_t tiles = shape.tiles_per_thread;
+    void* params[] = {(void*)&a, (void*)&tiles, (void*)&workspace};
+    return hip_status(hipLaunchKernel((const void*)fast_kernel(layout, variant, shape.threads), dim3(shape.blocks),
+                                      dim3(shape.threads), params, lds, s));
   }
-  return hip_status(hipGetLastError());
+  uint32_t tiles = shape.tiles_per_thread;
+  void* params[] = {(void*)&a, (void*)&tiles};
+  return hip_status(hipLaunchKernel((const void*)any_kernel(layout, shape.threads), dim3(shape.blocks),
+                                    dim3(shape.threads), params, any_kernel_lds(layout, shape.threads), s));
 }
 
 q1_status launch_zero(void* p, uint64_t bytes, void* stream) {

@@ -1482,6 +1482,10 @@ __device__ __forceinline__ void finish_scan(const ScanArgs& a) {
     } else if (lane < 48 && !high && sum) {
       atomicAdd((unsigned long long*)(d + lane), (unsigned long long)sum);
     }
+    if (a.done) {
+      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (lane == 0) store_host(a.done, a.sequence);
+    }
     return;
   }
   // Everything but the sequence number, then the number.
