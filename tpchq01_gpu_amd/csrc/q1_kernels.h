@@ -25,6 +25,11 @@ bool domain_is_tpch(q1_layout layout, const Domain& d);
 constexpr uint64_t kRowAlign = 128;
 inline uint64_t align_rows_down(uint64_t row) { return row / kRowAlign * kRowAlign; }
 
+// The tiles the host counts in (q1_launch's tuples_per_thread is a whole number of them), each
+// split into the smaller tiles the kernels read.
+template <int L>
+constexpr int kHostTileRows = L == Q1_LAYOUT_REFERENCE ? 4 : L == Q1_LAYOUT_UNCOMPRESSED ? 8 : 16;
+
 struct LaunchShape {
   uint32_t blocks, threads, tiles_per_thread;
 };

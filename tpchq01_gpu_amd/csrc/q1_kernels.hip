@@ -232,7 +232,9 @@ uint32_t any_kernel_lds(q1_layout l, uint32_t threads) {
 }
 
 uint32_t tile_rows(q1_layout l) {
-  return l == Q1_LAYOUT_REFERENCE ? 4u : (l == Q1_LAYOUT_UNCOMPRESSED ? 8u : 16u);
+  return l == Q1_LAYOUT_REFERENCE      ? kHostTileRows<Q1_LAYOUT_REFERENCE>
+         : l == Q1_LAYOUT_UNCOMPRESSED ? kHostTileRows<Q1_LAYOUT_UNCOMPRESSED>
+                                       : kHostTileRows<Q1_LAYOUT_COMPRESSED>;
 }
 
 q1_status hip_status(hipError_t e) { return e == hipSuccess ? Q1_OK : Q1_EDEVICE; }

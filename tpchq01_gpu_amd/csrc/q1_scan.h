@@ -2,21 +2,19 @@
 // shared by the translation units that instantiate it, one per column layout
 // (q1_scan_<layout>.hip), so the layouts compile in parallel.
 //
-//
 // Work decomposition (all layouts, all placements):
-//   * rows are cut into lane tiles of TILE consecutive rows (16 for the compressed layouts,
-//     8 for the uncompressed one, 4 for the reference layout); the shared placement reads
-//     the compressed layouts in 4-row tiles instead, four in flight per lane, so that every
-//     load instruction of a wavefront reads whole cache lines and the loads can be
+//   * rows are cut into lane tiles of consecutive rows (4 for the compressed layouts, 2 for
+//     the uncompressed and reference ones), four in flight per lane, so that every load
+//     instruction of a wavefront reads whole cache lines of its column and the loads can be
 //     non-temporal;
 //   * a block owns tiles_per_thread * blockDim consecutive tiles; in iteration k thread i
 //     takes tile base + k*blockDim + i, so each load instruction of a wavefront covers one
-//     contiguous stretch of every column (coalesced 16-byte loads);
-//   * only the first and the last tile of a range can be partial: those take a guarded
-//     per-row path, every other tile reads whole vectors;
+//     contiguous stretch of a column;
+//   * only the first and the last tile of a range can be partial: groups of tiles at the
+//     range's ends take a guarded path, every other one straight-line loads and rows;
 //   * each placement keeps its partial aggregation table in its own memory space
 //     (registers, scratch, LDS or global memory); at the end of the block the per-lane
-//     partials are reduced across the wavefront with ds_bpermute butterflies, across the
+//     partials are reduced across the wavefront, across the
 //     block through LDS in 128-bit arithmetic, and merged into the destination table with
 //     one set of 64-bit atomics per block (128-bit sums as carry-propagating word pairs).
 //
@@ -135,111 +133,7 @@ __device__ __forceinline__ uint2 nt_load(const uint2* p) {
 __device__ __forceinline__ uint32_t nt_load(const uint32_t* p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ uint32_t nt_load(const uint16_t* p) { return __builtin_nontemporal_load(p); }
 
-// Q1_LAYOUT_COMPRESSED / Q1_LAYOUT_COMPRESSED_PUSHDOWN: 16 rows per tile.
-template <bool PUSHDOWN>
-struct CompressedTile {
-  static constexpr int TILE = 16;
-  static constexpr int GROUP = 1;
-  uint4 sd[2];      // 16 x uint16 ship dates (unused for pushdown)
-  uint4 q, d, x;    // 16 x uint8 quantity, discount, tax
-  uint4 p[4];       // 16 x uint32 extended price
-  uint32_t rf;      // 16 x 2-bit return flag codes
-  uint32_t ls;      // 16 x 1-bit line status codes (low half-word)
-  uint32_t flt;     // 16 x filter bits (pushdown)
-
-  __device__ __forceinline__ void load(const q1_columns& c, uint64_t t) {
-    if (!PUSHDOWN) {
-      const uint4* s = reinterpret_cast<const uint4*>(c.ship_date);
-      sd[0] = s[2 * t];
-      sd[1] = s[2 * t + 1];
-    } else {
-      flt = reinterpret_cast<const uint16_t*>(c.filter)[t];
-    }
-    q = reinterpret_cast<const uint4*>(c.quantity)[t];
-    d = reinterpret_cast<const uint4*>(c.discount)[t];
-    x = reinterpret_cast<const uint4*>(c.tax)[t];
-    const uint4* pp = reinterpret_cast<const uint4*>(c.extended_price);
-#pragma unroll
-    for (int k = 0; k < 4; k++) p[k] = pp[4 * t + k];
-    rf = reinterpret_cast<const uint32_t*>(c.return_flag)[t];
-    ls = reinterpret_cast<const uint16_t*>(c.line_status)[t];
-  }
-  __device__ __forceinline__ void load_edge(const q1_columns& c, uint64_t t, uint32_t valid) {
-    sd[0] = sd[1] = q = d = x = p[0] = p[1] = p[2] = p[3] = make_uint4(0, 0, 0, 0);
-    rf = ls = flt = 0;
-    // The packed words of a tile hold rows of the tile only, so reading them for a tile
-    // that has at least one valid row stays inside the column.
-    if (valid) {
-      rf = reinterpret_cast<const uint32_t*>(c.return_flag)[t];
-      ls = reinterpret_cast<const uint16_t*>(c.line_status)[t];
-      if (PUSHDOWN) flt = reinterpret_cast<const uint16_t*>(c.filter)[t];
-    }
-#pragma unroll
-    for (int j = 0; j < TILE; j++) {
-      if (valid >> j & 1) {
-        const uint64_t r = t * TILE + j;
-        if (!PUSHDOWN) {
-          const uint32_t s = reinterpret_cast<const uint16_t*>(c.ship_date)[r];
-          comp_or(sd[j >> 3], (j >> 1) & 3, s << (16 * (j & 1)));
-        }
-        comp_or(q, j >> 2, (uint32_t)reinterpret_cast<const uint8_t*>(c.quantity)[r] << (8 * (j & 3)));
-        comp_or(d, j >> 2, (uint32_t)reinterpret_cast<const uint8_t*>(c.discount)[r] << (8 * (j & 3)));
-        comp_or(x, j >> 2, (uint32_t)reinterpret_cast<const uint8_t*>(c.tax)[r] << (8 * (j & 3)));
-        comp_set(p[j >> 2], j & 3, reinterpret_cast<const uint32_t*>(c.extended_price)[r]);
-      }
-    }
-  }
-  // `cut` is the cutoff relative to the frame of reference (may be < 0 or > 65535).
-  __device__ __forceinline__ bool pass(int j, int32_t cut) const {
-    if (PUSHDOWN) return (flt >> j) & 1;
-    const uint32_t s = (comp(sd[j >> 3], (j >> 1) & 3) >> (16 * (j & 1))) & 0xFFFFu;
-    return (int32_t)s <= cut;
-  }
-  __device__ __forceinline__ uint32_t gid(int j) const {
-    return __builtin_amdgcn_ubfe(rf, 2 * j, 2) << 1 | __builtin_amdgcn_ubfe(ls, j, 1);
-  }
-  __device__ __forceinline__ uint32_t byte(const uint4& v, int j) const {
-    return (comp(v, j >> 2) >> (8 * (j & 3))) & 0xFFu;
-  }
-  // Rows carrying the unused return-flag code 3 (slot 6 or 7): bit 2j set for row j.
-  __device__ __forceinline__ uint32_t bad_codes() const { return rf & (rf >> 1) & 0x55555555u; }
-  // Turns those rows into rows that fail the filter (ship date 0xFFFF, above every
-  // cutoff below 65535; pushdown: filter bit cleared) with code 0, so every row's slot is
-  // below 6.
-  __device__ void drop_bad_codes() {
-    const uint32_t inv = bad_codes();
-    rf &= ~(inv * 3u);
-#pragma unroll
-    for (int j = 0; j < TILE; j++) {
-      if (inv >> (2 * j) & 1) {
-        if (PUSHDOWN)
-          flt &= ~(1u << j);
-        else
-          comp_or(sd[j >> 3], (j >> 1) & 3, 0xFFFFu << (16 * (j & 1)));
-      }
-    }
-  }
-  template <int U>
-  __device__ __forceinline__ static void load_group(CompressedTile (&g)[U], const q1_columns& c, uint64_t t0,
-                                                    uint64_t stride) {
-#pragma unroll
-    for (int m = 0; m < U; m++) g[m].load(c, t0 + (uint64_t)m * stride);
-  }
-  template <bool EDGE>
-  __device__ __forceinline__ FastRow fast(int j, int32_t cut, uint32_t valid) const {
-    FastRow r;
-    r.pass = EDGE ? ((valid >> j & 1) && pass(j, cut)) : pass(j, cut);
-    r.gid = gid(j);
-    r.qty = byte(q, j);
-    r.disc = byte(d, j);
-    r.tax = byte(x, j);
-    r.price = comp(p[j >> 2], j & 3);
-    return r;
-  }
-};
-
-// Streaming variant for the compressed layouts (used with the shared placement): 4 rows
-// per tile, so that each load
+// Q1_LAYOUT_COMPRESSED / Q1_LAYOUT_COMPRESSED_PUSHDOWN: 4 rows per tile, so that each load
 // instruction of a wavefront reads one contiguous, line-aligned stretch of its column:
 // 64 lanes x 8 bytes of ship dates, x 4 bytes of quantity / discount / tax, x 16 bytes of
 // prices.  The 4 rows' return flags are one byte of the packed column (2 bits per row)
@@ -351,82 +245,7 @@ struct CompressedStreamTile {
   }
 };
 
-// Q1_LAYOUT_UNCOMPRESSED: int32 ship, int32 qty, int64 price, int8 disc/tax, char rf/ls.
-struct UncompressedTile {
-  static constexpr int TILE = 8;
-  static constexpr int GROUP = 1;
-  uint4 s[2], q[2], p[4];
-  uint2 d, x, rf, ls;
-
-  __device__ __forceinline__ void load(const q1_columns& c, uint64_t t) {
-    const uint4* ss = reinterpret_cast<const uint4*>(c.ship_date);
-    const uint4* qq = reinterpret_cast<const uint4*>(c.quantity);
-    const uint4* pp = reinterpret_cast<const uint4*>(c.extended_price);
-    s[0] = ss[2 * t]; s[1] = ss[2 * t + 1];
-    q[0] = qq[2 * t]; q[1] = qq[2 * t + 1];
-#pragma unroll
-    for (int k = 0; k < 4; k++) p[k] = pp[4 * t + k];
-    d = reinterpret_cast<const uint2*>(c.discount)[t];
-    x = reinterpret_cast<const uint2*>(c.tax)[t];
-    rf = reinterpret_cast<const uint2*>(c.return_flag)[t];
-    ls = reinterpret_cast<const uint2*>(c.line_status)[t];
-  }
-  __device__ __forceinline__ void load_edge(const q1_columns& c, uint64_t t, uint32_t valid) {
-    s[0] = s[1] = q[0] = q[1] = p[0] = p[1] = p[2] = p[3] = make_uint4(0, 0, 0, 0);
-    d = x = rf = ls = make_uint2(0, 0);
-#pragma unroll
-    for (int j = 0; j < TILE; j++) {
-      if (valid >> j & 1) {
-        const uint64_t r = t * TILE + j;
-        comp_set(s[j >> 2], j & 3, (uint32_t)reinterpret_cast<const int32_t*>(c.ship_date)[r]);
-        comp_set(q[j >> 2], j & 3, (uint32_t)reinterpret_cast<const int32_t*>(c.quantity)[r]);
-        const uint64_t pr = (uint64_t)reinterpret_cast<const int64_t*>(c.extended_price)[r];
-        comp_set(p[j >> 1], 2 * (j & 1), (uint32_t)pr);
-        comp_set(p[j >> 1], 2 * (j & 1) + 1, (uint32_t)(pr >> 32));
-        const int sh = 8 * (j & 3);
-        uint32_t* dd = (j < 4) ? &d.x : &d.y;
-        uint32_t* xx = (j < 4) ? &x.x : &x.y;
-        uint32_t* rr = (j < 4) ? &rf.x : &rf.y;
-        uint32_t* ll = (j < 4) ? &ls.x : &ls.y;
-        *dd |= (uint32_t)reinterpret_cast<const uint8_t*>(c.discount)[r] << sh;
-        *xx |= (uint32_t)reinterpret_cast<const uint8_t*>(c.tax)[r] << sh;
-        *rr |= (uint32_t)reinterpret_cast<const uint8_t*>(c.return_flag)[r] << sh;
-        *ll |= (uint32_t)reinterpret_cast<const uint8_t*>(c.line_status)[r] << sh;
-      }
-    }
-  }
-  __device__ __forceinline__ static uint32_t byte8(const uint2& v, int j) {
-    return ((j < 4 ? v.x : v.y) >> (8 * (j & 3))) & 0xFFu;
-  }
-  __device__ __forceinline__ uint32_t gid(int j) const {
-    return encode_return_flag(byte8(rf, j)) << 1 | encode_line_status(byte8(ls, j));
-  }
-  __device__ __forceinline__ bool pass(int j, int32_t cut) const {
-    return (int32_t)comp(s[j >> 2], j & 3) <= cut;
-  }
-  // Character flags encode to slots 0..5 only.
-  __device__ __forceinline__ static constexpr uint32_t bad_codes() { return 0; }
-  __device__ __forceinline__ void drop_bad_codes() {}
-  template <int U>
-  __device__ __forceinline__ static void load_group(UncompressedTile (&g)[U], const q1_columns& c, uint64_t t0,
-                                                    uint64_t stride) {
-#pragma unroll
-    for (int m = 0; m < U; m++) g[m].load(c, t0 + (uint64_t)m * stride);
-  }
-  template <bool EDGE>
-  __device__ __forceinline__ FastRow fast(int j, int32_t cut, uint32_t valid) const {
-    FastRow r;
-    r.pass = EDGE ? ((valid >> j & 1) && pass(j, cut)) : pass(j, cut);
-    r.gid = gid(j);
-    r.qty = comp(q[j >> 2], j & 3);
-    r.disc = byte8(d, j);
-    r.tax = byte8(x, j);
-    r.price = comp(p[j >> 1], 2 * (j & 1));
-    return r;
-  }
-};
-
-// Streaming variant for the uncompressed layout (used with the shared placement): 2 rows
+// Q1_LAYOUT_UNCOMPRESSED: int32 ship, int32 qty, int64 price, int8 disc/tax, char rf/ls; 2 rows
 // per tile, so that each load instruction of a wavefront reads one contiguous stretch of
 // its column with at most 16 bytes per lane: 64 lanes x 8 bytes of ship dates and
 // quantities, x 16 bytes of prices, x 2 bytes of discounts, taxes, return flags and line
@@ -505,83 +324,7 @@ struct UncompressedStreamTile {
   }
 };
 
-// Q1_LAYOUT_REFERENCE: int32 ship, int64 qty/price/disc/tax, char rf/ls.
-struct ReferenceTile {
-  static constexpr int TILE = 4;
-  static constexpr int GROUP = 1;
-  uint4 s, q[2], p[2], d[2], x[2];
-  uint32_t rf, ls;
-
-  __device__ __forceinline__ void load(const q1_columns& c, uint64_t t) {
-    s = reinterpret_cast<const uint4*>(c.ship_date)[t];
-    const uint4* qq = reinterpret_cast<const uint4*>(c.quantity);
-    const uint4* pp = reinterpret_cast<const uint4*>(c.extended_price);
-    const uint4* dd = reinterpret_cast<const uint4*>(c.discount);
-    const uint4* xx = reinterpret_cast<const uint4*>(c.tax);
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-      q[k] = qq[2 * t + k];
-      p[k] = pp[2 * t + k];
-      d[k] = dd[2 * t + k];
-      x[k] = xx[2 * t + k];
-    }
-    rf = reinterpret_cast<const uint32_t*>(c.return_flag)[t];
-    ls = reinterpret_cast<const uint32_t*>(c.line_status)[t];
-  }
-  __device__ __forceinline__ static void put64(uint4* v, int j, uint64_t val) {
-    comp_set(v[j >> 1], 2 * (j & 1), (uint32_t)val);
-    comp_set(v[j >> 1], 2 * (j & 1) + 1, (uint32_t)(val >> 32));
-  }
-  __device__ __forceinline__ void load_edge(const q1_columns& c, uint64_t t, uint32_t valid) {
-    s = q[0] = q[1] = p[0] = p[1] = d[0] = d[1] = x[0] = x[1] = make_uint4(0, 0, 0, 0);
-    rf = ls = 0;
-#pragma unroll
-    for (int j = 0; j < TILE; j++) {
-      if (valid >> j & 1) {
-        const uint64_t r = t * TILE + j;
-        comp_set(s, j, (uint32_t)reinterpret_cast<const int32_t*>(c.ship_date)[r]);
-        put64(q, j, (uint64_t)reinterpret_cast<const int64_t*>(c.quantity)[r]);
-        put64(p, j, (uint64_t)reinterpret_cast<const int64_t*>(c.extended_price)[r]);
-        put64(d, j, (uint64_t)reinterpret_cast<const int64_t*>(c.discount)[r]);
-        put64(x, j, (uint64_t)reinterpret_cast<const int64_t*>(c.tax)[r]);
-        rf |= (uint32_t)reinterpret_cast<const uint8_t*>(c.return_flag)[r] << (8 * j);
-        ls |= (uint32_t)reinterpret_cast<const uint8_t*>(c.line_status)[r] << (8 * j);
-      }
-    }
-  }
-  __device__ __forceinline__ static uint32_t lo32(const uint4* v, int j) {
-    return comp(v[j >> 1], 2 * (j & 1));
-  }
-  __device__ __forceinline__ static int64_t get64(const uint4* v, int j) {
-    return (int64_t)((uint64_t)comp(v[j >> 1], 2 * (j & 1) + 1) << 32 | comp(v[j >> 1], 2 * (j & 1)));
-  }
-  __device__ __forceinline__ uint32_t gid(int j) const {
-    return encode_return_flag((rf >> (8 * j)) & 0xFFu) << 1 | encode_line_status((ls >> (8 * j)) & 0xFFu);
-  }
-  __device__ __forceinline__ bool pass(int j, int32_t cut) const { return (int32_t)comp(s, j) <= cut; }
-  // Character flags encode to slots 0..5 only.
-  __device__ __forceinline__ static constexpr uint32_t bad_codes() { return 0; }
-  __device__ __forceinline__ void drop_bad_codes() {}
-  template <int U>
-  __device__ __forceinline__ static void load_group(ReferenceTile (&g)[U], const q1_columns& c, uint64_t t0,
-                                                    uint64_t stride) {
-#pragma unroll
-    for (int m = 0; m < U; m++) g[m].load(c, t0 + (uint64_t)m * stride);
-  }
-  template <bool EDGE>
-  __device__ __forceinline__ FastRow fast(int j, int32_t cut, uint32_t valid) const {
-    FastRow r;
-    r.pass = EDGE ? ((valid >> j & 1) && pass(j, cut)) : pass(j, cut);
-    r.gid = gid(j);
-    r.qty = lo32(q, j);
-    r.disc = lo32(d, j);
-    r.tax = lo32(x, j);
-    r.price = lo32(p, j);
-    return r;
-  }
-};
-
-// Streaming variant for the reference layout (used with the shared placement): 2 rows per
+// Q1_LAYOUT_REFERENCE: int32 ship, int64 qty/price/disc/tax, char rf/ls; 2 rows per
 // tile, each load instruction of a wavefront one contiguous stretch of its column with at
 // most 16 bytes per lane (64 lanes x 8 bytes of ship dates, x 16 bytes of each int64
 // column, x 2 bytes of return flags and line statuses), all loads non-temporal.
@@ -662,18 +405,15 @@ struct ReferenceStreamTile {
   }
 };
 
+// Every placement reads these tiles.  The register placements read tiles of 16, 8 and 4 rows
+// with ordinary loads before, half a stretch per load instruction: 600M compressed rows per
+// thread / in registers / global 982 / 990 / 1007 us (now 873 / 929 / 930), 60M uncompressed
+// 210 / 208 / 210 (188 / 189 / 190), 60M reference 382 / 378 / 386 (345 / 344 / 346).
 template <int L> struct TileOf;
-template <> struct TileOf<Q1_LAYOUT_REFERENCE> { using T = ReferenceTile; };
-template <> struct TileOf<Q1_LAYOUT_UNCOMPRESSED> { using T = UncompressedTile; };
-template <> struct TileOf<Q1_LAYOUT_COMPRESSED> { using T = CompressedTile<false>; };
-template <> struct TileOf<Q1_LAYOUT_COMPRESSED_PUSHDOWN> { using T = CompressedTile<true>; };
-
-// The tile a scan_fast<L, P> kernel reads.  The LDS placement (little register state per
-// lane) streams small tiles with non-temporal loads, four tiles in flight per lane: 4 rows
-// for the compressed layouts, 2 for uncompressed and reference (specialisations below);
-// the register placements keep TileOf<L>, whose tile sizes are also the units the host
-// counts tiles in (tile_rows).
-template <int L, int P> struct ScanTileOf { using T = typename TileOf<L>::T; };
+template <> struct TileOf<Q1_LAYOUT_REFERENCE> { using T = ReferenceStreamTile; };
+template <> struct TileOf<Q1_LAYOUT_UNCOMPRESSED> { using T = UncompressedStreamTile; };
+template <> struct TileOf<Q1_LAYOUT_COMPRESSED> { using T = CompressedStreamTile<false>; };
+template <> struct TileOf<Q1_LAYOUT_COMPRESSED_PUSHDOWN> { using T = CompressedStreamTile<true>; };
 
 // A group of U lane tiles t0 + m * stride (m < U, at most `count` of them, below
 // `end_tile`), all loaded before any of their rows is used, so that a wavefront keeps
@@ -707,12 +447,7 @@ struct TileGroup {
 #pragma unroll
     for (int m = 0; m < U; m++) {
       const uint64_t t = t0 + (uint64_t)m * stride;
-      if (use[m] && edge[m]) {
-        if constexpr (U > 1)
-          tile[m].load_edge(c, t, EdgeRows{row_begin, row_end});
-        else
-          tile[m].load_edge(c, t, valid[m]);
-      }
+      if (use[m] && edge[m]) tile[m].load_edge(c, t, EdgeRows{row_begin, row_end});
     }
   }
 };
@@ -781,7 +516,7 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
 // 2^28 over a tile; the product in the high half, below 16 * 15 * 2^24 < 2^32), so a row
 // costs three adds per group: that word, the packed count|discount|quantity and the charge.
 struct AccRegisters {
-  static constexpr bool kWideRows = false;
+  static constexpr bool kWideRows = false, kCompactEnds = true;
   uint32_t ns[kNumGroups];
   uint64_t npd[kNumGroups];
   uint64_t ch[kNumGroups], pr[kNumGroups], dp[kNumGroups];
@@ -870,7 +605,7 @@ __device__ __forceinline__ uint64_t small_to_small64(uint32_t s) {
 // of it (real data fills four of the six groups), and its four 64-bit adds run under the
 // lanes' mask: count, discount and quantity share one word (pack_small64).
 struct AccPerThread {
-  static constexpr bool kWideRows = false;
+  static constexpr bool kWideRows = false, kCompactEnds = true;
   uint64_t sm[kNumGroups], pr[kNumGroups], dp[kNumGroups], ch[kNumGroups];
   __device__ __forceinline__ void init(char*) {
 #pragma unroll
@@ -921,7 +656,7 @@ struct AccPerThread {
 // 64 rows 1.46 ms, 256 rows 1.35 ms, 1024 rows 1.19 ms.
 constexpr uint32_t kLocalFlushRows = 1024;
 struct AccLocal {
-  static constexpr bool kWideRows = false;
+  static constexpr bool kWideRows = false, kCompactEnds = true;
   // Per group: narrow sums of at most 16 rows as in AccRegisters (pack_small word; price
   // and discount product in one 64-bit word), folded every 16 rows into 64-bit
   // register sums of at most kLocalFlushRows rows (count, discount and quantity in the
@@ -1089,7 +824,7 @@ constexpr uint32_t shared_table_bytes(uint32_t threads) { return 4u * kNumGroups
 // register pair to build per row); the slot's high word stays zero.
 template <int B, bool NARROW = false>
 struct AccShared {
-  static constexpr bool kWideRows = false;
+  static constexpr bool kWideRows = false, kCompactEnds = false;
   uint64_t* tab;  // dynamic LDS: 6 * 4 * B words
   __device__ __forceinline__ void init(char* lds) {
     tab = reinterpret_cast<uint64_t*>(lds);
@@ -1173,7 +908,7 @@ constexpr uint32_t packed_table_bytes(uint32_t threads) { return 3u * kNumGroups
 
 template <int B>
 struct AccSharedPacked {
-  static constexpr bool kWideRows = false;
+  static constexpr bool kWideRows = false, kCompactEnds = false;
   uint64_t* tab;  // dynamic LDS: 6 * 3 * B words
   __device__ __forceinline__ void init(char* lds) {
     tab = reinterpret_cast<uint64_t*>(lds);
@@ -1237,7 +972,7 @@ struct AccSharedPacked {
 // fits 64 bits (price < 2^46, discount product < 2^50, charge < 2^60).
 __device__ __forceinline__ void atomic_add128(uint64_t* lo_p, uint64_t* hi_p, uint64_t lo, uint64_t hi);
 struct AccGlobal {
-  static constexpr bool kWideRows = false;
+  static constexpr bool kWideRows = false, kCompactEnds = true;
   static constexpr int W = 5;  // words per group: count|disc, qty, price, dprod, charge
   AccRegisters regs;
   uint64_t* tab;               // [W][6] words of this block
@@ -1310,18 +1045,6 @@ template <int B> struct AccOf<kPlaceSharedNarrow, B> { using A = AccShared<B, tr
 // ... and, for the compressed layouts, the packed table with three slots per group.
 constexpr int kPlaceSharedPacked = 9;
 template <int B> struct AccOf<kPlaceSharedPacked, B> { using A = AccSharedPacked<B>; };
-
-template <> struct ScanTileOf<Q1_LAYOUT_COMPRESSED, Q1_PLACE_PER_THREAD_SHARED_MEM> { using T = CompressedStreamTile<false>; };
-template <> struct ScanTileOf<Q1_LAYOUT_COMPRESSED, kPlaceSharedNarrow> { using T = CompressedStreamTile<false>; };
-template <> struct ScanTileOf<Q1_LAYOUT_COMPRESSED_PUSHDOWN, Q1_PLACE_PER_THREAD_SHARED_MEM> {
-  using T = CompressedStreamTile<true>;
-};
-template <> struct ScanTileOf<Q1_LAYOUT_COMPRESSED_PUSHDOWN, kPlaceSharedNarrow> { using T = CompressedStreamTile<true>; };
-template <> struct ScanTileOf<Q1_LAYOUT_UNCOMPRESSED, Q1_PLACE_PER_THREAD_SHARED_MEM> { using T = UncompressedStreamTile; };
-template <> struct ScanTileOf<Q1_LAYOUT_UNCOMPRESSED, kPlaceSharedNarrow> { using T = UncompressedStreamTile; };
-template <> struct ScanTileOf<Q1_LAYOUT_REFERENCE, Q1_PLACE_PER_THREAD_SHARED_MEM> { using T = ReferenceStreamTile; };
-template <> struct ScanTileOf<Q1_LAYOUT_REFERENCE, kPlaceSharedNarrow> { using T = ReferenceStreamTile; };
-template <int L> struct ScanTileOf<L, kPlaceSharedPacked> { using T = typename ScanTileOf<L, kPlaceSharedNarrow>::T; };
 
 // ------------------------------------------------------------------------------------
 // Block merge and the single global merge per block.
@@ -1547,7 +1270,21 @@ __device__ __forceinline__ void add_any_group(const TileGroup<Tile, U>& grp, Acc
   }
 }
 
-// The tiles base + k * B + lane (k < tiles_per_thread) of a block's lanes into an LDS table.
+// A group at an end of the range for the register tables: tile by tile, so that the kernel
+// holds one guarded copy of a tile's rows beside the whole groups' (with a guarded copy of
+// every row of a group the compressed kernels take 142-180 registers and spill, 106-136 so).
+template <class Tile, int U, class Acc>
+__device__ __forceinline__ void add_end_tiles(const ScanArgs& a, uint64_t t0, uint64_t stride, uint32_t count,
+                                              uint64_t end_tile, Acc& acc, int32_t cut) {
+#pragma unroll 1
+  for (uint32_t m = 0; m < U; m++) {
+    TileGroup<Tile, 1> one;
+    one.load(a.cols, t0 + m * stride, stride, m < count ? 1 : 0, end_tile, a.row_begin, a.row_end);
+    add_any_group(one, acc, cut);
+  }
+}
+
+// The tiles base + k * B + lane (k < tiles_per_thread) of a block's lanes into a table.
 // Groups k in [k_lo, k_end) are whole and inside the range for every lane of the
 // block: the tiles of group k are base + (k + m) * B + lane, and they all lie in
 // [whole_begin, whole_end), the tiles with no row outside [row_begin, row_end).  They
@@ -1559,6 +1296,7 @@ __device__ __forceinline__ void add_tiles(const ScanArgs& a, uint64_t base, uint
                                           int32_t cut) {
   constexpr int TILE = Tile::TILE;
   constexpr int U = Tile::GROUP;
+  constexpr int FLUSH = U * TILE >= 16 ? 1 : 16 / (U * TILE);  // groups per 16 rows
   const uint64_t end_tile = (a.row_end + TILE - 1) / TILE;
   const uint64_t whole_begin = (a.row_begin + TILE - 1) / TILE, whole_end = a.row_end / TILE;
   uint32_t k_lo = 0, k_end = 0;
@@ -1572,23 +1310,30 @@ __device__ __forceinline__ void add_tiles(const ScanArgs& a, uint64_t base, uint
       k_end = (uint32_t)(klo + (kmax - klo) / U * U);
     }
   }
+  auto add_end_group = [&](uint32_t k) {
+    const uint64_t t0 = base + (uint64_t)k * B + thread_index();
+    if constexpr (Acc::kCompactEnds) {
+      add_end_tiles<Tile, U>(a, t0, B, tiles_per_thread - k, end_tile, acc, cut);
+    } else {
+      TileGroup<Tile, U> grp;
+      grp.load(a.cols, t0, B, tiles_per_thread - k, end_tile, a.row_begin, a.row_end);
+      add_any_group(grp, acc, cut);
+    }
+  };
   uint32_t k = 0;
   for (; k < k_lo; k += U) {
-    TileGroup<Tile, U> grp;
-    grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
-             a.row_end);
-    add_any_group(grp, acc, cut);
+    add_end_group(k);
+    if ((k / U + 1) % FLUSH == 0) acc.flush();
   }
   for (; k < k_end; k += U) {
     TileGroup<Tile, U> grp;
     grp.load_plain(a.cols, base + (uint64_t)k * B + thread_index(), B);
     add_whole_group(grp, acc, cut);
+    if ((k / U + 1) % FLUSH == 0) acc.flush();
   }
   for (; k < tiles_per_thread; k += U) {
-    TileGroup<Tile, U> grp;
-    grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
-             a.row_end);
-    add_any_group(grp, acc, cut);
+    add_end_group(k);
+    if ((k / U + 1) % FLUSH == 0) acc.flush();
   }
 }
 
@@ -1600,13 +1345,10 @@ __device__ __forceinline__ void add_tiles(const ScanArgs& a, uint64_t base, uint
 template <int L, int P, int B>
 __device__ __forceinline__ void scan_block(const ScanArgs& a, uint64_t block, uint32_t host_tiles_per_thread,
                                            uint64_t* ws, uint64_t* lds, q1_device_aggregates* out) {
-  using Tile = typename ScanTileOf<L, P>::T;
+  using Tile = typename TileOf<L>::T;
   using Acc = typename AccOf<P, B>::A;
   constexpr int TILE = Tile::TILE;
-  constexpr int U = Tile::GROUP;                       // tiles loaded together per lane
-  constexpr int FLUSH = U * TILE >= 16 ? 1 : 16 / (U * TILE);  // groups per 16 rows
-  // The host counts tiles of TileOf<L> (tile_rows); a smaller kernel tile splits each.
-  constexpr int SUB = TileOf<L>::T::TILE / TILE;
+  constexpr int SUB = kHostTileRows<L> / TILE;  // kernel tiles per tile the host counts
 
   const int32_t cut = column_cutoff<L>(a.cutoff_day);
   // Block b covers kernel tiles [first_tile + b*B*tpt, +B*tpt): SUB times the host's
@@ -1615,7 +1357,6 @@ __device__ __forceinline__ void scan_block(const ScanArgs& a, uint64_t block, ui
   static_assert(kRowAlign % TILE == 0, "kRowAlign is a whole number of tiles");
   const uint32_t tiles_per_thread = host_tiles_per_thread * SUB;
   const uint64_t first_tile = a.row_begin / kRowAlign * kRowAlign / TILE;
-  const uint64_t end_tile = (a.row_end + TILE - 1) / TILE;
   const uint64_t base = first_tile + block * B * tiles_per_thread;
 
   Acc acc;
@@ -1627,31 +1368,7 @@ __device__ __forceinline__ void scan_block(const ScanArgs& a, uint64_t block, ui
   else
     acc.init(reinterpret_cast<char*>(lds));
 
-  constexpr bool kSplit = P == Q1_PLACE_PER_THREAD_SHARED_MEM || P == kPlaceSharedNarrow || P == kPlaceSharedPacked;
-  if constexpr (kSplit) {
-    add_tiles<L, Tile, B>(a, base, tiles_per_thread, acc, cut);
-  } else {
-    // The register-table placements keep one guarded loop: a second copy of the row body
-    // costs them registers (spills, lower occupancy) that the saved instructions do not
-    // repay.
-    for (uint32_t k = 0, n = 0; k < tiles_per_thread; k += U, n++) {
-      TileGroup<Tile, U> grp;
-      grp.load(a.cols, base + (uint64_t)k * B + thread_index(), B, tiles_per_thread - k, end_tile, a.row_begin,
-               a.row_end);
-#pragma unroll
-      for (int m = 0; m < U; m++) {
-        if (!grp.use[m]) continue;
-        if (!grp.edge[m]) {
-#pragma unroll
-          for (int j = 0; j < TILE; j++) acc.add(grp.tile[m].template fast<false>(j, cut, 0));
-        } else {
-#pragma unroll
-          for (int j = 0; j < TILE; j++) acc.add(grp.tile[m].template fast<true>(j, cut, grp.valid[m]));
-        }
-      }
-      if ((n + 1) % FLUSH == 0) acc.flush();  // at most 16 rows per lane between flushes
-    }
-  }
+  add_tiles<L, Tile, B>(a, base, tiles_per_thread, acc, cut);
   acc.flush(true);
 
   const uint64_t qty_scale =
@@ -1662,7 +1379,7 @@ __device__ __forceinline__ void scan_block(const ScanArgs& a, uint64_t block, ui
   } else {
     // The reduction scratch follows the placement's own LDS table.
     uint64_t* red = lds + Acc::lds_bytes(B) / 8;
-    if constexpr (kSplit) {
+    if constexpr (P == Q1_PLACE_PER_THREAD_SHARED_MEM || P == kPlaceSharedNarrow || P == kPlaceSharedPacked) {
       acc.wave_totals(red);
     } else {
       LaneTotals tot;
@@ -1722,11 +1439,12 @@ __device__ __forceinline__ uint32_t high24(uint64_t w) { return (uint32_t)((w - 
 // Two multiplications a row beyond the narrow table's, both with a 64-bit result.
 template <int B>
 struct AnyCompressed {
-  static constexpr bool kWideRows = false;
+  static constexpr bool kWideRows = false, kCompactEnds = false;
   static constexpr int W = 3;
   static_assert(any_value_lane_rows(Q1_LAYOUT_COMPRESSED) <= 128, "the fields' widths");
   static constexpr uint32_t kFactorBias = 55025;
   uint64_t* tab;
+  __device__ __forceinline__ void flush(bool = false) {}
   __device__ __forceinline__ void init(uint64_t* lds) {
     tab = lds;
     clear_wave_table<B, W>(tab);
@@ -1794,10 +1512,11 @@ __device__ __forceinline__ uint64_t mul_64_s32(uint64_t a, int32_t f) {
 //   word 4: price (wrapping)
 template <int B>
 struct AnyUncompressed {
-  static constexpr bool kWideRows = true;
+  static constexpr bool kWideRows = true, kCompactEnds = false;
   static constexpr int W = 5;
   static_assert(any_value_lane_rows(Q1_LAYOUT_UNCOMPRESSED) <= 256, "the fields' widths");
   uint64_t* tab;
+  __device__ __forceinline__ void flush(bool = false) {}
   __device__ __forceinline__ void init(uint64_t* lds) {
     tab = lds;
     clear_wave_table<B, W>(tab);
@@ -1862,10 +1581,11 @@ struct AnyUncompressed {
 // price, quantity and discount.
 template <int B>
 struct AnyReference {
-  static constexpr bool kWideRows = true;
+  static constexpr bool kWideRows = true, kCompactEnds = false;
   static constexpr int W = 7;
   static_assert(any_value_lane_rows(Q1_LAYOUT_REFERENCE) <= 256, "the fields' widths");
   uint64_t* tab;
+  __device__ __forceinline__ void flush(bool = false) {}
   __device__ __forceinline__ void init(uint64_t* lds) {
     tab = lds;
     clear_wave_table<B, W>(tab);
@@ -1944,10 +1664,10 @@ __device__ __forceinline__ void any_merge(const uint64_t* red, q1_device_aggrega
 template <int L, int B>
 __global__ void __launch_bounds__(B)
 scan_any(ScanArgs a, uint32_t host_tiles_per_thread) {
-  using Tile = typename ScanTileOf<L, kPlaceSharedNarrow>::T;
+  using Tile = typename TileOf<L>::T;
   using Acc = typename AnyOf<L, B>::A;
   constexpr int TILE = Tile::TILE;
-  constexpr int SUB = TileOf<L>::T::TILE / TILE;  // the host counts tiles of TileOf<L>
+  constexpr int SUB = kHostTileRows<L> / TILE;  // kernel tiles per tile the host counts
   constexpr uint64_t kQtyScale =
       (L == Q1_LAYOUT_COMPRESSED || L == Q1_LAYOUT_COMPRESSED_PUSHDOWN) ? kQuantityScaleCompressed : 1;
   extern __shared__ uint64_t lds[];
