@@ -321,7 +321,7 @@ q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const
                                                             : (int)placement;
     uint32_t lds = variant == kPlaceSharedPacked ? packed_table_bytes(shape.threads)
                    : shared                     ? shared_table_bytes(shape.threads)
-                                                : 0;
+                                                : stage_bytes(shape.threads);
     lds += nwaves * kNumGroups * NF * 8;
     uint32_t tiles = shape.tiles_per_thread;
     void* params[] = {(void*)&a, (void*)&tiles, (void*)&workspace};
@@ -400,7 +400,7 @@ static void* batch_kernel(q1_layout layout, q1_placement p) {
 
 static uint32_t batch_lds(q1_layout layout, q1_placement p) {
   const bool units = layout == Q1_LAYOUT_COMPRESSED || layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN;
-  uint32_t lds = p != Q1_PLACE_PER_THREAD_SHARED_MEM ? 0
+  uint32_t lds = p != Q1_PLACE_PER_THREAD_SHARED_MEM ? stage_bytes(kBatchBlock)
                  : units                            ? packed_table_bytes(kBatchBlock)
                                                     : shared_table_bytes(kBatchBlock);
   return lds + kBatchBlock / 64 * kNumGroups * NF * 8;

@@ -469,9 +469,11 @@ __device__ __forceinline__ int32_t column_cutoff(int32_t cutoff_day) {
 // ------------------------------------------------------------------------------------
 enum { F_QTY, F_PRICE, F_DISC, F_CNT, F_DPROD, F_CHARGE, NF };
 
-struct LaneTotals {
-  uint64_t v[kNumGroups][NF];
-};
+// A lane's sums as the register tables hand them over: per group the packed (count |
+// discount | quantity) word (pack_small64), price, discount product and charge.
+typedef uint64_t LaneWords[kNumGroups][4];
+// The LDS rows that their sum over a wavefront goes through (sum_lane_words).
+constexpr uint32_t stage_bytes(uint32_t threads) { return 2u * kNumGroups * 8u * threads; }
 
 __device__ __forceinline__ uint32_t pack_small(const FastRow& r) {
   return 1u | r.disc << 5 | r.qty << 13;
@@ -490,24 +492,6 @@ __device__ __forceinline__ uint64_t dpp_u64(uint64_t v) {
   const uint2 r = make_uint2((uint32_t)__builtin_amdgcn_mov_dpp((int)w.x, CTRL, 0xF, 0xF, false),
                              (uint32_t)__builtin_amdgcn_mov_dpp((int)w.y, CTRL, 0xF, 0xF, false));
   return __builtin_bit_cast(uint64_t, r);
-}
-__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int lane) {
-  const uint2 w = __builtin_bit_cast(uint2, v);
-  const uint2 r = make_uint2((uint32_t)__builtin_amdgcn_readlane((int)w.x, lane),
-                             (uint32_t)__builtin_amdgcn_readlane((int)w.y, lane));
-  return __builtin_bit_cast(uint64_t, r);
-}
-
-// Sum of a 64-bit value over the 64 lanes of a wavefront (all lanes active); the result
-// is wavefront-uniform.  Within each row of 16 lanes: quad butterflies (quad_perm
-// [1,0,3,2] and [2,3,0,1]) then rotations by 4 and 8 leave the row total in every lane;
-// the four row totals are read into scalar registers and added there.
-__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
-  v += dpp_u64<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_u64<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_u64<0x124>(v);  // row_ror:4
-  v += dpp_u64<0x128>(v);  // row_ror:8
-  return readlane_u64(v, 0) + readlane_u64(v, 16) + readlane_u64(v, 32) + readlane_u64(v, 48);
 }
 
 // Q1_PLACE_IN_REGISTERS: narrow per-tile accumulators in registers; a group's block of
@@ -566,18 +550,16 @@ struct AccRegisters {
       }
     }
   }
-  __device__ __forceinline__ void totals(LaneTotals& t, char*) const {
+  __device__ __forceinline__ void words(LaneWords& w) const {
 #pragma unroll
     for (int g = 0; g < kNumGroups; g++) {
-      t.v[g][F_QTY] = qty[g];
-      t.v[g][F_PRICE] = pr[g];
-      t.v[g][F_DISC] = dsc[g];
-      t.v[g][F_CNT] = cnt[g];
-      t.v[g][F_DPROD] = dp[g];
-      t.v[g][F_CHARGE] = ch[g];
+      w[g][0] = (uint64_t)cnt[g] | (uint64_t)dsc[g] << 17 | (uint64_t)qty[g] << 37;
+      w[g][1] = pr[g];
+      w[g][2] = dp[g];
+      w[g][3] = ch[g];
     }
   }
-  static constexpr uint32_t lds_bytes(uint32_t) { return 0; }
+  static constexpr uint32_t lds_bytes(uint32_t threads) { return stage_bytes(threads); }
 };
 
 // Packed (count | discount | quantity) in 64 bits for the per-lane 64-bit tables:
@@ -631,16 +613,16 @@ struct AccPerThread {
     }
   }
   __device__ __forceinline__ void flush(bool = false) {}
-  __device__ __forceinline__ void totals(LaneTotals& t, char*) const {
+  __device__ __forceinline__ void words(LaneWords& w) const {
 #pragma unroll
     for (int g = 0; g < kNumGroups; g++) {
-      unpack_small64(sm[g], t.v[g]);
-      t.v[g][F_PRICE] = pr[g];
-      t.v[g][F_DPROD] = dp[g];
-      t.v[g][F_CHARGE] = ch[g];
+      w[g][0] = sm[g];
+      w[g][1] = pr[g];
+      w[g][2] = dp[g];
+      w[g][3] = ch[g];
     }
   }
-  static constexpr uint32_t lds_bytes(uint32_t) { return 0; }
+  static constexpr uint32_t lds_bytes(uint32_t threads) { return stage_bytes(threads); }
 };
 
 // Q1_PLACE_LOCAL_MEM: the per-thread table of the reference
@@ -747,17 +729,13 @@ struct AccLocal {
     }
   }
   // The private table (after the last flush).
-  __device__ __forceinline__ void totals(LaneTotals& o, char*) const {
+  __device__ __forceinline__ void words(LaneWords& w) const {
 #pragma unroll
-    for (int g = 0; g < kNumGroups; g++) {
-      const uint64_t* w = t + g * 4;
-      unpack_small64(w[0], o.v[g]);
-      o.v[g][F_PRICE] = w[1];
-      o.v[g][F_DPROD] = w[2];
-      o.v[g][F_CHARGE] = w[3];
-    }
+    for (int g = 0; g < kNumGroups; g++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) w[g][j] = t[g * 4 + j];
   }
-  static constexpr uint32_t lds_bytes(uint32_t) { return 0; }
+  static constexpr uint32_t lds_bytes(uint32_t threads) { return stage_bytes(threads); }
 };
 
 // The LDS tables of the shared placement: [group][word][thread] words of 64 bits, W words per
@@ -960,6 +938,42 @@ struct AccSharedPacked {
   static constexpr uint32_t lds_bytes(uint32_t) { return packed_table_bytes(B); }
 };
 
+// The register tables' sums over a wavefront, through LDS like the LDS tables' own: two of a
+// lane's four words per group at a time are staged in rows of 64 lanes (6 KB per wavefront,
+// so that registers, not LDS, go on limiting the wavefronts of a compute unit), and eight
+// lanes per group add them.  A butterfly over all lanes for each word of each
+// group took 3 us more of every launch: 1M compressed rows per thread 15.2 us, now 12.0; 6M
+// uncompressed rows 31.9, now 28.8.
+__device__ __forceinline__ void sum_lane_words(const LaneWords& w, uint64_t* stage, uint64_t* red) {
+  const uint32_t wave = thread_index() >> 6, lane = thread_index() & 63, g = lane >> 3, k = lane & 7;
+  uint64_t* mine = stage + wave * (2 * kNumGroups * 64);
+  typename AccShared<64>::GroupSums sums;
+  uint64_t v[8][4];
+#pragma unroll
+  for (int half = 0; half < 4; half += 2) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < kNumGroups; i++) {
+      mine[(2 * i) * 64 + lane] = w[i][half];
+      mine[(2 * i + 1) * 64 + lane] = w[i][half + 1];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t row = g < kNumGroups ? g : 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; i++) {
+      const uint32_t at = 2 * row * 64 + k + 8 * ((i + g) & 7);
+      v[i][half] = mine[at];
+      v[i][half + 1] = mine[at + 64];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i++) sums.add(v[i]);
+  sums.reduce([](auto& x) { add_eight(x); });
+  if (g < kNumGroups && k == 0) sums.store(red + (wave * kNumGroups + g) * NF);
+}
+
 // Q1_PLACE_GLOBAL: the block's aggregation table lives in global memory (the kernel's
 // workspace, one table per block), as the reference's table does
 // (src/kernels/ht_in_global_mem.hpp:12-52).  The reference adds every row into it with
@@ -985,28 +999,24 @@ struct AccGlobal {
   __device__ __forceinline__ void init(char* lds) { regs.init(lds); }
   __device__ __forceinline__ void add(const FastRow& r) { regs.add(r); }
   __device__ __forceinline__ void flush(bool = false) { regs.flush(); }
-  // The block's whole merge (called by every thread of the block).
-  __device__ __forceinline__ void merge(q1_device_aggregates* out, uint64_t qty_scale) const {
-    LaneTotals o;
-    regs.totals(o, nullptr);
-    const uint32_t lane = thread_index() & 63;
-#pragma unroll
-    for (int g = 0; g < kNumGroups; g++) {
-      if (ballot(o.v[g][F_CNT] != 0)) {
-        // a lane's count is at most 16384 and its discount sum at most 15 * 16384
-        const uint64_t cd = wave_sum_u64(o.v[g][F_CNT] | o.v[g][F_DISC] << 24);
-        const uint64_t q = wave_sum_u64(o.v[g][F_QTY]);
-        const uint64_t p = wave_sum_u64(o.v[g][F_PRICE]);
-        const uint64_t d = wave_sum_u64(o.v[g][F_DPROD]);
-        const uint64_t c = wave_sum_u64(o.v[g][F_CHARGE]);
-        if (lane == 0) {
-          atomicAdd((unsigned long long*)(tab + g), (unsigned long long)cd);
-          atomicAdd((unsigned long long*)(tab + kNumGroups + g), (unsigned long long)q);
-          atomicAdd((unsigned long long*)(tab + 2 * kNumGroups + g), (unsigned long long)p);
-          atomicAdd((unsigned long long*)(tab + 3 * kNumGroups + g), (unsigned long long)d);
-          atomicAdd((unsigned long long*)(tab + 4 * kNumGroups + g), (unsigned long long)c);
-        }
-      }
+  // The block's whole merge (called by every thread of the block; `stage` is its LDS).
+  __device__ __forceinline__ void merge(uint64_t* stage, uint64_t* red, q1_device_aggregates* out,
+                                        uint64_t qty_scale) const {
+    LaneWords o;
+    regs.words(o);
+    sum_lane_words(o, stage, red);
+    const uint32_t wave = thread_index() >> 6, lane = thread_index() & 63;
+    // lane 5g + w adds word w of group g into the block's table (a wavefront's count is below
+    // 2^21 and its discount sum below 2^24)
+    if (lane < W * kNumGroups) {
+      const uint32_t g = lane / W, w = lane % W;
+      const uint64_t* r = red + (wave * kNumGroups + g) * NF;
+      const uint64_t v = w == 0   ? r[F_CNT] | r[F_DISC] << 24
+                         : w == 1 ? r[F_QTY]
+                         : w == 2 ? r[F_PRICE]
+                         : w == 3 ? r[F_DPROD]
+                                  : r[F_CHARGE];
+      if (v) atomicAdd((unsigned long long*)(tab + w * kNumGroups + g), (unsigned long long)v);
     }
     // Only this block reads its table back, and every wave of the block shares one L2 (where
     // the atomics are performed): the barrier's workgroup-scope release and acquire order
@@ -1030,7 +1040,7 @@ struct AccGlobal {
       }
     }
   }
-  static constexpr uint32_t lds_bytes(uint32_t) { return 0; }
+  static constexpr uint32_t lds_bytes(uint32_t threads) { return stage_bytes(threads); }
 };
 
 template <int P, int B> struct AccOf;
@@ -1057,21 +1067,6 @@ __device__ __forceinline__ void atomic_add128(uint64_t* lo_p, uint64_t* hi_p, ui
     carry = (old + lo) < old;
   }
   if (hi + carry) atomicAdd((unsigned long long*)hi_p, (unsigned long long)(hi + carry));
-}
-
-// A wavefront's sums of LaneTotals (exact: they fit uint64) into red[wave][group][NF].
-__device__ void sum_lane_totals(const LaneTotals& t, uint64_t* red) {
-  const uint32_t wave = thread_index() >> 6, lane = thread_index() & 63;
-#pragma unroll
-  for (int g = 0; g < kNumGroups; g++) {
-    const bool any = ballot(t.v[g][F_CNT] != 0) != 0;
-    uint64_t* r = red + (wave * kNumGroups + g) * NF;
-#pragma unroll
-    for (int f = 0; f < NF; f++) {
-      const uint64_t sum = any ? wave_sum_u64(t.v[g][f]) : 0;
-      if (lane == 0) r[f] = sum;
-    }
-  }
 }
 
 // The block's merge into `out`: the wavefronts' sums red[wave][group][NF] are added in 128
@@ -1373,18 +1368,17 @@ __device__ __forceinline__ void scan_block(const ScanArgs& a, uint64_t block, ui
 
   const uint64_t qty_scale =
       (L == Q1_LAYOUT_COMPRESSED || L == Q1_LAYOUT_COMPRESSED_PUSHDOWN) ? kQuantityScaleCompressed : 1;
+  // The reduction scratch follows the placement's own LDS table or staging rows.
+  uint64_t* red = lds + Acc::lds_bytes(B) / 8;
   if constexpr (P == Q1_PLACE_GLOBAL) {
-    // through the block's table in global memory
-    acc.merge(out, qty_scale);
+    acc.merge(lds, red, out, qty_scale);  // through the block's table in global memory
   } else {
-    // The reduction scratch follows the placement's own LDS table.
-    uint64_t* red = lds + Acc::lds_bytes(B) / 8;
     if constexpr (P == Q1_PLACE_PER_THREAD_SHARED_MEM || P == kPlaceSharedNarrow || P == kPlaceSharedPacked) {
       acc.wave_totals(red);
     } else {
-      LaneTotals tot;
-      acc.totals(tot, reinterpret_cast<char*>(lds));
-      sum_lane_totals(tot, red);
+      LaneWords w;
+      acc.words(w);
+      sum_lane_words(w, lds, red);
     }
     block_merge(red, out, qty_scale);
   }
