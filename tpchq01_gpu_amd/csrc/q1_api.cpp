@@ -254,11 +254,22 @@ static const void* colc(const q1_columns& c, int i) { return col(const_cast<q1_c
 // pushdown table are those of a compressed one.
 static q1_status measure_domain(q1_ctx* ctx, q1_table* t) {
   const q1_layout l = t->layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? Q1_LAYOUT_COMPRESSED : t->layout;
-  *ctx->h_outside = 0;
-  q1_status s = launch_domain_check(l, t->dev, t->rows, ctx->d_outside, ctx->stream);
+  if (t->rows == 0) {
+    t->fast = true;
+    return Q1_OK;
+  }
+  const Completion done{ctx->set, ctx->d_result, ++ctx->sequence};
+  bool counted = false;
+  ctx->h_result->outside = 0;
+  q1_status s = launch_domain_check(l, t->dev, t->rows, done, ctx->stream, &counted);
   if (s != Q1_OK) return fail(ctx, s, "domain check kernel launch failed");
-  Q1_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  t->fast = *ctx->h_outside == 0;
+  if (!counted) {
+    Q1_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  } else {
+    s = wait_sequence(ctx, &ctx->h_result->sequence, done.sequence);
+    if (s != Q1_OK) return s;
+  }
+  t->fast = ctx->h_result->outside == 0;
   return Q1_OK;
 }
 
@@ -335,9 +346,8 @@ static void load_tuning_file(q1_ctx* ctx) {
 // holds it when a creation fails).
 static void release_table(q1_table* t) {
   if (q1_ctx* ctx = t->ctx) {
-    if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     for (void* p : t->owned)
-      if (p) (void)hipFree(p);
+      if (p) (void)hipFree(p);  // waits for the device, which may still read it
     ctx->tables.erase(t);
   }
   delete t;
@@ -397,8 +407,6 @@ q1_status q1_init(int device, q1_ctx** out) {
   ok = ok && hipEventCreate(&ctx->ev_h2d_begin) == hipSuccess && hipEventCreate(&ctx->ev_h2d_end) == hipSuccess;
   ok = ok && hipMalloc(&ctx->d_aggr, sizeof(q1_device_aggregates)) == hipSuccess;
   ok = ok && hipHostMalloc(&ctx->h_aggr, sizeof(q1_device_aggregates), hipHostMallocDefault) == hipSuccess;
-  ok = ok && hipHostMalloc(&ctx->h_outside, sizeof(uint32_t), hipHostMallocMapped) == hipSuccess &&
-       hipHostGetDevicePointer((void**)&ctx->d_outside, ctx->h_outside, 0) == hipSuccess;
   ok = ok && hipHostMalloc(&ctx->h_result, sizeof(HostResult), hipHostMallocMapped) == hipSuccess &&
        hipHostGetDevicePointer((void**)&ctx->d_result, ctx->h_result, 0) == hipSuccess;
   if (ok) std::memset(ctx->h_result, 0, sizeof(HostResult));
@@ -450,7 +458,6 @@ void q1_shutdown(q1_ctx* ctx) {
   if (ctx->pool.sets) (void)hipFree(ctx->pool.sets);
   if (ctx->pool.done) (void)hipHostFree(ctx->pool.done);
   if (ctx->h_aggr) (void)hipHostFree(ctx->h_aggr);
-  if (ctx->h_outside) (void)hipHostFree(ctx->h_outside);
   if (ctx->h_result) (void)hipHostFree(ctx->h_result);
   if (ctx->d_aggr) (void)hipFree(ctx->d_aggr);
   for (hipEvent_t e : {ctx->ev_begin, ctx->ev_end, ctx->ev_h2d_begin, ctx->ev_h2d_end})

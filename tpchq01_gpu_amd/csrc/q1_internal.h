@@ -61,8 +61,6 @@ struct q1_ctx {
   int32_t clock_khz = 0;                   // rate of the device clock in h_result
   q1_device_aggregates* d_aggr = nullptr;  // the table q1_run_streaming's chunks add into
   q1_device_aggregates* h_aggr = nullptr;  // pinned host copy
-  uint32_t* h_outside = nullptr;           // pinned word the domain check writes
-  uint32_t* d_outside = nullptr;           // ... as the device addresses it
   void* workspace = nullptr;
   uint64_t workspace_bytes = 0;
   q1_timing last{};

@@ -64,13 +64,22 @@ inline uint32_t merge_tables(uint64_t blocks) {
 struct MergeSet {
   MergeTable table[kSpreadTables];
   uint64_t clock_begin;       // device clock at the start of block 0
+  uint32_t outside;           // the domain check's finding
 };
 
 // What a launch leaves in pinned host memory for a caller that waits for it.
 struct HostResult {
   q1_device_aggregates sums;
   uint64_t clock_begin, clock_end;  // device clock at the start of block 0 and at the fold
+  uint64_t outside;                 // domain check: whether a value lies outside the TPC-H domain
   uint64_t sequence;                // the launch's number, written after everything else
+};
+// How a kernel that leaves no sums tells the host that all its blocks are done: through the
+// counters of a merge set, into a HostResult.
+struct Completion {
+  MergeSet* set;
+  HostResult* host;           // as the device addresses it
+  uint64_t sequence;
 };
 
 // Kernel-level request: accumulate rows [row_begin, row_end) of `cols` into `out`.
@@ -124,10 +133,11 @@ q1_status launch_zero(void* p, uint64_t bytes, void* stream);
 q1_status launch_generate(q1_layout layout, uint64_t seed, uint64_t rows, const q1_columns& cols,
                           void* stream);
 
-// Device-side domain check of a table's columns: *outside (device-visible) is set to 1 if any
-// value lies outside the TPC-H domain, and not written otherwise.
-q1_status launch_domain_check(q1_layout layout, const q1_columns& cols, uint64_t rows, uint32_t* outside,
-                              void* stream);
+// Device-side domain check of a table's columns (rows > 0): host->outside, 0 before, becomes 1
+// if any value lies outside the TPC-H domain.  *counted: `done` tells when; otherwise the
+// kernel's end does.
+q1_status launch_domain_check(q1_layout layout, const q1_columns& cols, uint64_t rows, const Completion& done,
+                              void* stream, bool* counted);
 
 // Device-side pushdown producer: filter bitmap of a compressed ship_date column.
 q1_status launch_build_filter(const uint16_t* ship, uint64_t rows, int32_t cutoff_day,

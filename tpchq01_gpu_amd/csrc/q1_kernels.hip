@@ -1,5 +1,7 @@
 // gfx950 utility kernels (zero fill, generator, domain check, pushdown producer), kernel dispatch and the host-side launch helpers of the TPC-H Q1
 // path.  The scan kernels themselves are in q1_scan.h, instantiated per layout.
+#include <type_traits>
+
 #include "q1_scan.h"
 
 namespace q1 {
@@ -58,8 +60,21 @@ __global__ void generate_rows(uint64_t seed, uint64_t rows, q1_columns c) {
   }
 }
 
-// The value-domain check: *outside becomes 1 if any discount, tax, quantity or price lies
-// outside the TPC-H domain (domain_is_tpch's limits), and is left alone otherwise.
+// The end of a kernel that leaves no sums, called by wavefront 0 of a block: the count of
+// finished blocks, whose last one tells the host.
+__device__ __forceinline__ void end_counted(const Completion& c) {
+  MergeSet* const set = c.set;
+  const uint32_t grid = gridDim.x, b = blockIdx.x, mask = kSpreadTables - 1;
+  const uint32_t used = grid < kSpreadTables ? grid : kSpreadTables;
+  if (!count_block(set->table, b & mask, blocks_sharing(grid, b, mask), used)) return;
+  clear_counts(set->table, used);
+  if ((threadIdx.x & 63) == 0) store_host(&c.host->outside, atomicExch(&set->outside, 0u));
+  __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if ((threadIdx.x & 63) == 0) store_host(&c.host->sequence, c.sequence);
+}
+
+// The value-domain check: host->outside becomes whether any discount, tax, quantity or price
+// lies outside the TPC-H domain (domain_is_tpch's limits).
 // HBM bounds it: 7 (compressed), 14 or 32 bytes per row are read once and nothing is written
 // for a table inside the domain.  Each column is read as 16-byte vectors with no regard to
 // rows: a limit of the form 2^k - 1 is a test of bits, so a lane ORs what it reads of such a
@@ -145,8 +160,14 @@ __device__ __forceinline__ bool block_outside(const q1_columns& c, uint64_t rows
   return tail | d.outside() | x.outside() | q.outside() | p.outside();
 }
 
-template <int L>
-__global__ void __launch_bounds__(256) domain_check(q1_columns c, uint64_t rows, uint32_t* outside) {
+// Larger grids do not count their blocks: a block lives for one round of loads, which the
+// count lengthens.  Check and wait, counted / not: 1M compressed rows (123 blocks) 10.1 / 12.3
+// us, 60M (7,325 blocks) 77 / 77, 600M 694 / 672.
+constexpr uint64_t kDomainCountedBlocks = 4096;
+// COUNTED: the last of its blocks tells the host; otherwise the caller waits for the kernel's
+// end, host->outside being 0 before.
+template <int L, bool COUNTED>
+__global__ void __launch_bounds__(256) domain_check(q1_columns c, uint64_t rows, Completion done) {
   bool bad;
   if constexpr (L == Q1_LAYOUT_REFERENCE)
     bad = block_outside<int64_t, int64_t, 6300, int64_t, kDomainRows<L>>(c, rows);
@@ -154,10 +175,16 @@ __global__ void __launch_bounds__(256) domain_check(q1_columns c, uint64_t rows,
     bad = block_outside<int8_t, int32_t, 6300, int64_t, kDomainRows<L>>(c, rows);
   else
     bad = block_outside<uint8_t, uint8_t, 63, uint32_t, kDomainRows<L>>(c, rows);
-  // The word is in host memory: a wavefront writes it once, and only if nobody has yet.
-  if (ballot(bad) && (threadIdx.x & 63) == 0 &&
-      __hip_atomic_load(outside, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0)
-    __hip_atomic_store(outside, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (COUNTED) {
+    const bool outside = __syncthreads_or(bad);
+    if (threadIdx.x < 64) {
+      if (outside && threadIdx.x == 0) atomicOr(&done.set->outside, 1u);
+      end_counted(done);
+    }
+  } else if (ballot(bad) && (threadIdx.x & 63) == 0 &&
+             __hip_atomic_load(&done.host->outside, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0) {
+    store_host(&done.host->outside, 1);
+  }
 }
 
 // The pushdown producer (src/main.cu:362-389 semantics, runtime cutoff).  A lane turns the
@@ -356,9 +383,9 @@ q1_status launch_generate(q1_layout layout, uint64_t seed, uint64_t rows, const 
   return hip_status(hipGetLastError());
 }
 
-q1_status launch_domain_check(q1_layout layout, const q1_columns& cols, uint64_t rows, uint32_t* outside,
-                              void* stream) {
-  if (rows == 0) return Q1_OK;
+q1_status launch_domain_check(q1_layout layout, const q1_columns& cols, uint64_t rows, const Completion& done,
+                              void* stream, bool* counted) {
+  if (rows == 0) return Q1_EINVAL;
   const uint64_t per = layout == Q1_LAYOUT_REFERENCE      ? kDomainRows<Q1_LAYOUT_REFERENCE>
                        : layout == Q1_LAYOUT_UNCOMPRESSED ? kDomainRows<Q1_LAYOUT_UNCOMPRESSED>
                                                           : kDomainRows<Q1_LAYOUT_COMPRESSED>;
@@ -366,10 +393,18 @@ q1_status launch_domain_check(q1_layout layout, const q1_columns& cols, uint64_t
   if (blocks * 256 > 0xFFFFFFFFull) return Q1_EINVAL;  // HIP counts work-items in 32 bits
   const dim3 grid((uint32_t)blocks), block(256);
   const hipStream_t s = (hipStream_t)stream;
+  *counted = blocks <= kDomainCountedBlocks;
+  auto run = [&](auto layout_const) {
+    constexpr int L = decltype(layout_const)::value;
+    if (*counted)
+      hipLaunchKernelGGL((domain_check<L, true>), grid, block, 0, s, cols, rows, done);
+    else
+      hipLaunchKernelGGL((domain_check<L, false>), grid, block, 0, s, cols, rows, done);
+  };
   switch (layout) {
-    case Q1_LAYOUT_REFERENCE: hipLaunchKernelGGL(domain_check<Q1_LAYOUT_REFERENCE>, grid, block, 0, s, cols, rows, outside); break;
-    case Q1_LAYOUT_UNCOMPRESSED: hipLaunchKernelGGL(domain_check<Q1_LAYOUT_UNCOMPRESSED>, grid, block, 0, s, cols, rows, outside); break;
-    default: hipLaunchKernelGGL(domain_check<Q1_LAYOUT_COMPRESSED>, grid, block, 0, s, cols, rows, outside); break;
+    case Q1_LAYOUT_REFERENCE: run(std::integral_constant<int, Q1_LAYOUT_REFERENCE>()); break;
+    case Q1_LAYOUT_UNCOMPRESSED: run(std::integral_constant<int, Q1_LAYOUT_UNCOMPRESSED>()); break;
+    default: run(std::integral_constant<int, Q1_LAYOUT_COMPRESSED>()); break;
   }
   return hip_status(hipGetLastError());
 }

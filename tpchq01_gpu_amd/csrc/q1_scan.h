@@ -1111,7 +1111,7 @@ __device__ __forceinline__ void block_merge(const uint64_t* red, q1_device_aggre
 // The end of a block that merged into table t of the tables its range's blocks share, called
 // by wavefront 0 of the block, which issued the merge atomics; `sharing` blocks merge into
 // table t, and `used` tables have blocks.  Returns whether this is the last block of the
-// range: lane w then holds word w of the sums (w < 48), and the tables are zero again.
+// range (count_block): lane w then holds word w of the sums (w < 48), and the tables are zero again.
 // Ordering: the tables and the counters are only ever touched by device-scope
 // atomics, which are performed at memory, past the XCDs' L2 caches.  A block counts itself
 // only after its own atomics have been performed (the wait below), so the block that draws
@@ -1123,17 +1123,26 @@ __device__ __forceinline__ void block_merge(const uint64_t* red, q1_device_aggre
 // host after it, each 2-5 us of a short call: q1_run of 5,003 rows 32.3 -> 18.9 us, of 1M
 // rows 39.0 -> 23.9.  A block's own part is two waits for an atomic; the other blocks of
 // its compute unit cover them (600M rows, 18,311 blocks: 862 -> 847 us per call).
-__device__ __forceinline__ bool finish_tables(MergeTable* tables, uint32_t t, uint32_t sharing, uint32_t used,
-                                              uint64_t& sum) {
-  const uint32_t lane = thread_index() & 63;
+__device__ __forceinline__ bool count_block(MergeTable* tables, uint32_t t, uint32_t sharing, uint32_t used) {
   __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   uint32_t last = 0;
-  if (lane == 0) {
+  if ((thread_index() & 63) == 0) {
     last = sharing == 1 || atomicAdd(&tables[t].merged, 1u) == sharing - 1;
     if (last && used > 1) last = atomicAdd(&tables[0].tables_merged, 1u) == used - 1;
   }
-  if (!__builtin_amdgcn_readfirstlane(last)) return false;
+  last = (uint32_t)__builtin_amdgcn_readfirstlane((int)last);
   __asm__ volatile("" ::: "memory");
+  return last;
+}
+__device__ __forceinline__ void clear_counts(MergeTable* tables, uint32_t used) {
+  const uint32_t lane = thread_index() & 63;
+  if (lane < used) atomicExch(&tables[lane].merged, 0u);
+  if (lane == 0) atomicExch(&tables[0].tables_merged, 0u);
+}
+__device__ __forceinline__ bool finish_tables(MergeTable* tables, uint32_t t, uint32_t sharing, uint32_t used,
+                                              uint64_t& sum) {
+  if (!count_block(tables, t, sharing, used)) return false;
+  const uint32_t lane = thread_index() & 63;
   // Lane w sums word w of the tables in use.  A 128-bit field is two words: the lane of the
   // low one counts its carries, which then go to the lane of the high one, 6 lanes on.
   constexpr uint32_t kWords = sizeof(q1_device_aggregates) / 8;
@@ -1156,8 +1165,7 @@ __device__ __forceinline__ bool finish_tables(MergeTable* tables, uint32_t t, ui
   }
   const uint64_t carried = __shfl(carry, (int)lane - kNumGroups, 64);  // lanes below 6 ignore it
   if ((lane >= 18 && lane < 24) || (lane >= 30 && lane < 36)) s += carried;
-  if (lane < used) atomicExch(&tables[lane].merged, 0u);
-  if (lane == 0) atomicExch(&tables[0].tables_merged, 0u);
+  clear_counts(tables, used);
   sum = s;
   return true;
 }
