@@ -64,7 +64,7 @@ inline uint32_t merge_tables(uint64_t blocks) {
 struct MergeSet {
   MergeTable table[kSpreadTables];
   uint64_t clock_begin;       // device clock at the start of block 0
-  uint32_t outside;           // the domain check's finding
+  uint64_t outside;           // number of the last domain check that found a value outside
 };
 
 // What a launch leaves in pinned host memory for a caller that waits for it.

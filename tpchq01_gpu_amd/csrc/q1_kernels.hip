@@ -68,7 +68,6 @@ __device__ __forceinline__ void end_counted(const Completion& c) {
   const uint32_t used = grid < kSpreadTables ? grid : kSpreadTables;
   if (!count_block(set->table, b & mask, blocks_sharing(grid, b, mask), used)) return;
   clear_counts(set->table, used);
-  if ((threadIdx.x & 63) == 0) store_host(&c.host->outside, atomicExch(&set->outside, 0u));
   __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if ((threadIdx.x & 63) == 0) store_host(&c.host->sequence, c.sequence);
 }
@@ -175,15 +174,22 @@ __global__ void __launch_bounds__(256) domain_check(q1_columns c, uint64_t rows,
     bad = block_outside<int8_t, int32_t, 6300, int64_t, kDomainRows<L>>(c, rows);
   else
     bad = block_outside<uint8_t, uint8_t, 63, uint32_t, kDomainRows<L>>(c, rows);
+  // The first block to find a value outside tells the host: a table with many would have
+  // every wavefront write to it over PCIe (1.1 ms at 60M rows).
+  auto report = [&] {
+    uint64_t* const seen = &done.set->outside;
+    if (__hip_atomic_load(seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != done.sequence &&
+        atomicExch((unsigned long long*)seen, (unsigned long long)done.sequence) != done.sequence)
+      store_host(&done.host->outside, 1);
+  };
   if (COUNTED) {
     const bool outside = __syncthreads_or(bad);
     if (threadIdx.x < 64) {
-      if (outside && threadIdx.x == 0) atomicOr(&done.set->outside, 1u);
+      if (outside && threadIdx.x == 0) report();
       end_counted(done);
     }
-  } else if (ballot(bad) && (threadIdx.x & 63) == 0 &&
-             __hip_atomic_load(&done.host->outside, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0) {
-    store_host(&done.host->outside, 1);
+  } else if (ballot(bad) && (threadIdx.x & 63) == 0) {
+    report();
   }
 }
 
