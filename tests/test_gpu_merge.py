@@ -1,6 +1,7 @@
-"""The merge at the end of a scan kernel: grids of one block, around the 64 tables of a merge
-set, around the 144 blocks from which q1_enqueue merges through a set, and of many blocks per
-table; twice in a row, since every launch must leave its set zero."""
+"""The merge at the end of a scan kernel: grids of one block, around the 8 blocks up to which
+q1_run's blocks each leave a record for the host, around the 64 tables of a merge set, around
+the 144 blocks from which q1_enqueue merges through a set, and of many blocks per table; twice
+in a row, since every launch must leave its set zero."""
 import ctypes as C
 
 import numpy as np
@@ -10,7 +11,7 @@ from tpchq01_gpu_amd import q1
 
 pytestmark = pytest.mark.gpu
 
-BLOCKS = [1, 2, 17, 63, 64, 65, 129, 143, 144, 1000]
+BLOCKS = [1, 2, 8, 9, 17, 63, 64, 65, 129, 143, 144, 1000]
 LANES, LANE_ROWS = 64, 16
 
 

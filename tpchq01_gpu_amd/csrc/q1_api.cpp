@@ -184,12 +184,15 @@ q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bo
                        const LaunchShape& shape) {
   a.host = ctx->d_result;
   a.sequence = ++ctx->sequence;
+  const bool direct = can_launch_direct(placement, layout, fast, shape);
+  ctx->results = direct ? shape.blocks : 1;
   if (shape.blocks == 0) {
     std::memset(ctx->h_result, 0, sizeof(HostResult));
     ctx->h_result->sequence = a.sequence;
     return Q1_OK;
   }
-  const q1_status s = scan_on(ctx, placement, layout, fast, a, shape, (void*)ctx->stream);
+  const q1_status s = direct ? launch_direct(layout, a, shape, (void*)ctx->stream)
+                             : scan_on(ctx, placement, layout, fast, a, shape, (void*)ctx->stream);
   return s == Q1_OK ? Q1_OK : fail(ctx, s, "scan kernel launch failed");
 }
 
@@ -214,12 +217,35 @@ double clock_ms(const q1_ctx* ctx, uint64_t begin, uint64_t end) {
   return ctx->clock_khz > 0 ? (double)(end - begin) / ctx->clock_khz : 0.0;
 }
 
+// sum += other, the 128-bit fields as (lo, hi) pairs.
+static void add_aggregates(q1_device_aggregates* sum, const q1_device_aggregates& other) {
+  for (int g = 0; g < Q1_NUM_GROUPS; g++) {
+    sum->sum_qty[g] += other.sum_qty[g];
+    sum->sum_base_price[g] += other.sum_base_price[g];
+    sum->sum_disc[g] += other.sum_disc[g];
+    sum->count[g] += other.count[g];
+    sum->sum_disc_price_lo[g] += other.sum_disc_price_lo[g];
+    sum->sum_disc_price_hi[g] += other.sum_disc_price_hi[g] + (sum->sum_disc_price_lo[g] < other.sum_disc_price_lo[g]);
+    sum->sum_charge_lo[g] += other.sum_charge_lo[g];
+    sum->sum_charge_hi[g] += other.sum_charge_hi[g] + (sum->sum_charge_lo[g] < other.sum_charge_lo[g]);
+  }
+}
+
 q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms) {
   const HostResult* r = ctx->h_result;
-  const q1_status s = wait_sequence(ctx, &r->sequence, ctx->sequence);
-  if (s != Q1_OK) return s;
-  q1_aggregates_to_result(&r->sums, out);
-  *kernel_ms = clock_ms(ctx, r->clock_begin, r->clock_end);
+  for (uint32_t i = 0; i < ctx->results; i++) {
+    const q1_status s = wait_sequence(ctx, &r[i].sequence, ctx->sequence);
+    if (s != Q1_OK) return s;
+  }
+  q1_device_aggregates sum = r[0].sums;
+  uint64_t begin = r[0].clock_begin, end = r[0].clock_end;
+  for (uint32_t i = 1; i < ctx->results; i++) {
+    add_aggregates(&sum, r[i].sums);
+    begin = std::min(begin, r[i].clock_begin);
+    end = std::max(end, r[i].clock_end);
+  }
+  q1_aggregates_to_result(&sum, out);
+  *kernel_ms = clock_ms(ctx, begin, end);
   return Q1_OK;
 }
 
@@ -407,9 +433,9 @@ q1_status q1_init(int device, q1_ctx** out) {
   ok = ok && hipEventCreate(&ctx->ev_h2d_begin) == hipSuccess && hipEventCreate(&ctx->ev_h2d_end) == hipSuccess;
   ok = ok && hipMalloc(&ctx->d_aggr, sizeof(q1_device_aggregates)) == hipSuccess;
   ok = ok && hipHostMalloc(&ctx->h_aggr, sizeof(q1_device_aggregates), hipHostMallocDefault) == hipSuccess;
-  ok = ok && hipHostMalloc(&ctx->h_result, sizeof(HostResult), hipHostMallocMapped) == hipSuccess &&
+  ok = ok && hipHostMalloc(&ctx->h_result, kDirectBlocks * sizeof(HostResult), hipHostMallocMapped) == hipSuccess &&
        hipHostGetDevicePointer((void**)&ctx->d_result, ctx->h_result, 0) == hipSuccess;
-  if (ok) std::memset(ctx->h_result, 0, sizeof(HostResult));
+  if (ok) std::memset(ctx->h_result, 0, kDirectBlocks * sizeof(HostResult));
   ok = ok && hipDeviceGetAttribute(&ctx->clock_khz, hipDeviceAttributeWallClockRate, device) == hipSuccess;
   ok = ok && hipMalloc(&ctx->set, sizeof(MergeSet)) == hipSuccess;
   ok = ok && hipMemset(ctx->set, 0, sizeof(MergeSet)) == hipSuccess;

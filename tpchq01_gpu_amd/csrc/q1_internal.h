@@ -55,7 +55,8 @@ struct q1_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev_begin = nullptr, ev_end = nullptr, ev_h2d_begin = nullptr, ev_h2d_end = nullptr;
-  q1::HostResult* h_result = nullptr;      // pinned: what q1_run's kernel leaves for the host
+  q1::HostResult* h_result = nullptr;      // pinned, kDirectBlocks: what q1_run's kernel leaves
+  uint32_t results = 1;                    // records that the last launch leaves
   q1::HostResult* d_result = nullptr;      // ... as the device addresses it
   uint64_t sequence = 0;                   // number of the last launch that wrote h_result
   int32_t clock_khz = 0;                   // rate of the device clock in h_result

@@ -92,7 +92,8 @@ struct ScanArgs {
   // merges into the set's table b & table_mask, and the last block folds the tables into
   // *host (stored, with the clocks and `sequence`; host memory as the device addresses it),
   // or, when host is null, into *out (added; `sequence` then goes to *done if not null, once
-  // the set is zero again).
+  // the set is zero again).  A direct launch (launch_direct) leaves a record per block in
+  // host[0 ..].
   uint32_t table_mask;
   MergeSet* set;
   HostResult* host;
@@ -117,6 +118,13 @@ q1_status make_shape(q1_placement placement, q1_layout layout, bool fast, const 
 // through a set: 64 blocks 12.2 / 14.8 us, 128 blocks 14.5 / 15.1, 176 blocks 16.1 / 15.1,
 // 512 blocks 30.8 / 16.5, 4096 blocks 167 / 35.5.
 constexpr uint32_t kSpreadMinBlocks = 144;
+
+// The shortest fast launches of the LDS-table placement may instead leave each block's sums in a
+// record of its own, a.host[block], for the host to add.  The line: 5 blocks 14.3 us per q1_run
+// with a set, 12.4 with records; 10 blocks 13.7 / 12.8; 16 blocks 13.5 / 14.2.
+constexpr uint32_t kDirectBlocks = 8;
+bool can_launch_direct(q1_placement placement, q1_layout layout, bool fast, const LaunchShape& shape);
+q1_status launch_direct(q1_layout layout, const ScanArgs& a, const LaunchShape& shape, void* stream);
 
 // Where a scan's sums go.  host: stored into a.host (needs `set`; every grid merges through
 // it).  Otherwise added into *a.out, through `set` when there is one and the grid has at

@@ -246,6 +246,15 @@ FastFn fast_kernel(q1_layout l, int p, uint32_t threads) {
   }
 }
 
+GenFn direct_kernel(q1_layout l, uint32_t threads) {
+  switch (l) {
+    case Q1_LAYOUT_REFERENCE: return direct_kernel_reference(threads);
+    case Q1_LAYOUT_UNCOMPRESSED: return direct_kernel_uncompressed(threads);
+    case Q1_LAYOUT_COMPRESSED: return direct_kernel_compressed(threads);
+    default: return direct_kernel_pushdown(threads);
+  }
+}
+
 GenFn any_kernel(q1_layout l, uint32_t threads) {
   switch (l) {
     case Q1_LAYOUT_REFERENCE: return any_kernel_reference(threads);
@@ -335,31 +344,50 @@ uint64_t scan_workspace_bytes(q1_placement placement, const LaunchShape& shape) 
   return placement == Q1_PLACE_GLOBAL ? (uint64_t)shape.blocks * AccGlobal::W * kNumGroups * 8 : 0;
 }
 
+// The kernel variant of a fast launch, and its LDS.  The packed slot holds quantities in whole
+// units: the compressed layouts only.
+static int fast_variant(q1_placement placement, q1_layout layout, const LaunchShape& shape) {
+  const bool units = layout == Q1_LAYOUT_COMPRESSED || layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN;
+  if (placement != Q1_PLACE_PER_THREAD_SHARED_MEM || (uint64_t)shape.tiles_per_thread * tile_rows(layout) > 256)
+    return (int)placement;
+  return units ? kPlaceSharedPacked : kPlaceSharedNarrow;
+}
+
+static uint32_t fast_lds(int variant, const LaunchShape& shape) {
+  const bool shared = variant == kPlaceSharedNarrow || variant == (int)Q1_PLACE_PER_THREAD_SHARED_MEM;
+  const uint32_t table = variant == kPlaceSharedPacked ? packed_table_bytes(shape.threads)
+                         : shared                     ? shared_table_bytes(shape.threads)
+                                                      : stage_bytes(shape.threads);
+  return table + shape.threads / 64 * kNumGroups * NF * 8;
+}
+
+bool can_launch_direct(q1_placement placement, q1_layout layout, bool fast, const LaunchShape& shape) {
+  return fast && shape.blocks >= 1 && shape.blocks <= kDirectBlocks &&
+         fast_variant(placement, layout, shape) != (int)placement;
+}
+
+q1_status launch_direct(q1_layout layout, const ScanArgs& a, const LaunchShape& shape, void* stream) {
+  const int variant = fast_variant(Q1_PLACE_PER_THREAD_SHARED_MEM, layout, shape);
+  uint32_t tiles = shape.tiles_per_thread;
+  void* params[] = {(void*)&a, (void*)&tiles};
+  return hip_status(hipLaunchKernel((const void*)direct_kernel(layout, shape.threads), dim3(shape.blocks),
+                                    dim3(shape.threads), params, fast_lds(variant, shape), (hipStream_t)stream));
+}
+
 q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const ScanArgs& args,
                       const LaunchShape& shape, void* workspace, void* stream, MergeSet* set) {
   if (args.host && !set) return Q1_EINVAL;
   if (shape.blocks == 0) return Q1_OK;
   const hipStream_t s = (hipStream_t)stream;
-  const uint32_t nwaves = shape.threads / 64;
   ScanArgs a = args;
   a.set = set && (a.host || shape.blocks >= kSpreadMinBlocks) ? set : nullptr;
   a.table_mask = merge_tables(shape.blocks) - 1;
   if (fast) {
-    const uint64_t lane_rows = (uint64_t)shape.tiles_per_thread * tile_rows(layout);
-    const bool shared = placement == Q1_PLACE_PER_THREAD_SHARED_MEM;
-    // The packed slot holds quantities in whole units: the compressed layouts only.
-    const bool units = layout == Q1_LAYOUT_COMPRESSED || layout == Q1_LAYOUT_COMPRESSED_PUSHDOWN;
-    const int variant = shared && units && lane_rows <= 256 ? kPlaceSharedPacked
-                        : shared && lane_rows <= 256        ? kPlaceSharedNarrow
-                                                            : (int)placement;
-    uint32_t lds = variant == kPlaceSharedPacked ? packed_table_bytes(shape.threads)
-                   : shared                     ? shared_table_bytes(shape.threads)
-                                                : stage_bytes(shape.threads);
-    lds += nwaves * kNumGroups * NF * 8;
+    const int variant = fast_variant(placement, layout, shape);
     uint32_t tiles = shape.tiles_per_thread;
     void* params[] = {(void*)&a, (void*)&tiles, (void*)&workspace};
     return hip_status(hipLaunchKernel((const void*)fast_kernel(layout, variant, shape.threads), dim3(shape.blocks),
-                                      dim3(shape.threads), params, lds, s));
+                                      dim3(shape.threads), params, fast_lds(variant, shape), s));
   }
   uint32_t tiles = shape.tiles_per_thread;
   void* params[] = {(void*)&a, (void*)&tiles};

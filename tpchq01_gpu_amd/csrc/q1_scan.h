@@ -1069,8 +1069,35 @@ __device__ __forceinline__ void atomic_add128(uint64_t* lo_p, uint64_t* hi_p, ui
   if (hi + carry) atomicAdd((unsigned long long*)hi_p, (unsigned long long)(hi + carry));
 }
 
+// A store to pinned host memory.  System-scope stores go past every cache of the device, so
+// the wait for them (vmcnt 0) is all that orders them before a later one; a system-scope
+// fence would also write back the XCD's L2.
+__device__ __forceinline__ void store_host(uint64_t* p, uint64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A word, or a (lo, hi) pair, of a block's sums: added into a device table, or (DIRECT) stored
+// into the block's own record in host memory.
+template <bool DIRECT>
+__device__ __forceinline__ void put_word(uint64_t* p, uint64_t v) {
+  if (DIRECT)
+    store_host(p, v);
+  else
+    atomicAdd((unsigned long long*)p, (unsigned long long)v);
+}
+template <bool DIRECT>
+__device__ __forceinline__ void put_pair(uint64_t* lo_p, uint64_t* hi_p, uint64_t lo, uint64_t hi) {
+  if (DIRECT) {
+    store_host(lo_p, lo);
+    store_host(hi_p, hi);
+  } else {
+    atomic_add128(lo_p, hi_p, lo, hi);
+  }
+}
+
 // The block's merge into `out`: the wavefronts' sums red[wave][group][NF] are added in 128
 // bits.  qty_scale turns layout units into x100.
+template <bool DIRECT = false>
 __device__ __forceinline__ void block_merge(const uint64_t* red, q1_device_aggregates* out, uint64_t qty_scale) {
   const uint32_t nwaves = blockDim.x >> 6;
   __syncthreads();
@@ -1089,20 +1116,20 @@ __device__ __forceinline__ void block_merge(const uint64_t* red, q1_device_aggre
       plo += pv;
       phi += plo < pv;
     }
-    if (cnt) {
+    if (DIRECT || cnt) {
       switch (f) {
-        case F_QTY: atomicAdd((unsigned long long*)&out->sum_qty[g], (unsigned long long)(lo * qty_scale)); break;
-        case F_PRICE: atomicAdd((unsigned long long*)&out->sum_base_price[g], (unsigned long long)lo); break;
-        case F_DISC: atomicAdd((unsigned long long*)&out->sum_disc[g], (unsigned long long)lo); break;
-        case F_CNT: atomicAdd((unsigned long long*)&out->count[g], (unsigned long long)lo); break;
+        case F_QTY: put_word<DIRECT>(&out->sum_qty[g], lo * qty_scale); break;
+        case F_PRICE: put_word<DIRECT>(&out->sum_base_price[g], lo); break;
+        case F_DISC: put_word<DIRECT>(&out->sum_disc[g], lo); break;
+        case F_CNT: put_word<DIRECT>(&out->count[g], lo); break;
         case F_DPROD: {
           // sum_disc_price = 100 * sum_price - sum(disc * price), in 128 bits
           const unsigned __int128 p100 = ((unsigned __int128)phi << 64 | plo) * 100u;
           const unsigned __int128 dp = p100 - ((unsigned __int128)hi << 64 | lo);
-          atomic_add128(&out->sum_disc_price_lo[g], &out->sum_disc_price_hi[g], (uint64_t)dp, (uint64_t)(dp >> 64));
+          put_pair<DIRECT>(&out->sum_disc_price_lo[g], &out->sum_disc_price_hi[g], (uint64_t)dp, (uint64_t)(dp >> 64));
           break;
         }
-        default: atomic_add128(&out->sum_charge_lo[g], &out->sum_charge_hi[g], lo, hi); break;
+        default: put_pair<DIRECT>(&out->sum_charge_lo[g], &out->sum_charge_hi[g], lo, hi); break;
       }
     }
   }
@@ -1168,13 +1195,6 @@ __device__ __forceinline__ bool finish_tables(MergeTable* tables, uint32_t t, ui
   clear_counts(tables, used);
   sum = s;
   return true;
-}
-
-// A store to pinned host memory.  System-scope stores go past every cache of the device, so
-// the wait for them (vmcnt 0) is all that orders them before a later one; a system-scope
-// fence would also write back the XCD's L2.
-__device__ __forceinline__ void store_host(uint64_t* p, uint64_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Blocks of a range of `blocks` blocks that share the table of block b.
@@ -1345,7 +1365,7 @@ __device__ __forceinline__ void add_tiles(const ScanArgs& a, uint64_t base, uint
 // ------------------------------------------------------------------------------------
 // One block's share of a range: block `block` of the grid that launch_scan would run over
 // a's rows, merged into *out.  `lds` is the block's dynamic LDS.
-template <int L, int P, int B>
+template <int L, int P, int B, bool DIRECT = false>
 __device__ __forceinline__ void scan_block(const ScanArgs& a, uint64_t block, uint32_t host_tiles_per_thread,
                                            uint64_t* ws, uint64_t* lds, q1_device_aggregates* out) {
   using Tile = typename TileOf<L>::T;
@@ -1388,7 +1408,7 @@ __device__ __forceinline__ void scan_block(const ScanArgs& a, uint64_t block, ui
       acc.words(w);
       sum_lane_words(w, lds, red);
     }
-    block_merge(red, out, qty_scale);
+    block_merge<DIRECT>(red, out, qty_scale);
   }
 }
 
@@ -1399,6 +1419,28 @@ scan_fast(ScanArgs a, uint32_t host_tiles_per_thread, uint64_t* ws) {
   begin_scan(a);
   scan_block<L, P, B>(a, blockIdx.x, host_tiles_per_thread, ws, lds, merge_target(a));
   finish_scan(a);
+}
+
+// The shortest queries: a grid of at most kDirectBlocks blocks, each of which leaves its sums,
+// clocks and `sequence` in a host record of its own, for the host to add.  What it saves is the
+// chain at a short kernel's end of an atomic, the block count, the exchange and the store, each
+// waiting a microsecond for the last: 5,003 rows (2 blocks) 13.2 -> 11.5 us per call, kernel 5.5
+// -> 3.7; 5 blocks 14.3 -> 12.4; 10 blocks 13.7 -> 12.8.  At 16 blocks the host's reading of the
+// records costs more (13.5 -> 14.2 us).  A kernel of its own, without an argument for it: the
+// choice at run time in every kernel's tail, and one more word of ScanArgs, each made all
+// longer launches 0.3 us slower.
+template <int L, int P, int B>
+__global__ void __launch_bounds__(B)
+scan_direct(ScanArgs a, uint32_t host_tiles_per_thread) {
+  extern __shared__ uint64_t lds[];
+  HostResult* const mine = a.host + blockIdx.x;
+  if (thread_index() == 0) store_host(&mine->clock_begin, wall_clock64());
+  scan_block<L, P, B, true>(a, blockIdx.x, host_tiles_per_thread, nullptr, lds, &mine->sums);
+  if (thread_index() < 64) {  // wavefront 0 stored the sums
+    if (thread_index() == 0) store_host(&mine->clock_end, wall_clock64());
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (thread_index() == 0) store_host(&mine->sequence, a.sequence);
+  }
 }
 
 // ------------------------------------------------------------------------------------
@@ -1821,6 +1863,14 @@ FastFn fast_fn(int p, uint32_t threads) {
   return threads == 64 ? fast_fn_b<L, 64>(p) : threads == 128 ? fast_fn_b<L, 128>(p) : fast_fn_b<L, 256>(p);
 }
 
+// The direct kernel of the LDS table for at most 256 rows per lane.
+template <int L>
+GenFn direct_fn(uint32_t threads) {
+  constexpr bool units = L == Q1_LAYOUT_COMPRESSED || L == Q1_LAYOUT_COMPRESSED_PUSHDOWN;
+  constexpr int P = units ? kPlaceSharedPacked : kPlaceSharedNarrow;
+  return threads == 64 ? scan_direct<L, P, 64> : threads == 128 ? scan_direct<L, P, 128> : scan_direct<L, P, 256>;
+}
+
 template <int L>
 GenFn any_fn(uint32_t threads) {
   return threads == 64 ? scan_any<L, 64> : threads == 128 ? scan_any<L, 128> : scan_any<L, 256>;
@@ -1844,6 +1894,7 @@ void* batch_fn(q1_placement p) {
 // Kernel entry points of one layout, defined by that layout's translation unit.
 #define Q1_DECLARE_LAYOUT_KERNELS(NAME)                  \
   FastFn fast_kernel_##NAME(int placement, uint32_t threads); \
+  GenFn direct_kernel_##NAME(uint32_t threads);          \
   GenFn any_kernel_##NAME(uint32_t threads);             \
   uint32_t any_kernel_lds_##NAME(uint32_t threads);      \
   void* batch_kernel_##NAME(q1_placement placement);
@@ -1854,6 +1905,7 @@ Q1_DECLARE_LAYOUT_KERNELS(pushdown)
 
 #define Q1_DEFINE_LAYOUT_KERNELS(L, NAME)                                                          \
   FastFn fast_kernel_##NAME(int placement, uint32_t threads) { return fast_fn<L>(placement, threads); } \
+  GenFn direct_kernel_##NAME(uint32_t threads) { return direct_fn<L>(threads); }                   \
   GenFn any_kernel_##NAME(uint32_t threads) { return any_fn<L>(threads); }                         \
   uint32_t any_kernel_lds_##NAME(uint32_t threads) { return any_lds<L>(threads); }                 \
   void* batch_kernel_##NAME(q1_placement placement) { return batch_fn<L>(placement); }
