@@ -94,3 +94,22 @@ def test_grids_a_caller_chooses(ctx, layout):
             with pytest.raises(q1.Q1Error):
                 ctx.run(t, launch=q1.make_launch(tpb, tpt, least - 1))
     t.free()
+
+
+@pytest.mark.parametrize("layout,fit,most", [(q1.COMPRESSED, 1024, 1024), (q1.UNCOMPRESSED, 640, 512),
+                                             (q1.REFERENCE, 384, 256)])
+def test_default_rows_per_lane(ctx, oracle, layout, fit, most):
+    """The rows at which the default shape changes: 16 per lane up to `fit` lanes per compute
+    unit, one round of `most` lanes up to 128 rows each, then rounds of short blocks."""
+    units = 256
+    edges = [16 * units * fit, 2 * 16 * units * most, 128 * units * most]
+    rows = edges[-1] + 1
+    cols, ref = _case(layout, rows, None, np.random.default_rng(9))
+    t = ctx.upload(layout, cols, rows)
+    for n in sorted({e + d for e in edges for d in (0, 1)}):
+        print("case", q1.LAYOUT_NAMES[layout], n, flush=True)
+        want, _ = oracle.naive(ref, 0, n, 730100)
+        assert _as_dicts(ctx.run(t, 0, n, 730100)) == want, n
+        lane = ctx.last_timing().tuples_per_thread
+        assert lane == 16 if n <= edges[0] else 16 < lane <= 128
+    t.free()

@@ -50,20 +50,22 @@ q1_placement resolve_placement(q1_ctx* ctx, q1_layout layout, q1_placement p) {
 // The any-value kernel's shape.  Lanes per block: 256 for the compressed layouts, 128 for the
 // others, whose LDS tables of 61 and 86 KB per 256 lanes leave a compute unit two blocks or
 // one (60M reference rows 371 us with 256 lanes, 354 with 128; 2M compressed rows 10.0 and
-// 11.2 us, 600M 0.82 and 0.83 ms).  Rows per lane: 128, or 64 where 128 would give fewer than
-// 2048 lanes per compute unit (the last of few rounds of large blocks leaves compute units
-// idle), and less only to have half the lanes whose tables fit a compute unit's LDS (a
-// block's fixed cost shows; 2M reference rows 18.9 us with 32 rows per lane, 23.3 with 16,
-// whose 1,024 blocks are a third more than fit).
-// Compressed / uncompressed / reference: 60M rows with 64 rows per lane 94 / 190 / 341 us,
-// with 128 98 / 200 / 354; 6M rows with 32 18 / 33 / 46, with 64 21 / 30 / 45, with 128 29 /
-// 44 / 48; 1M rows with 16 12 / 14 / 15, with 64 15 / 21 / 21.
-constexpr uint32_t kAnyTuples = 128, kAnyManyLanes = 2048;
-static uint32_t any_value_lanes(q1_layout l) {
-  return l == Q1_LAYOUT_REFERENCE ? 192 : l == Q1_LAYOUT_UNCOMPRESSED ? 320 : 512;
-}
-static uint32_t any_value_threads(q1_layout l) {
-  return l == Q1_LAYOUT_COMPRESSED || l == Q1_LAYOUT_COMPRESSED_PUSHDOWN ? 256 : 128;
+// 11.2 us).  Rows per lane: what makes the grid one round of the chip, since the last of two
+// or three rounds leaves compute units idle (8.4M reference rows 56 us with 128 rows per lane,
+// one round, and 63 with 64; 12M uncompressed rows 47 with 96 and 55 with 64; 20M compressed
+// rows 38 with 80 and 41 with 64): 16 while all lanes' tables fit the LDS (`fit` lanes per
+// compute unit), else the fewest for which `lanes` do, an even share of its four SIMDs, at
+// most 128.  Above that, many rounds of short blocks, whose last round is short: 60M rows with
+// 32 / 64 / 128 per lane: compressed 101 / 98 / 102, uncompressed 193 / 197 / 207, reference
+// 345 / 349 / 353.
+struct AnyShape {
+  uint32_t threads, fit, lanes, many;
+};
+constexpr uint32_t kAnyTuples = 128;
+static AnyShape any_value_shape(q1_layout l) {
+  return l == Q1_LAYOUT_REFERENCE      ? AnyShape{128, 384, 256, 32}
+         : l == Q1_LAYOUT_UNCOMPRESSED ? AnyShape{128, 640, 512, 32}
+                                       : AnyShape{256, 1024, 1024, 64};
 }
 
 // The tuned shape for a range of `rows` rows: of the shapes tuned at several row counts,
@@ -88,7 +90,8 @@ static q1_launch tuned_for_rows(const q1_ctx* ctx, q1_layout layout, q1_placemen
 
 void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, uint64_t rows, const q1_launch* in,
                     q1_launch* out, bool table) {
-  q1_launch t{any_value_threads(layout), kAnyTuples, 0, 0};
+  const AnyShape any = any_value_shape(layout);
+  q1_launch t{any.threads, kAnyTuples, 0, 0};
   if (fast)
     t = tuned_for_rows(ctx, layout, p, rows);
   else if (in && in->num_blocks)
@@ -100,21 +103,23 @@ void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, ui
   out->flags = in ? in->flags : 0;
   // A caller-chosen value is kept as given.
   if ((in && in->tuples_per_thread) || out->num_blocks) return;
-  // A range smaller than the row counts the shape was tuned at halves its tuples_per_thread
-  // until the grid has at least `lanes` lanes (for the tuned shapes 4 blocks) per compute unit,
-  // so small requests still spread over the whole chip.
-  const uint64_t tpb = out->threads_per_block ? out->threads_per_block : 256;
-  auto halve = [&](uint64_t lanes, uint32_t least) {
-    const uint64_t want = lanes * (uint64_t)(ctx->compute_units > 0 ? ctx->compute_units : 256);
-    while (out->tuples_per_thread > least && rows < want * out->tuples_per_thread)
-      out->tuples_per_thread = std::max<uint32_t>(16, (out->tuples_per_thread / 2) & ~15u);
-  };
-  if (fast) {
-    halve(4 * tpb, 16);
-  } else {
-    halve(kAnyManyLanes, kAnyTuples / 2);
-    halve(any_value_lanes(layout), 16);
+  const uint64_t units = ctx->compute_units > 0 ? ctx->compute_units : 256;
+  if (!fast) {
+    const uint64_t a_round = 16 * units * any.lanes;
+    if (rows <= 16 * units * any.fit)
+      out->tuples_per_thread = 16;
+    else if (rows <= a_round * (kAnyTuples / 16))
+      out->tuples_per_thread = 16 * (uint32_t)((rows + a_round - 1) / a_round);
+    else
+      out->tuples_per_thread = any.many;
+    return;
   }
+  // A range smaller than the row counts the shape was tuned at halves its tuples_per_thread
+  // until the grid has at least 4 blocks per compute unit, so small requests still spread over
+  // the whole chip.
+  const uint64_t tpb = out->threads_per_block ? out->threads_per_block : 256;
+  while (out->tuples_per_thread > 16 && rows < 4 * tpb * units * out->tuples_per_thread)
+    out->tuples_per_thread = std::max<uint32_t>(16, (out->tuples_per_thread / 2) & ~15u);
 }
 
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
