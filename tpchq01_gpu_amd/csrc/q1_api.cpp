@@ -122,6 +122,22 @@ void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, ui
     out->tuples_per_thread = std::max<uint32_t>(16, (out->tuples_per_thread / 2) & ~15u);
 }
 
+static void give_back_spare(q1_ctx* ctx) {
+  if (ctx->spare.p) (void)hipFree(ctx->spare.p);
+  ctx->spare = SpareFilter{};
+}
+
+// hipMalloc that gives the spare bitmap back when there is no more memory.
+static hipError_t device_malloc(q1_ctx* ctx, void** p, uint64_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && ctx->spare.p) {
+    (void)hipGetLastError();
+    give_back_spare(ctx);
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
   if (bytes <= ctx->workspace_bytes) return Q1_OK;
   if (ctx->workspace) {
@@ -130,7 +146,7 @@ q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
     ctx->workspace = nullptr;
     ctx->workspace_bytes = 0;
   }
-  Q1_HIP(ctx, hipMalloc(&ctx->workspace, bytes));
+  Q1_HIP(ctx, device_malloc(ctx, &ctx->workspace, bytes));
   ctx->workspace_bytes = bytes;
   return Q1_OK;
 }
@@ -373,10 +389,32 @@ static void load_tuning_file(q1_ctx* ctx) {
   }
 }
 
+// A bitmap of at least `bytes` bytes.  The context stream runs the launches that read the spare
+// one before those of its next table; for launches on other streams the device is waited for,
+// as hipFree would have.
+static bool filter_malloc(q1_ctx* ctx, uint64_t bytes, q1_table* t) {
+  if (ctx->spare.bytes >= bytes && (!ctx->spare.shared || hipDeviceSynchronize() == hipSuccess)) {
+    t->owned[7] = ctx->spare.p;
+    t->filter_bytes = ctx->spare.bytes;
+    ctx->spare = SpareFilter{};
+    return true;
+  }
+  void* p = nullptr;
+  if (device_malloc(ctx, &p, bytes) != hipSuccess) return false;
+  t->owned[7] = p;
+  t->filter_bytes = bytes;
+  return true;
+}
+
 // Frees a table with its context's lock held (every entry point that creates tables
 // holds it when a creation fails).
 static void release_table(q1_table* t) {
   if (q1_ctx* ctx = t->ctx) {
+    if (t->filter_bytes > ctx->spare.bytes && t->filter_bytes <= kSpareFilterBytes) {
+      const SpareFilter kept{t->owned[7], t->filter_bytes, t->shared};
+      t->owned[7] = ctx->spare.p;
+      ctx->spare = kept;
+    }
     for (void* p : t->owned)
       if (p) (void)hipFree(p);  // waits for the device, which may still read it
     ctx->tables.erase(t);
@@ -478,6 +516,7 @@ void q1_shutdown(q1_ctx* ctx) {
     t->rows = 0;
   }
   ctx->tables.clear();
+  give_back_spare(ctx);
   if (ctx->batch) {
     batch_free(ctx->batch);
     delete ctx->batch;
@@ -543,7 +582,7 @@ static q1_status alloc_table(q1_ctx* ctx, q1_layout layout, uint64_t rows, q1_ta
   for (int i = 0; i < 8; i++) {
     if (!b[i]) continue;
     void* p = nullptr;
-    const hipError_t e = hipMalloc(&p, b[i]);
+    const hipError_t e = device_malloc(ctx, &p, b[i]);
     if (e != hipSuccess) {
       release_table(t);
       return fail(ctx, Q1_ENOMEM, "device allocation of a table column failed");
@@ -663,7 +702,10 @@ q1_status q1_table_info(const q1_table* t, q1_layout* layout, uint64_t* rows, q1
   if (!t) return Q1_EINVAL;
   if (layout) *layout = t->layout;
   if (rows) *rows = t->rows;
-  if (device) *device = t->dev;
+  if (device) {
+    t->shared = true;
+    *device = t->dev;
+  }
   return Q1_OK;
 }
 
@@ -702,6 +744,7 @@ q1_status q1_build_filter(q1_ctx* ctx, const q1_table* compressed, int32_t cutof
   *out = nullptr;
   GUARD_BEGIN
   std::lock_guard<std::mutex> g(ctx->lock);
+  Q1_HIP(ctx, hipSetDevice(ctx->device));
   q1_table* t = new q1_table();
   t->ctx = ctx;
   t->layout = Q1_LAYOUT_COMPRESSED_PUSHDOWN;
@@ -713,13 +756,11 @@ q1_status q1_build_filter(q1_ctx* ctx, const q1_table* compressed, int32_t cutof
   ctx->tables.insert(t);
   const uint64_t words = (t->rows + 31) / 32;
   if (words) {
-    void* f = nullptr;
-    if (hipMalloc(&f, words * 4) != hipSuccess) {
-      ctx->tables.erase(t);
-      delete t;
+    if (!filter_malloc(ctx, words * 4, t)) {
+      release_table(t);
       return fail(ctx, Q1_ENOMEM, "filter allocation failed");
     }
-    t->owned[7] = f;
+    void* const f = t->owned[7];
     t->dev.filter = f;
     t->device_bytes = words * 4;
     q1_status s = hipEventRecord(ctx->ev_begin, ctx->stream) == hipSuccess ? Q1_OK : Q1_EDEVICE;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <mutex>
 #include <string>
 #include <unordered_set>
@@ -20,6 +21,10 @@ struct q1_table {
   bool fast = false;             // inside the TPC-H value domain
   uint64_t device_bytes = 0;
   int32_t filter_cutoff = 0;     // pushdown tables: the cutoff their bitmap encodes
+  uint64_t filter_bytes = 0;     // ... and what is allocated for it
+  // Whether work on other streams than the context's may read the table (its pointers were
+  // handed out, or a server got a request on it).
+  mutable std::atomic<bool> shared{false};
 };
 
 // q1_run_streaming's chunk rows and stream count when neither the caller nor the tuning
@@ -43,6 +48,16 @@ struct SetPool {
   uint64_t sequence = 0;
   size_t cursor = 0;
   bool stalled = false;           // the last wait for a set was in vain
+};
+// The filter bitmap of a freed table, kept for the next q1_build_filter (a query per cutoff
+// builds, reads and frees one: hipMalloc and hipFree were 40 of the 160 us of such a query over
+// 60M rows).  At most kSpareFilterBytes (a bitmap of 512M rows), given back when an allocation
+// fails and with the context.
+constexpr uint64_t kSpareFilterBytes = 64ull << 20;
+struct SpareFilter {
+  void* p = nullptr;
+  uint64_t bytes = 0;
+  bool shared = false;            // as its table was
 };
 // A launch shape tuned on ranges of `rows` rows ("launch_at" lines of the tuning file).
 struct SizedLaunch {
@@ -84,6 +99,7 @@ struct q1_ctx {
   q1::StreamState* streaming = nullptr;    // cached staging buffers and streams of q1_run_streaming
   q1::MergeSet* set = nullptr;             // merge set of the context stream
   q1::SetPool pool;                        // merge sets of launches on callers' streams
+  q1::SpareFilter spare;                   // a freed table's filter bitmap, for the next one
   std::unordered_set<q1_table*> tables;    // live tables (released device memory at shutdown)
   std::mutex lock;                         // serialises calls that share the context stream
 };

@@ -395,6 +395,7 @@ q1_status q1_server_submit(q1_server* sv, const q1_request* req, uint64_t* ticke
   std::unique_lock<std::mutex> lk(sv->m);
   if (sv->stop) return Q1_ECANCELED;
   if (sv->queue.size() >= sv->cfg.queue_capacity) return Q1_EBUSY;
+  t->shared = true;
   Pending p{sv->next_ticket++, *req, Clock::now()};
   *ticket = p.ticket;
   // An idle server launches the request from this thread, with no hand-off to the
