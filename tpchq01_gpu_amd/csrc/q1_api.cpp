@@ -763,20 +763,15 @@ q1_status q1_build_filter(q1_ctx* ctx, const q1_table* compressed, int32_t cutof
     void* const f = t->owned[7];
     t->dev.filter = f;
     t->device_bytes = words * 4;
-    q1_status s = hipEventRecord(ctx->ev_begin, ctx->stream) == hipSuccess ? Q1_OK : Q1_EDEVICE;
-    if (s == Q1_OK)
-      s = launch_build_filter((const uint16_t*)compressed->dev.ship_date, t->rows, cutoff_day, (uint32_t*)f,
-                              ctx->stream);
-    if (s == Q1_OK && hipEventRecord(ctx->ev_end, ctx->stream) != hipSuccess) s = Q1_EDEVICE;
-    if (s == Q1_OK && hipStreamSynchronize(ctx->stream) != hipSuccess) s = Q1_EDEVICE;
+    q1_status s = launch_build_filter((const uint16_t*)compressed->dev.ship_date, t->rows, cutoff_day, (uint32_t*)f,
+                                      ctx->d_result, ++ctx->sequence, ctx->stream);
+    if (s == Q1_OK) s = wait_sequence(ctx, &ctx->h_result->sequence, ctx->sequence);
     if (s != Q1_OK) {
       release_table(t);
       return fail(ctx, s, "building the filter bitmap failed");
     }
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end);
     ctx->last = q1_timing{};
-    ctx->last.kernel_ms = ms;
+    ctx->last.kernel_ms = clock_ms(ctx, ctx->h_result->clock_begin, ctx->h_result->clock_end);
     ctx->last.rows = t->rows;
     ctx->last.bytes_read = 2 * t->rows + 4 * words;
   }

@@ -147,9 +147,10 @@ q1_status launch_generate(q1_layout layout, uint64_t seed, uint64_t rows, const 
 q1_status launch_domain_check(q1_layout layout, const q1_columns& cols, uint64_t rows, const Completion& done,
                               void* stream, bool* counted);
 
-// Device-side pushdown producer: filter bitmap of a compressed ship_date column.
-q1_status launch_build_filter(const uint16_t* ship, uint64_t rows, int32_t cutoff_day,
-                              uint32_t* filter, void* stream);
+// Device-side pushdown producer: filter bitmap of a compressed ship_date column; the clocks and
+// `sequence` in *host once it is there.
+q1_status launch_build_filter(const uint16_t* ship, uint64_t rows, int32_t cutoff_day, uint32_t* filter,
+                              HostResult* host, uint64_t sequence, void* stream);
 
 // Batched scan: one launch over many requests of one layout, TPC-H domain.  The device
 // buffer starts with a BatchHeader followed by `n` BatchDesc records and the n first blocks.
