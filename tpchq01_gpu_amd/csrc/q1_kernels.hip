@@ -67,7 +67,6 @@ __device__ __forceinline__ void end_counted(const Completion& c) {
   const uint32_t grid = gridDim.x, b = blockIdx.x, mask = kSpreadTables - 1;
   const uint32_t used = grid < kSpreadTables ? grid : kSpreadTables;
   if (!count_block(set->table, b & mask, blocks_sharing(grid, b, mask), used)) return;
-  clear_counts(set->table, used);
   __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if ((threadIdx.x & 63) == 0) store_host(&c.host->sequence, c.sequence);
 }

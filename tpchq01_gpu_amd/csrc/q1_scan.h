@@ -1138,7 +1138,8 @@ __device__ __forceinline__ void block_merge(const uint64_t* red, q1_device_aggre
 // The end of a block that merged into table t of the tables its range's blocks share, called
 // by wavefront 0 of the block, which issued the merge atomics; `sharing` blocks merge into
 // table t, and `used` tables have blocks.  Returns whether this is the last block of the
-// range (count_block): lane w then holds word w of the sums (w < 48), and the tables are zero again.
+// range (count_block): lane w then holds word w of the sums (w < 48), lane 48 what was in *extra
+// (if not null), and all of it is zero again.
 // Ordering: the tables and the counters are only ever touched by device-scope
 // atomics, which are performed at memory, past the XCDs' L2 caches.  A block counts itself
 // only after its own atomics have been performed (the wait below), so the block that draws
@@ -1149,32 +1150,31 @@ __device__ __forceinline__ void block_merge(const uint64_t* red, q1_device_aggre
 // What it replaces is a zero-fill launch before the scan, a fold launch and a copy to the
 // host after it, each 2-5 us of a short call: q1_run of 5,003 rows 32.3 -> 18.9 us, of 1M
 // rows 39.0 -> 23.9.  A block's own part is two waits for an atomic; the other blocks of
-// its compute unit cover them (600M rows, 18,311 blocks: 862 -> 847 us per call).
+// its compute unit cover them (600M rows, 18,311 blocks: 862 -> 847 us per call).  The start
+// clock is read with the tables and the counts clear themselves: 10 blocks 14.4 -> 13.8 us, 1M
+// rows 15.8 -> 15.3, a launch of 2M rows on a caller's stream 22.7 -> 22.2.
 __device__ __forceinline__ bool count_block(MergeTable* tables, uint32_t t, uint32_t sharing, uint32_t used) {
   __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   uint32_t last = 0;
   if ((thread_index() & 63) == 0) {
-    last = sharing == 1 || atomicAdd(&tables[t].merged, 1u) == sharing - 1;
-    if (last && used > 1) last = atomicAdd(&tables[0].tables_merged, 1u) == used - 1;
+    // atomicInc goes from its second argument back to 0: the last one clears the count.
+    last = sharing == 1 || atomicInc(&tables[t].merged, sharing - 1) == sharing - 1;
+    if (last && used > 1) last = atomicInc(&tables[0].tables_merged, used - 1) == used - 1;
   }
   last = (uint32_t)__builtin_amdgcn_readfirstlane((int)last);
   __asm__ volatile("" ::: "memory");
   return last;
 }
-__device__ __forceinline__ void clear_counts(MergeTable* tables, uint32_t used) {
-  const uint32_t lane = thread_index() & 63;
-  if (lane < used) atomicExch(&tables[lane].merged, 0u);
-  if (lane == 0) atomicExch(&tables[0].tables_merged, 0u);
-}
 __device__ __forceinline__ bool finish_tables(MergeTable* tables, uint32_t t, uint32_t sharing, uint32_t used,
-                                              uint64_t& sum) {
+                                              uint64_t& sum, uint64_t* extra = nullptr) {
   if (!count_block(tables, t, sharing, used)) return false;
   const uint32_t lane = thread_index() & 63;
   // Lane w sums word w of the tables in use.  A 128-bit field is two words: the lane of the
   // low one counts its carries, which then go to the lane of the high one, 6 lanes on.
   constexpr uint32_t kWords = sizeof(q1_device_aggregates) / 8;
   static_assert(kWords == 48 && kNumGroups == 6, "8 fields of 6 groups, the 128-bit ones at words 12..35");
-  uint64_t s = 0, carry = 0;
+  uint64_t s = 0, carry = 0, other = 0;
+  if (extra && lane == kWords) other = atomicExch((unsigned long long*)extra, 0ull);
   if (lane < kWords) {
     for (uint32_t k = 0; k < used; k += 16) {
       uint64_t v[16];
@@ -1192,8 +1192,7 @@ __device__ __forceinline__ bool finish_tables(MergeTable* tables, uint32_t t, ui
   }
   const uint64_t carried = __shfl(carry, (int)lane - kNumGroups, 64);  // lanes below 6 ignore it
   if ((lane >= 18 && lane < 24) || (lane >= 30 && lane < 36)) s += carried;
-  clear_counts(tables, used);
-  sum = s;
+  sum = lane == kWords ? other : s;
   return true;
 }
 
@@ -1217,8 +1216,14 @@ __device__ __forceinline__ void finish_scan(const ScanArgs& a) {
   const uint32_t lane = thread_index() & 63;
   const uint32_t grid = gridDim.x, b = blockIdx.x, used = grid <= a.table_mask ? grid : a.table_mask + 1;
   uint64_t sum;
-  if (!finish_tables(set->table, b & a.table_mask, blocks_sharing(grid, b, a.table_mask), used, sum)) return;
+  if (!finish_tables(set->table, b & a.table_mask, blocks_sharing(grid, b, a.table_mask), used, sum,
+                     a.host ? &set->clock_begin : nullptr))
+    return;
   if (!a.host) {
+    if (a.done) {
+      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the set is zero
+      if (lane == 0) store_host(a.done, a.sequence);
+    }
     uint64_t* d = reinterpret_cast<uint64_t*>(a.out);
     const uint64_t hi = __shfl(sum, (int)lane + kNumGroups, 64);  // of a low lane: its high word
     const bool low = (lane >= 12 && lane < 18) || (lane >= 24 && lane < 30);
@@ -1228,18 +1233,12 @@ __device__ __forceinline__ void finish_scan(const ScanArgs& a) {
     } else if (lane < 48 && !high && sum) {
       atomicAdd((unsigned long long*)(d + lane), (unsigned long long)sum);
     }
-    if (a.done) {
-      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (lane == 0) store_host(a.done, a.sequence);
-    }
     return;
   }
   // Everything but the sequence number, then the number.
-  if (lane < 48) store_host(reinterpret_cast<uint64_t*>(&a.host->sums) + lane, sum);
-  if (lane == 0) {
-    store_host(&a.host->clock_begin, atomicExch((unsigned long long*)&set->clock_begin, 0ull));
-    store_host(&a.host->clock_end, wall_clock64());
-  }
+  static_assert(offsetof(HostResult, clock_begin) == sizeof(q1_device_aggregates), "word 48");
+  if (lane < 49) store_host(reinterpret_cast<uint64_t*>(&a.host->sums) + lane, sum);
+  if (lane == 0) store_host(&a.host->clock_end, wall_clock64());
   __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (lane == 0) store_host(&a.host->sequence, a.sequence);
 }
