@@ -2,11 +2,11 @@
 scripts/try_grid_params.py and the hand-entered optimum table of
 scripts/benchmark_with_optimal_params.py:39-55).
 
-Scan shapes: for every row count asked (by default 600M, 200M, 60M, 20M and 6M rows) and every
+Scan shapes: for every row count asked (by default ten from 600M to 20,000 rows) and every
 (layout, placement) it sweeps threads_per_block x tuples_per_thread, times the kernel alone
 (q1_last_timing().kernel_ms, the minimum over repetitions), skips shapes that leave fewer
 than 2 blocks per compute unit (as try_grid_params.py:78-80 does) or fewer than 8
-wavefronts, whose time depends on how their one round of blocks happens to fit the row
+wavefronts (below 5M rows fewer than 6 wavefronts, but 16 rows per lane always), whose time depends on how their one round of blocks happens to fit the row
 count (64 x 512 is 1.4 % faster than 128 x 64 at 60M compressed rows, 6 % slower at 100M
 and 11 % at 180M), and rotates between table copies when the table is smaller than the
 256 MB Infinity Cache so the timing reflects HBM.  The best shape differs with the row count: shorter launches
@@ -51,9 +51,11 @@ import time
 from . import PACKAGE_DIR, q1
 
 THREADS = [64, 128, 256]
-TUPLES = [16, 32, 64, 128, 256, 512, 1024, 2048, 4096, 8192, 16384]
-ROWS = [600_000_000, 200_000_000, 60_000_000, 20_000_000, 6_000_000]
+TUPLES = [16, 32, 48, 64, 96, 128, 256, 512, 1024, 2048, 4096, 8192, 16384]
+ROWS = [600_000_000, 200_000_000, 60_000_000, 20_000_000, 10_000_000, 6_000_000, 4_000_000, 2_000_000, 150_000,
+        20_000]
 PLACEMENT_TIE = 0.01
+SHORT_ROWS, MANY_ROWS = 5_000_000, 20_000_000
 BATCH_BLOCKS_PER_CU = [4, 8, 16, 32, 64]
 STREAM_CHUNKS = [1 << 20, 1 << 21, 1 << 22, 1 << 23, 1 << 24, 1 << 25, 1 << 26]
 STREAM_COUNTS = [1, 2, 3, 4, 6, 8]
@@ -82,7 +84,10 @@ def sweep(ctx: q1.Context, layout: int, rows: int, placements, reps: int, seed: 
             for tpb in threads:
                 for tpt in tuples:
                     blocks = -(-rows // (tpb * tpt))
-                    if blocks < 2 * cus or blocks * tpb < 8 * 64 * cus:
+                    if rows < SHORT_ROWS:
+                        if tpt > 16 and blocks * tpb < 6 * 64 * cus:
+                            continue
+                    elif blocks < 2 * cus or blocks * tpb < 8 * 64 * cus:
                         continue
                     launch = q1.make_launch(tpb, tpt)
                     best = float("inf")
@@ -176,7 +181,12 @@ def best_table(results, rows=None):
     """The fastest shape per (layout, placement) at `rows` rows (default: the largest row
     count measured), and the fastest placement per layout among those; the LDS table if no
     other is more than 1 % faster, since it is the fastest on shorter ranges (6M reference rows
-    41 us, 44 in registers)."""
+    41 us, 44 in registers).  Below 5M rows, of the shapes within 3 % of the fastest (5 % below
+    100,000 rows), the one with the fewest blocks, whose fixed cost shows on the still shorter
+    ranges that take it (1M compressed rows 15.4 us in 256 x 16, 17.2 in 64 x 16, which tie at
+    2M) and in the host's part of the shortest calls; then up to 20M rows, of those within 2 %,
+    the one with the most, whose last round is shorter on the ranges beside it (5M reference
+    rows 42.8 us in 256 x 16, 45.2 in 256 x 32, 2 % faster at 6M)."""
     if rows is None and results:
         rows = sizes_of(results)[0]
     best = {}
@@ -186,6 +196,14 @@ def best_table(results, rows=None):
         k = (r["layout"], r["placement"])
         if k not in best or r["kernel_ms"] < best[k]["kernel_ms"]:
             best[k] = r
+    if rows is not None and rows < MANY_ROWS:
+        fewest = 1 if rows < SHORT_ROWS else -1
+        tie = 0.05 if rows < 100_000 else 0.03 if rows < SHORT_ROWS else 0.02
+        near = {k: r["kernel_ms"] * (1 + tie) for k, r in best.items()}
+        for r in results:
+            k = (r["layout"], r["placement"])
+            if r["rows"] == rows and r["kernel_ms"] <= near[k] and fewest * r["blocks"] < fewest * best[k]["blocks"]:
+                best[k] = r
     per_layout = {}
     for (l, p), r in best.items():
         if l not in per_layout or r["kernel_ms"] < per_layout[l]["kernel_ms"]:
