@@ -195,7 +195,7 @@ def batch_leg(q1, ctx, spec, headline=None):
     tables = [ctx.generate(q1.COMPRESSED, spec[r][0], int(sizes[r])) for r in range(n)]
     reqs = (q1.Request * n)(*[q1.Request(tables[r].handle, 0, int(sizes[r]), int(cutoffs[r]), 0) for r in range(n)])
     outs = (q1.Result * n)()
-    # Build the graph, then warm: over the first ten or so back-to-back batches the device
+    # The first call makes the buffers; then warm: over the first ten or so back-to-back batches the device
     # time rises and falls again by 4-6 %, whatever ran before.
     for _ in range(8):
         ctx.check(q1.lib.q1_run_batch(ctx.handle, reqs, n, None, outs), "q1_run_batch")
@@ -224,7 +224,6 @@ def batch_leg(q1, ctx, spec, headline=None):
                 bms.append(b)
                 sms.append(ctx.last_timing().kernel_ms)
         one_table = {"rows": trows, "batch_kernel_ms": sum(bms) / len(bms), "scan_kernel_ms": sum(sms) / len(sms)}
-        # the 256-request graph is rebuilt on the next call of that size
     singles = []
     for r in range(n):   # warm the per-request path
         ctx.run_raw(tables[r], 0, int(sizes[r]), int(cutoffs[r]), q1.AUTO)

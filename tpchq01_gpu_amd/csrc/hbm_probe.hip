@@ -310,8 +310,8 @@ int main(int argc, char** argv) {
     std::printf("%s{\"threads_per_block\": %d, \"tuples_per_thread\": %d, \"ms\": %.4f, \"gbps\": %.1f}", s ? ", " : "",
                 b, stream_shapes[s][1], ms, bytes / ms / 1e6);
   }
-  // the batched kernel's tuned structure: 8 blocks per compute unit x 256 lanes, entries of
-  // 192 rows per lane taken with a fixed stride
+  // the batched kernel's entries (256 lanes x 192 rows), taken with a fixed stride by a resident
+  // grid of 8 blocks per compute unit
   int cus = 0;
   CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0));
   const uint32_t res_blocks = 8u * (uint32_t)cus, res_tiles = 192 / 4;

@@ -203,9 +203,9 @@ q1_status launch_batch(q1_layout layout, q1_placement placement, const BatchHead
                        void* stream);
 
 // The scratch of q1_enqueue_noalloc (q1_noalloc.hip): a static per-device array holding the
-// spread tables and kNoallocWorkspaceBytes of per-block tables for the global placement.
+// merge set and kNoallocWorkspaceBytes of per-block tables for the global placement.
 // noalloc_setup looks up the array's address on `device` (which must be current) and
-// clears its spread tables, once per device; noalloc_launch_scan is launch_scan with the
+// clears its merge set, once per device; noalloc_launch_scan is launch_scan with the
 // array as its scratch, refusing launches that need more (*why says which).
 constexpr uint64_t kNoallocWorkspaceBytes = 8ull << 20;
 q1_status noalloc_setup(int device, void* stream);
