@@ -136,7 +136,9 @@ typedef struct {
 typedef struct {
   double kernel_ms;      /* device time of the last run: q1_run, q1_run_split and q1_run_batch
                             by the device's clock, from the first block's start to the folded
-                            result; the others by HIP events around the kernels */
+                            result (q1_build_filter and a q1_run_streaming of one chunk too,
+                            the latter with its copies); the others by HIP events around the
+                            kernels */
   double h2d_ms;         /* device time of host-to-device copies of the last call */
   double wall_ms;        /* host wall-clock of the last call */
   uint64_t bytes_read;   /* algorithmic column bytes the last run read */

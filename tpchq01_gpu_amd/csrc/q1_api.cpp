@@ -253,7 +253,7 @@ static void add_aggregates(q1_device_aggregates* sum, const q1_device_aggregates
   }
 }
 
-q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms) {
+q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms, uint64_t* begin_clock) {
   const HostResult* r = ctx->h_result;
   for (uint32_t i = 0; i < ctx->results; i++) {
     const q1_status s = wait_sequence(ctx, &r[i].sequence, ctx->sequence);
@@ -268,6 +268,7 @@ q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms) {
   }
   q1_aggregates_to_result(&sum, out);
   *kernel_ms = clock_ms(ctx, begin, end);
+  if (begin_clock) *begin_clock = begin;
   return Q1_OK;
 }
 
@@ -477,9 +478,9 @@ q1_status q1_init(int device, q1_ctx** out) {
   ok = ok && hipEventCreate(&ctx->ev_h2d_begin) == hipSuccess && hipEventCreate(&ctx->ev_h2d_end) == hipSuccess;
   ok = ok && hipMalloc(&ctx->d_aggr, sizeof(q1_device_aggregates)) == hipSuccess;
   ok = ok && hipHostMalloc(&ctx->h_aggr, sizeof(q1_device_aggregates), hipHostMallocDefault) == hipSuccess;
-  ok = ok && hipHostMalloc(&ctx->h_result, kDirectBlocks * sizeof(HostResult), hipHostMallocMapped) == hipSuccess &&
+  ok = ok && hipHostMalloc(&ctx->h_result, (kDirectBlocks + 1) * sizeof(HostResult), hipHostMallocMapped) == hipSuccess &&
        hipHostGetDevicePointer((void**)&ctx->d_result, ctx->h_result, 0) == hipSuccess;
-  if (ok) std::memset(ctx->h_result, 0, kDirectBlocks * sizeof(HostResult));
+  if (ok) std::memset(ctx->h_result, 0, (kDirectBlocks + 1) * sizeof(HostResult));
   ok = ok && hipDeviceGetAttribute(&ctx->clock_khz, hipDeviceAttributeWallClockRate, device) == hipSuccess;
   ok = ok && hipMalloc(&ctx->set, sizeof(MergeSet)) == hipSuccess;
   ok = ok && hipMemset(ctx->set, 0, sizeof(MergeSet)) == hipSuccess;

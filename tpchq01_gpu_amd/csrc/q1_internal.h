@@ -70,7 +70,8 @@ struct q1_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev_begin = nullptr, ev_end = nullptr, ev_h2d_begin = nullptr, ev_h2d_end = nullptr;
-  q1::HostResult* h_result = nullptr;      // pinned, kDirectBlocks: what q1_run's kernel leaves
+  q1::HostResult* h_result = nullptr;      // pinned, kDirectBlocks: what q1_run's kernel leaves (and
+                                           // a copy's start clock behind them)
   uint32_t results = 1;                    // records that the last launch leaves
   q1::HostResult* d_result = nullptr;      // ... as the device addresses it
   uint64_t sequence = 0;                   // number of the last launch that wrote h_result
@@ -125,7 +126,7 @@ q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fa
 // blocks leaves zeros.
 q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, ScanArgs a,
                        const LaunchShape& shape);
-q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms);
+q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms, uint64_t* begin = nullptr);
 // Waits until a launch on the context stream has written `sequence` to *word (pinned).
 q1_status wait_sequence(q1_ctx* ctx, const uint64_t* word, uint64_t sequence);
 double clock_ms(const q1_ctx* ctx, uint64_t begin, uint64_t end);

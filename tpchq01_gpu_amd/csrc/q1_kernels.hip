@@ -1,5 +1,6 @@
 // gfx950 utility kernels (zero fill, generator, domain check, pushdown producer), kernel dispatch and the host-side launch helpers of the TPC-H Q1
 // path.  The scan kernels themselves are in q1_scan.h, instantiated per layout.
+#include <algorithm>
 #include <type_traits>
 
 #include "q1_scan.h"
@@ -237,6 +238,50 @@ __global__ void __launch_bounds__(256) build_filter(const uint16_t* ship, uint64
   if (blockIdx.x == 0) __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clock is there before report_end's
 }
 
+// Columns out of pinned host memory.  PCIe bounds it (57 GB/s), or its latency.  A block takes
+// pieces of 16 KiB of one column, every lane's loads all issued before any is stored: 512 blocks
+// keep 8 MiB in flight, far more than the 57 GB/s need, and leave most of every compute unit to
+// the scans of other streams.  System-scope loads go past the caches, where lines of host memory
+// that the caller has written since may be, and do not wait for them: 45 GB/s with ordinary ones.
+__device__ __forceinline__ uint64_t load_host(const uint64_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+constexpr uint32_t kFetchPiece = 256 * 8 * 8, kFetchBlocks = 512;
+inline uint64_t fetch_pieces(const FetchArgs& f) {
+  uint64_t n = 0;
+  for (uint64_t bytes : f.bytes) n += (bytes + kFetchPiece - 1) / kFetchPiece;
+  return n;
+}
+__global__ void __launch_bounds__(256) fetch_columns(FetchArgs f, uint64_t pieces) {
+  if (blockIdx.x == 0 && threadIdx.x == 0 && f.clock_begin) {
+    store_host(f.clock_begin, wall_clock64());
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  for (uint64_t next = blockIdx.x; next < pieces; next += gridDim.x) {
+    uint64_t piece = next;
+    int k = 0;
+    for (;; k++) {
+      const uint64_t n = (f.bytes[k] + kFetchPiece - 1) / kFetchPiece;
+      if (piece < n) break;
+      piece -= n;
+    }
+    const uint64_t bytes = f.bytes[k], words = bytes / 8, w0 = piece * (kFetchPiece / 8) + threadIdx.x;
+    const uint64_t* src = reinterpret_cast<const uint64_t*>(f.src[k]);
+    uint64_t* dst = reinterpret_cast<uint64_t*>(f.dst[k]);
+    uint64_t v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = w0 + i * 256 < words ? load_host(src + w0 + i * 256) : 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      if (w0 + i * 256 < words) dst[w0 + i * 256] = v[i];
+    // the column's last bytes behind its last whole word, with its last piece
+    const uint64_t tail = words * 8 + threadIdx.x;
+    if ((piece + 1) * kFetchPiece >= bytes && tail < bytes)
+      reinterpret_cast<uint8_t*>(f.dst[k])[tail] = __hip_atomic_load(
+          reinterpret_cast<const uint8_t*>(f.src[k]) + tail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // ------------------------------------------------------------------------------------
 // Dispatch
 // ------------------------------------------------------------------------------------
@@ -396,6 +441,13 @@ q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const
   void* params[] = {(void*)&a, (void*)&tiles};
   return hip_status(hipLaunchKernel((const void*)any_kernel(layout, shape.threads), dim3(shape.blocks),
                                     dim3(shape.threads), params, any_kernel_lds(layout, shape.threads), s));
+}
+
+q1_status launch_fetch(const FetchArgs& f, void* stream) {
+  const uint64_t pieces = fetch_pieces(f);
+  const uint32_t blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(pieces, kFetchBlocks));
+  hipLaunchKernelGGL(fetch_columns, dim3(blocks), dim3(256), 0, (hipStream_t)stream, f, pieces);
+  return hip_status(hipGetLastError());
 }
 
 q1_status launch_zero(void* p, uint64_t bytes, void* stream) {

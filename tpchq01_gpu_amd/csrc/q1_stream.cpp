@@ -2,7 +2,8 @@
 // host-resident streaming pipeline (src/main.cu:567-724): chunks of host columns are
 // copied into per-stream device staging buffers and aggregated by the scan kernel on the
 // same stream, so copies of one chunk overlap kernels of others; all launches add into
-// one device table.
+// one device table.  A call of one chunk runs on the context stream alone.
+#include <algorithm>
 #include <chrono>
 #include <cstring>
 #include <thread>
@@ -40,6 +41,20 @@ static void stream_state_free(StreamState* st) {
 void stream_state_release(q1_ctx* ctx) {
   stream_state_free(ctx->streaming);
   ctx->streaming = nullptr;
+}
+
+// Whether a kernel can read the bytes at p: pinned memory, at the address the host uses.
+static bool kernel_reads(const void* p, uint64_t bytes) {
+  if ((uintptr_t)p % 8) return false;
+  for (const char* q : {(const char*)p, (const char*)p + bytes - 1}) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, q) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    if (a.type != hipMemoryTypeHost || a.devicePointer != q) return false;
+  }
+  return true;
 }
 
 static void column_bytes_local(q1_layout layout, uint64_t n, uint64_t b[8]) {
@@ -118,6 +133,8 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
     q1_launch l;
     const bool fast = in_domain_flag(launch);
     resolve_launch(ctx, layout, p, fast, chunk_rows, launch, &l, false);
+    // A call of fewer rows than a chunk takes the shape for its rows.
+    const uint64_t most = std::min(rows, chunk_rows);
     StreamState* st = nullptr;
     q1_status s = prepare(ctx, layout, chunk_rows, num_streams, &st);
     if (s != Q1_OK) return s;
@@ -125,8 +142,13 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
     const char* why = "";
     s = make_shape(p, layout, fast, &l, 0, chunk_rows, &full_shape, &why);
     if (s != Q1_OK) return fail(ctx, s, why);
+    if (most < chunk_rows) {
+      if (!l.num_blocks) resolve_launch(ctx, layout, p, fast, most, launch, &l, false);
+      s = make_shape(p, layout, fast, &l, 0, most, &full_shape, &why);
+      if (s != Q1_OK) return fail(ctx, s, why);
+    }
     const uint64_t ws_bytes = scan_workspace_bytes(p, full_shape);
-    if (ws_bytes > st->workspace_bytes) {
+    if (rows > chunk_rows && ws_bytes > st->workspace_bytes) {
       for (auto& w : st->workspace) {
         if (w) (void)hipFree(w);
         w = nullptr;
@@ -145,64 +167,118 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
       (void)hipStreamSynchronize(ctx->stream);
       return fail(ctx, code, why);
     };
-    s = launch_zero(ctx->d_aggr, sizeof(q1_device_aggregates), ctx->stream);
-    if (s != Q1_OK) return fail(ctx, s, "zero kernel failed");
-    if (hipEventRecord(ctx->ev_begin, ctx->stream) != hipSuccess) return fail(ctx, Q1_EDEVICE, "event record failed");
-    for (hipStream_t ss : st->s)
-      if (hipStreamWaitEvent(ss, ctx->ev_begin, 0) != hipSuccess) return drain_fail(Q1_EDEVICE, "stream wait failed");
     const void* hsrc[8] = {host->ship_date, host->quantity, host->extended_price, host->discount,
                            host->tax, host->return_flag, host->line_status, host->filter};
-    uint64_t bytes = 0;
-    int idx = 0;
-    for (uint64_t off = 0; off < rows; off += chunk_rows, idx = (idx + 1) % num_streams) {
-      const uint64_t n = rows - off < chunk_rows ? rows - off : chunk_rows;
-      const q1_columns& dst = st->staging[(size_t)idx];
+    // Column k's share of the n rows from `off`.
+    struct Piece {
+      const char* src;
+      void* dst;
+      uint64_t len;
+    };
+    auto piece = [&](const q1_columns& dst, int k, uint64_t off, uint64_t n) {
       const void* ddst[8] = {dst.ship_date, dst.quantity, dst.extended_price, dst.discount,
                              dst.tax, dst.return_flag, dst.line_status, dst.filter};
-      hipStream_t ss = st->s[(size_t)idx];
-      for (int k = 0; k < 8; k++) {
-        if (!ddst[k]) continue;
-        uint64_t src_off, len;
-        if (packed && k == 5) {          // return flags: 16 rows per word
-          src_off = off / 16 * 4;
-          len = (n + 15) / 16 * 4;
-        } else if (packed && k >= 6) {   // line status / filter: 32 rows per word
-          src_off = off / 32 * 4;
-          len = (n + 31) / 32 * 4;
-        } else {
-          src_off = off * elem[k];
-          len = n * elem[k];
-        }
-        if (!hsrc[k]) return drain_fail(Q1_EINVAL, "a column required by the layout is NULL");
-        if (hipMemcpyAsync((void*)ddst[k], (const char*)hsrc[k] + src_off, len, hipMemcpyHostToDevice, ss) != hipSuccess)
-          return drain_fail(Q1_EDEVICE, "chunk copy failed");
-        bytes += len;
+      Piece c{(const char*)hsrc[k], (void*)ddst[k], 0};
+      if (!c.dst || !c.src) return c;
+      if (packed && k == 5) {          // return flags: 16 rows per word
+        c.src += off / 16 * 4;
+        c.len = (n + 15) / 16 * 4;
+      } else if (packed && k >= 6) {   // line status / filter: 32 rows per word
+        c.src += off / 32 * 4;
+        c.len = (n + 31) / 32 * 4;
+      } else {
+        c.src += off * elem[k];
+        c.len = n * elem[k];
       }
-      LaunchShape shape;
-      s = make_shape(p, layout, fast, &l, 0, n, &shape, &why);
-      if (s != Q1_OK) return drain_fail(s, why);
+      return c;
+    };
+    uint64_t bytes = 0;
+    double ms = 0;
+    if (rows <= chunk_rows) {
+      // One chunk: copies, scan and result one after another on the context stream, as q1_run.
+      // The join of six streams, the table's clearing and its copy back took 80 us of such a
+      // call (5,003 rows 146 -> 66 us).
+      const q1_columns& dst = st->staging[0];
+      FetchArgs f{};
+      f.clock_begin = &ctx->d_result[kDirectBlocks].clock_begin;
+      Piece c[8];
+      for (int k = 0; k < 8; k++) {
+        c[k] = piece(dst, k, 0, rows);
+        if (!c[k].dst || !rows) continue;
+        if (!c[k].src) return fail(ctx, Q1_EINVAL, "a column required by the layout is NULL");
+        bytes += c[k].len;
+        f.src[k] = c[k].src;
+        f.dst[k] = c[k].dst;
+        f.bytes[k] = c[k].len;
+      }
+      bool fetch = true;
+      for (int k = 0; k < 8 && fetch; k++) fetch = !f.bytes[k] || kernel_reads(f.src[k], f.bytes[k]);
+      if (!fetch) std::memset(f.bytes, 0, sizeof(f.bytes));
+      if (rows && launch_fetch(f, ctx->stream) != Q1_OK) return drain_fail(Q1_EDEVICE, "chunk copy failed");
+      for (int k = 0; k < 8 && !fetch; k++)
+        if (c[k].len && hipMemcpyAsync(c[k].dst, c[k].src, c[k].len, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
+          return drain_fail(Q1_EDEVICE, "chunk copy failed");
+      s = ensure_workspace(ctx, ws_bytes);
+      if (s != Q1_OK) return drain_fail(s, "workspace allocation failed");
       ScanArgs a{};
       a.cols = dst;
-      a.row_begin = 0;
-      a.row_end = n;
+      a.row_end = rows;
       a.cutoff_day = cutoff_day;
-      a.out = ctx->d_aggr;
-      s = launch_scan(p, layout, fast, a, shape, st->workspace[(size_t)idx], ss, st->set[(size_t)idx]);
+      s = scan_to_host(ctx, p, layout, fast, a, full_shape);
       if (s != Q1_OK) return drain_fail(s, "scan kernel launch failed");
+      double scan_ms = 0;
+      uint64_t begin = 0;
+      s = wait_result(ctx, out, &scan_ms, &begin);
+      if (s != Q1_OK) return s;
+      if (rows) ms = scan_ms + clock_ms(ctx, ctx->h_result[kDirectBlocks].clock_begin, begin);
+    } else {
+      const int used = (int)std::min<uint64_t>((uint64_t)num_streams, (rows + chunk_rows - 1) / chunk_rows);
+      s = launch_zero(ctx->d_aggr, sizeof(q1_device_aggregates), ctx->stream);
+      if (s != Q1_OK) return fail(ctx, s, "zero kernel failed");
+      if (hipEventRecord(ctx->ev_begin, ctx->stream) != hipSuccess) return fail(ctx, Q1_EDEVICE, "event record failed");
+      for (int i = 0; i < used; i++)
+        if (hipStreamWaitEvent(st->s[(size_t)i], ctx->ev_begin, 0) != hipSuccess)
+          return drain_fail(Q1_EDEVICE, "stream wait failed");
+      int idx = 0;
+      for (uint64_t off = 0; off < rows; off += chunk_rows, idx = (idx + 1) % num_streams) {
+        const uint64_t n = rows - off < chunk_rows ? rows - off : chunk_rows;
+        const q1_columns& dst = st->staging[(size_t)idx];
+        hipStream_t ss = st->s[(size_t)idx];
+        for (int k = 0; k < 8; k++) {
+          const Piece c = piece(dst, k, off, n);
+          if (!c.dst) continue;
+          if (!c.src) return drain_fail(Q1_EINVAL, "a column required by the layout is NULL");
+          if (hipMemcpyAsync(c.dst, c.src, c.len, hipMemcpyHostToDevice, ss) != hipSuccess)
+            return drain_fail(Q1_EDEVICE, "chunk copy failed");
+          bytes += c.len;
+        }
+        LaunchShape shape;
+        s = make_shape(p, layout, fast, &l, 0, n, &shape, &why);
+        if (s != Q1_OK) return drain_fail(s, why);
+        ScanArgs a{};
+        a.cols = dst;
+        a.row_begin = 0;
+        a.row_end = n;
+        a.cutoff_day = cutoff_day;
+        a.out = ctx->d_aggr;
+        s = launch_scan(p, layout, fast, a, shape, st->workspace[(size_t)idx], ss, st->set[(size_t)idx]);
+        if (s != Q1_OK) return drain_fail(s, "scan kernel launch failed");
+      }
+      for (int i = 0; i < used; i++) {
+        if (hipEventRecord(st->done[(size_t)i], st->s[(size_t)i]) != hipSuccess ||
+            hipStreamWaitEvent(ctx->stream, st->done[(size_t)i], 0) != hipSuccess)
+          return drain_fail(Q1_EDEVICE, "stream join failed");
+      }
+      if (hipEventRecord(ctx->ev_end, ctx->stream) != hipSuccess ||
+          hipMemcpyAsync(ctx->h_aggr, ctx->d_aggr, sizeof(q1_device_aggregates), hipMemcpyDeviceToHost, ctx->stream) !=
+              hipSuccess ||
+          hipStreamSynchronize(ctx->stream) != hipSuccess)
+        return drain_fail(Q1_EDEVICE, "final copy failed");
+      q1_aggregates_to_result(ctx->h_aggr, out);
+      float device_ms = 0;
+      (void)hipEventElapsedTime(&device_ms, ctx->ev_begin, ctx->ev_end);
+      ms = device_ms;
     }
-    for (int i = 0; i < num_streams; i++) {
-      if (hipEventRecord(st->done[(size_t)i], st->s[(size_t)i]) != hipSuccess ||
-          hipStreamWaitEvent(ctx->stream, st->done[(size_t)i], 0) != hipSuccess)
-        return drain_fail(Q1_EDEVICE, "stream join failed");
-    }
-    if (hipEventRecord(ctx->ev_end, ctx->stream) != hipSuccess ||
-        hipMemcpyAsync(ctx->h_aggr, ctx->d_aggr, sizeof(q1_device_aggregates), hipMemcpyDeviceToHost, ctx->stream) !=
-            hipSuccess ||
-        hipStreamSynchronize(ctx->stream) != hipSuccess)
-      return drain_fail(Q1_EDEVICE, "final copy failed");
-    q1_aggregates_to_result(ctx->h_aggr, out);
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, ctx->ev_begin, ctx->ev_end);
     ctx->last = q1_timing{};
     ctx->last.kernel_ms = ms;
     ctx->last.h2d_ms = ms;
