@@ -152,7 +152,7 @@ q1_status launch_domain_check(q1_layout layout, const q1_columns& cols, uint64_t
 // *clock_begin (host memory) if not null.
 // Each of seven copies through the copy engine costs a few microseconds to start and to wait for:
 // a whole q1_run_streaming call of 5,003 compressed rows takes 66 us with copies, 29 with this;
-// 300,000 rows (2.8 MB) 160 / 77; 1M (9.4 MB) 275 / 198; 4M 770 / 697; 10M (94 MB) 1762 / 1682.
+// 300,000 rows (2.8 MB) 160 / 77; 1M (9.4 MB) 275 / 198; 4M 770 / 697; 10M (94 MB) 1762 / 1682; 60M in two chunks 10100-10170 / 9930.
 struct FetchArgs {
   const void* src[8];
   void* dst[8];

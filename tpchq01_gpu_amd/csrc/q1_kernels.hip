@@ -239,14 +239,14 @@ __global__ void __launch_bounds__(256) build_filter(const uint16_t* ship, uint64
 }
 
 // Columns out of pinned host memory.  PCIe bounds it (57 GB/s), or its latency.  A block takes
-// pieces of 16 KiB of one column, every lane's loads all issued before any is stored: 512 blocks
-// keep 8 MiB in flight, far more than the 57 GB/s need, and leave most of every compute unit to
-// the scans of other streams.  System-scope loads go past the caches, where lines of host memory
+// pieces of 16 KiB of one column, every lane's loads all issued before any is stored: 128 blocks
+// keep 2 MiB in flight, which PCIe fills (200M rows 32.8-33.0 ms, as with 512; 64 blocks 33.2-33.4),
+// and leave the compute units to the scans of other streams.  System-scope loads go past the caches, where lines of host memory
 // that the caller has written since may be, and do not wait for them: 45 GB/s with ordinary ones.
 __device__ __forceinline__ uint64_t load_host(const uint64_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-constexpr uint32_t kFetchPiece = 256 * 8 * 8, kFetchBlocks = 512;
+constexpr uint32_t kFetchPiece = 256 * 8 * 8, kFetchBlocks = 128;
 inline uint64_t fetch_pieces(const FetchArgs& f) {
   uint64_t n = 0;
   for (uint64_t bytes : f.bytes) n += (bytes + kFetchPiece - 1) / kFetchPiece;

@@ -244,14 +244,23 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
         const uint64_t n = rows - off < chunk_rows ? rows - off : chunk_rows;
         const q1_columns& dst = st->staging[(size_t)idx];
         hipStream_t ss = st->s[(size_t)idx];
+        FetchArgs f{};
+        Piece c[8];
+        bool fetch = true;
         for (int k = 0; k < 8; k++) {
-          const Piece c = piece(dst, k, off, n);
-          if (!c.dst) continue;
-          if (!c.src) return drain_fail(Q1_EINVAL, "a column required by the layout is NULL");
-          if (hipMemcpyAsync(c.dst, c.src, c.len, hipMemcpyHostToDevice, ss) != hipSuccess)
-            return drain_fail(Q1_EDEVICE, "chunk copy failed");
-          bytes += c.len;
+          c[k] = piece(dst, k, off, n);
+          if (!c[k].dst) continue;
+          if (!c[k].src) return drain_fail(Q1_EINVAL, "a column required by the layout is NULL");
+          fetch = fetch && kernel_reads(c[k].src, c[k].len);
+          f.src[k] = c[k].src;
+          f.dst[k] = c[k].dst;
+          f.bytes[k] = c[k].len;
+          bytes += c[k].len;
         }
+        if (fetch && launch_fetch(f, ss) != Q1_OK) return drain_fail(Q1_EDEVICE, "chunk copy failed");
+        for (int k = 0; k < 8 && !fetch; k++)
+          if (c[k].len && hipMemcpyAsync(c[k].dst, c[k].src, c[k].len, hipMemcpyHostToDevice, ss) != hipSuccess)
+            return drain_fail(Q1_EDEVICE, "chunk copy failed");
         LaunchShape shape;
         s = make_shape(p, layout, fast, &l, 0, n, &shape, &why);
         if (s != Q1_OK) return drain_fail(s, why);
