@@ -218,11 +218,12 @@ q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bo
   return s == Q1_OK ? Q1_OK : fail(ctx, s, "scan kernel launch failed");
 }
 
-// The kernel's last store is the launch's number in pinned host memory: a short launch is
-// awaited by watching for it (an empty kernel launched and awaited so takes 6.2 us, 10.9
-// with the stream's wait), a longer one, after kWatchMicroseconds, by the stream's own wait,
-// which lets the processor go and then costs at most 5 % of the call.
-constexpr int kWatchMicroseconds = 100;
+// The kernel's last store is the launch's number in pinned host memory, for which the host
+// watches: an empty kernel launched and awaited so takes 6.2 us, 10.9 with the stream's wait,
+// and a call of 820 us 5 us less.  The stream's wait keeps the processor as busy (1.00 of a core
+// over such calls), so nothing is lost by watching for as long as a scan of 1.4G compressed rows
+// takes; then the stream's wait, which also tells when the launch has failed.
+constexpr int kWatchMicroseconds = 2000;
 q1_status wait_sequence(q1_ctx* ctx, const uint64_t* word, uint64_t sequence) {
   auto arrived = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) == sequence; };
   const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(kWatchMicroseconds);
