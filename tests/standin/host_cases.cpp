@@ -1,0 +1,137 @@
+// Cases of the library's host code over the stand-in runtime (hip_standin.h), each run in a
+// process of its own: host_cases NAME.  A failed expectation prints its line and exits with 1.
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+
+#include <sys/mman.h>
+
+#include "../../tpchq01_gpu_amd/csrc/q1_internal.h"
+#include "hip_standin.h"
+
+using namespace q1;
+using standin::state;
+
+#define EXPECT(x)                                                     \
+  do {                                                                \
+    if (!(x)) {                                                       \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #x);             \
+      std::exit(1);                                                   \
+    }                                                                 \
+  } while (0)
+
+namespace {
+
+q1_ctx* context() {
+  q1_ctx* ctx = nullptr;
+  EXPECT(q1_init(0, &ctx) == Q1_OK);
+  state().launches.clear();
+  state().copies.clear();
+  return ctx;
+}
+
+// The columns of `rows` rows of a layout at one address each.
+struct HostColumns {
+  q1_columns c{};
+  uint64_t bytes[8] = {};
+  const void** slot(int i) {
+    const void** s[8] = {&c.ship_date, &c.quantity, &c.extended_price, &c.discount,
+                         &c.tax, &c.return_flag, &c.line_status, &c.filter};
+    return s[i];
+  }
+  HostColumns(q1_layout layout, uint64_t rows) {
+    q1_layout_column_bytes(layout, rows, bytes);
+    for (int i = 0; i < 8; i++)
+      if (bytes[i]) {
+        *slot(i) = mmap(nullptr, bytes[i], PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+        EXPECT(*slot(i) != MAP_FAILED);
+      }
+  }
+};
+
+const ScanArgs& scan_args(const standin::Launch& l) { return *(const ScanArgs*)l.scan_args.data(); }
+
+// The bytes that copy kernels read from host memory.
+uint64_t fetched() {
+  uint64_t n = 0;
+  for (const standin::Launch& l : state().launches)
+    if (l.is("fetch_columns"))
+      for (uint64_t b : ((const FetchArgs*)l.fetch_args.data())->bytes) n += b;
+  return n;
+}
+uint64_t copied_in() {
+  uint64_t n = 0;
+  for (const standin::Copy& c : state().copies) n += c.to_device ? c.bytes : 0;
+  return n;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Host columns pinned in pieces, with pageable memory between them: no kernel may read them.
+void streaming_columns_pinned_in_pieces() {
+  const uint64_t rows = 1u << 20;
+  for (uint64_t chunk : {rows, rows / 4}) {
+    for (int holed = 0; holed < 7; holed++) {
+      q1_ctx* ctx = context();
+      HostColumns h(Q1_LAYOUT_COMPRESSED, rows);
+      for (int i = 0; i < 7; i++) {
+        const char* p = (const char*)*h.slot(i);
+        if (i != holed) {
+          standin::pin(p, h.bytes[i]);
+          continue;
+        }
+        // every chunk's first and last 4 KiB pinned, the middle of it not
+        const uint64_t piece = h.bytes[i] / (rows / chunk);
+        for (uint64_t at = 0; at < h.bytes[i]; at += piece) {
+          standin::pin(p + at, 4096);
+          standin::pin(p + at + piece - 4096, 4096);
+        }
+      }
+      q1_result r;
+      EXPECT(q1_run_streaming(ctx, Q1_LAYOUT_COMPRESSED, &h.c, rows, 729999, Q1_PLACE_AUTO, nullptr, chunk, 2, &r) == Q1_OK);
+      uint64_t all = 0;
+      for (uint64_t b : h.bytes) all += b;
+      EXPECT(fetched() == 0);
+      EXPECT(copied_in() == all);
+      q1_shutdown(ctx);
+    }
+  }
+}
+
+// Pinned columns, also where they begin inside their range, are read by the copy kernel.
+void streaming_pinned_columns() {
+  const uint64_t rows = 1u << 20;
+  q1_ctx* ctx = context();
+  HostColumns h(Q1_LAYOUT_COMPRESSED, rows);
+  uint64_t all = 0;
+  for (int i = 0; i < 7; i++) {
+    char* range = (char*)std::calloc(1, h.bytes[i] + 16);
+    standin::pin(range, h.bytes[i] + 16);
+    *h.slot(i) = range + (i % 2 ? 16 : 0);
+    all += h.bytes[i];
+  }
+  q1_result r;
+  EXPECT(q1_run_streaming(ctx, Q1_LAYOUT_COMPRESSED, &h.c, rows, 729999, Q1_PLACE_AUTO, nullptr, rows / 4, 2, &r) == Q1_OK);
+  EXPECT(fetched() == all && copied_in() == 0);
+  q1_shutdown(ctx);
+}
+
+const std::map<std::string, void (*)()> kCases = {
+    {"streaming_columns_pinned_in_pieces", streaming_columns_pinned_in_pieces},
+    {"streaming_pinned_columns", streaming_pinned_columns},
+};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  if (argc < 2) {
+    for (const auto& c : kCases) std::printf("%s\n", c.first.c_str());
+    return 0;
+  }
+  const auto it = kCases.find(argv[1]);
+  if (it == kCases.end()) return 2;
+  it->second();
+  return 0;
+}

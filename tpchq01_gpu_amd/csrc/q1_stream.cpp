@@ -43,18 +43,21 @@ void stream_state_release(q1_ctx* ctx) {
   ctx->streaming = nullptr;
 }
 
-// Whether a kernel can read the bytes at p: pinned memory, at the address the host uses.
+// Whether a kernel can read the bytes at p: pinned memory, at the address the host uses, and all of
+// them in the one range that holds the first (a buffer may be pinned in pieces, with pageable
+// memory between them).
 static bool kernel_reads(const void* p, uint64_t bytes) {
   if ((uintptr_t)p % 8) return false;
-  for (const char* q : {(const char*)p, (const char*)p + bytes - 1}) {
-    hipPointerAttribute_t a{};
-    if (hipPointerGetAttributes(&a, q) != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-    if (a.type != hipMemoryTypeHost || a.devicePointer != q) return false;
+  hipPointerAttribute_t a{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeHost || a.devicePointer != p ||
+      hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
   }
-  return true;
+  const uint64_t offset = (uint64_t)((const char*)p - (const char*)base);
+  return (const char*)p >= (const char*)base && offset <= size && bytes <= size - offset;
 }
 
 static void column_bytes_local(q1_layout layout, uint64_t n, uint64_t b[8]) {
