@@ -118,7 +118,43 @@ void streaming_pinned_columns() {
   q1_shutdown(ctx);
 }
 
+// Device columns that nothing reads.
+q1_columns device_columns(q1_layout layout, uint64_t rows) { return HostColumns(layout, rows).c; }
+
+const standin::Launch& last_scan() {
+  for (size_t i = state().launches.size(); i-- > 0;)
+    if (!state().launches[i].scan_args.empty()) return state().launches[i];
+  std::printf("no scan was launched\n");
+  std::exit(1);
+}
+
+// A launch that a graph records uses no merge set, on the context's stream as on a caller's: its
+// replays may overlap whatever else uses the set.
+void enqueue_under_capture() {
+  q1_ctx* ctx = context();
+  const uint64_t rows = 1u << 20;
+  const q1_columns cols = device_columns(Q1_LAYOUT_COMPRESSED, rows);
+  static q1_device_aggregates sums;
+  hipStream_t own = nullptr;
+  EXPECT(hipStreamCreateWithFlags(&own, 0) == hipSuccess);
+  for (uint32_t flags : {0u, Q1_LAUNCH_ASSUME_TPCH_DOMAIN})
+    for (void* stream : {q1_stream(ctx), (void*)own})
+      for (bool capture : {false, true, false}) {
+        const q1_launch l{64, 16, 0, flags};  // 1024 blocks
+        state().capturing = capture ? stream : nullptr;
+        EXPECT(q1_enqueue(ctx, Q1_PLACE_IN_REGISTERS, Q1_LAYOUT_COMPRESSED, &l, &sums, &cols, 0, rows, 729999, stream) ==
+               Q1_OK);
+        state().capturing = nullptr;
+        const standin::Launch& scan = last_scan();
+        EXPECT(scan.captured == capture && scan.grid == 1024 && scan.stream == stream);
+        EXPECT((scan_args(scan).set == nullptr) == capture);
+        EXPECT(!capture || scan_args(scan).done == nullptr);
+      }
+  q1_shutdown(ctx);
+}
+
 const std::map<std::string, void (*)()> kCases = {
+    {"enqueue_under_capture", enqueue_under_capture},
     {"streaming_columns_pinned_in_pieces", streaming_columns_pinned_in_pieces},
     {"streaming_pinned_columns", streaming_pinned_columns},
 };

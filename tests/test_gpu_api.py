@@ -191,6 +191,44 @@ def test_enqueue_under_graph_capture(ctx, oracle):
     t.free()
 
 
+def test_enqueue_captured_on_the_context_stream(oracle):
+    """q1_enqueue captured on the context's own stream merges directly too: replays on that stream
+    in order with q1_run, and on another stream beside q1_run and eager launches, each add exactly
+    one result and leave the others' results alone."""
+    import torch
+    rows = 1_500_007
+    ref = q1.generate_host(q1.REFERENCE, SEED + 7, rows)
+    comp = q1.generate_host(q1.COMPRESSED, SEED + 7, rows)
+    want, _ = oracle.naive(ref, 0, rows, 729999)
+    with q1.Context(0) as c:
+        t = c.upload(q1.COMPRESSED, comp, rows)
+        cols = t.device_columns()
+        l = q1.make_launch(64, 16, 0, q1.LAUNCH_ASSUME_TPCH_DOMAIN)   # 1465 blocks
+        replayed, eager = (torch.zeros(48, dtype=torch.int64, device="cuda") for _ in range(2))
+        own, other = torch.cuda.ExternalStream(c.stream()), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        note("case capture on the context stream")
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=own):
+            _enqueue(c, q1.PER_THREAD_SHARED_MEM, cols, replayed, rows, None, l)
+        torch.cuda.synchronize()
+        _assert_times(replayed, want, 0, "captured, not run")
+        k = 0
+        for stream in (own, other):
+            for rep in range(3):
+                note("case replay", stream is own, rep)
+                with torch.cuda.stream(stream):
+                    g.replay()
+                _enqueue(c, q1.IN_REGISTERS, cols, eager, rows, None, l)
+                assert as_dicts(c.run(t, 0, rows, 729999)) == want
+                torch.cuda.synchronize()
+                k += 1
+                _assert_times(replayed, want, k, ("replay", rep))
+                _assert_times(eager, want, k, ("eager", rep))
+        del g
+        t.free()
+
+
 def test_wrap_torch_columns(ctx, oracle):
     import torch
     rows = 123_457

@@ -155,11 +155,8 @@ q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
 constexpr int kPoolWaitMs = 2;  // longer than any scan of 1.5G compressed rows
 
 // A free set of the pool for a large launch on a caller's stream, its index in *index; nullptr
-// (merge directly) while the stream is being captured into a graph, whose replays would use
-// the set again, or when the sets stay in flight.
-static MergeSet* pool_set(q1_ctx* ctx, void* stream, size_t* index) {
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
+// (merge directly) when the sets stay in flight.
+static MergeSet* pool_set(q1_ctx* ctx, size_t* index) {
   SetPool& pool = ctx->pool;
   // Launches on one stream end in order, so the set after the last one given is the first to
   // come free unless streams of very different pace share the pool.
@@ -186,19 +183,30 @@ static MergeSet* pool_set(q1_ctx* ctx, void* stream, size_t* index) {
   return nullptr;
 }
 
+// Whether a launch on the stream goes into a graph, whose replays, on any stream and beside any
+// other launch, would use its merge set again: it merges directly.
+static bool captured(void* stream) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+}
+
 q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& args,
                   const LaunchShape& shape, void* stream) {
-  if (stream == (void*)ctx->stream)  // its launches run one after another
-    return launch_scan(placement, layout, fast, args, shape, ctx->workspace, stream, ctx->set);
   ScanArgs a = args;
   size_t i = 0;
-  MergeSet* set = shape.blocks >= kSpreadMinBlocks ? pool_set(ctx, stream, &i) : nullptr;
-  if (set) {
+  MergeSet *set = nullptr, *pooled = nullptr;
+  if (shape.blocks >= kSpreadMinBlocks && !captured(stream)) {
+    if (stream == (void*)ctx->stream)  // its launches run one after another
+      set = ctx->set;
+    else
+      set = pooled = pool_set(ctx, &i);
+  }
+  if (pooled) {
     a.done = ctx->pool.done_dev + i;
     a.sequence = ++ctx->pool.sequence;
   }
   const q1_status s = launch_scan(placement, layout, fast, a, shape, ctx->workspace, stream, set);
-  if (s == Q1_OK && set) ctx->pool.last[i] = a.sequence;
+  if (s == Q1_OK && pooled) ctx->pool.last[i] = a.sequence;
   return s;
 }
 
@@ -214,7 +222,7 @@ q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bo
     return Q1_OK;
   }
   const q1_status s = direct ? launch_direct(layout, a, shape, (void*)ctx->stream)
-                             : scan_on(ctx, placement, layout, fast, a, shape, (void*)ctx->stream);
+                             : launch_scan(placement, layout, fast, a, shape, ctx->workspace, (void*)ctx->stream, ctx->set);
   return s == Q1_OK ? Q1_OK : fail(ctx, s, "scan kernel launch failed");
 }
 

@@ -117,11 +117,11 @@ void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, ui
 inline bool in_domain_flag(const q1_launch* l) { return l && (l->flags & Q1_LAUNCH_ASSUME_TPCH_DOMAIN); }
 uint64_t algorithmic_bytes(q1_layout layout, uint64_t rows);
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes);
-// launch_scan with the context's merge set on the context stream, one of the pool's on a
-// caller's.
+// launch_scan for q1_enqueue: with the context's merge set on the context stream, one of the
+// pool's on a caller's, none on a stream that is being captured.
 q1_status scan_on(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
                   const LaunchShape& shape, void* stream);
-// The same on the context stream with the sums going to ctx->h_result, and the wait for
+// launch_scan on the context stream with the sums going to ctx->h_result, and the wait for
 // them: fills *out and returns the kernel's device time in *kernel_ms.  A launch with no
 // blocks leaves zeros.
 q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bool fast, ScanArgs a,
