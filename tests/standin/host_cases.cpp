@@ -153,7 +153,30 @@ void enqueue_under_capture() {
   q1_shutdown(ctx);
 }
 
+// A launch that ends without its result leaves no partial sums or block counts behind for the
+// launches after it.
+void merge_set_after_a_lost_result() {
+  q1_ctx* ctx = context();
+  HostColumns h(Q1_LAYOUT_COMPRESSED, 1u << 20);
+  q1_table* t = nullptr;
+  EXPECT(q1_table_wrap(ctx, Q1_LAYOUT_COMPRESSED, &h.c, 1u << 20, &t) == Q1_OK);
+  std::memset((void*)ctx->set, 0x55, sizeof(MergeSet));
+  state().silent = true;
+  q1_result r;
+  EXPECT(q1_run(ctx, t, 0, 1u << 20, 729999, Q1_PLACE_AUTO, nullptr, &r) == Q1_EDEVICE);
+  state().silent = false;
+  for (uint32_t i = 0; i < kSpreadTables; i++) {
+    EXPECT(ctx->set->table[i].merged == 0 && ctx->set->table[i].tables_merged == 0);
+    EXPECT(ctx->set->table[i].sums.count[0] == 0);
+  }
+  EXPECT(ctx->set->clock_begin == 0);
+  EXPECT(q1_run(ctx, t, 0, 1u << 20, 729999, Q1_PLACE_AUTO, nullptr, &r) == Q1_OK);
+  q1_table_free(t);
+  q1_shutdown(ctx);
+}
+
 const std::map<std::string, void (*)()> kCases = {
+    {"merge_set_after_a_lost_result", merge_set_after_a_lost_result},
     {"enqueue_under_capture", enqueue_under_capture},
     {"streaming_columns_pinned_in_pieces", streaming_columns_pinned_in_pieces},
     {"streaming_pinned_columns", streaming_pinned_columns},

@@ -239,7 +239,11 @@ q1_status wait_sequence(q1_ctx* ctx, const uint64_t* word, uint64_t sequence) {
     for (int i = 0; i < 16 && !arrived(); i++) __builtin_ia32_pause();
   if (!arrived()) {
     Q1_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (!arrived()) return fail(ctx, Q1_EDEVICE, "the scan kernel ended without a result");
+    if (!arrived()) {
+      // The launch's blocks were not counted to the end: the set may hold partial sums.
+      (void)launch_zero(ctx->set, sizeof(MergeSet), ctx->stream);
+      return fail(ctx, Q1_EDEVICE, "the scan kernel ended without a result");
+    }
   }
   return Q1_OK;
 }
