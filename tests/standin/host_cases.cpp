@@ -175,7 +175,43 @@ void merge_set_after_a_lost_result() {
   q1_shutdown(ctx);
 }
 
+// Calls of q1_enqueue_noalloc that overlapped spoil their own results only: whatever they left in
+// the merge set they share is cleared, in the later call's own stream, before its scan.
+void noalloc_after_an_overlap() {
+  q1_ctx* ctx = context();
+  const uint64_t rows = 1u << 20;
+  const q1_columns cols = device_columns(Q1_LAYOUT_COMPRESSED, rows);
+  static q1_device_aggregates sums;
+  hipStream_t own = nullptr;
+  EXPECT(hipStreamCreateWithFlags(&own, 0) == hipSuccess);
+  for (uint32_t flags : {0u, Q1_LAUNCH_ASSUME_TPCH_DOMAIN})
+    for (void* stream : {q1_stream(ctx), (void*)own})
+      for (bool capture : {false, true}) {
+        const q1_launch l{64, 16, 0, flags};  // 1024 blocks
+        auto enqueue = [&] {
+          return q1_enqueue_noalloc(ctx, Q1_PLACE_IN_REGISTERS, Q1_LAYOUT_COMPRESSED, &l, &sums, &cols, 0, rows, 729999,
+                                    stream);
+        };
+        EXPECT(enqueue() == Q1_OK);
+        MergeSet* set = scan_args(last_scan()).set;
+        EXPECT(set != nullptr);
+        std::memset((void*)set, 0x55, sizeof(MergeSet));
+        state().launches.clear();
+        state().capturing = capture ? stream : nullptr;
+        EXPECT(enqueue() == Q1_OK);
+        state().capturing = nullptr;
+        EXPECT(scan_args(last_scan()).set == set);
+        EXPECT(state().launches.size() == 2 && state().launches[0].is("zero_words"));
+        for (const standin::Launch& k : state().launches) EXPECT(k.stream == stream && k.captured == capture);
+        EXPECT(state().launches[0].grid * state().launches[0].block * 8ull >= sizeof(MergeSet));
+        const MergeSet clear{};
+        EXPECT(capture || std::memcmp(set, &clear, sizeof(MergeSet)) == 0);
+      }
+  q1_shutdown(ctx);
+}
+
 const std::map<std::string, void (*)()> kCases = {
+    {"noalloc_after_an_overlap", noalloc_after_an_overlap},
     {"merge_set_after_a_lost_result", merge_set_after_a_lost_result},
     {"enqueue_under_capture", enqueue_under_capture},
     {"streaming_columns_pinned_in_pieces", streaming_columns_pinned_in_pieces},

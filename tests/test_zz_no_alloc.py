@@ -59,3 +59,38 @@ def test_noalloc_matches_enqueue_on_two_calls_in_a_row():
         assert st == q1.EINVAL
         assert b"static array" in q1.lib.q1_last_error(ctx.handle)
         t.free()
+
+
+def test_noalloc_in_a_graph():
+    """Captured with a grid that merges through the static set: every replay adds one result, with
+    eager calls of another grid between the replays."""
+    import torch
+    with q1.Context(0) as ctx:
+        rows = 1_500_007
+        t = ctx.generate(q1.COMPRESSED, SEED + 1, rows)
+        cols = t.device_columns()
+        grids = [q1.make_launch(64, 16, 0, q1.LAUNCH_ASSUME_TPCH_DOMAIN), q1.make_launch(128, 32)]   # 1465, 367 blocks
+        once = run(q1.lib.q1_enqueue, ctx, q1.IN_REGISTERS, q1.COMPRESSED, grids[0], cols, 0, rows, 729999, torch)
+        agg = torch.zeros(48, dtype=torch.int64, device="cuda")
+        stream = torch.cuda.Stream()
+
+        def enqueue(launch):
+            ctx.check(q1.lib.q1_enqueue_noalloc(ctx.handle, q1.IN_REGISTERS, q1.COMPRESSED, C.byref(launch),
+                                                C.c_void_p(agg.data_ptr()), C.byref(cols), 0, rows, 729999,
+                                                C.c_void_p(stream.cuda_stream)), "q1_enqueue_noalloc")
+
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            enqueue(grids[0])
+        torch.cuda.synchronize()
+        for rep in range(3):
+            note(f"case noalloc replay {rep}")
+            g.replay()
+            torch.cuda.synchronize()
+            assert (agg.cpu().numpy() == (2 * rep + 1) * once).all(), rep   # sums of these rows stay below 2^64
+            enqueue(grids[1])
+            torch.cuda.synchronize()
+            assert (agg.cpu().numpy() == (2 * rep + 2) * once).all(), rep
+        del g
+        t.free()

@@ -8,8 +8,9 @@
 // In host code `scratch` names a host-side stand-in, not a device address: q1_init looks up
 // each device's address once (hipGetSymbolAddress, with that device current) and every use
 // goes through that address.  All calls on one GPU share the array, which keeps the last
-// call's contents: the merge set is cleared at set-up and left clear by every launch that
-// uses it, and the global placement's per-block tables are cleared by the kernel itself.  Calls that overlap on one GPU race.
+// call's contents: the merge set is cleared before every launch that uses it, and the global
+// placement's per-block tables are cleared by the kernel itself.  Calls that overlap on one GPU race:
+// their own results are wrong, those of later calls are not.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -65,8 +66,16 @@ q1_status noalloc_launch_scan(int device, q1_placement placement, q1_layout layo
     return Q1_EINVAL;
   }
   void* workspace = static_cast<char*>(base) + sizeof(MergeSet);
-  const q1_status s =
-      launch_scan(placement, layout, fast, a, shape, workspace, stream, static_cast<MergeSet*>(base));
+  MergeSet* const set = static_cast<MergeSet*>(base);
+  // A launch leaves the set clear if it had it to itself; block counts that two overlapping grids
+  // left would make every later one fold its tables too early.  The fill kernel is recorded into a
+  // caller's graph with the scan.  It costs 1.5 us of queued launches (512 blocks of 4,096 rows 13.1
+  // -> 14.6 us) and 2.8 of a lone one.
+  if (shape.blocks >= kSpreadMinBlocks && launch_zero(set, sizeof(MergeSet), stream) != Q1_OK) {
+    *why = "clearing the merge tables failed";
+    return Q1_EDEVICE;
+  }
+  const q1_status s = launch_scan(placement, layout, fast, a, shape, workspace, stream, set);
   if (s != Q1_OK) *why = "scan kernel launch failed";
   return s;
 }
