@@ -210,7 +210,33 @@ void noalloc_after_an_overlap() {
   q1_shutdown(ctx);
 }
 
+// The global placement's workspaces of the streaming pipeline grow until memory runs out: the next
+// call, which needs no more than the first had, launches no kernel without one.
+void streaming_workspace_after_a_failed_growth() {
+  q1_ctx* ctx = context();
+  const uint64_t rows = 1u << 22, chunk = 1u << 20;
+  HostColumns h(Q1_LAYOUT_COMPRESSED, rows);
+  auto stream = [&](uint32_t threads, uint32_t tuples) {
+    const q1_launch l{threads, tuples, 0, Q1_LAUNCH_ASSUME_TPCH_DOMAIN};
+    q1_result r;
+    state().launches.clear();
+    const q1_status s =
+        q1_run_streaming(ctx, Q1_LAYOUT_COMPRESSED, &h.c, rows, 729999, Q1_PLACE_GLOBAL, &l, chunk, 2, &r);
+    for (const standin::Launch& k : state().launches) EXPECT(!k.is("scan_fast") || k.workspace != nullptr);
+    return s;
+  };
+  EXPECT(stream(256, 1024) == Q1_OK);
+  const uint64_t larger = 1024 * 240;  // the tables of a chunk's 1024 blocks
+  state().budget = state().device_bytes + larger;
+  EXPECT(stream(64, 16) == Q1_ENOMEM);
+  state().budget = UINT64_MAX;
+  EXPECT(stream(256, 1024) == Q1_OK);
+  EXPECT(stream(64, 16) == Q1_OK);
+  q1_shutdown(ctx);
+}
+
 const std::map<std::string, void (*)()> kCases = {
+    {"streaming_workspace_after_a_failed_growth", streaming_workspace_after_a_failed_growth},
     {"noalloc_after_an_overlap", noalloc_after_an_overlap},
     {"merge_set_after_a_lost_result", merge_set_after_a_lost_result},
     {"enqueue_under_capture", enqueue_under_capture},

@@ -152,10 +152,13 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
     }
     const uint64_t ws_bytes = scan_workspace_bytes(p, full_shape);
     if (rows > chunk_rows && ws_bytes > st->workspace_bytes) {
+      st->workspace_bytes = 0;  // until every stream has its own
       for (auto& w : st->workspace) {
         if (w) (void)hipFree(w);
         w = nullptr;
-        if (hipMalloc(&w, ws_bytes) != hipSuccess) return fail(ctx, Q1_ENOMEM, "workspace allocation failed");
+        void* grown = nullptr;
+        if (hipMalloc(&grown, ws_bytes) != hipSuccess) return fail(ctx, Q1_ENOMEM, "workspace allocation failed");
+        w = grown;
       }
       st->workspace_bytes = ws_bytes;
     }
