@@ -200,7 +200,8 @@ q1_status q1_table_download(q1_ctx* ctx, const q1_table* t, const q1_columns* ho
 uint64_t q1_table_device_bytes(const q1_table* t);
 /* Frees the table's device memory (if its context is still alive) and the handle.  Of freed
  * pushdown tables the context keeps one bitmap, of at most 64 MiB, for the next
- * q1_build_filter; it is given back when an allocation fails and with the context. */
+ * q1_build_filter; it is given back when an allocation of the context or of its servers fails,
+ * and with the context. */
 void q1_table_free(q1_table* t);
 /* Pushdown producer on the device: builds a COMPRESSED_PUSHDOWN table sharing the
  * compressed table's columns plus a filter bitmap for `cutoff_day`.  The pushdown table

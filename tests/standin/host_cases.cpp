@@ -235,7 +235,52 @@ void streaming_workspace_after_a_failed_growth() {
   q1_shutdown(ctx);
 }
 
+// The bitmap of a freed pushdown table, kept for the next one, is given back to whatever allocation
+// of the library finds no memory left.
+void spare_bitmap_given_back() {
+  const uint64_t rows = 1u << 26;  // a bitmap of 8 MiB
+  static HostColumns h(Q1_LAYOUT_COMPRESSED, rows);
+  auto with_spare = [&](q1_ctx* ctx, const q1_table* t) {
+    q1_table* f = nullptr;
+    EXPECT(q1_build_filter(ctx, t, 729999, &f) == Q1_OK);
+    q1_table_free(f);
+    EXPECT(ctx->spare.bytes == rows / 8);
+    state().budget = state().device_bytes;
+  };
+  auto given_back = [&](const q1_ctx* ctx) {
+    state().budget = UINT64_MAX;
+    return ctx->spare.p == nullptr;
+  };
+  q1_ctx* ctx = context();
+  q1_table* t = nullptr;
+  EXPECT(q1_table_wrap(ctx, Q1_LAYOUT_COMPRESSED, &h.c, rows, &t) == Q1_OK);
+  q1_result r[2];
+  // a table's columns
+  with_spare(ctx, t);
+  q1_table* made = nullptr;
+  EXPECT(q1_table_generate(ctx, Q1_LAYOUT_COMPRESSED, 1, 10000, &made) == Q1_OK && given_back(ctx));
+  q1_table_free(made);
+  // the staging buffers of the streaming pipeline, and its workspaces
+  const q1_launch few{256, 16, 0, Q1_LAUNCH_ASSUME_TPCH_DOMAIN};
+  for (q1_placement p : {Q1_PLACE_IN_REGISTERS, Q1_PLACE_GLOBAL}) {
+    with_spare(ctx, t);
+    EXPECT(q1_run_streaming(ctx, Q1_LAYOUT_COMPRESSED, &h.c, 4096, 729999, p, &few, 1024, 2, r) == Q1_OK && given_back(ctx));
+  }
+  // the buffers of a batch
+  with_spare(ctx, t);
+  const q1_request reqs[2] = {{t, 0, 1000, 729999, 0}, {t, 5, 1000, 729999, 0}};
+  EXPECT(q1_run_batch(ctx, reqs, 2, nullptr, r) == Q1_OK && given_back(ctx));
+  // a server's merge sets
+  with_spare(ctx, t);
+  q1_server* sv = nullptr;
+  EXPECT(q1_server_create(ctx, nullptr, &sv) == Q1_OK && given_back(ctx));
+  q1_server_destroy(sv);
+  q1_table_free(t);
+  q1_shutdown(ctx);
+}
+
 const std::map<std::string, void (*)()> kCases = {
+    {"spare_bitmap_given_back", spare_bitmap_given_back},
     {"streaming_workspace_after_a_failed_growth", streaming_workspace_after_a_failed_growth},
     {"noalloc_after_an_overlap", noalloc_after_an_overlap},
     {"merge_set_after_a_lost_result", merge_set_after_a_lost_result},

@@ -123,20 +123,22 @@ void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, ui
     out->tuples_per_thread = (out->tuples_per_thread / 2 + 15) & ~15u;
 }
 
-static void give_back_spare(q1_ctx* ctx) {
-  if (ctx->spare.p) (void)hipFree(ctx->spare.p);
-  ctx->spare = SpareFilter{};
+// The spare bitmap if it holds at least `bytes` bytes; it is then the caller's.
+static SpareFilter take_spare(q1_ctx* ctx, uint64_t bytes) {
+  std::lock_guard<std::mutex> g(ctx->spare_lock);
+  SpareFilter spare;
+  if (ctx->spare.bytes >= bytes) std::swap(spare, ctx->spare);
+  return spare;
 }
 
-// hipMalloc that gives the spare bitmap back when there is no more memory.
-static hipError_t device_malloc(q1_ctx* ctx, void** p, uint64_t bytes) {
+hipError_t device_malloc(q1_ctx* ctx, void** p, uint64_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess && ctx->spare.p) {
-    (void)hipGetLastError();
-    give_back_spare(ctx);
-    e = hipMalloc(p, bytes);
-  }
-  return e;
+  if (e == hipSuccess) return e;
+  const SpareFilter spare = take_spare(ctx, 0);
+  if (!spare.p) return e;
+  (void)hipGetLastError();
+  (void)hipFree(spare.p);
+  return hipMalloc(p, bytes);
 }
 
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
@@ -408,12 +410,13 @@ static void load_tuning_file(q1_ctx* ctx) {
 // one before those of its next table; for launches on other streams the device is waited for,
 // as hipFree would have.
 static bool filter_malloc(q1_ctx* ctx, uint64_t bytes, q1_table* t) {
-  if (ctx->spare.bytes >= bytes && (!ctx->spare.shared || hipDeviceSynchronize() == hipSuccess)) {
-    t->owned[7] = ctx->spare.p;
-    t->filter_bytes = ctx->spare.bytes;
-    ctx->spare = SpareFilter{};
+  const SpareFilter spare = take_spare(ctx, bytes);
+  if (spare.p && (!spare.shared || hipDeviceSynchronize() == hipSuccess)) {
+    t->owned[7] = spare.p;
+    t->filter_bytes = spare.bytes;
     return true;
   }
+  if (spare.p) (void)hipFree(spare.p);
   void* p = nullptr;
   if (device_malloc(ctx, &p, bytes) != hipSuccess) return false;
   t->owned[7] = p;
@@ -425,10 +428,13 @@ static bool filter_malloc(q1_ctx* ctx, uint64_t bytes, q1_table* t) {
 // holds it when a creation fails).
 static void release_table(q1_table* t) {
   if (q1_ctx* ctx = t->ctx) {
-    if (t->filter_bytes > ctx->spare.bytes && t->filter_bytes <= kSpareFilterBytes) {
-      const SpareFilter kept{t->owned[7], t->filter_bytes, t->shared};
-      t->owned[7] = ctx->spare.p;
-      ctx->spare = kept;
+    if (t->filter_bytes && t->filter_bytes <= kSpareFilterBytes) {
+      std::lock_guard<std::mutex> g(ctx->spare_lock);
+      if (t->filter_bytes > ctx->spare.bytes) {
+        const SpareFilter kept{t->owned[7], t->filter_bytes, t->shared};
+        t->owned[7] = ctx->spare.p;
+        ctx->spare = kept;
+      }
     }
     for (void* p : t->owned)
       if (p) (void)hipFree(p);  // waits for the device, which may still read it
@@ -531,7 +537,7 @@ void q1_shutdown(q1_ctx* ctx) {
     t->rows = 0;
   }
   ctx->tables.clear();
-  give_back_spare(ctx);
+  if (ctx->spare.p) (void)hipFree(ctx->spare.p);
   if (ctx->batch) {
     batch_free(ctx->batch);
     delete ctx->batch;

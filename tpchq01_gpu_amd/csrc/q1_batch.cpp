@@ -54,7 +54,8 @@ static uint64_t request_blocks(const q1_request& r, uint32_t lane_rows) {
 
 // Makes room for n requests and `tables` merge tables.  The stream's earlier launches with
 // the buffers have finished.
-static q1_status reserve(BatchBuffers* b, uint32_t n, uint32_t tables, hipStream_t stream, const char** why) {
+static q1_status reserve(q1_ctx* ctx, BatchBuffers* b, uint32_t n, uint32_t tables, hipStream_t stream,
+                         const char** why) {
   auto give_up = [&](q1_status s, const char* text) {
     *why = text;
     return s;
@@ -72,7 +73,7 @@ static q1_status reserve(BatchBuffers* b, uint32_t n, uint32_t tables, hipStream
     if (hipHostMalloc(&b->h_buf, buf_bytes(cap), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc(&b->h_out, out_bytes, hipHostMallocMapped) != hipSuccess ||
         hipHostGetDevicePointer((void**)&b->h_out_dev, b->h_out, 0) != hipSuccess ||
-        hipMalloc(&b->d_buf, buf_bytes(cap)) != hipSuccess)
+        device_malloc(ctx, (void**)&b->d_buf, buf_bytes(cap)) != hipSuccess)
       return give_up(Q1_ENOMEM, "batch buffers could not be allocated");
     std::memset((void*)b->h_out, 0, out_bytes);
     b->capacity = cap;
@@ -84,7 +85,7 @@ static q1_status reserve(BatchBuffers* b, uint32_t n, uint32_t tables, hipStream
     b->control = nullptr;
     b->tables = 0;
     const uint64_t bytes = sizeof(BatchControl) + (uint64_t)t * sizeof(MergeTable);
-    if (hipMalloc(&b->control, bytes) != hipSuccess)
+    if (device_malloc(ctx, (void**)&b->control, bytes) != hipSuccess)
       return give_up(Q1_ENOMEM, "batch tables could not be allocated");
     if (launch_zero(b->control, bytes, stream) != Q1_OK) {
       (void)hipFree(b->control);
@@ -130,7 +131,7 @@ q1_status batch_launch(q1_ctx* ctx, BatchBuffers* b, const q1_request* reqs, uin
     if (tables <= kBatchMaxTables || most == 1) break;
   }
   if (entries >= (1ull << 31)) return give_up(Q1_EINVAL, "batch too large (2^31 blocks of rows)");
-  const q1_status s = reserve(b, n, (uint32_t)tables, stream, why);
+  const q1_status s = reserve(ctx, b, n, (uint32_t)tables, stream, why);
   if (s != Q1_OK) return s;
   BatchDesc* d = reinterpret_cast<BatchDesc*>(b->h_buf + 1);
   uint32_t* first = reinterpret_cast<uint32_t*>(d + n);

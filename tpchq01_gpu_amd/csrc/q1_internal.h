@@ -52,7 +52,7 @@ struct SetPool {
 // The filter bitmap of a freed table, kept for the next q1_build_filter (a query per cutoff
 // builds, reads and frees one: hipMalloc and hipFree were 40 of the 160 us of such a query over
 // 60M rows).  At most kSpareFilterBytes (a bitmap of 512M rows), given back when an allocation
-// fails and with the context.
+// of the library on the device fails (device_malloc) and with the context.
 constexpr uint64_t kSpareFilterBytes = 64ull << 20;
 struct SpareFilter {
   void* p = nullptr;
@@ -101,6 +101,7 @@ struct q1_ctx {
   q1::MergeSet* set = nullptr;             // merge set of the context stream
   q1::SetPool pool;                        // merge sets of launches on callers' streams
   q1::SpareFilter spare;                   // a freed table's filter bitmap, for the next one
+  std::mutex spare_lock;                   // guards it: server threads allocate without `lock`
   std::unordered_set<q1_table*> tables;    // live tables (released device memory at shutdown)
   std::mutex lock;                         // serialises calls that share the context stream
 };
@@ -116,6 +117,8 @@ void resolve_launch(q1_ctx* ctx, q1_layout layout, q1_placement p, bool fast, ui
                     q1_launch* out, bool table = true);
 inline bool in_domain_flag(const q1_launch* l) { return l && (l->flags & Q1_LAUNCH_ASSUME_TPCH_DOMAIN); }
 uint64_t algorithmic_bytes(q1_layout layout, uint64_t rows);
+// hipMalloc that gives the spare bitmap back when there is no more memory; needs no lock held.
+hipError_t device_malloc(q1_ctx* ctx, void** p, uint64_t bytes);
 q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes);
 // launch_scan for q1_enqueue: with the context's merge set on the context stream, one of the
 // pool's on a caller's, none on a stream that is being captured.
@@ -151,7 +154,7 @@ void batch_free(BatchBuffers* b);
 // b->sequence, or the stream has got there.  lane_rows and grid of 0 take the tuned rows per
 // lane, less for a batch too small to fill the chip, and a block per entry up to the tuned
 // grid.  *lane_rows_planned, *grid_planned: the tuned shape or the caller's.  *why: what
-// failed (ctx is only read: the server's threads launch without its lock).
+// failed (of ctx only the spare bitmap is changed: the server's threads launch without its lock).
 q1_status batch_launch(q1_ctx* ctx, BatchBuffers* b, const q1_request* reqs, uint32_t n, q1_placement placement,
                        uint32_t lane_rows, uint32_t grid, hipStream_t stream, uint32_t* lane_rows_planned,
                        uint32_t* grid_planned, const char** why);

@@ -367,7 +367,7 @@ q1_status q1_server_create(q1_ctx* ctx, const q1_server_config* cfg, q1_server**
           hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess ||
           hipHostMalloc(&s.h_result, sizeof(q1::HostResult), hipHostMallocMapped) != hipSuccess ||
           hipHostGetDevicePointer((void**)&s.h_result_dev, s.h_result, 0) != hipSuccess ||
-          hipMalloc(&s.set, sizeof(q1::MergeSet)) != hipSuccess ||
+          q1::device_malloc(ctx, (void**)&s.set, sizeof(q1::MergeSet)) != hipSuccess ||
           hipMemset(s.set, 0, sizeof(q1::MergeSet)) != hipSuccess) {
         q1_server_destroy(sv);
         return q1::fail(ctx, Q1_EDEVICE, "stream or merge-set creation failed");

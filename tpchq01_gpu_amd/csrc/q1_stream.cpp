@@ -90,7 +90,8 @@ static q1_status prepare(q1_ctx* ctx, q1_layout layout, uint64_t chunk_rows, int
     if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return give_up(Q1_EDEVICE, "event creation failed");
     st->done.push_back(e);
     MergeSet* set = nullptr;
-    if (hipMalloc(&set, sizeof(MergeSet)) != hipSuccess) return give_up(Q1_ENOMEM, "staging allocation failed");
+    if (device_malloc(ctx, (void**)&set, sizeof(MergeSet)) != hipSuccess)
+      return give_up(Q1_ENOMEM, "staging allocation failed");
     st->set.push_back(set);
     if (launch_zero(set, sizeof(MergeSet), s) != Q1_OK) return give_up(Q1_EDEVICE, "zero kernel failed");
     q1_columns c{};
@@ -99,7 +100,7 @@ static q1_status prepare(q1_ctx* ctx, q1_layout layout, uint64_t chunk_rows, int
     for (int k = 0; k < 8; k++) {
       if (!b[k]) continue;
       void* p = nullptr;
-      if (hipMalloc(&p, b[k]) != hipSuccess) return give_up(Q1_ENOMEM, "staging allocation failed");
+      if (device_malloc(ctx, &p, b[k]) != hipSuccess) return give_up(Q1_ENOMEM, "staging allocation failed");
       st->allocs.push_back(p);
       *slots[k] = p;
     }
@@ -157,7 +158,8 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
         if (w) (void)hipFree(w);
         w = nullptr;
         void* grown = nullptr;
-        if (hipMalloc(&grown, ws_bytes) != hipSuccess) return fail(ctx, Q1_ENOMEM, "workspace allocation failed");
+        if (device_malloc(ctx, &grown, ws_bytes) != hipSuccess)
+          return fail(ctx, Q1_ENOMEM, "workspace allocation failed");
         w = grown;
       }
       st->workspace_bytes = ws_bytes;
