@@ -279,7 +279,40 @@ void spare_bitmap_given_back() {
   q1_shutdown(ctx);
 }
 
+// Launches of the any-value kernel need no per-block tables, whatever the placement and however
+// many blocks the kernel's own limit of rows per lane makes of the launch: q1_enqueue_noalloc takes
+// them, except for grids of more than 34952 blocks that the caller asks for itself.
+void any_value_launches_need_no_workspace() {
+  q1_ctx* ctx = context();
+  static q1_device_aggregates sums;
+  const uint64_t rows = 600'000'000;
+  for (q1_layout layout : {Q1_LAYOUT_REFERENCE, Q1_LAYOUT_UNCOMPRESSED, Q1_LAYOUT_COMPRESSED, Q1_LAYOUT_COMPRESSED_PUSHDOWN}) {
+    const q1_columns cols = device_columns(layout, rows);
+    auto noalloc = [&](uint32_t threads, uint32_t tuples, uint32_t blocks, uint32_t flags = 0) {
+      const q1_launch l{threads, tuples, blocks, flags};
+      return q1_enqueue_noalloc(ctx, Q1_PLACE_GLOBAL, layout, &l, &sums, &cols, 0, rows, 729999, q1_stream(ctx));
+    };
+    EXPECT(q1_enqueue_noalloc(ctx, Q1_PLACE_GLOBAL, layout, nullptr, &sums, &cols, 0, rows, 729999, nullptr) == Q1_OK);
+    EXPECT(noalloc(0, 0, 0) == Q1_OK);
+    EXPECT(noalloc(256, 1024, 0) == Q1_OK);   // 2289 blocks asked for
+    EXPECT(noalloc(64, 16384, 0) == Q1_OK);
+    EXPECT(noalloc(64, 512, 0) == Q1_OK);     // 18311
+    EXPECT(noalloc(0, 0, 3000) == Q1_OK);
+    EXPECT(noalloc(64, 1024, 34952) == Q1_OK);
+    EXPECT(noalloc(64, 1024, 34953) == Q1_EINVAL);
+    EXPECT(noalloc(64, 256, 0) == Q1_EINVAL);  // 36622
+    EXPECT(noalloc(64, 16, 0) == Q1_EINVAL);
+    EXPECT(noalloc(64, 256, 0, Q1_LAUNCH_ASSUME_TPCH_DOMAIN) == Q1_EINVAL);
+    // nor does the launch that may allocate
+    const uint64_t before = state().device_bytes;
+    EXPECT(q1_enqueue(ctx, Q1_PLACE_GLOBAL, layout, nullptr, &sums, &cols, 0, rows, 729999, nullptr) == Q1_OK);
+    EXPECT(state().device_bytes == before);
+  }
+  q1_shutdown(ctx);
+}
+
 const std::map<std::string, void (*)()> kCases = {
+    {"any_value_launches_need_no_workspace", any_value_launches_need_no_workspace},
     {"spare_bitmap_given_back", spare_bitmap_given_back},
     {"streaming_workspace_after_a_failed_growth", streaming_workspace_after_a_failed_growth},
     {"noalloc_after_an_overlap", noalloc_after_an_overlap},

@@ -854,7 +854,7 @@ static q1_status run_locked(q1_ctx* ctx, const q1_table* t, uint64_t row_begin, 
   const char* why = "";
   q1_status s = make_shape(p, t->layout, t->fast, &l, row_begin, row_begin + row_count, &shape, &why);
   if (s != Q1_OK) return fail(ctx, s, why);
-  s = ensure_workspace(ctx, scan_workspace_bytes(p, shape));
+  s = ensure_workspace(ctx, scan_workspace_bytes(p, t->fast, shape));
   if (s != Q1_OK) return s;
   ScanArgs a{};
   a.cols = t->dev;
@@ -916,6 +916,16 @@ q1_status q1_enqueue_noalloc(q1_ctx* ctx, q1_placement placement, q1_layout layo
   const char* why = "";
   q1_status s = make_shape(p, layout, fast, &l, row_begin, row_begin + num_tuples, &shape, &why);
   if (s != Q1_OK) return fail(ctx, s, why);
+  if (!fast && p == Q1_PLACE_GLOBAL) {
+    // The any-value kernel runs this launch without per-block tables, with as many blocks as its
+    // rows per lane make; the limit on the caller's own grid holds all the same.
+    const q1_launch own{launch && launch->threads_per_block ? launch->threads_per_block : 256,
+                        launch && launch->tuples_per_thread ? launch->tuples_per_thread : 1024, l.num_blocks, 0};
+    LaunchShape asked;
+    s = make_shape(p, layout, true, &own, row_begin, row_begin + num_tuples, &asked, &why);
+    if (s != Q1_OK) return fail(ctx, s, why);
+    if (scan_workspace_bytes(p, true, asked) > kNoallocWorkspaceBytes) return fail(ctx, Q1_EINVAL, kNoallocRefused);
+  }
   ScanArgs a{};
   a.cols = *device;
   a.row_begin = row_begin;
@@ -957,7 +967,7 @@ q1_status q1_enqueue(q1_ctx* ctx, q1_placement placement, q1_layout layout, cons
   // share it ordered on the context stream.
   if (p == Q1_PLACE_GLOBAL && stream != (void*)ctx->stream)
     return fail(ctx, Q1_EINVAL, "the global placement enqueues on the context stream only");
-  s = ensure_workspace(ctx, scan_workspace_bytes(p, shape));
+  s = ensure_workspace(ctx, scan_workspace_bytes(p, fast, shape));
   if (s != Q1_OK) return s;
   ScanArgs a{};
   a.cols = *device;

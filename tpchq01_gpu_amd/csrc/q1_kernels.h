@@ -132,7 +132,9 @@ q1_status launch_direct(q1_layout layout, const ScanArgs& a, const LaunchShape& 
 // fast: the rows lie inside the TPC-H domain.  Otherwise the any-value kernel runs.
 q1_status launch_scan(q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
                       const LaunchShape& shape, void* workspace, void* stream, MergeSet* set = nullptr);
-uint64_t scan_workspace_bytes(q1_placement placement, const LaunchShape& shape);
+// The workspace launch_scan needs: the global placement's per-block tables, which the any-value
+// kernel does without.
+uint64_t scan_workspace_bytes(q1_placement placement, bool fast, const LaunchShape& shape);
 
 // Zero device memory (whole 64-bit words; a fill kernel, safe inside graph capture).
 q1_status launch_zero(void* p, uint64_t bytes, void* stream);
@@ -222,6 +224,8 @@ q1_status launch_batch(q1_layout layout, q1_placement placement, const BatchHead
 // clears its merge set, once per device; noalloc_launch_scan is launch_scan with the
 // array as its scratch, refusing launches that need more (*why says which).
 constexpr uint64_t kNoallocWorkspaceBytes = 8ull << 20;
+constexpr const char* kNoallocRefused =
+    "the launch needs more scratch than the static array holds (the global placement: at most 34952 blocks)";
 q1_status noalloc_setup(int device, void* stream);
 q1_status noalloc_launch_scan(int device, q1_placement placement, q1_layout layout, bool fast, const ScanArgs& a,
                               const LaunchShape& shape, void* stream, const char** why);

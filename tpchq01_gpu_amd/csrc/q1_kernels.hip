@@ -388,8 +388,8 @@ q1_status make_shape(q1_placement placement, q1_layout layout, bool fast, const 
   return Q1_OK;
 }
 
-uint64_t scan_workspace_bytes(q1_placement placement, const LaunchShape& shape) {
-  return placement == Q1_PLACE_GLOBAL ? (uint64_t)shape.blocks * AccGlobal::W * kNumGroups * 8 : 0;
+uint64_t scan_workspace_bytes(q1_placement placement, bool fast, const LaunchShape& shape) {
+  return fast && placement == Q1_PLACE_GLOBAL ? (uint64_t)shape.blocks * AccGlobal::W * kNumGroups * 8 : 0;
 }
 
 // The kernel variant of a fast launch, and its LDS.  The packed slot holds quantities in whole

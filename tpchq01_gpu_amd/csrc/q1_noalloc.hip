@@ -60,9 +60,8 @@ q1_status noalloc_launch_scan(int device, q1_placement placement, q1_layout layo
     *why = "the scratch array of this device is not set up (q1_init does it)";
     return Q1_EDEVICE;
   }
-  if (scan_workspace_bytes(placement, shape) > kNoallocWorkspaceBytes) {
-    *why = "the launch needs more scratch than the static array holds (the global placement: at most "
-           "34952 blocks)";
+  if (scan_workspace_bytes(placement, fast, shape) > kNoallocWorkspaceBytes) {
+    *why = kNoallocRefused;
     return Q1_EINVAL;
   }
   void* workspace = static_cast<char*>(base) + sizeof(MergeSet);

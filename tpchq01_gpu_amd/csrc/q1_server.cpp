@@ -123,7 +123,7 @@ q1_status launch_slot(q1_server* sv, Slot& s) {
     const char* why = "";
     q1_status st = q1::make_shape(p, t0->layout, !s.single, &l, r.row_begin, r.row_begin + r.row_count, &shape, &why);
     if (s.single && st != Q1_OK) return st;
-    if (st == Q1_OK && q1::scan_workspace_bytes(p, shape) == 0) {
+    if (st == Q1_OK && q1::scan_workspace_bytes(p, !s.single, shape) == 0) {
       q1::ScanArgs a{};
       a.cols = t0->dev;
       a.row_begin = r.row_begin;

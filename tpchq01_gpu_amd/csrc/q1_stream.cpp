@@ -151,7 +151,7 @@ q1_status q1_run_streaming(q1_ctx* ctx, q1_layout layout, const q1_columns* host
       s = make_shape(p, layout, fast, &l, 0, most, &full_shape, &why);
       if (s != Q1_OK) return fail(ctx, s, why);
     }
-    const uint64_t ws_bytes = scan_workspace_bytes(p, full_shape);
+    const uint64_t ws_bytes = scan_workspace_bytes(p, fast, full_shape);
     if (rows > chunk_rows && ws_bytes > st->workspace_bytes) {
       st->workspace_bytes = 0;  // until every stream has its own
       for (auto& w : st->workspace) {
@@ -332,7 +332,7 @@ q1_status q1_run_split(q1_ctx* ctx, const q1_table* t, const q1_columns* host, u
     const char* why = "";
     q1_status s = make_shape(p, t->layout, t->fast, &l, 0, split, &shape, &why);
     if (s != Q1_OK) return fail(ctx, s, why);
-    s = ensure_workspace(ctx, scan_workspace_bytes(p, shape));
+    s = ensure_workspace(ctx, scan_workspace_bytes(p, t->fast, shape));
     if (s != Q1_OK) return s;
     ScanArgs a{};
     a.cols = t->dev;
