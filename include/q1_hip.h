@@ -198,7 +198,8 @@ q1_status q1_table_info(const q1_table* t, q1_layout* layout, uint64_t* rows, q1
 /* (new) Copies the device columns back into caller host buffers of the layout's sizes. */
 q1_status q1_table_download(q1_ctx* ctx, const q1_table* t, const q1_columns* host_out);
 uint64_t q1_table_device_bytes(const q1_table* t);
-/* Frees the table's device memory (if its context is still alive) and the handle.  Of freed
+/* Frees the table's device memory (if its context is still alive) and the handle, once work
+ * on the context's stream that may read the table has ended.  Of freed
  * pushdown tables the context keeps one bitmap, of at most 64 MiB, for the next
  * q1_build_filter; it is given back when an allocation of the context or of its servers fails,
  * and with the context. */

@@ -311,7 +311,62 @@ void any_value_launches_need_no_workspace() {
   q1_shutdown(ctx);
 }
 
+// q1_table_free returns once the work that may read the table has ended, as freeing its memory did:
+// queued on the context's stream, which callers can also get and use themselves, or for a filter
+// bitmap whose address was handed out, on any stream.
+void table_free_waits() {
+  const uint64_t rows = 1u << 20;
+  HostColumns h(Q1_LAYOUT_COMPRESSED, rows);
+  static q1_device_aggregates sums;
+  q1_result r;
+  auto wrapped = [&](q1_ctx* ctx) {
+    q1_table* t = nullptr;
+    EXPECT(q1_table_wrap(ctx, Q1_LAYOUT_COMPRESSED, &h.c, rows, &t) == Q1_OK);
+    return t;
+  };
+  auto waits_for_stream = [&](q1_table* t) {
+    state().stream_waits = 0;
+    q1_table_free(t);
+    return state().stream_waits > 0;
+  };
+  q1_ctx* ctx = context();
+  auto enqueue = [&](bool noalloc) {
+    EXPECT((noalloc ? q1_enqueue_noalloc : q1_enqueue)(ctx, Q1_PLACE_IN_REGISTERS, Q1_LAYOUT_COMPRESSED, nullptr, &sums,
+                                                       &h.c, 0, rows, 729999, nullptr) == Q1_OK);
+  };
+  for (bool noalloc : {false, true}) {
+    q1_table* t = wrapped(ctx);
+    enqueue(noalloc);
+    EXPECT(waits_for_stream(t));
+    // calls without rows launch nothing that could be waited for
+    t = wrapped(ctx);
+    enqueue(noalloc);
+    EXPECT(q1_run(ctx, t, 0, 0, 729999, Q1_PLACE_AUTO, nullptr, &r) == Q1_OK);
+    const q1_request none{t, 5, 0, 729999, 0};
+    EXPECT(q1_run_batch(ctx, &none, 1, nullptr, &r) == Q1_OK);
+    EXPECT(waits_for_stream(t));
+    // nothing is queued behind a query's result
+    t = wrapped(ctx);
+    enqueue(noalloc);
+    EXPECT(q1_run(ctx, t, 0, rows, 729999, Q1_PLACE_AUTO, nullptr, &r) == Q1_OK);
+    EXPECT(!waits_for_stream(t));
+  }
+  // a bitmap on other streams
+  q1_table *t = wrapped(ctx), *f = nullptr;
+  EXPECT(q1_build_filter(ctx, t, 729999, &f) == Q1_OK);
+  q1_columns dev;
+  EXPECT(q1_table_info(f, nullptr, nullptr, &dev) == Q1_OK);
+  state().device_waits = state().frees = 0;
+  q1_table_free(f);
+  EXPECT(state().device_waits + state().frees > 0);
+  // the caller's own work on the context's stream
+  EXPECT(q1_stream(ctx) != nullptr);
+  EXPECT(waits_for_stream(t));
+  q1_shutdown(ctx);
+}
+
 const std::map<std::string, void (*)()> kCases = {
+    {"table_free_waits", table_free_waits},
     {"any_value_launches_need_no_workspace", any_value_launches_need_no_workspace},
     {"spare_bitmap_given_back", spare_bitmap_given_back},
     {"streaming_workspace_after_a_failed_growth", streaming_workspace_after_a_failed_growth},

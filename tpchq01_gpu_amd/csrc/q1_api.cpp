@@ -217,12 +217,8 @@ q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bo
   a.host = ctx->d_result;
   a.sequence = ++ctx->sequence;
   const bool direct = can_launch_direct(placement, layout, fast, shape);
-  ctx->results = direct ? shape.blocks : 1;
-  if (shape.blocks == 0) {
-    std::memset(ctx->h_result, 0, sizeof(HostResult));
-    ctx->h_result->sequence = a.sequence;
-    return Q1_OK;
-  }
+  ctx->results = direct ? shape.blocks : shape.blocks ? 1 : 0;
+  if (shape.blocks == 0) return Q1_OK;
   const q1_status s = direct ? launch_direct(layout, a, shape, (void*)ctx->stream)
                              : launch_scan(placement, layout, fast, a, shape, ctx->workspace, (void*)ctx->stream, ctx->set);
   return s == Q1_OK ? Q1_OK : fail(ctx, s, "scan kernel launch failed");
@@ -247,6 +243,7 @@ q1_status wait_sequence(q1_ctx* ctx, const uint64_t* word, uint64_t sequence) {
       return fail(ctx, Q1_EDEVICE, "the scan kernel ended without a result");
     }
   }
+  ctx->queued = false;  // what was before the launch on the stream has ended too
   return Q1_OK;
 }
 
@@ -274,8 +271,13 @@ q1_status wait_result(q1_ctx* ctx, q1_result* out, double* kernel_ms, uint64_t* 
     const q1_status s = wait_sequence(ctx, &r[i].sequence, ctx->sequence);
     if (s != Q1_OK) return s;
   }
-  q1_device_aggregates sum = r[0].sums;
-  uint64_t begin = r[0].clock_begin, end = r[0].clock_end;
+  q1_device_aggregates sum{};
+  uint64_t begin = 0, end = 0;
+  if (ctx->results) {
+    sum = r[0].sums;
+    begin = r[0].clock_begin;
+    end = r[0].clock_end;
+  }
   for (uint32_t i = 1; i < ctx->results; i++) {
     add_aggregates(&sum, r[i].sums);
     begin = std::min(begin, r[i].clock_begin);
@@ -406,17 +408,14 @@ static void load_tuning_file(q1_ctx* ctx) {
   }
 }
 
-// A bitmap of at least `bytes` bytes.  The context stream runs the launches that read the spare
-// one before those of its next table; for launches on other streams the device is waited for,
-// as hipFree would have.
+// A bitmap of at least `bytes` bytes.
 static bool filter_malloc(q1_ctx* ctx, uint64_t bytes, q1_table* t) {
   const SpareFilter spare = take_spare(ctx, bytes);
-  if (spare.p && (!spare.shared || hipDeviceSynchronize() == hipSuccess)) {
+  if (spare.p) {
     t->owned[7] = spare.p;
     t->filter_bytes = spare.bytes;
     return true;
   }
-  if (spare.p) (void)hipFree(spare.p);
   void* p = nullptr;
   if (device_malloc(ctx, &p, bytes) != hipSuccess) return false;
   t->owned[7] = p;
@@ -425,19 +424,25 @@ static bool filter_malloc(q1_ctx* ctx, uint64_t bytes, q1_table* t) {
 }
 
 // Frees a table with its context's lock held (every entry point that creates tables
-// holds it when a creation fails).
+// holds it when a creation fails).  Whatever may still read the table ends first: hipFree waits
+// for the device, and where nothing may be freed, the waits here are those that are needed.
 static void release_table(q1_table* t) {
   if (q1_ctx* ctx = t->ctx) {
+    if (ctx->queued || ctx->stream_out) {
+      (void)hipStreamSynchronize(ctx->stream);
+      ctx->queued = false;
+    }
     if (t->filter_bytes && t->filter_bytes <= kSpareFilterBytes) {
+      if (t->shared) (void)hipDeviceSynchronize();
       std::lock_guard<std::mutex> g(ctx->spare_lock);
       if (t->filter_bytes > ctx->spare.bytes) {
-        const SpareFilter kept{t->owned[7], t->filter_bytes, t->shared};
+        const SpareFilter kept{t->owned[7], t->filter_bytes};
         t->owned[7] = ctx->spare.p;
         ctx->spare = kept;
       }
     }
     for (void* p : t->owned)
-      if (p) (void)hipFree(p);  // waits for the device, which may still read it
+      if (p) (void)hipFree(p);
     ctx->tables.erase(t);
   }
   delete t;
@@ -581,7 +586,11 @@ q1_status q1_synchronize(q1_ctx* ctx) {
   return Q1_OK;
 }
 
-void* q1_stream(q1_ctx* ctx) { return ctx ? (void*)ctx->stream : nullptr; }
+void* q1_stream(q1_ctx* ctx) {
+  if (!ctx) return nullptr;
+  ctx->stream_out = true;
+  return (void*)ctx->stream;
+}
 
 q1_status q1_layout_column_bytes(q1_layout layout, uint64_t rows, uint64_t bytes_out[8]) {
   if (!valid_layout(layout) || !bytes_out) return Q1_EINVAL;
@@ -932,6 +941,7 @@ q1_status q1_enqueue_noalloc(q1_ctx* ctx, q1_placement placement, q1_layout layo
   a.row_end = row_begin + num_tuples;
   a.cutoff_day = cutoff_day;
   a.out = aggregates;
+  if (!hip_stream) ctx->queued = true;
   // the device's static scratch array instead of the context's merge set and workspace
   s = noalloc_launch_scan(ctx->device, p, layout, fast, a, shape,
                           hip_stream ? hip_stream : (void*)ctx->stream, &why);
@@ -975,6 +985,7 @@ q1_status q1_enqueue(q1_ctx* ctx, q1_placement placement, q1_layout layout, cons
   a.row_end = row_begin + num_tuples;
   a.cutoff_day = cutoff_day;
   a.out = aggregates;
+  if (stream == (void*)ctx->stream) ctx->queued = true;
   s = scan_on(ctx, p, layout, fast, a, shape, stream);
   return s == Q1_OK ? Q1_OK : fail(ctx, s, "scan kernel launch failed");
   GUARD_END(ctx)

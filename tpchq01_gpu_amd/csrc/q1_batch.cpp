@@ -229,7 +229,9 @@ extern "C" q1_status q1_run_batch(q1_ctx* ctx, const q1_request* reqs, uint32_t 
     const char* why = "";
     q1_status s = batch_launch(ctx, b, reqs, n, p, lane_rows, grid, ctx->stream, &plan_rows, &plan_grid, &why);
     if (s != Q1_OK) return fail(ctx, s, why);
-    s = wait_sequence(ctx, &b->done()->sequence, b->sequence);
+    // a batch without rows has launched nothing to wait for
+    if (__atomic_load_n(&b->done()->sequence, __ATOMIC_ACQUIRE) != b->sequence)
+      s = wait_sequence(ctx, &b->done()->sequence, b->sequence);
     if (s != Q1_OK) {
       // The tables may hold partial sums: the next call makes new ones.
       batch_free(b);

@@ -57,7 +57,6 @@ constexpr uint64_t kSpareFilterBytes = 64ull << 20;
 struct SpareFilter {
   void* p = nullptr;
   uint64_t bytes = 0;
-  bool shared = false;            // as its table was
 };
 // A launch shape tuned on ranges of `rows` rows ("launch_at" lines of the tuning file).
 struct SizedLaunch {
@@ -69,10 +68,14 @@ struct SizedLaunch {
 struct q1_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
+  // Work may be on the stream that no call has waited for: q1_enqueue's since the last wait, or
+  // the caller's own once it has got the stream (q1_stream).
+  bool queued = false;
+  std::atomic<bool> stream_out{false};
   hipEvent_t ev_begin = nullptr, ev_end = nullptr, ev_h2d_begin = nullptr, ev_h2d_end = nullptr;
   q1::HostResult* h_result = nullptr;      // pinned, kDirectBlocks: what q1_run's kernel leaves (and
                                            // a copy's start clock behind them)
-  uint32_t results = 1;                    // records that the last launch leaves
+  uint32_t results = 0;                    // records that the last launch leaves
   q1::HostResult* d_result = nullptr;      // ... as the device addresses it
   uint64_t sequence = 0;                   // number of the last launch that wrote h_result
   int32_t clock_khz = 0;                   // rate of the device clock in h_result
