@@ -365,7 +365,37 @@ void table_free_waits() {
   q1_shutdown(ctx);
 }
 
+// A process that asked for blocking waits (hipDeviceScheduleBlockingSync) gets the runtime's wait,
+// which sleeps, for a result that takes a while; by default the host watches for it.
+void waits_follow_the_device_flags() {
+  q1_ctx* ctx = context();
+  const uint64_t rows = 1u << 20;
+  HostColumns h(Q1_LAYOUT_COMPRESSED, rows);
+  q1_table* t = nullptr;
+  EXPECT(q1_table_wrap(ctx, Q1_LAYOUT_COMPRESSED, &h.c, rows, &t) == Q1_OK);
+  state().late_stream = (void*)ctx->stream;
+  state().late_us = 300;
+  for (unsigned flags : {(unsigned)hipDeviceScheduleAuto, (unsigned)hipDeviceScheduleSpin,
+                         (unsigned)(hipDeviceScheduleBlockingSync | hipDeviceMapHost)}) {
+    state().device_flags = flags;
+    const bool blocking = flags & hipDeviceScheduleBlockingSync;
+    q1_result r;
+    state().stream_waits = 0;
+    EXPECT(q1_run(ctx, t, 0, rows, 729999, Q1_PLACE_AUTO, nullptr, &r) == Q1_OK);
+    EXPECT((state().stream_waits > 0) == blocking);
+    const q1_request reqs[2] = {{t, 0, rows, 729999, 0}, {t, 32, 1000, 729999, 0}};
+    q1_result rs[2];
+    state().stream_waits = 0;
+    EXPECT(q1_run_batch(ctx, reqs, 2, nullptr, rs) == Q1_OK);
+    EXPECT((state().stream_waits > 0) == blocking);
+  }
+  state().late_us = 0;
+  q1_table_free(t);
+  q1_shutdown(ctx);
+}
+
 const std::map<std::string, void (*)()> kCases = {
+    {"waits_follow_the_device_flags", waits_follow_the_device_flags},
     {"table_free_waits", table_free_waits},
     {"any_value_launches_need_no_workspace", any_value_launches_need_no_workspace},
     {"spare_bitmap_given_back", spare_bitmap_given_back},

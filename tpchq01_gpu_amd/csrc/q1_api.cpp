@@ -226,14 +226,25 @@ q1_status scan_to_host(q1_ctx* ctx, q1_placement placement, q1_layout layout, bo
 
 // The kernel's last store is the launch's number in pinned host memory, for which the host
 // watches: an empty kernel launched and awaited so takes 6.2 us, 10.9 with the stream's wait,
-// and a call of 820 us 5 us less.  The stream's wait keeps the processor as busy (1.00 of a core
-// over such calls), so nothing is lost by watching for as long as a scan of 1.4G compressed rows
-// takes; then the stream's wait, which also tells when the launch has failed.
+// and a call of 820 us 5 us less.  Under HIP's default schedule the stream's wait keeps the
+// processor as busy (1.00 of a core over such calls), so nothing is lost by watching for as long as
+// a scan of 1.4G compressed rows takes; then the stream's wait, which also tells when the launch
+// has failed.  A process that asked for blocking waits gets the stream's at once.
+static bool blocking_waits(const q1_ctx* ctx) {
+  int current = ctx->device;
+  unsigned flags = 0;
+  (void)hipGetDevice(&current);
+  if (current != ctx->device) (void)hipSetDevice(ctx->device);
+  const bool got = hipGetDeviceFlags(&flags) == hipSuccess;
+  if (current != ctx->device) (void)hipSetDevice(current);
+  return got && (flags & hipDeviceScheduleMask) == hipDeviceScheduleBlockingSync;
+}
 constexpr int kWatchMicroseconds = 2000;
 q1_status wait_sequence(q1_ctx* ctx, const uint64_t* word, uint64_t sequence) {
   auto arrived = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) == sequence; };
   const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(kWatchMicroseconds);
-  while (!arrived() && std::chrono::steady_clock::now() < until)
+  const bool watch = !arrived() && !blocking_waits(ctx);
+  while (watch && !arrived() && std::chrono::steady_clock::now() < until)
     for (int i = 0; i < 16 && !arrived(); i++) __builtin_ia32_pause();
   if (!arrived()) {
     Q1_HIP(ctx, hipStreamSynchronize(ctx->stream));
