@@ -349,9 +349,11 @@ typedef struct {
                                   another batch is on the device (0: launch at once) */
   uint64_t memory_budget;      /* admission: device bytes the in-flight work may pin -- the
                                   columns of every table with requests in flight (once per
-                                  table) plus 480 B of descriptor and result per request;
+                                  table) plus a fixed 480 B per request for its own state;
                                   0 = three quarters of the device's memory.  A request whose
-                                  table alone does not fit gets Q1_ENOMEM at submit. */
+                                  table alone does not fit gets Q1_ENOMEM at submit.  Not
+                                  counted: the merge tables that each of the max_inflight slots
+                                  keeps for its batches (512 B per table, at most 32 MiB). */
   uint64_t exclusive_bytes;    /* a request that scans at least this many column bytes is
                                   large: it runs alone (the scan kernel with its tuned launch),
                                   and large requests run one at a time, in arrival order, while

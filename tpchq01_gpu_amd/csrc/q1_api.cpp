@@ -154,7 +154,9 @@ q1_status ensure_workspace(q1_ctx* ctx, uint64_t bytes) {
   return Q1_OK;
 }
 
-constexpr int kPoolWaitMs = 2;  // longer than any scan of 1.5G compressed rows
+// The longest wait for a set, with the context's lock held: beyond it a launch merges directly.  The
+// oldest of 256 launches in flight usually ends within its own few microseconds.
+constexpr int kPoolWaitMs = 2;
 
 // A free set of the pool for a large launch on a caller's stream, its index in *index; nullptr
 // (merge directly) when the sets stay in flight.

@@ -39,7 +39,7 @@ struct StreamState;     // q1_stream.cpp: the host-resident streaming pipeline
 // nothing orders the streams (or a destroyed stream and one made at its address).  A launch's
 // last block writes the launch's number to its set's word in `done`, and a set is free again
 // once the number is there.
-constexpr size_t kPoolSets = 256;  
+constexpr size_t kPoolSets = 256;
 struct SetPool {
   MergeSet* sets = nullptr;       // kPoolSets
   uint64_t* done = nullptr;       // pinned words

@@ -1,5 +1,6 @@
-// gfx950 utility kernels (zero fill, generator, domain check, pushdown producer), kernel dispatch and the host-side launch helpers of the TPC-H Q1
-// path.  The scan kernels themselves are in q1_scan.h, instantiated per layout.
+// gfx950 utility kernels (zero fill, generator, domain check, pushdown producer), kernel dispatch
+// and the host-side launch helpers of the TPC-H Q1 path.  The scan kernels themselves are in
+// q1_scan.h, instantiated per layout.
 #include <algorithm>
 #include <type_traits>
 
@@ -521,7 +522,6 @@ q1_status launch_build_filter(const uint16_t* ship, uint64_t rows, int32_t cutof
   hipLaunchKernelGGL(report_end, dim3(1), dim3(64), 0, (hipStream_t)stream, host, sequence);
   return hip_status(hipGetLastError());
 }
-
 
 uint32_t layout_tile_rows(q1_layout layout) { return tile_rows(layout); }
 

@@ -40,7 +40,6 @@ using GenFn = void (*)(ScanArgs, uint32_t);
 
 namespace {
 
-constexpr int kMaxBlock = 256;
 constexpr int kBatchBlock = (int)kBatchThreads;  // the batched kernel's block size
 
 // ------------------------------------------------------------------------------------
@@ -62,9 +61,6 @@ __device__ __forceinline__ uint32_t thread_index() {
 }
 __device__ __forceinline__ uint32_t comp(const uint4& v, int i) {
   return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
-}
-__device__ __forceinline__ void comp_or(uint4& v, int i, uint32_t bits) {
-  if (i == 0) v.x |= bits; else if (i == 1) v.y |= bits; else if (i == 2) v.z |= bits; else v.w |= bits;
 }
 __device__ __forceinline__ void comp_set(uint4& v, int i, uint32_t bits) {
   if (i == 0) v.x = bits; else if (i == 1) v.y = bits; else if (i == 2) v.z = bits; else v.w = bits;
@@ -112,7 +108,8 @@ struct WideRow {
 
 // ------------------------------------------------------------------------------------
 // Tile loaders, one per layout.  load() reads a whole tile with vector loads; load_edge()
-// reads only the rows inside [lo, hi) (guarded, per row) into the same vector form.
+// reads a partial tile row by row into the same vector form, its rows outside the range replaced by
+// the nearest one inside (EdgeRows).
 // Accessors extract row j (j is a compile-time constant after unrolling).
 // ------------------------------------------------------------------------------------
 
@@ -416,8 +413,8 @@ template <> struct TileOf<Q1_LAYOUT_COMPRESSED> { using T = CompressedStreamTile
 template <> struct TileOf<Q1_LAYOUT_COMPRESSED_PUSHDOWN> { using T = CompressedStreamTile<true>; };
 
 // A group of U lane tiles t0 + m * stride (m < U, at most `count` of them, below
-// `end_tile`), all loaded before any of their rows is used, so that a wavefront keeps
-// 16 rows' worth of loads per lane in flight whatever the tile size.
+// `end_tile`), all loaded before any of their rows is used, so that a wavefront keeps 16 rows'
+// (4-row tiles) or 8 rows' (2-row tiles) worth of loads per lane in flight.
 template <class Tile, int U>
 struct TileGroup {
   Tile tile[U];
@@ -1793,9 +1790,11 @@ __device__ __forceinline__ uint32_t next_request(const uint32_t* first, uint32_t
 // next entry lies past the list.
 // The header and descriptors come as read-only pointers, so they load through the scalar
 // cache into scalar registers.
-// The default grid is one block per entry, up to 64 per compute unit: the hardware's dispatch
-// then balances the list.  256 requests of 754M rows in all: 1.03 ms (6.87 TB/s, 64 blocks
-// per compute unit x 192 rows per lane), 1.08 ms striding with 8 blocks per compute unit.
+// On the layouts with a tuned batch shape (the compressed one) the default grid is one block per
+// entry, up to 64 per compute unit: the hardware's dispatch then balances the list.  256 requests
+// of 754M rows in all: 1.03 ms (6.87 TB/s, 64 blocks per compute unit x 192 rows per lane), 1.08 ms
+// striding with 8 blocks per compute unit.  Batches of the other layouts stride with as many blocks
+// as are resident.
 // The descriptors and results used to travel through a graph of a copy, the kernel and a
 // fold, rebuilt for every power of two of requests: 16 requests of 10,000 rows 50 -> 21 us.
 template <int L, int P>

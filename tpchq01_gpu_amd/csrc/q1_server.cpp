@@ -18,7 +18,7 @@
 // request that arrives while a large one runs starts at once instead of queueing behind it.
 // A batch runs the batched kernel as q1_run_batch does.
 // Admission by device memory: a request pins its table's columns (counted once per table
-// while any of its requests is in flight) and its descriptor and result table.
+// while any of its requests is in flight) and a fixed 480 bytes for its own state.
 // Requests on tables outside the TPC-H value domain run alone through the any-value kernel.
 #include <algorithm>
 #include <chrono>
@@ -52,8 +52,10 @@ struct Where {
   uint32_t batch_id;
 };
 
-// A request's share of the memory budget beside its table (stated in q1_hip.h).
-uint64_t request_state_bytes() { return 480; }
+// A request's share of the memory budget beside its table, as stated in q1_hip.h: what is refused
+// depends on it, so it does not follow the size of the descriptor, which it covers.
+constexpr uint64_t request_state_bytes() { return 480; }
+static_assert(sizeof(q1::BatchDesc) + sizeof(uint32_t) <= request_state_bytes(), "a descriptor and its first block");
 
 // Device bytes of a table's columns (what a request on it keeps resident).
 uint64_t table_bytes(const q1_table* t) {
