@@ -2,14 +2,13 @@
 //
 // Reads the nine compressed Q1 columns of N rows (u16 ship date, u8 quantity, u32 price,
 // u8 discount, u8 tax, 2-bit return flags, 1-bit line statuses: 9.375 bytes per row) with
-// the scan kernel's own access pattern and launch shapes, but with no filter and no
-// aggregation (each lane only XORs what it loads), and then the same number of bytes as
-// one flat buffer, and with the streaming pattern of the shared placement (4-row tiles,
-// non-temporal loads); then the columns of the uncompressed (20 B/row) and reference
-// (38 B/row) layouts with the patterns of their kernels, and a plain 2 GiB device copy
-// (read + write rate), and the batched kernel's resident-grid structure over the compressed
-// columns.  Each shape is timed as 20 back-to-back launches, as bench.py
-// times the scan.  The fastest of these is the rate the scan could reach if its arithmetic
+// the scan kernels' access pattern (4-row tiles, non-temporal loads) in several launch
+// shapes, but with no filter and no aggregation (each lane only XORs what it loads); with
+// 16-row tiles and ordinary loads; and the same number of bytes as one flat buffer.  Then
+// the columns of the uncompressed (20 B/row) and reference (38 B/row) layouts in the same
+// two ways, a plain 2 GiB device copy (read + write rate), and the striding batch kernel's
+// resident-grid structure over the compressed columns.  Each shape is timed as 20
+// back-to-back launches, as bench.py times the scan.  The fastest of these is the rate the scan could reach if its arithmetic
 // were free; the scan's own rate is compared with it and with the published 8 TB/s.
 //
 //   hbm_probe [rows]     (default 600000000; prints one JSON line)
@@ -45,7 +44,7 @@ constexpr uint32_t kSentinel = 0x9E3779B9u;  // a lane stores only if its XOR hi
 
 __device__ __forceinline__ uint32_t fold(uint4 v) { return v.x ^ v.y ^ v.z ^ v.w; }
 
-// The scan kernel's pattern: in iteration k thread i reads lane tile base + k*B + i.
+// 16-row tiles: in iteration k thread i reads lane tile base + k*B + i.
 template <int B>
 __global__ __launch_bounds__(B) void read_columns(Columns c, uint64_t tiles, uint32_t tiles_per_thread,
                                                   uint32_t* sink) {
@@ -62,7 +61,7 @@ __global__ __launch_bounds__(B) void read_columns(Columns c, uint64_t tiles, uin
   if (acc == kSentinel) sink[0] = acc;
 }
 
-// The streaming pattern: 4-row tiles (lane i of a wavefront reads tile base + i, so every
+// The scan kernels' streaming pattern: 4-row tiles (lane i of a wavefront reads tile base + i, so every
 // load instruction covers whole cache lines), non-temporal loads for the five value
 // columns and plain byte loads for the packed flag columns.
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
@@ -126,9 +125,8 @@ __global__ __launch_bounds__(B) void copy_flat(const uint4* src, uint4* dst, uin
 
 // The wide layouts' columns: lane tiles of TILE rows, column k holding W[k] bytes per
 // tile.  With TILE = 2 every column load of a wavefront is one contiguous stretch with at
-// most 16 bytes per lane, loaded non-temporally (the pattern of the LDS placement's
-// kernels); with TILE = 8 (uncompressed) or 4 (reference) and ordinary loads it is the
-// pattern of the register placements.
+// most 16 bytes per lane, loaded non-temporally (the scan kernels' pattern); with TILE = 8
+// (uncompressed) or 4 (reference) and ordinary loads a lane reads whole 32- or 64-byte pieces.
 template <int W, bool NT>
 __device__ __forceinline__ uint32_t load_bytes(const char* col, uint64_t t) {
   const char* p = col + t * W;
@@ -296,8 +294,8 @@ int main(int argc, char** argv) {
   std::printf("], \"columns_streaming\": [");
   const uint64_t tiles4 = rows / 4;
   double best_stream = 1e30;
-  const int stream_shapes[3][2] = {{256, 256}, {256, 1024}, {64, 1024}};
-  for (int s = 0; s < 3; s++) {
+  const int stream_shapes[4][2] = {{256, 128}, {256, 256}, {256, 1024}, {64, 1024}};
+  for (int s = 0; s < 4; s++) {
     const int b = stream_shapes[s][0];
     const uint32_t tpt = stream_shapes[s][1] / 4;  // 4-row tiles per thread
     const uint64_t blocks = (tiles4 + (uint64_t)b * tpt - 1) / ((uint64_t)b * tpt);
@@ -350,9 +348,17 @@ int main(int argc, char** argv) {
   CHECK(hipMemset(wide, 0x5A, rows * 38 + 8 * 256));
   const double unc_bytes = (double)rows * 20, ref_bytes = (double)rows * 38;
   const double u8 = wide_pass<256, 1, 8, false, 32, 32, 64, 8, 8, 8, 8>(wide, rows, 256, sink, reps);
-  const double u2 = wide_pass<256, 4, 2, true, 8, 8, 16, 2, 2, 2, 2>(wide, rows, 256, sink, reps);
   const double r4 = wide_pass<256, 1, 4, false, 16, 32, 32, 32, 32, 4, 4>(wide, rows, 256, sink, reps);
-  const double r2 = wide_pass<256, 4, 2, true, 8, 16, 16, 16, 16, 2, 2>(wide, rows, 256, sink, reps);
+  // The best shape is another one for each layout and machine, as the scan's is.
+  constexpr int kShapes = 5;
+  const uint32_t shape[kShapes] = {32, 64, 128, 256, 1024};
+  double u2[kShapes], r2[kShapes], best_u = u8, best_r = r4;
+  for (int s = 0; s < kShapes; s++) {
+    u2[s] = wide_pass<256, 4, 2, true, 8, 8, 16, 2, 2, 2, 2>(wide, rows, shape[s], sink, reps);
+    r2[s] = wide_pass<256, 4, 2, true, 8, 16, 16, 16, 16, 2, 2>(wide, rows, shape[s], sink, reps);
+    best_u = std::min(best_u, u2[s]);
+    best_r = std::min(best_r, r2[s]);
+  }
   CHECK(hipFree(wide));
 
   // Stream copy of 2 GiB into another 2 GiB: bytes read plus bytes written per second.
@@ -367,23 +373,27 @@ int main(int argc, char** argv) {
       back_to_back_ms([&] { copy_flat<256><<<dim3((uint32_t)cblocks), dim3(256)>>>(csrc, cdst, n16c, cpt); }, reps);
   CHECK(hipFree(csrc));
   CHECK(hipFree(cdst));
-  const char* fmt = "{\"tile_rows\": %d, \"nontemporal\": %s, \"threads_per_block\": 256, \"tuples_per_thread\": 256, "
+  const char* fmt = "{\"tile_rows\": %d, \"nontemporal\": %s, \"threads_per_block\": 256, \"tuples_per_thread\": %u, "
                     "\"ms\": %.4f, \"gbps\": %.1f}";
   std::printf("], \"uncompressed\": [");
-  std::printf(fmt, 8, "false", u8, unc_bytes / u8 / 1e6);
-  std::printf(", ");
-  std::printf(fmt, 2, "true", u2, unc_bytes / u2 / 1e6);
+  std::printf(fmt, 8, "false", 256u, u8, unc_bytes / u8 / 1e6);
+  for (int s = 0; s < kShapes; s++) {
+    std::printf(", ");
+    std::printf(fmt, 2, "true", shape[s], u2[s], unc_bytes / u2[s] / 1e6);
+  }
   std::printf("], \"reference\": [");
-  std::printf(fmt, 4, "false", r4, ref_bytes / r4 / 1e6);
-  std::printf(", ");
-  std::printf(fmt, 2, "true", r2, ref_bytes / r2 / 1e6);
+  std::printf(fmt, 4, "false", 256u, r4, ref_bytes / r4 / 1e6);
+  for (int s = 0; s < kShapes; s++) {
+    std::printf(", ");
+    std::printf(fmt, 2, "true", shape[s], r2[s], ref_bytes / r2[s] / 1e6);
+  }
   std::printf("], \"copy\": {\"bytes\": %llu, \"ms\": %.4f, \"gbps\": %.1f}", (unsigned long long)copy_bytes,
               copy_ms, 2.0 * copy_bytes / copy_ms / 1e6);
   std::printf(", \"resident_gbps\": %.1f", bytes / res_ms / 1e6);
   std::printf(", \"best_columns_gbps\": %.1f, \"best_streaming_gbps\": %.1f, \"best_flat_gbps\": %.1f, "
               "\"best_uncompressed_gbps\": %.1f, \"best_reference_gbps\": %.1f, \"copy_gbps\": %.1f}\n",
               bytes / best_cols / 1e6, bytes / best_stream / 1e6, n16 * 16 / best_flat / 1e6,
-              unc_bytes / std::min(u8, u2) / 1e6, ref_bytes / std::min(r4, r2) / 1e6, 2.0 * copy_bytes / copy_ms / 1e6);
+              unc_bytes / best_u / 1e6, ref_bytes / best_r / 1e6, 2.0 * copy_bytes / copy_ms / 1e6);
   CHECK(hipFree(sink));
   return 0;
 }
